@@ -370,7 +370,7 @@ class RequestManager:
                 w, ascending = np.ascontiguousarray(w, np.int32), False
                 order.append(rows + back.reshape(-1))
             else:
-                order.append(range(rows, rows + len(w)))
+                order.append(np.arange(rows, rows + len(w)))  # (whole numbers, also of no rows)
             keep += [t, w]
             a.id, a.num_tokens, a.num_want = rid, len(t), len(w)
             a.tokens = ctypes.cast(t.ctypes.data, ctypes.POINTER(ctypes.c_int32))

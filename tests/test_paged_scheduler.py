@@ -91,6 +91,18 @@ def test_replay_returns_the_order_asked_for():
     assert len(rm.replay_step(m, [(2, [5], [])])) == 0
 
 
+@pytest.mark.parametrize("want", [[4, 0, 2], [3, 3], [1, 2, 4], []])
+@pytest.mark.parametrize("first", [True, False])
+def test_replay_portion_without_rows_beside_any_order(want, first):
+    """A prompt's portion that wants no row, in one step with rows in any order."""
+    rm, m = replay_setup()
+    toks = prompts(3)[2]
+    ref = picks(rm.replay_step(m, [(1, toks, range(len(toks)))]))
+    rm.replay_end(m, 1)
+    step = [(2, [7, 8], []), (3, toks, want)]
+    assert picks(rm.replay_step(m, step if first else step[::-1])) == [ref[i] for i in want]
+
+
 def test_replay_slots_and_pages_run_out_and_come_back():
     rm, m = replay_setup(pages=4, page=8, slots=2)
     rm.replay_step(m, [(1, [5] * 16, []), (2, [6] * 9, [])])
