@@ -16,6 +16,7 @@
 #include <climits>
 
 #include "ffmi_internal.h"
+#include "runtime/graph_workspace.h"
 #include "collective.h"
 
 // ---------------------------------------------------------------------------
@@ -513,35 +514,38 @@ extern "C" ffmi_status ffmi_linear_ws(const void *X, const void *W_packed, void 
 }
 
 static std::mutex g_ws_mu;
-static void *g_ws = nullptr;
-static size_t g_ws_bytes = 0;
+static ffmi::GraphWorkspace g_ws;
 
 extern "C" ffmi_status ffmi_linear(const void *X, const void *W_packed, void *Y, int T,
                                    int out_dim, int in_dim, int epilogue, ffmi_stream stream) {
   FFMI_CHECK(X && W_packed && Y && T >= 0 && out_dim > 0, FFMI_ERR_INVALID);
   FFMI_CHECK(in_dim > 0 && in_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
-  // (a captured call keeps to the slabs: a graph outlives a workspace that grows)
+  // a captured call takes its slabs alone: a graph's share of the workspace is kept
+  // for good (up to 64 rows there are no slabs without a consumer of them)
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (stream && T > 128) FFMI_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
-  const bool slabs_only = cap != hipStreamCaptureStatusNone;
-  const size_t need = slabs_only ? ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue)
-                                 : ffmi_linear_workspace_bytes(T, out_dim, in_dim, epilogue);
+  if (stream && T > 64) FFMI_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  const size_t need = captured ? ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue)
+                               : ffmi_linear_workspace_bytes(T, out_dim, in_dim, epilogue);
   void *ws = nullptr;
   size_t ws_bytes = 0;
   {
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    if (need > g_ws_bytes) {
-      if (g_ws) {
-        FFMI_HIP(hipDeviceSynchronize());
-        (void)hipFree(g_ws);
-        g_ws = nullptr;
-        g_ws_bytes = 0;
-      }
-      if (hipMalloc(&g_ws, need) != hipSuccess) return FFMI_ERR_OOM;
-      g_ws_bytes = need;
-    }
-    ws = g_ws;
-    ws_bytes = slabs_only ? need : g_ws_bytes;
+    hipError_t err = hipSuccess;
+    ws = g_ws.get(
+        need, captured && need > 0,
+        [](size_t n) {
+          void *p = nullptr;
+          return hipMalloc(&p, n) == hipSuccess ? p : nullptr;
+        },
+        [&](void *p) {
+          err = hipDeviceSynchronize();
+          if (err == hipSuccess) (void)hipFree(p);
+          return err == hipSuccess;
+        });
+    FFMI_HIP(err);
+    if (need > 0 && !ws) return FFMI_ERR_OOM;
+    ws_bytes = captured ? need : g_ws.bytes();
   }
   return ffmi_linear_ws(X, W_packed, Y, T, out_dim, in_dim, epilogue, ws, ws_bytes, stream);
 }

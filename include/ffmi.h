@@ -189,8 +189,10 @@ ffmi_status ffmi_linear_pack_weight(const void *W, int out_dim, int in_dim,
 ffmi_status ffmi_linear_pack_gate_up(const void *Wg, const void *Wu, int out_dim,
                                      int in_dim, void *W_packed, ffmi_stream stream);
 /* Y[T][out] = X[T][in] . W^T, fp16 in/out, fp32 accumulate.  Uses a
- * library-owned split-K workspace: calls on different streams must not
- * overlap (use ffmi_linear_ws for that). */
+ * library-owned workspace (split-K slabs, and row-major X packed where that
+ * pays): calls on different streams must not overlap (use ffmi_linear_ws for
+ * that).  A call under stream capture records its place in the workspace,
+ * which then stays valid for the life of the process. */
 ffmi_status ffmi_linear(const void *X, const void *W_packed, void *Y, int T,
                         int out_dim, int in_dim, int epilogue, ffmi_stream stream);
 /* Linear on DT_FLOAT (linear_kernels.cu:450-582 with the full-precision

@@ -97,3 +97,33 @@ def test_buffers_off_16_bytes(T, N, k):
                                  ctypes.c_void_p(ws.ptr.value + off), n, None))
         got.append(y.get())
     K.close16(got[1], got[0].astype(np.float32))
+
+
+@pytest.mark.parametrize("T,later", [(168, (168,)), (256, (257, 384))])
+def test_graph_before_eager_growth(T, later):
+    """A graph's slabs stay valid when eager calls after the capture ask the library's
+    workspace for more: the same call (its packed activations), and longer ones."""
+    L, H, N, k = K.L, hip(), 4096, 11008
+    rng = np.random.default_rng(T)
+    X, W = f16(rng.standard_normal((max(later), k))), Buf(f16(rng.uniform(-0.05, 0.05, (N, k))))
+    Wp = Buf.empty((L.ffmi_linear_packed_bytes(N, k) // 2,), np.uint16)
+    F.check(L.ffmi_linear_pack_weight(W.ptr, N, k, Wp.ptr, None))
+    x, y = Buf(X), Buf(np.full((T, N), np.nan, np.float16))
+    s, g, ex = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert H.hipStreamCreate(ctypes.byref(s)) == 0
+    sync()
+    assert H.hipStreamBeginCapture(s, 2) == 0
+    F.check(L.ffmi_linear(x.ptr, Wp.ptr, y.ptr, T, N, k, 0, s))
+    assert H.hipStreamEndCapture(s, ctypes.byref(g)) == 0
+    assert H.hipGraphInstantiate(ctypes.byref(ex), g, None, None, ctypes.c_size_t(0)) == 0
+    z = Buf(np.full((max(later), N), np.nan, np.float16))
+    for t in (*later, T):
+        F.check(L.ffmi_linear(x.ptr, Wp.ptr, z.ptr, t, N, k, 0, None))
+        sync()
+        # whoever is given memory now keeps what is written there
+        others = [Buf(np.full((n << 20,), 7, np.uint8)) for n in (8, 22, 26, 34)]
+        assert H.hipGraphLaunch(ex, s) == 0
+        assert H.hipStreamSynchronize(s) == 0
+        assert all((b.get() == 7).all() for b in others)
+    assert np.array_equal(y.get().view(np.uint16), z.get()[:T].view(np.uint16))
+    H.hipGraphExecDestroy(ex), H.hipGraphDestroy(g)
