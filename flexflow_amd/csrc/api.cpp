@@ -181,6 +181,11 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
     b->max_kv = std::max(b->max_kv, (int)d->work[wi].kv_len);
     if (wi > 0 && d->work[wi].req == d->work[wi - 1].req) b->one_item_per_req = false;
   }
+  // (a request's place in the key split's scratch is for one item)
+  if (b->max_q == 1 && b->max_kv > 256)
+    for (int wi = 1; wi < d->num_work; ++wi)
+      for (int wj = 0; wj < wi; ++wj)
+        if (d->work[wi].req == d->work[wj].req) b->max_kv = 0;
   b->commit_overlap = false;
   for (int c = 0; c < d->num_commits && !b->commit_overlap; ++c)
     for (int t = 0; t < d->num_tokens; ++t)
@@ -296,10 +301,9 @@ extern "C" ffmi_status ffmi_attn_create(const ffmi_attn_cfg *cfg, ffmi_attn **ou
   std::vector<float> tab;
   rope_table(tab, h->slots, cfg->head_dim, cfg);
   const size_t table = tab.size();
-  if (!f32) tab.resize(table + ffmi::kKvSplitSlots, 0.f);  // the counters start at zero
-  if (ok)
-    ok = hipMalloc((void **)&h->rope,
-                   (table + (f32 ? 0 : ffmi::kv_split_floats(cfg->head_dim))) * sizeof(float)) == hipSuccess;
+  const size_t split = f32 ? 0 : ffmi::kv_split_floats(cfg->max_requests, cfg->num_heads, cfg->head_dim);
+  if (!f32) tab.resize(table + (size_t)cfg->max_requests * cfg->num_heads, 0.f);  // the counters start at zero
+  if (ok) ok = hipMalloc((void **)&h->rope, (table + split) * sizeof(float)) == hipSuccess;
   if (!f32) h->zscratch = h->rope + table;
   if (!ok) {
     ffmi_attn_destroy(h);
@@ -413,7 +417,7 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
                                   (const uint16_t *)qkv, qkvp, stage_wr, stage_rd, h->rope,
                                   h->slots, oproj ? opa : nullptr,
                                   fused && !oproj ? ffmi::attn_kv_split(b->num_work, heads, b->max_q, b->max_kv) : 1,
-                                  h->zscratch, b->one_item_per_req ? 0 : b->num_blocks));
+                                  h->zscratch, h->cfg.max_requests, b->one_item_per_req ? 0 : b->num_blocks));
   if (oproj) opa->done = true;
   return FFMI_OK;
 }

@@ -313,11 +313,17 @@ struct OprojArgs {
   size_t wts = 0, wks = 0;       // packed-block strides (w_tile_stride / w_k_stride)
   bool done = false;             // out: the launch projected (else run the o GEMM)
 };
-// An item's keys over Z = attn_kv_split(...) workgroups: scratch of
-// kKvSplitSlots counters (zero between launches), then as many partial outputs
-// [d] with max and sum
-constexpr int kMaxKvSplit = 8, kKvSplitSlots = 256;
-inline size_t kv_split_floats(int d) { return (size_t)kKvSplitSlots * (d + 3); }
+// An item's keys over Z = attn_kv_split(...) <= kv_split_most(heads) workgroups.
+// Scratch: a counter per (request, head) (zero between launches), then per counter
+// kv_split_most partial outputs [d] with max and sum
+constexpr int kMaxKvSplit = 8, kKvSplitWgs = 256;
+inline int kv_split_most(int heads) {
+  const int z = kKvSplitWgs / heads;
+  return z > kMaxKvSplit ? kMaxKvSplit : z;
+}
+inline size_t kv_split_floats(int requests, int heads, int d) {
+  return (size_t)requests * heads * (1 + (size_t)kv_split_most(heads) * (d + 2));
+}
 int attn_kv_split(int W, int heads, int max_q, int max_kv);
 hipError_t launch_attention(const char *blob, int W, int max_q, uint16_t *qbuf, uint16_t *kc,
                             uint16_t *vc, uint16_t *out, int heads, int d, int slots, float scale,
@@ -325,7 +331,7 @@ hipError_t launch_attention(const char *blob, int W, int max_q, uint16_t *qbuf, 
                             const uint16_t *qkv, Partials qkvp, uint16_t *stage_wr,
                             const uint16_t *stage_rd, const float *rope, int max_rope_pos,
                             const OprojArgs *opa = nullptr, int Z = 1, float *zscratch = nullptr,
-                            int blocks = 0);
+                            int requests = 0, int blocks = 0);
 
 uint64_t weight_key(const char *name, uint64_t seed);
 
@@ -344,7 +350,7 @@ struct ffmi_batch_dev {
   bool lds_tail = false;  // every item's writes fit the fused kernel's LDS tail and
                           // its commits the work item (else the two-launch path)
   int max_q = 0;                  // largest work item
-  int max_kv = 0;                 // most keys an item scans
+  int max_kv = 0;                 // most keys an item scans (0: no split of them, see batch_stage)
   int num_blocks = 0;             // WorkDev::block of the prompt attention
   hipEvent_t uploaded = nullptr;  // guards reuse of the pinned staging
 };

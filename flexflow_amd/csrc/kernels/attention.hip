@@ -478,10 +478,13 @@ struct KvUpdateArgs {
   const float *rope;
   int max_rope_pos;
   long long *stamps;  // ST kernels: per-wave timeline (diagnostics)
-  // ZS kernels: per workgroup the partial output [D] and its max and sum, then
-  // per (item, head) the count of partials that are there (zero between launches)
+  // ZS kernels: per (request, head) and sharing workgroup (at most zmax) the partial
+  // output [D] and its max and sum, and per (request, head) the count of partials
+  // that are there (zero between launches).  (By request, not by item: steps of
+  // different requests may run side by side.)
   float *zpart;
   unsigned *zcount;
+  int zmax;
 };
 
 // One workgroup per (work item = <= 16*QT consecutive queries of a request,
@@ -892,8 +895,8 @@ __global__ __launch_bounds__(64 * NW, 1) void attention_kernel(
     }
     if constexpr (ZS) {
       // the partial outputs past every cache, then the count; the last one merges
-      const int pair = (int)(blockIdx.y * gridDim.x + blockIdx.x), Z = (int)gridDim.z;
-      float *mine = kv.zpart + (size_t)(pair * Z + (int)blockIdx.z) * (D + 2);
+      const int pair = w.req * heads + h, Z = (int)gridDim.z;
+      float *mine = kv.zpart + ((size_t)pair * kv.zmax + blockIdx.z) * (D + 2);
       if (wave < DT && qi == 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -919,7 +922,7 @@ __global__ __launch_bounds__(64 * NW, 1) void attention_kernel(
       __syncthreads();
       const int dd = (int)threadIdx.x * 2;
       if (!sMrec[0].w || dd >= D || w.q_count == 0) return;
-      const float *all = kv.zpart + (size_t)pair * Z * (D + 2);
+      const float *all = kv.zpart + (size_t)pair * kv.zmax * (D + 2);
       float zm[kMaxKvSplit], zl[kMaxKvSplit], za[kMaxKvSplit], zb[kMaxKvSplit];
 #pragma unroll
       for (int z = 0; z < kMaxKvSplit; ++z) {  // (all in flight; past Z the last one again)
@@ -1183,7 +1186,7 @@ static bool attn_split_fits(int wgs) { return 2 * wgs <= attn_cus(); }
 
 int attn_kv_split(int W, int heads, int max_q, int max_kv) {
   if (max_q != 1 || W <= 0) return 1;
-  const int room = std::min(attn_cus(), kKvSplitSlots) / (W * heads), chunks = (max_kv + 31) / 32;
+  const int room = std::min(attn_cus(), kKvSplitWgs) / (W * heads), chunks = (max_kv + 31) / 32;
   const int Z = std::max(1, std::min(std::min(room, (chunks + 7) / 8), kMaxKvSplit));
   const char *e = Z > 1 ? getenv("FFMI_ATTN_KVSPLIT") : nullptr;
   return e && !atoi(e) ? 1 : Z;
@@ -1350,15 +1353,16 @@ hipError_t launch_attention(const char *blob, int W, int max_q, uint16_t *qbuf, 
                             hipStream_t s, bool out_packed, bool fused, int T, int C,
                             const uint16_t *qkv, Partials qkvp, uint16_t *stage_wr,
                             const uint16_t *stage_rd, const float *rope, int max_rope_pos,
-                            const OprojArgs *opa, int Z, float *zscratch, int blocks) {
+                            const OprojArgs *opa, int Z, float *zscratch, int requests, int blocks) {
   if (W <= 0) return hipSuccess;
   if (out_packed && (heads * d) % 32) return hipErrorInvalidValue;
   if (max_q > FFMI_ATTN_QTILE) return hipErrorInvalidValue;
+  const int zmax = kv_split_most(heads);
   const KvUpdateArgs kv{T,        C,        qkv,  qkvp.S > 0 ? qkvp.p : nullptr,
                         qkvp.S,   qkvp.NP,  stage_wr, stage_rd,
                         rope,     max_rope_pos, attn_stamp_buf(W * heads),
-                        zscratch ? zscratch + kKvSplitSlots : nullptr, (unsigned *)zscratch};
-  if (Z > 1 && (!fused || !zscratch || max_q != 1 || Z > kMaxKvSplit || W * heads * Z > kKvSplitSlots))
+                        zscratch ? zscratch + (size_t)requests * heads : nullptr, (unsigned *)zscratch, zmax};
+  if (Z > 1 && (!fused || !zscratch || max_q != 1 || Z > zmax))
     return hipErrorInvalidValue;
   const int op = out_packed ? 1 : 0;
   if (opa) {  // output projection folded in (the caller checked fused, d, max_q, N)

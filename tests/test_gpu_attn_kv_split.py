@@ -55,3 +55,45 @@ def test_split_keys(d, lens, layout, monkeypatch):
     # one rounding to fp16 of two fp32 sums of at most 2083 terms in other orders
     assert (np.abs(split - whole) <= 2.0 ** -10 * np.abs(whole) + 2e-6).all()
     assert (split == whole).mean() > 0.97
+
+
+def step_on(c, batch, stream, infos, qkv, out):
+    """One decode step of c's handle on a stream, from a batch of its own."""
+    toks = (F.TokenInfo * len(infos))(*[F.TokenInfo(*i, 0) for i in infos])
+    work = (F.AttnWork * len(infos))(*[F.AttnWork(i[2], t, 1, i[4]) for t, i in enumerate(infos)])
+    desc = F.BatchDesc(len(infos), len(infos), 0, 0, toks, work, (F.CommitInfo * 1)(), (ctypes.c_uint64 * 1)())
+    F.check(K.L.ffmi_batch_upload(batch, ctypes.byref(desc), stream))
+    F.check(K.L.ffmi_attn_inc(c.h, batch, qkv.ptr, out.ptr, stream))
+
+
+@pytest.mark.parametrize("heads,lens", [(2, [2080, 700, 1300, 400]), (16, [1025, 513, 2000, 300])])
+def test_two_streams_on_one_handle(heads, lens):
+    """Steps of different requests side by side: splits of different widths (the first
+    request alone, the other three together) count for themselves."""
+    d, H = 128, hip()
+    c = AttnCase(F.ATTN_INC, heads=heads, d=d, max_seq=2176, max_tokens=1024)
+    rng = np.random.default_rng(heads)
+    for r, n in enumerate(lens):
+        for a in range(0, n, 1024):
+            c.run([(3, p, r, p, p + 1, 0, 0, 0) for p in range(a, min(n, a + 1024))], rng=rng)
+    groups, sides = [[0], [1, 2, 3]], []
+    for g in groups:
+        b, s = ctypes.c_void_p(), ctypes.c_void_p()
+        F.check(K.L.ffmi_batch_create(64, 4, ctypes.byref(b)))
+        assert H.hipStreamCreate(ctypes.byref(s)) == 0
+        infos = [(7, lens[r], r, lens[r], lens[r] + 1, 0, 0, 0) for r in g]
+        qkv = K.Buf(K.f16(rng.standard_normal((len(g), 3 * c.Hl))))
+        sides.append((b, s, infos, qkv, [K.Buf.empty((16, c.Hl), np.float16) for _ in range(41)]))
+    for b, s, infos, qkv, outs in sides:  # one after the other
+        step_on(c, b, s, infos, qkv, outs[0])
+        assert H.hipStreamSynchronize(s) == 0
+    for i in range(1, 41):  # side by side, the same step again and again
+        for b, s, infos, qkv, outs in sides:
+            step_on(c, b, s, infos, qkv, outs[i])
+    for _, s, _, _, _ in sides:
+        assert H.hipStreamSynchronize(s) == 0
+    for g, (b, s, infos, qkv, outs) in zip(groups, sides):
+        want = outs[0].get()[:len(g)].view(np.uint16)
+        assert want.any()
+        for o in outs[1:]:
+            assert np.array_equal(o.get()[:len(g)].view(np.uint16), want)
