@@ -134,8 +134,11 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
       }
       wd[wi] = x;
     }
-    b->num_blocks = 0;
-    for (int wi = 0; wi < d->num_work; ++wi) {
+    b->one_item_per_req = true;
+    for (int wi = 1; wi < d->num_work; ++wi)
+      if (d->work[wi].req == d->work[wi - 1].req) b->one_item_per_req = false;
+    b->num_blocks = 0;  // (of prompt items only)
+    for (int wi = 0; wi < d->num_work && !b->one_item_per_req; ++wi) {
       const bool two = wi + 1 < d->num_work && d->work[wi + 1].req == d->work[wi].req;
       wd[b->num_blocks++].block = wi << 1 | (int)two;
       wi += two;
@@ -173,13 +176,11 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
   b->num_commits = d->num_commits;
   b->num_mask_reqs = d->num_mask_reqs;
   b->max_q = b->max_kv = 0;
-  b->one_item_per_req = true;
   for (int wi = 0; wi < d->num_work; ++wi) {
     FFMI_CHECK(d->work[wi].q_count >= 0 && d->work[wi].q_count <= FFMI_ATTN_QTILE,
                FFMI_ERR_INVALID);
     b->max_q = std::max(b->max_q, (int)d->work[wi].q_count);
     b->max_kv = std::max(b->max_kv, (int)d->work[wi].kv_len);
-    if (wi > 0 && d->work[wi].req == d->work[wi - 1].req) b->one_item_per_req = false;
   }
   // (a request's place in the key split's scratch is for one item)
   if (b->max_q == 1 && b->max_kv > 256)
@@ -417,7 +418,7 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
                                   (const uint16_t *)qkv, qkvp, stage_wr, stage_rd, h->rope,
                                   h->slots, oproj ? opa : nullptr,
                                   fused && !oproj ? ffmi::attn_kv_split(b->num_work, heads, b->max_q, b->max_kv) : 1,
-                                  h->zscratch, h->cfg.max_requests, b->one_item_per_req ? 0 : b->num_blocks));
+                                  h->zscratch, h->cfg.max_requests, b->num_blocks));
   if (oproj) opa->done = true;
   return FFMI_OK;
 }
@@ -483,38 +484,55 @@ static bool pack_first(int T, int out_dim, int in_dim, int epilogue) {
   return !(epilogue & FFMI_X_PACKED) && T > 128 && in_dim % 32 == 0 &&
          (double)T * out_dim * in_dim * (pair ? 2 : 1) >= 2.5e9;
 }
-// the split-K slabs, before the packed activations
+// Bytes of the split-K slabs, and of slabs and packed activations behind them.
+// (Planned once a call: about 1 us above 64 rows.  Up to 64 there are no slabs
+// without a consumer of them.)
 static size_t linear_slab_bytes(int T, int out_dim, int in_dim, int epilogue) {
-  return (ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue) + 255) & ~(size_t)255;
+  return T <= 64 ? 0 : ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue);
 }
+static size_t packed_behind(size_t slab) { return (slab + 255) & ~(size_t)255; }
 
 extern "C" size_t ffmi_linear_workspace_bytes(int T, int out_dim, int in_dim, int epilogue) {
   if (T <= 0 || out_dim <= 0 || in_dim <= 0) return 0;
-  if (pack_first(T, out_dim, in_dim, epilogue))
-    return linear_slab_bytes(T, out_dim, in_dim, epilogue) + ffmi::packed_act_bytes(T, in_dim);
-  return ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue);
+  const size_t slab = ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue);
+  return pack_first(T, out_dim, in_dim, epilogue) ? packed_behind(slab) + ffmi::packed_act_bytes(T, in_dim) : slab;
+}
+
+static ffmi_status linear_check(const void *X, const void *W_packed, void *Y, int T, int out_dim, int in_dim,
+                                int epilogue) {
+  FFMI_CHECK(X && W_packed && Y && T >= 0 && out_dim > 0, FFMI_ERR_INVALID);
+  FFMI_CHECK(in_dim > 0 && in_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
+  const int epi_base = epilogue & ~(FFMI_X_PACKED | FFMI_W_STREAM | FFMI_Y_PACKED);
+  FFMI_CHECK(epi_base == FFMI_EPI_NONE || epi_base == FFMI_EPI_SILU_MUL, FFMI_ERR_INVALID);
+  FFMI_CHECK(!(epilogue & FFMI_Y_PACKED) || out_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
+  return FFMI_OK;
+}
+
+// packed: where in the workspace row-major activations are packed first (nullptr: not)
+static ffmi_status linear_run(const void *X, const void *W_packed, void *Y, int T, int out_dim, int in_dim,
+                              int epilogue, void *ws, size_t slab, void *packed, hipStream_t s) {
+  if (packed) {
+    FFMI_HIP(ffmi::launch_pack_act((const uint16_t *)X, (uint16_t *)packed, T, in_dim, s));
+    X = packed, epilogue |= FFMI_X_PACKED;
+  }
+  FFMI_HIP(ffmi::launch_gemm((const uint16_t *)X, (const uint16_t *)W_packed, (uint16_t *)Y, (float *)ws, slab, T,
+                             out_dim, in_dim, epilogue, s));
+  return FFMI_OK;
 }
 
 extern "C" ffmi_status ffmi_linear_ws(const void *X, const void *W_packed, void *Y, int T,
                                       int out_dim, int in_dim, int epilogue, void *workspace,
                                       size_t workspace_bytes, ffmi_stream stream) {
-  FFMI_CHECK(X && W_packed && Y && T >= 0 && out_dim > 0, FFMI_ERR_INVALID);
-  FFMI_CHECK(in_dim > 0 && in_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
-  const int epi = epilogue & ~(FFMI_X_PACKED | FFMI_W_STREAM);
-  const int epi_base = epi & ~FFMI_Y_PACKED;
-  FFMI_CHECK(epi_base == FFMI_EPI_NONE || epi_base == FFMI_EPI_SILU_MUL, FFMI_ERR_INVALID);
-  FFMI_CHECK(!(epilogue & FFMI_Y_PACKED) || out_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
-  const size_t slab = linear_slab_bytes(T, out_dim, in_dim, epilogue);
-  if (workspace && ((uintptr_t)workspace & 15) == 0 && pack_first(T, out_dim, in_dim, epilogue) &&
-      workspace_bytes >= slab + ffmi::packed_act_bytes(T, in_dim)) {
-    uint16_t *xp = (uint16_t *)((char *)workspace + slab);
-    FFMI_HIP(ffmi::launch_pack_act((const uint16_t *)X, xp, T, in_dim, (hipStream_t)stream));
-    X = xp, epilogue |= FFMI_X_PACKED, workspace_bytes = slab;
+  const ffmi_status st = linear_check(X, W_packed, Y, T, out_dim, in_dim, epilogue);
+  if (st != FFMI_OK) return st;
+  void *packed = nullptr;
+  if (workspace && ((uintptr_t)workspace & 15) == 0 && pack_first(T, out_dim, in_dim, epilogue)) {
+    const size_t at = packed_behind(linear_slab_bytes(T, out_dim, in_dim, epilogue));
+    if (workspace_bytes >= at + ffmi::packed_act_bytes(T, in_dim))
+      packed = (char *)workspace + at, workspace_bytes = at;
   }
-  FFMI_HIP(ffmi::launch_gemm((const uint16_t *)X, (const uint16_t *)W_packed, (uint16_t *)Y,
-                             (float *)workspace, workspace_bytes, T, out_dim, in_dim, epilogue,
-                             (hipStream_t)stream));
-  return FFMI_OK;
+  return linear_run(X, W_packed, Y, T, out_dim, in_dim, epilogue, workspace, workspace_bytes, packed,
+                    (hipStream_t)stream);
 }
 
 static std::mutex g_ws_mu;
@@ -522,22 +540,24 @@ static ffmi::GraphWorkspace g_ws;
 
 extern "C" ffmi_status ffmi_linear(const void *X, const void *W_packed, void *Y, int T,
                                    int out_dim, int in_dim, int epilogue, ffmi_stream stream) {
-  FFMI_CHECK(X && W_packed && Y && T >= 0 && out_dim > 0, FFMI_ERR_INVALID);
-  FFMI_CHECK(in_dim > 0 && in_dim % 32 == 0, FFMI_ERR_UNSUPPORTED);
-  // a captured call takes its slabs alone: a graph's share of the workspace is kept
-  // for good (up to 64 rows there are no slabs without a consumer of them)
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (stream && T > 64) FFMI_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
-  const bool captured = cap != hipStreamCaptureStatusNone;
-  const size_t need = captured ? ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue)
-                               : ffmi_linear_workspace_bytes(T, out_dim, in_dim, epilogue);
+  const ffmi_status st = linear_check(X, W_packed, Y, T, out_dim, in_dim, epilogue);
+  if (st != FFMI_OK) return st;
+  const size_t slab = linear_slab_bytes(T, out_dim, in_dim, epilogue);
+  bool pack = pack_first(T, out_dim, in_dim, epilogue), captured = false;
+  if (stream && (slab > 0 || pack)) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    FFMI_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
+    captured = cap != hipStreamCaptureStatusNone;
+    // a captured call takes its slabs alone: a graph's share of the workspace is kept for good
+    if (captured) pack = false;
+  }
+  const size_t need = pack ? packed_behind(slab) + ffmi::packed_act_bytes(T, in_dim) : slab;
   void *ws = nullptr;
-  size_t ws_bytes = 0;
-  {
+  if (need > 0) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     hipError_t err = hipSuccess;
     ws = g_ws.get(
-        need, captured && need > 0,
+        need, captured,
         [](size_t n) {
           void *p = nullptr;
           return hipMalloc(&p, n) == hipSuccess ? p : nullptr;
@@ -548,10 +568,10 @@ extern "C" ffmi_status ffmi_linear(const void *X, const void *W_packed, void *Y,
           return err == hipSuccess;
         });
     FFMI_HIP(err);
-    if (need > 0 && !ws) return FFMI_ERR_OOM;
-    ws_bytes = captured ? need : g_ws.bytes();
+    if (!ws) return FFMI_ERR_OOM;
   }
-  return ffmi_linear_ws(X, W_packed, Y, T, out_dim, in_dim, epilogue, ws, ws_bytes, stream);
+  return linear_run(X, W_packed, Y, T, out_dim, in_dim, epilogue, ws, slab,
+                    pack ? (char *)ws + packed_behind(slab) : nullptr, (hipStream_t)stream);
 }
 
 extern "C" ffmi_status ffmi_rmsnorm(const void *x, const void *w, void *out, int T, int H,

@@ -232,7 +232,8 @@ __device__ __forceinline__ float silu_glu(float gate, float up) {
 hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                        size_t ws_bytes, int T, int N, int K, int epilogue, hipStream_t s,
                        Partials *defer = nullptr, int wpitch = 0, const FuseArgs *fuse = nullptr);
-size_t gemm_workspace_bytes(int T, int N, int K, int epilogue);
+// (aligned: X on a 16-byte boundary)
+size_t gemm_workspace_bytes(int T, int N, int K, int epilogue, bool aligned = false);
 // The same GEMM on bf16 operands in packed activation tiles, one entry per
 // epilogue: Y bf16; Y bf16 = relu(x)^2; or fp32 slabs in `ws` (*defer, or one
 // unsplit [T][ceil16(N)] slab when defer is null).  flags: FFMI_X_PACKED |

@@ -3,8 +3,8 @@
 
 namespace ffmi {
 
-size_t gemm_workspace_bytes(int T, int N, int K, int epilogue) {
-  return gemm_slab_bytes(T, N, K, epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM));
+size_t gemm_workspace_bytes(int T, int N, int K, int epilogue, bool aligned) {
+  return gemm_slab_bytes(T, N, K, epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM), false, aligned);
 }
 
 hipError_t launch_partials_reduce(const Partials &p, uint16_t *Y, int T, int N, hipStream_t s) {

@@ -1337,18 +1337,23 @@ static bool use_tiles(int T, int N, int K, bool paired) {
   return mode == 2 || (mode == 1 && !msplit_ahead(T, N, K, paired));
 }
 
-static bool use_tiles(int T, int N, int K, bool paired);
-// split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums
-static inline size_t gemm_slab_bytes(int T, int N, int K, int epilogue, bool f32 = false) {
+// split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;
+// aligned: activations on 16-byte boundaries, as a model's own are (those the tile
+// kernel takes it takes always: the M-split plans, a microsecond, are not asked for)
+static inline size_t gemm_slab_bytes(int T, int N, int K, int epilogue, bool f32 = false, bool aligned = false) {
   const int mtiles = (T + 15) / 16;
   if (mtiles <= 4) {
     const int S = skinny_split(T, N, K, epilogue, true);
     return S > 1 ? (size_t)S * T * ((N + 15) / 16) * 16 * sizeof(float) : 0;
   }
   const int ntiles = (N + 15) / 16 * (epilogue ? 2 : 1);
-  int S = std::max(mid_plan(T, N, K, epilogue, false).S,
-                   epilogue ? 1 : mid_plan(T, N, K, epilogue, true).S);
-  if (K % 32 == 0 && use_tiles(T, N, K, epilogue != 0)) {
+  const bool tiles = K % 32 == 0 && use_tiles(T, N, K, epilogue != 0);
+  int S = 1;
+  if (!tiles || !aligned) {
+    S = mid_plan(T, N, K, epilogue, false).S;
+    if (!epilogue) S = std::max(S, mid_plan(T, N, K, epilogue, true).S);
+  }
+  if (tiles) {
     if (!f32) S = std::max(S, tile_plan(T, N, K, epilogue != 0, false, false).S);
     if (!epilogue) S = std::max(S, tile_plan(T, N, K, false, f32, true).S);
   }

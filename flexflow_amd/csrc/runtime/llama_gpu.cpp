@@ -584,11 +584,11 @@ struct LlamaGPU : public ffmi_model {
       // the split-K factor depends on the row-block count, so take the max
       // over every batch size the model can see
       for (int t = 16; t <= Tm; t += 16) {
-        const size_t w1 = ffmi::gemm_workspace_bytes(t, 3 * Hl, H, FFMI_EPI_NONE);
-        const size_t w2 = ffmi::gemm_workspace_bytes(t, H, Hl, FFMI_EPI_NONE);
-        const size_t w3 = ffmi::gemm_workspace_bytes(t, Fl, H, FFMI_EPI_SILU_MUL);
-        const size_t w4 = ffmi::gemm_workspace_bytes(t, H, Fl, FFMI_EPI_NONE);
-        const size_t w5 = ffmi::gemm_workspace_bytes(t, Vl, H, FFMI_EPI_NONE);
+        const size_t w1 = ffmi::gemm_workspace_bytes(t, 3 * Hl, H, FFMI_EPI_NONE, true);
+        const size_t w2 = ffmi::gemm_workspace_bytes(t, H, Hl, FFMI_EPI_NONE, true);
+        const size_t w3 = ffmi::gemm_workspace_bytes(t, Fl, H, FFMI_EPI_SILU_MUL, true);
+        const size_t w4 = ffmi::gemm_workspace_bytes(t, H, Fl, FFMI_EPI_NONE, true);
+        const size_t w5 = ffmi::gemm_workspace_bytes(t, Vl, H, FFMI_EPI_NONE, true);
         ws_bytes = std::max(ws_bytes, std::max(std::max(std::max(w1, w2), std::max(w3, w4)), w5));
       }
       // the row-parallel column chunks over the xGMI transport defer their
@@ -597,8 +597,8 @@ struct LlamaGPU : public ffmi_model {
       if (peer && ar_slabs && tp_chunks > 1) {
         const int Hc = H / tp_chunks;
         for (int t = 16; t <= Tm; t += 16)
-          ws_chunk = std::max(ws_chunk, std::max(ffmi::gemm_workspace_bytes(t, Hc, Hl, FFMI_EPI_NONE),
-                                                 ffmi::gemm_workspace_bytes(t, Hc, Fl, FFMI_EPI_NONE)));
+          ws_chunk = std::max(ws_chunk, std::max(ffmi::gemm_workspace_bytes(t, Hc, Hl, FFMI_EPI_NONE, true),
+                                                 ffmi::gemm_workspace_bytes(t, Hc, Fl, FFMI_EPI_NONE, true)));
         ws_chunk = (ws_chunk + 255) & ~(size_t)255;
         ws_bytes = std::max(ws_bytes, ws_chunk * tp_chunks);
       }
