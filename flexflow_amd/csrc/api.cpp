@@ -360,6 +360,19 @@ extern "C" ffmi_status ffmi_attn_kv_ptrs(ffmi_attn *h, void **k, void **v, int *
 }
 
 namespace ffmi {
+static bool attn_fused(const ffmi_batch_dev *b) {
+  return b->one_item_per_req && b->lds_tail && getenv("FFMI_ATTN_NO_FUSE") == nullptr;
+}
+// (fused, one query tile, d = 64, N <= 1024 columns)
+static bool attn_oproj(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
+  return opa && opa->wo && opa->slab && attn_fused(b) && h->cfg.head_dim == 64 && b->max_q <= 16 &&
+         opa->N % 16 == 0 && opa->N <= 1024 && b->num_tokens <= opa->max_T;
+}
+int attn_key_split(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
+  if (!attn_fused(b) || attn_oproj(h, b, opa)) return 1;
+  return attn_kv_split(b->num_work, h->cfg.num_heads, b->max_q, b->max_kv);
+}
+
 ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv, Partials qkvp,
                          void *out, ffmi_stream stream, int parity, OprojArgs *opa) {
   FFMI_CHECK(h && b && (qkv || qkvp.S > 0) && out, FFMI_ERR_INVALID);
@@ -396,8 +409,7 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
   // slot this step stores go first in their own launch (the reference's
   // commit-then-store order).  FFMI_ATTN_NO_FUSE=1 forces the two-launch path
   // (A/B and parity tests).
-  const bool no_fuse = getenv("FFMI_ATTN_NO_FUSE") != nullptr;
-  const bool fused = b->one_item_per_req && b->lds_tail && !no_fuse;
+  const bool fused = attn_fused(b);
   if (C > 0 && b->commit_overlap) {
     FFMI_HIP(ffmi::launch_commit(b->dev, C, stage_rd, h->kc, h->vc, heads, d, h->slots, s));
     C = 0;
@@ -408,16 +420,15 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
                                     stage_rd, h->rope, heads, d, h->slots, h->slots, s));
     C = 0;
   }
-  // the output projection rides along where its launch allows it (fused,
-  // one query tile, d = 64, N <= 1024 columns); otherwise the caller runs it
-  const bool oproj = opa && opa->wo && opa->slab && fused && d == 64 && b->max_q <= 16 &&
-                     opa->N % 16 == 0 && opa->N <= 1024 && b->num_tokens <= opa->max_T;
+  // the output projection rides along where its launch allows it; otherwise the
+  // caller runs it
+  const bool oproj = attn_oproj(h, b, opa);
   FFMI_HIP(ffmi::launch_attention(b->dev, b->num_work, b->max_q, h->qbuf, h->kc, h->vc,
                                   (uint16_t *)out, heads, d, h->slots, h->cfg.qk_scale, s,
                                   h->cfg.out_layout == 1, fused, b->num_tokens, C,
                                   (const uint16_t *)qkv, qkvp, stage_wr, stage_rd, h->rope,
                                   h->slots, oproj ? opa : nullptr,
-                                  fused && !oproj ? ffmi::attn_kv_split(b->num_work, heads, b->max_q, b->max_kv) : 1,
+                                  attn_key_split(h, b, opa),
                                   h->zscratch, h->cfg.max_requests, b->num_blocks));
   if (oproj) opa->done = true;
   return FFMI_OK;

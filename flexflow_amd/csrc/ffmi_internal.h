@@ -181,6 +181,9 @@ hipError_t launch_logit_rows(const void *logits, bool half, size_t ld, const Log
 hipError_t launch_softmax_topk_f32(const float *logits, int T, int V, int k, int32_t *ids,
                                    float *probs, hipStream_t s, int ld = 0);  // (0: ld = V)
 ffmi_status attn_rope_fault(ffmi_attn *h, int from_pos);
+// workgroups that share an item's keys where attn_forward runs this step
+struct OprojArgs;
+int attn_key_split(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa);
 // Packed weights (weights.hip): 1 KiB block (tile t, k-step kt) at
 // t * w_tile_stride(KT) + kt * w_k_stride(P) halves, P = tiles per k-row of
 // the allocation.  K-major unless FFMI_W_TILE_MAJOR=1 (A/B runs).

@@ -38,6 +38,8 @@ extern "C" long ffmi_model_debug_tensor(ffmi_model *m, int which, int layer, flo
   return m->debug_tensor(which, layer, out, cap);
 }
 
+extern "C" long ffmi_model_debug_graphs(ffmi_model *m) { return m ? m->debug_graphs() : -1; }
+
 extern "C" long ffmi_model_debug_width(ffmi_model *m, int which) {
   if (!m) return -1;
   return m->debug_width(which);

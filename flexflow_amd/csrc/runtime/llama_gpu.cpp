@@ -851,11 +851,27 @@ struct LlamaGPU : public ffmi_model {
              std::tie(o.T, o.W, o.C, o.k, o.parity, o.overlap, o.fused, o.max_q, o.slot, o.bytes);
     }
   };
-  // how a step's attention is launched
-  int attn_form() const {
+  // how a step's attention is launched (as attn_forward decides: what it does not
+  // split is captured once, however many keys there are)
+  int attn_form(int T) const {
+    if (layers.empty()) return 0;
+    const ffmi::OprojArgs oa = oproj_args(layers[0], T);
     return (batch->one_item_per_req ? 1 : 0) | (batch->lds_tail ? 2 : 0) |
-           ffmi::attn_kv_split(batch->num_work, heads_l, batch->max_q, batch->max_kv) << 2 |
-           batch->num_blocks << 6;
+           ffmi::attn_key_split(layers[0].attn, batch, oa.wo ? &oa : nullptr) << 2 | batch->num_blocks << 6;
+  }
+  // the residual norms folded into the GEMMs around them (see fuse_norms)
+  bool fused_norms(int T) const {
+    const int H = c.hidden;
+    return (fuse_norms == 2 || (fuse_norms == 1 && H >= 2048)) && !dbg && o.tp_size == 1 && T <= 32 &&
+           H % 32 == 0 && Hl % 32 == 0 && H <= 4096;
+  }
+  ffmi::OprojArgs oproj_args(const Layer &L, int T) const {
+    ffmi::OprojArgs oa;
+    if (fuse_ao && !fused_norms(T)) {
+      oa.wo = L.wo, oa.slab = oslab, oa.N = c.hidden, oa.max_T = oslab_T;
+      oa.wts = ffmi::w_tile_stride(Hl / 32), oa.wks = ffmi::w_k_stride(c.hidden / 16);
+    }
+    return oa;
   }
   // TREE steps write alternate halves of the attention staging (commits of
   // the next step read the half this one wrote); kept here so graph replays
@@ -941,7 +957,7 @@ struct LlamaGPU : public ffmi_model {
     if (graph) {
       const GraphKey key{T, batch->num_work, batch->num_commits, k, tree_parity,
                          batch->commit_overlap ? 1 : 0,
-                         attn_form(),
+                         attn_form(T),
                          batch->max_q, cur_slot, bytes};
       auto it = graphs.find(key);
       if (it == graphs.end()) {
@@ -993,7 +1009,7 @@ struct LlamaGPU : public ffmi_model {
     pend.push_back({slot, T, k, bytes,
                     GraphKey{T, batch->num_work, batch->num_commits, k, tree_parity,
                              batch->commit_overlap ? 1 : 0,
-                             attn_form(),
+                             attn_form(T),
                              batch->max_q, slot, bytes}});
     return FFMI_OK;
   }
@@ -1062,6 +1078,7 @@ struct LlamaGPU : public ffmi_model {
     return FFMI_OK;
   }
 
+  long debug_graphs() const override { return (long)(graphs.size() + group_graphs.size()); }
   void clear_graphs() {
     for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
     graphs.clear();
@@ -1090,8 +1107,7 @@ struct LlamaGPU : public ffmi_model {
     static const int marker_h = getenv("FFMI_MARKERS") ? atoi(getenv("FFMI_MARKERS")) : 0;
     static const int marker_t = getenv("FFMI_MARKERS_T") ? atoi(getenv("FFMI_MARKERS_T")) : 0;
     int mark_i = 0;
-    const bool fuse = (fuse_norms == 2 || (fuse_norms == 1 && H >= 2048)) && !dbg &&
-                      o.tp_size == 1 && T <= 32 && H % 32 == 0 && Hl % 32 == 0 && H <= 4096;
+    const bool fuse = fused_norms(T);
     // the residual norms inside the transport's all-reduces (tp_fuse_norm)
     const bool arn = peer && !solo && o.tp_size > 1 && (tp_fuse_norm == 2 || (tp_fuse_norm == 1 && !dbg));
     for (int l = 0; l < c.num_layers; ++l) {
@@ -1155,11 +1171,7 @@ struct LlamaGPU : public ffmi_model {
       mk();
       if (dbg) TRY(dbg_gemm_out(FFMI_DBG_QKV, l, qkv, qkv_part, T));
       pr = prof_begin(on);
-      ffmi::OprojArgs oa;
-      if (fuse_ao && !fuse) {
-        oa.wo = L.wo, oa.slab = oslab, oa.N = H, oa.max_T = oslab_T;
-        oa.wts = ffmi::w_tile_stride(Hl / 32), oa.wks = ffmi::w_k_stride(H / 16);
-      }
+      ffmi::OprojArgs oa = oproj_args(L, T);
       TRY(ffmi::attn_forward(L.attn, batch, qkv, qkv_part, att, s,
                              mode == FFMI_MODEL_TREE ? tree_parity : -1,
                              oa.wo ? &oa : nullptr));

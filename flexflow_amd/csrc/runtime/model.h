@@ -139,6 +139,7 @@ struct ffmi_model {
     (void)which;
     return -1;
   }
+  virtual long debug_graphs() const { return -1; }
 };
 
 namespace ffmi {

@@ -207,6 +207,7 @@ SIGNATURES = {
     "ffmi_model_set_debug": (c_int, [c_void_p, c_int]),
     "ffmi_model_debug_tensor": (ctypes.c_long, [c_void_p, c_int, c_int, c_void_p, ctypes.c_long]),
     "ffmi_model_debug_width": (ctypes.c_long, [c_void_p, c_int]),
+    "ffmi_model_debug_graphs": (ctypes.c_long, [c_void_p]),
     "ffmi_model_debug_fault": (c_int, [c_void_p, c_int, c_int, c_int]),
     "ffmi_set_device": (c_int, [c_int]),
     "ffmi_rm_create": (c_int, [ctypes.POINTER(RMConfig), ctypes.POINTER(c_void_p)]),

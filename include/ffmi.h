@@ -505,6 +505,8 @@ int ffmi_model_op_stats(ffmi_model *m, ffmi_op_stat *out, int cap);
 ffmi_status ffmi_model_set_debug(ffmi_model *m, int enable);
 long ffmi_model_debug_tensor(ffmi_model *m, int which, int layer, float *out, long cap);
 long ffmi_model_debug_width(ffmi_model *m, int which);
+/* Test hook: step graphs that the model holds (-1: this kind of model does not say). */
+long ffmi_model_debug_graphs(ffmi_model *m);
 /* Negative-control fault injection (tests only; never set in serving): the
  * parity tests must FAIL on a model with a deliberate bug.
  *   FFMI_FAULT_ROPE_POS, layer, arg: that layer's RoPE rotates tokens at
