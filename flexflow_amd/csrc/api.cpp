@@ -1205,6 +1205,12 @@ extern "C" ffmi_status ffmi_allreduce_rmsnorm(ffmi_comm *c, const void *in, int 
                                    (flags & FFMI_Y_PACKED) != 0, two, (hipStream_t)stream);
 }
 
+extern "C" int ffmi_debug_linear_tiles(int T, int out_dim, int in_dim, int epilogue, int *slices) {
+  int one = 1;
+  if (T <= 0 || out_dim <= 0 || in_dim <= 0) return -1;
+  return ffmi::gemm_tile_form(T, out_dim, in_dim, epilogue, slices ? slices : &one);
+}
+
 extern "C" long ffmi_debug_gemm_stamps(long long *dst, long max_waves) {
   return ffmi::gemm_debug_stamps(dst, max_waves);
 }

@@ -235,6 +235,9 @@ __device__ __forceinline__ float silu_glu(float gate, float up) {
 hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                        size_t ws_bytes, int T, int N, int K, int epilogue, hipStream_t s,
                        Partials *defer = nullptr, int wpitch = 0, const FuseArgs *fuse = nullptr);
+// The form (kTileForms) and K slices in which the tile kernel takes a product of its
+// own (no consumer of slabs), -1 where another kernel takes it
+int gemm_tile_form(int T, int N, int K, int epilogue, int *slices);
 // (aligned: X on a 16-byte boundary)
 size_t gemm_workspace_bytes(int T, int N, int K, int epilogue, bool aligned = false);
 // The same GEMM on bf16 operands in packed activation tiles, one entry per

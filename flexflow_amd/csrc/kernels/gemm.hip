@@ -32,6 +32,15 @@ hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float
   return launch_gemm_kind<0>(X, Wp, Y, ws, ws_bytes, T, N, K, epilogue, s, defer, wpitch, fuse);
 }
 
+int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
+  const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
+  *slices = 1;
+  if (T <= 64 || K % 32 || !use_tiles(T, N, K, paired, false, false)) return -1;
+  const TilePlan p = tile_plan(T, N, K, paired, false, false);
+  *slices = p.S;
+  return p.form;
+}
+
 // Packed activation tiles: Xp[mt][kt][lane][8] = X[mt*16 + (lane&15)][kt*32 + 8(lane>>4) + e]
 // (rows >= T zero) -- the MFMA operand fragment order of the weights (weights.hip),
 // so a GEMM reads each activation fragment as one contiguous 1 KiB.

@@ -1276,7 +1276,32 @@ static constexpr TileForm kTileForms[] = {
 static constexpr int kNumTileForms = sizeof(kTileForms) / sizeof(kTileForms[0]);
 struct TilePlan {
   int form, S, nbm, nbn;
+  bool msplit;  // the M-split kernel is the faster one (msplit_ahead)
 };
+// Where the M-split kernel stays ahead of the tile forms (us).
+//  * Up to 192 rows, one row block whose non-temporal weight stream is the time (in
+//    the model, at T = 168, o_proj and down with the norms that read their slabs 55.7
+//    against 57.2, N 32000 x K 4096 58 against 65, 12288 x 4096 32 against 36; at
+//    T = 82 K 9600 x N 4096 20.0 against 23.7).
+//  * Two blocks of up to 192 rows of a large unpaired weight (12288 x 4096 at T = 384
+//    46.3 against 51.6, 4096 x 11008 44.9 against 47.5; but gate/up 90.6 against 78.8).
+//  * Two such blocks of a small product: narrow waves, all in one round, up to 44
+//    k-steps a slice and no more slices than the tiles take (or few columns, whose
+//    slabs are small).  The tile kernel fills its ring of stages first, which costs it
+//    about 0.5 us and is not won back in so few steps.  At T = 257 and 384: 2304 x 768
+//    7.1 and 7.2 against 7.6, 2048 x 512 5.8 and 6.0 against 6.3 and 6.4, 8192 x 1024 10.8
+//    and 10.3 against 11.2, 512 x 4096 10.2 and 11.3 against 10.8 and 11.8; but 768 x 768, split by
+//    one kernel only, 8.4 and 8.5 against 7.2, and 6144 x 2048, longer slices, 20.1 and 20.1
+//    against 20.0 and 20.2.
+static bool msplit_ahead(int mtiles, int ntiles, int N, int K, bool paired, bool deferred, const TilePlan &t) {
+  if (mtiles <= 12) return true;
+  if (mtiles <= 16 || mtiles > 24) return false;
+  if ((long)ntiles * 16 * K >= 1L << 25) return !paired && ntiles <= 1024;
+  const MidPlan m = mid_plan(mtiles * 16, N, K, paired, deferred && !paired);
+  const int steps = (K / 32 + m.S - 1) / m.S;
+  return m.NTW <= 4 && steps <= 44 && (long)m.nblk * m.S * m.mblocks <= 256 &&
+         (m.S <= t.S || (ntiles <= 32 && t.S > 4));
+}
 // f32: the output is slabs in any case; deferred: the consumer sums the slabs
 // (else a reduce pass).  Depends on T by its row tiles only, as workspaces are
 // sized.  The search takes about a microsecond; a thread keeps what it found,
@@ -1308,33 +1333,23 @@ static TilePlan tile_plan(int T, int N, int K, bool paired, bool f32, bool defer
       if (S > 1) t += 4.0 * S * mb / 4.5;
       for (int d = 0; d < 2; ++d)
         if (t + (S > 1 && !d ? 3.0 : 0.0) < least[d])
-          least[d] = t + (S > 1 && !d ? 3.0 : 0.0), best[d] = TilePlan{f, S, nbm, nbn};
+          least[d] = t + (S > 1 && !d ? 3.0 : 0.0), best[d] = TilePlan{f, S, nbm, nbn, false};
     }
   }
+  for (int d = 0; d < 2; ++d)
+    best[d].msplit = msplit_ahead(mtiles, ntiles, N, K, paired, d != 0, best[d]);
   at = Found{mtiles, ntiles, KT, flags, {best[0], best[1]}};
   return best[deferred];
-}
-// Where the M-split kernel stays ahead of the tile forms (us): up to 192 rows,
-// one row block whose non-temporal weight stream is the time (in the model, at
-// T = 168, o_proj and down with the norms that read their slabs 55.7 against
-// 57.2, N 32000 x K 4096 58 against 65, 12288 x 4096 32 against 36; at T = 82
-// K 9600 x N 4096 20.0 against 23.7), and two blocks of up to 192 rows of a
-// large unpaired weight (12288 x 4096 at T = 384 46.3 against 51.6, 4096 x 11008
-// 44.9 against 47.5; but gate/up 90.6 against 78.8).
-static bool msplit_ahead(int T, int N, int K, bool paired) {
-  const int mtiles = (T + 15) / 16, ntiles = (N + 15) / 16 * (paired ? 2 : 1);
-  const bool large = (long)ntiles * 16 * K >= 1L << 25;
-  if (mtiles <= 12) return true;
-  return large && !paired && mtiles > 16 && mtiles <= 24 && ntiles <= 1024;
 }
 // FFMI_TILE_GEMM: 0 never, 2 whatever the size (A/B runs and tests; read per call)
 static int tile_mode() {
   const char *e = getenv("FFMI_TILE_GEMM");
   return e ? atoi(e) : 1;
 }
-static bool use_tiles(int T, int N, int K, bool paired) {
+static bool use_tiles(int T, int N, int K, bool paired, bool f32, bool deferred) {
   const int mode = tile_mode();
-  return mode == 2 || (mode == 1 && !msplit_ahead(T, N, K, paired));
+  if (mode != 1) return mode == 2;
+  return T > 192 && !tile_plan(T, N, K, paired, f32, deferred).msplit;
 }
 
 // split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;
@@ -1347,15 +1362,11 @@ static inline size_t gemm_slab_bytes(int T, int N, int K, int epilogue, bool f32
     return S > 1 ? (size_t)S * T * ((N + 15) / 16) * 16 * sizeof(float) : 0;
   }
   const int ntiles = (N + 15) / 16 * (epilogue ? 2 : 1);
-  const bool tiles = K % 32 == 0 && use_tiles(T, N, K, epilogue != 0);
   int S = 1;
-  if (!tiles || !aligned) {
-    S = mid_plan(T, N, K, epilogue, false).S;
-    if (!epilogue) S = std::max(S, mid_plan(T, N, K, epilogue, true).S);
-  }
-  if (tiles) {
-    if (!f32) S = std::max(S, tile_plan(T, N, K, epilogue != 0, false, false).S);
-    if (!epilogue) S = std::max(S, tile_plan(T, N, K, false, f32, true).S);
+  for (int deferred = f32 ? 1 : 0; deferred <= (epilogue ? 0 : 1); ++deferred) {
+    const bool tiles = K % 32 == 0 && use_tiles(T, N, K, epilogue != 0, f32, deferred);
+    if (tiles) S = std::max(S, tile_plan(T, N, K, epilogue != 0, f32, deferred).S);
+    if (!tiles || !aligned) S = std::max(S, mid_plan(T, N, K, epilogue, deferred).S);
   }
   return S > 1 ? (size_t)S * T * ntiles * 16 * sizeof(float) : 0;
 }
@@ -1510,7 +1521,8 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   }
   // (the tile kernel's copies to LDS are of 16 bytes)
   const bool aligned = (((uintptr_t)X | (uintptr_t)Wp) & 15) == 0;
-  if (mtiles > 4 && K % 32 == 0 && aligned && (xp || E < 2) && use_tiles(T, N, K, paired))
+  if (mtiles > 4 && K % 32 == 0 && aligned && (xp || E < 2) &&
+      use_tiles(T, N, K, paired, epi_f32<E>, defer != nullptr && !paired))
     return run_tiles<E>(X, Wp, Y, ws, ws_bytes, T, N, K, s, xp, yp, defer, wpitch, lim);
   if (mtiles > 4) {
     const MidPlan p = mid_plan(T, N, K, paired, defer != nullptr && !paired);

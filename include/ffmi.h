@@ -662,6 +662,10 @@ ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const float *ss_i
                                          void *Y, int T, int out_dim, int in_dim, int epilogue,
                                          ffmi_stream stream);
 
+/* Test hook: the tile size (0 ..) and K slices in which ffmi_linear's tile kernel
+ * takes a product on 16-byte boundaries, -1 where another kernel takes it. */
+int ffmi_debug_linear_tiles(int T, int out_dim, int in_dim, int epilogue, int *slices);
+
 /* Diagnostics: with FFMI_GEMM_STAMP set in the environment, M-split GEMM
  * launches record per-wave timestamps; copies the last launch's records
  * ({start, prologue done, k-loop done, end} at 100 MHz, HW_ID, XCC_ID) and

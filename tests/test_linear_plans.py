@@ -1,0 +1,41 @@
+"""Which kernel takes a dense layer's product (gemm_kernels.h tile_plan, msplit_ahead), on
+the CPU: the plan is host code."""
+import ctypes
+from concurrent.futures import ThreadPoolExecutor
+
+import pytest
+
+import flexflow_amd.ffmi as F
+
+
+def tiles(T, N, K, epi=0):
+    """(form, slices) of the tile kernel, None where another kernel takes the product"""
+    s = ctypes.c_int()
+    form = F.lib().ffmi_debug_linear_tiles(T, N, K, epi, ctypes.byref(s))
+    return (form, s.value) if form >= 0 else None
+
+
+# two blocks of up to 192 rows: short slices in narrow waves stay with the M-split kernel
+@pytest.mark.parametrize("T", [257, 300, 352, 384])
+@pytest.mark.parametrize("N,K,epi,ours", [
+    (2304, 768, 0, True), (2048, 512, 0, True), (8192, 1024, 0, True), (1024, 256, 0, True), (2816, 1024, 1, True),
+    (512, 4096, 0, True), (256, 2048, 0, True), (128, 2048, 0, True), (64, 4096, 0, True),
+    (768, 768, 0, False), (768, 3072, 0, False), (1024, 1024, 0, False), (32000, 768, 0, False),
+    (2304, 2048, 0, False), (6144, 2048, 0, False), (4096, 2048, 0, False), (128, 512, 0, False),
+    (12288, 4096, 0, True), (11008, 4096, 1, False)])
+def test_two_row_blocks(T, N, K, epi, ours):
+    assert (tiles(T, N, K, epi) is None) == ours
+
+
+@pytest.mark.parametrize("T", [1, 64, 65, 192, 193, 256, 385, 1024])
+def test_row_range(T):
+    assert (tiles(T, 2304, 768) is not None) == (T > 192)
+
+
+@pytest.mark.parametrize("N,K", [(2304, 768), (512, 2048), (4096, 4096), (1536, 4096)])
+def test_row_tiles_alone_decide(N, K):
+    """A thread keeps its plans by row tiles: they must not depend on which T asked first."""
+    def asked(first):
+        with ThreadPoolExecutor(1) as one:  # (a thread that has kept none)
+            return one.submit(lambda: [tiles(16 * t + first, N, K) for t in range(12, 30)]).result()
+    assert all(asked(r) == asked(16) for r in range(1, 16))
