@@ -999,7 +999,11 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // equal splits of K.  Blocks are remapped so the row blocks of a weight tile
 // and slice share an XCD (bijective remap): its weights come from HBM once per
 // XCD L2.
-template <int EPI, int MI, int NJ, int WR, int WC, int NB>
+// NTL (FFMI_W_STREAM, one row block: each weight is read once): non-temporal weight
+// copies.  T = 216: K 11008 x N 4096 35.4 us either way, 12288 x 4096 39.2 and 39.1; with
+// two row blocks the second one's reads miss (4096 x 4096 21.3 -> 25.3, gate/up 55.3
+// -> 63.6), which therefore go without the hint.
+template <int EPI, int MI, int NJ, int WR, int WC, int NB, bool NTL>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
     const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wp, uint16_t *__restrict__ Y,
     float *__restrict__ Yf, int T, int N, int KT, int NTILES, int nbm, int S, int xp, int yp,
@@ -1007,6 +1011,7 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
   constexpr int NW = WR * WC, FX = MI * WR, F = FX + NJ * WC;  // waves; fragments of a stage
   constexpr int PW = (F + NW - 1) / NW;                        // DMAs per wave and stage
   static_assert(NB >= 3 && (NB - 1) * PW < 64, "stages in flight");
+  static_assert(!NTL || FX % NW == 0, "a wave's copy is of X or of weights, known to the compiler");
   __shared__ __attribute__((aligned(1024))) h8 lds[NB][F][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1036,10 +1041,11 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
     }
   }
   auto issue = [&](int kt, int slot, int p) {
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kt * step[p]),
-        (__attribute__((address_space(3))) void *)(&lds[slot][min(wave + NW * p, F - 1)][0]), 16, 0,
-        0);
+    const auto from = (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kt * step[p]);
+    const auto to = (__attribute__((address_space(3))) void *)(&lds[slot][min(wave + NW * p, F - 1)][0]);
+    // (cache policy 2: non-temporal)
+    if (NTL && wave + NW * p >= FX) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
+    else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
   };
   const int wm = wave / WC, wn = wave % WC;
   f4 acc[MI][NJ];
@@ -1456,7 +1462,7 @@ static hipError_t run_mid(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, fl
 template <int E>
 static hipError_t run_tiles(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                             size_t ws_bytes, int T, int N, int K, hipStream_t s, bool xp, int yp,
-                            Partials *defer, int wpitch, float lim) {
+                            Partials *defer, bool nt, int wpitch, float lim) {
   constexpr bool paired = epi_paired<E>, f32 = epi_f32<E>;
   const int KT = K / 32, ntiles = (N + 15) / 16 * (paired ? 2 : 1);
   TilePlan p = tile_plan(T, N, K, paired, f32, defer != nullptr && !paired);
@@ -1466,10 +1472,16 @@ static hipError_t run_tiles(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, 
   static_for<kNumTileForms>([&](auto Fc) {
     constexpr int f = decltype(Fc)::value;
     constexpr TileForm F = kTileForms[f];
-    if (p.form == f)
-      hipLaunchKernelGGL((gemm_tile_kernel<E, F.MI, F.NJ, F.WR, F.WC, F.NB>), dim3(p.nbm * p.nbn * p.S),
-                         dim3(F.WR * F.WC * 64), 0, s, X, Wp, Y, ws, T, N, KT, ntiles, p.nbm, p.S,
-                         xp ? 1 : 0, yp, wts, wks, lim);
+    if (p.form != f) return;
+    const dim3 grid(p.nbm * p.nbn * p.S), block(F.WR * F.WC * 64);
+    if constexpr (F.MI * F.WR == 16)  // (the forms of which one row block holds more than 192 rows)
+      if (nt && p.nbm == 1) {
+        hipLaunchKernelGGL((gemm_tile_kernel<E, F.MI, F.NJ, F.WR, F.WC, F.NB, true>), grid, block, 0, s, X, Wp, Y,
+                           ws, T, N, KT, ntiles, p.nbm, p.S, xp ? 1 : 0, yp, wts, wks, lim);
+        return;
+      }
+    hipLaunchKernelGGL((gemm_tile_kernel<E, F.MI, F.NJ, F.WR, F.WC, F.NB, false>), grid, block, 0, s, X, Wp, Y, ws,
+                       T, N, KT, ntiles, p.nbm, p.S, xp ? 1 : 0, yp, wts, wks, lim);
   });
   if (defer && ((p.S > 1 && !paired) || f32)) {
     defer->p = ws, defer->S = p.S, defer->NP = ntiles * 16;
@@ -1523,7 +1535,7 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   const bool aligned = (((uintptr_t)X | (uintptr_t)Wp) & 15) == 0;
   if (mtiles > 4 && K % 32 == 0 && aligned && (xp || E < 2) &&
       use_tiles(T, N, K, paired, epi_f32<E>, defer != nullptr && !paired))
-    return run_tiles<E>(X, Wp, Y, ws, ws_bytes, T, N, K, s, xp, yp, defer, wpitch, lim);
+    return run_tiles<E>(X, Wp, Y, ws, ws_bytes, T, N, K, s, xp, yp, defer, nt, wpitch, lim);
   if (mtiles > 4) {
     const MidPlan p = mid_plan(T, N, K, paired, defer != nullptr && !paired);
 #define FFMI_RUN(M, NW) \

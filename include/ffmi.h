@@ -171,7 +171,9 @@ typedef enum {
 #define FFMI_Y_PACKED 0x20
 /* OR into `epilogue`: the weights are a once-read stream (a model larger than
  * the 256 MiB Infinity Cache): their loads carry the non-temporal hint so they
- * do not evict the KV cache, activations or a small model's weights.  Long-K
+ * do not evict the KV cache, activations or a small model's weights -- in
+ * launches that read each weight once: up to 192 rows, and up to 256 where one
+ * block of rows is taken at a time.  Long-K
  * launches of <= 64 rows then split K over 4 waves instead of 8 (faster under
  * the hint): results within the GEMM tolerance of the default policy, and
  * still independent of T within the <= 64-row regime. */

@@ -60,3 +60,26 @@ def test_tile_edges(T, N, K, epi, monkeypatch):
         assert (np.abs(y[:T] - ref) <= tol).all(), np.abs(y[:T] - ref).max()
     else:
         close16(y[:T], O.linear(X.astype(np.float32), W.astype(np.float32), fp16=1))
+
+
+# the sizes of one row block, in and out of K slices: the hint of a weight stream changes
+# where the weights are kept, not what is computed
+@pytest.mark.parametrize("T,N,K,epi,form", [(193, 4104, 11008, 0, 6), (200, 20008, 512, 0, 6), (193, 8200, 11008, 0, 7),
+                                            (193, 12296, 8192, 0, 9), (200, 12320, 288, 1, 6), (193, 20032, 512, 1, 7),
+                                            (193, 6176, 8192, 1, 9)])
+def test_weight_stream(T, N, K, epi, form):
+    L = F.lib()
+    assert L.ffmi_debug_linear_tiles(T, N, K, epi, None) == form
+    rng = np.random.default_rng(T)
+    X = Buf(pack_act_np(f16(rng.standard_normal((T, K)))))
+    W = [Buf(f16(rng.uniform(-0.05, 0.05, (N, K)))) for _ in range(1 + epi)]
+    Wp = Buf.empty(((1 + epi) * L.ffmi_linear_packed_bytes(N, K) // 2,), np.uint16)
+    F.check(L.ffmi_linear_pack_gate_up(W[0].ptr, W[1].ptr, N, K, Wp.ptr, None) if epi else
+            L.ffmi_linear_pack_weight(W[0].ptr, N, K, Wp.ptr, None))
+    got = []
+    for hint in (0, F.W_STREAM):
+        y = Buf(np.full((T + 1, N), np.nan, np.float16))
+        F.check(L.ffmi_linear(X.ptr, Wp.ptr, y.ptr, T, N, K, epi | F.X_PACKED | hint, None))
+        got.append(y.get())
+        assert np.isfinite(got[-1][:T]).all() and np.isnan(got[-1][T]).all()
+    assert np.array_equal(*(g[:T].view(np.uint16) for g in got))
