@@ -1,7 +1,9 @@
 """The tile form of the dense layers (gemm_tile_kernel, T > 64) where it can go
 wrong: rows and columns past a tile's edge, fewer k-steps than ring stages, every
-tile size, K slices summed by the reduce pass, row-major and packed activations.
+tile size by itself and in K slices summed by the reduce pass, row-major and packed
+activations, both epilogues.
 Tolerance as test_gpu_kernels.close16."""
+import ctypes
 import zlib
 
 import numpy as np
@@ -14,8 +16,8 @@ from test_gpu_kernels import close16, pack_act_np, unpack_act_np
 
 pytestmark = pytest.mark.gpu
 
-# (T, N, K): small ones with one to a few k-steps, then one for each tile size that
-# the plan takes at about this shape (64 columns by 128 rows up to 256 x 256)
+# (T, N, K): small ones with one to a few k-steps, then what the plan gives most tile
+# sizes (FORMS has the others)
 CASES = [(65, 8, 32), (129, 40, 64), (193, 136, 96), (257, 72, 160), (513, 264, 288),
          (170, 2040, 2048), (161, 4104, 4096), (1009, 4104, 1024), (1009, 6152, 1024), (377, 5624, 1024),
          (529, 12296, 1024), (241, 20008, 1024), (1009, 12296, 1024), (313, 20008, 1024), (849, 20008, 1024)]
@@ -60,6 +62,28 @@ def test_tile_edges(T, N, K, epi, monkeypatch):
         assert (np.abs(y[:T] - ref) <= tol).all(), np.abs(y[:T] - ref).max()
     else:
         close16(y[:T], O.linear(X.astype(np.float32), W.astype(np.float32), fp16=1))
+
+
+# (T, N, K, epilogue, form, in K slices): with CASES, every form in and out of slices, for
+# both epilogues (test_linear_plans.py checks that), at remainders of rows and columns
+FORMS = [(849, 10008, 512, 0, 7, False), (513, 20008, 288, 0, 8, False), (289, 8224, 2048, 1, 5, False),
+         (193, 12320, 288, 1, 6, False), (513, 10016, 288, 1, 8, False),
+         (193, 3000, 4096, 0, 2, True), (193, 5624, 5632, 0, 3, True), (129, 5624, 5632, 0, 4, True),
+         (289, 4104, 8192, 0, 5, True), (193, 4104, 11008, 0, 6, True), (193, 8200, 11008, 0, 7, True),
+         (129, 8200, 11008, 0, 8, True), (193, 12296, 8192, 0, 9, True),
+         (65, 64, 1024, 1, 0, True), (65, 3008, 2048, 1, 1, True), (193, 1024, 11008, 1, 2, True),
+         (193, 3008, 5632, 1, 3, True), (129, 3008, 8192, 1, 4, True), (289, 3008, 8192, 1, 5, True),
+         (193, 4128, 5632, 1, 6, True), (193, 4128, 11008, 1, 7, True), (129, 8224, 4096, 1, 8, True),
+         (193, 6176, 8192, 1, 9, True)]
+
+
+@pytest.mark.parametrize("T,N,K,epi,form,sliced", FORMS)
+def test_forms(T, N, K, epi, form, sliced, monkeypatch):
+    monkeypatch.setenv("FFMI_TILE_GEMM", "2")
+    slices = ctypes.c_int()
+    assert F.lib().ffmi_debug_linear_tiles(T, N, K, epi, ctypes.byref(slices)) == form
+    assert (slices.value > 1) == sliced
+    test_tile_edges(T, N * 2 if epi and N > 8000 else N, K, epi, monkeypatch)  # (which halves such N)
 
 
 # the sizes of one row block, in and out of K slices: the hint of a weight stream changes

@@ -39,3 +39,19 @@ def test_row_tiles_alone_decide(N, K):
         with ThreadPoolExecutor(1) as one:  # (a thread that has kept none)
             return one.submit(lambda: [tiles(16 * t + first, N, K) for t in range(12, 30)]).result()
     assert all(asked(r) == asked(16) for r in range(1, 16))
+
+
+@pytest.mark.parametrize("epi", [0, 1])
+def test_every_tile_form_is_tested(epi, monkeypatch):
+    """test_gpu_tile_gemm.py meets every form, in and out of K slices."""
+    import test_gpu_tile_gemm as G
+    monkeypatch.setenv("FFMI_TILE_GEMM", "2")
+    met = {(form, sliced) for _, _, _, e, form, sliced in G.FORMS if e == epi}
+    for T, N, K in G.CASES:
+        N = N // 2 if epi and N > 8000 else N
+        form, slices = tiles(T, N + (-N % 32 if epi else 0), K, epi)
+        met.add((form, slices > 1))
+    assert met == {(form, sliced) for form in range(10) for sliced in (False, True)}
+    for T, N, K, e, form, sliced in G.FORMS:
+        got = tiles(T, N, K, e)
+        assert (got[0], got[1] > 1) == (form, sliced)
