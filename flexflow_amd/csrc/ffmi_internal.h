@@ -73,7 +73,7 @@ __device__ __forceinline__ int packed_lane(int lane, int rows) {
 }
 
 // Layout of the packed per-step metadata blob (device copy of ffmi_batch_desc):
-// [header 32 B][work items, 32 B each][tokens][commits].  The work array sits
+// [header 32 B][work items (WorkDev)][tokens][commits].  The work array sits
 // at a FIXED offset, so a kernel's first two loads (header, its work item)
 // are independent instead of a dependent chain.
 struct BatchHeader {

@@ -716,7 +716,7 @@ __global__ __launch_bounds__(64 * NW, 1) void attention_kernel(
           for (int i = 0; i < TV; ++i) {
             const int e = threadIdx.x + i * NT, dd = e / 4, s8 = (e % 4) * 8;
             if (dd < D && s8 < told) {
-              uint2 *dst = reinterpret_cast<uint2 *>(&sVt[dd][s8]);  // rows are 8-B aligned
+              uint2 *dst = reinterpret_cast<uint2 *>(&sVt[dd][s8]);
               dst[0] = make_uint2(tv[i].x, tv[i].y);
               dst[1] = make_uint2(tv[i].z, tv[i].w);
             }
@@ -997,10 +997,6 @@ __global__ __launch_bounds__(64 * NW, 1) void attention_kernel(
   }
 }
 
-// Query split (attention_kernel QS == 2) of a fused launch with more than 16
-// queries per item: when the (item, head) grid leaves half the CUs idle
-// (TP >= 2 verify steps).  FFMI_ATTN_QSPLIT: 0 off, 1 auto (default), 2
-// always (tests; read at every launch, so a test can switch it).
 // Prompt items (several work items of a request): one workgroup per (two
 // consecutive items of a request, head), its keys through LDS in stages of 128,
 // the next stage on its way while one is computed.  Waves 0-3 attend the first
@@ -1166,11 +1162,6 @@ static bool attn_block() {
   return !e || atoi(e);
 }
 
-// Workgroups that share an item's keys in a step of one query per request: as
-// many as the chip has room for, at least a chunk of 32 keys per wave each (4
-// requests x 16 heads, d = 128, about 1500 keys: 29.8 us with one each, 16.3
-// with four).  With 12 heads x 8 requests and up to 256 keys, or a workgroup on
-// every CU, there is nothing to gain.  FFMI_ATTN_KVSPLIT=0: one (A/B, tests).
 static int attn_cus() {
   static int cus = 0;
   if (!cus) {
@@ -1184,6 +1175,11 @@ static int attn_cus() {
 // a doubled grid still fits one wave of the device's CUs
 static bool attn_split_fits(int wgs) { return 2 * wgs <= attn_cus(); }
 
+// Workgroups that share an item's keys in a step of one query per request: as
+// many as the chip has room for, at least a chunk of 32 keys per wave each (4
+// requests x 16 heads, d = 128, about 1500 keys: 29.8 us with one each, 16.3
+// with four).  With 12 heads x 8 requests and up to 256 keys, or a workgroup on
+// every CU, there is nothing to gain.  FFMI_ATTN_KVSPLIT=0: one (A/B, tests).
 int attn_kv_split(int W, int heads, int max_q, int max_kv) {
   if (max_q != 1 || W <= 0) return 1;
   const int room = std::min(attn_cus(), kKvSplitWgs) / (W * heads), chunks = (max_kv + 31) / 32;
@@ -1192,6 +1188,10 @@ int attn_kv_split(int W, int heads, int max_q, int max_kv) {
   return e && !atoi(e) ? 1 : Z;
 }
 
+// Query split (attention_kernel QS == 2) of a fused launch with more than 16
+// queries per item: when the (item, head) grid leaves half the CUs idle
+// (TP >= 2 verify steps).  FFMI_ATTN_QSPLIT: 0 off, 1 auto (default), 2
+// always (tests; read at every launch, so a test can switch it).
 static bool attn_qsplit(int wgs) {
   const char *e = getenv("FFMI_ATTN_QSPLIT");
   const int mode = e ? atoi(e) : 1;
