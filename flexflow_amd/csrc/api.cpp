@@ -363,14 +363,16 @@ namespace ffmi {
 static bool attn_fused(const ffmi_batch_dev *b) {
   return b->one_item_per_req && b->lds_tail && getenv("FFMI_ATTN_NO_FUSE") == nullptr;
 }
-// (fused, one query tile, d = 64, N <= 1024 columns)
-static bool attn_oproj(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
-  return opa && opa->wo && opa->slab && attn_fused(b) && h->cfg.head_dim == 64 && b->max_q <= 16 &&
-         opa->N % 16 == 0 && opa->N <= 1024 && b->num_tokens <= opa->max_T;
+// a fused launch would project: one query tile, d = 64, N <= 1024 columns
+static bool attn_oproj_fits(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
+  return opa && opa->wo && opa->slab && h->cfg.head_dim == 64 && b->max_q <= 16 && opa->N % 16 == 0 &&
+         opa->N <= 1024 && b->num_tokens <= opa->max_T;
 }
+// (asked for every step: the environment, 0.3 us a question, only where there is a split)
 int attn_key_split(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
-  if (!attn_fused(b) || attn_oproj(h, b, opa)) return 1;
-  return attn_kv_split(b->num_work, h->cfg.num_heads, b->max_q, b->max_kv);
+  if (!b->one_item_per_req || !b->lds_tail || attn_oproj_fits(h, b, opa)) return 1;
+  const int Z = attn_kv_split(b->num_work, h->cfg.num_heads, b->max_q, b->max_kv);
+  return Z > 1 && attn_fused(b) ? Z : 1;
 }
 
 ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv, Partials qkvp,
@@ -422,7 +424,7 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
   }
   // the output projection rides along where its launch allows it; otherwise the
   // caller runs it
-  const bool oproj = attn_oproj(h, b, opa);
+  const bool oproj = fused && attn_oproj_fits(h, b, opa);
   FFMI_HIP(ffmi::launch_attention(b->dev, b->num_work, b->max_q, h->qbuf, h->kc, h->vc,
                                   (uint16_t *)out, heads, d, h->slots, h->cfg.qk_scale, s,
                                   h->cfg.out_layout == 1, fused, b->num_tokens, C,
