@@ -265,6 +265,10 @@ static void rope_table(std::vector<float> &tab, int max_pos, int d, const ffmi_a
 }
 
 extern "C" ffmi_status ffmi_attn_create(const ffmi_attn_cfg *cfg, ffmi_attn **out) {
+  return ffmi::attn_create(cfg, nullptr, out);
+}
+
+ffmi_status ffmi::attn_create(const ffmi_attn_cfg *cfg, const ffmi_attn *first, ffmi_attn **out) {
   FFMI_CHECK(cfg && out, FFMI_ERR_INVALID);
   // head sizes of the reference's kernels: 32 / 64 / 128 for incremental
   // decoding (inc_multihead_self_attention.cu:911-926), 64 / 128 for tree
@@ -302,10 +306,11 @@ extern "C" ffmi_status ffmi_attn_create(const ffmi_attn_cfg *cfg, ffmi_attn **ou
   std::vector<float> tab;
   rope_table(tab, h->slots, cfg->head_dim, cfg);
   const size_t table = tab.size();
-  const size_t split = f32 ? 0 : ffmi::kv_split_floats(cfg->max_requests, cfg->num_heads, cfg->head_dim);
-  if (!f32) tab.resize(table + (size_t)cfg->max_requests * cfg->num_heads, 0.f);  // the counters start at zero
+  const bool own = !f32 && !first;
+  const size_t split = own ? ffmi::kv_split_floats(cfg->max_requests, cfg->num_heads, cfg->head_dim) : 0;
+  if (own) tab.resize(table + (size_t)cfg->max_requests * cfg->num_heads, 0.f);  // the counters start at zero
   if (ok) ok = hipMalloc((void **)&h->rope, (table + split) * sizeof(float)) == hipSuccess;
-  if (!f32) h->zscratch = h->rope + table;
+  if (!f32) h->zscratch = own ? h->rope + table : first->zscratch;
   if (!ok) {
     ffmi_attn_destroy(h);
     ffmi_set_last_error("attention cache alloc", __FILE__, __LINE__);

@@ -181,6 +181,10 @@ hipError_t launch_logit_rows(const void *logits, bool half, size_t ld, const Log
 hipError_t launch_softmax_topk_f32(const float *logits, int T, int V, int k, int32_t *ids,
                                    float *probs, hipStream_t s, int ld = 0);  // (0: ld = V)
 ffmi_status attn_rope_fault(ffmi_attn *h, int from_pos);
+// ffmi_attn_create; first: a handle of the same sizes whose scratch of the key split
+// this one shares (a model's layers, which follow one another on its stream: one
+// allocation per model, not one per layer), and which outlives it
+ffmi_status attn_create(const ffmi_attn_cfg *cfg, const ffmi_attn *first, ffmi_attn **out);
 // workgroups that share an item's keys where attn_forward runs this step
 struct OprojArgs;
 int attn_key_split(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa);

@@ -711,7 +711,7 @@ struct LlamaGPU : public ffmi_model {
       ac.rope_high_freq_factor = c.rope_high_freq_factor;
       ac.rope_original_max_pos = c.rope_original_max_pos;
       ac.out_layout = packed ? 1 : 0;
-      TRY(ffmi_attn_create(&ac, &L.attn));
+      TRY(ffmi::attn_create(&ac, &L == &layers[0] ? nullptr : layers[0].attn, &L.attn));
       int sl = 0;
       ffmi_attn_kv_ptrs(L.attn, nullptr, nullptr, &sl);
       slots = sl;
