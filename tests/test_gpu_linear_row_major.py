@@ -82,8 +82,8 @@ def test_packed_rows_past_the_last(T, epi):
 
 @pytest.mark.parametrize("T,N,k", [(200, 704, 1024), (300, 2050, 256), (200, 4100, 4096), (40, 704, 1024)])
 def test_buffers_off_16_bytes(T, N, k):
-    """Activations and a workspace that are 4 bytes off a 16-byte boundary: as before, in
-    the forms that load them as they are."""
+    """Activations and a workspace that are both 4 bytes off a 16-byte boundary: the forms
+    that load them as they are."""
     L = K.L
     rng = np.random.default_rng(T)
     X, W = f16(rng.standard_normal((T, k))), Buf(f16(rng.uniform(-0.05, 0.05, (N, k))))
@@ -97,6 +97,29 @@ def test_buffers_off_16_bytes(T, N, k):
                                  ctypes.c_void_p(ws.ptr.value + off), n, None))
         got.append(y.get())
     K.close16(got[1], got[0].astype(np.float32))
+
+
+@pytest.mark.parametrize("off_x,off_ws", [(4, 0), (2, 0), (0, 4), (4, 4)])
+@pytest.mark.parametrize("T,N,k", [(200, 4100, 4096), (300, 3000, 288)])
+def test_one_buffer_off_16_bytes(T, N, k, off_x, off_ws):
+    """Each by itself: activations off a 16-byte boundary are packed as others are (the pass
+    loads them as they lie) where the workspace is on one, and a workspace that is off one
+    holds slabs alone."""
+    L = K.L
+    rng = np.random.default_rng(T + off_x)
+    X, W = f16(rng.standard_normal((T, k))), Buf(f16(rng.uniform(-0.05, 0.05, (N, k))))
+    Wp = Buf.empty((L.ffmi_linear_packed_bytes(N, k) // 2,), np.uint16)
+    F.check(L.ffmi_linear_pack_weight(W.ptr, N, k, Wp.ptr, None))
+    n, got = L.ffmi_linear_workspace_bytes(T, N, k, 0), []
+    for ox, ow in ((0, 0), (off_x, off_ws)):
+        x = Buf(np.concatenate([np.zeros(ox // 2, np.float16), X.ravel().view(np.float16), np.zeros(8, np.float16)]))
+        y, ws = Buf(np.full((T, N), np.nan, np.float16)), Buf.empty((n + 64,), np.uint8)
+        F.check(L.ffmi_linear_ws(ctypes.c_void_p(x.ptr.value + ox), Wp.ptr, y.ptr, T, N, k, 0,
+                                 ctypes.c_void_p(ws.ptr.value + ow), n, None))
+        got.append(y.get())
+    K.close16(got[1], got[0].astype(np.float32))
+    if k == 4096 and not off_ws:  # packed both times
+        assert np.array_equal(got[1].view(np.uint16), got[0].view(np.uint16))
 
 
 @pytest.mark.parametrize("T,later", [(168, (168,)), (256, (257, 384))])
