@@ -90,6 +90,8 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
     for (int wi = 0; wi < d->num_work; ++wi) {
       ffmi::WorkDev x{};
       x.w = d->work[wi];
+      // kernels load an item's first row whether or not it has one
+      if (x.w.q_count == 0) x.w.q_start = std::max(0, std::min((int)x.w.q_start, d->num_tokens - 1));
       int clean = INT32_MAX, hi = -1;
       for (int t = 0; t < d->num_tokens; ++t)
         if (d->tokens[t].req == x.w.req && d->tokens[t].store_slot >= 0) {

@@ -3,6 +3,8 @@
 one query, contexts at the edges of its 128-key stages, tree masks over two items, and
 decode steps of more (request, head) pairs than CUs, against the oracle's rows and against
 one workgroup per item."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -97,3 +99,25 @@ def test_decode_of_many_pairs(d):
         infos = [(7, n + step, r, n + step, n + step + 1, 0, 0, 0) for r, n in enumerate(lens)]
         out, qs = c.run(infos, rng=rng)
         c.check(out[:9], np.stack([c.ref_row(qs[t], t, range(i[1] + 1)) for t, i in enumerate(infos)]))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("empty", [[], [(0, 288, 0, 0)], [(0, 288, 0, 288), (1, 288, 0, 0)], [(1, 288, 0, 40)]])
+def test_items_without_queries(d, empty):
+    """Items of no query behind the last row of a full batch, in a block of their own or as
+    another's second: nothing of theirs is read or written."""
+    T, L = 288, K.L
+    c = AttnCase(F.ATTN_INC, heads=32, d=d, max_requests=2, max_seq=320, max_tokens=T)
+    rng = np.random.default_rng(d)
+    toks = (F.TokenInfo * T)(*[F.TokenInfo(3, p, 0, p, p + 1, 0, 0, 0, 0) for p in range(T)])
+    qkv, got = K.Buf(K.f16(rng.standard_normal((T, 3 * c.Hl)))), []
+    for extra in ([], empty):
+        items = [(0, p, 32, p + 32) for p in range(0, T, 32)] + extra
+        desc = F.BatchDesc(T, len(items), 0, 0, toks, (F.AttnWork * len(items))(*[F.AttnWork(*i) for i in items]),
+                           (F.CommitInfo * 1)(), (ctypes.c_uint64 * 1)())
+        F.check(L.ffmi_batch_upload(c.b, ctypes.byref(desc), None))
+        out = K.Buf(np.full((T + 16, c.Hl), np.nan, np.float16))
+        F.check(L.ffmi_attn_inc(c.h, c.b, qkv.ptr, out.ptr, None))
+        got.append(out.get())
+        assert np.isfinite(got[-1][:T]).all() and np.isnan(got[-1][T:]).all()
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
