@@ -378,7 +378,7 @@ static bool attn_oproj_fits(const ffmi_attn *h, const ffmi_batch_dev *b, const O
 // (asked for every step: the environment, 0.3 us a question, only where there is a split)
 int attn_key_split(const ffmi_attn *h, const ffmi_batch_dev *b, const OprojArgs *opa) {
   if (!b->one_item_per_req || !b->lds_tail || attn_oproj_fits(h, b, opa)) return 1;
-  const int Z = attn_kv_split(b->num_work, h->cfg.num_heads, b->max_q, b->max_kv);
+  const int Z = attn_kv_split(b->num_work, h->cfg.num_heads, h->cfg.head_dim, b->max_q, b->max_kv);
   return Z > 1 && attn_fused(b) ? Z : 1;
 }
 

@@ -335,7 +335,7 @@ inline int kv_split_most(int heads) {
 inline size_t kv_split_floats(int requests, int heads, int d) {
   return (size_t)requests * heads * (1 + (size_t)kv_split_most(heads) * (d + 2));
 }
-int attn_kv_split(int W, int heads, int max_q, int max_kv);
+int attn_kv_split(int W, int heads, int d, int max_q, int max_kv);
 hipError_t launch_attention(const char *blob, int W, int max_q, uint16_t *qbuf, uint16_t *kc,
                             uint16_t *vc, uint16_t *out, int heads, int d, int slots, float scale,
                             hipStream_t s, bool out_packed, bool fused, int T, int C,

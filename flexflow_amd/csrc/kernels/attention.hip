@@ -1178,11 +1178,16 @@ static bool attn_split_fits(int wgs) { return 2 * wgs <= attn_cus(); }
 // Workgroups that share an item's keys in a step of one query per request: as
 // many as the chip has room for, at least a chunk of 32 keys per wave each (4
 // requests x 16 heads, d = 128, about 1500 keys: 29.8 us with one each, 16.3
-// with four).  With 12 heads x 8 requests and up to 256 keys, or a workgroup on
-// every CU, there is nothing to gain.  FFMI_ATTN_KVSPLIT=0: one (A/B, tests).
-int attn_kv_split(int W, int heads, int max_q, int max_kv) {
-  if (max_q != 1 || W <= 0) return 1;
-  const int room = std::min(attn_cus(), kKvSplitWgs) / (W * heads), chunks = (max_kv + 31) / 32;
+// with four), where that saves more than the merge's 1.3-2 us.  A round of 8 chunks
+// is 3.3 us at d = 128, 1.5 at 64 and 0.5 at 32, so from how many chunks on it pays
+// depends on d (one workgroup each / shared, 4 requests x 16 heads: d = 128, 300 keys 11.4 /
+// 11.2, 450 11.7 / 10.4; d = 64, 300 keys 8.1 / 8.7, 513 8.6 / 8.5, 700 10.4 / 8.9; d = 32,
+// 513 keys 6.2 / 7.7, 1025 7.2 / 8.1).  With a workgroup on every CU there is nothing to gain.
+// FFMI_ATTN_KVSPLIT=0: one (A/B, tests).
+int attn_kv_split(int W, int heads, int d, int max_q, int max_kv) {
+  const int chunks = (max_kv + 31) / 32;
+  if (max_q != 1 || W <= 0 || chunks <= (d >= 128 ? 8 : d >= 64 ? 16 : 40)) return 1;
+  const int room = std::min(attn_cus(), kKvSplitWgs) / (W * heads);
   const int Z = std::max(1, std::min(std::min(room, (chunks + 7) / 8), kMaxKvSplit));
   const char *e = Z > 1 ? getenv("FFMI_ATTN_KVSPLIT") : nullptr;
   return e && !atoi(e) ? 1 : Z;

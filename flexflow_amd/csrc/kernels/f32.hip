@@ -252,7 +252,16 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
 #define FFMI_F32_GEMM(MT, NT, PF)                                                                \
   hipLaunchKernelGGL((f32_gemm_lds_kernel<MT, NT, PF>), tiles(MT, NT), dim3(256), 0, s, X, W, Y, \
                      T, N, K)
-  if (T <= 16) FFMI_F32_GEMM(1, 1, 4);  // (N = 2048, K = 5632: 13.9 us, 22.7 from registers)
+  // Up to 16 rows: a ring of four k-blocks (N = 2048, K = 5632: 13.9 us, 22.7 from registers)
+  // takes 64 KiB, two workgroups to a CU, which is too few where each has little to
+  // read: of two for short K (N = 32000, T = 8: K = 512 14.3 us, 18.1 with four, 16.0 from
+  // registers; K = 2048, T = 1 48.2 and 46.1), and up to 4 rows, which fall into one access
+  // of a load, registers for the shortest (N = 32000, K = 256, T = 1: 7.6, ring of two 8.8,
+  // of four 11.7; T = 16 10.4, 9.5 and 12.6).
+  if (T <= 4 && K <= 256)
+    hipLaunchKernelGGL((f32_gemm_kernel<1, 1>), tiles(1, 1), dim3(256), 0, s, X, W, Y, T, N, K);
+  else if (T <= 16 && (K <= 512 || (K <= 1024 && N >= 4096))) FFMI_F32_GEMM(1, 1, 2);
+  else if (T <= 16) FFMI_F32_GEMM(1, 1, 4);
   else if (best == 0) FFMI_F32_GEMM(4, 4, 2);
   else if (best == 1) FFMI_F32_GEMM(3, 4, 2);
   else if (best == 2) FFMI_F32_GEMM(2, 4, 2);

@@ -28,7 +28,8 @@ def caches(c):
 
 
 @pytest.mark.parametrize("d", [32, 64, 128])
-@pytest.mark.parametrize("lens", [[255], [256], [511, 3, 300], [513, 512, 40, 257], [1793, 1], [2080]])
+@pytest.mark.parametrize("lens", [[255], [256], [511, 3, 300], [513, 512, 40, 257], [1793, 1], [2080],
+                                  [1279, 1, 1280]])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_split_keys(d, lens, layout, monkeypatch):
     def scenario(oracle):

@@ -49,6 +49,13 @@ def test_linear_forms(T, N, k):
     assert (np.abs(got[0] - ref) <= 2e-6 * mag + 1e-30).all()
 
 
+# both sides of the lines between registers and rings of two and of four k-blocks
+@pytest.mark.parametrize("T,N,k", [(4, 100, 256), (5, 100, 256), (4, 100, 288), (16, 2050, 512), (16, 2050, 544),
+                                   (3, 4096, 1024), (3, 4095, 1024), (16, 4100, 1056)])
+def test_linear_of_few_rows(T, N, k):
+    test_linear_forms(T, N, k)
+
+
 @pytest.mark.parametrize("H", [4, 102, 1020, 1024, 1028, 2048, 4096, 8192, 8196])
 @pytest.mark.parametrize("form", ["plain", "residual", "alias", "unaligned"])
 def test_norm_widths(H, form):
