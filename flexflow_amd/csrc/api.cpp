@@ -494,15 +494,15 @@ extern "C" ffmi_status ffmi_linear_pack_gate_up(const void *Wg, const void *Wu, 
 }
 
 // Row-major activations are packed first where the GEMM is long enough to pay for
-// it (T > 128 and 2.5e9 products): an operand load of row-major rows sends
-// neighbouring lanes to 16 of them, which costs the GEMM 10-35%, the pass about 3 us.
-// T = 168, K = 4096: N = 12288 42.7 -> 37.6 us, gate and up of 11008 66.8 -> 53.3,
-// N = 32000 73.5 -> 63.7; but N = 4096 at T = 130 20.4 -> 23.0 and K = 2048, N = 6144
-// at T = 168 19.8 -> 21.0.
+// it: an operand load of row-major rows sends neighbouring lanes to 16 of them, which
+// costs the GEMM 10-35%, the pass about 3 us.  T > 128 and 2.5e9 products: T = 168,
+// K = 4096: N = 12288 42.7 -> 37.6 us, gate and up of 11008 66.8 -> 53.3, N = 32000 73.5 ->
+// 63.7; but N = 4096 at T = 130 20.4 -> 23.0 and K = 2048, N = 6144 at T = 168 19.8 -> 21.0.
+// Fewer products where the tile kernel takes them: gemm_pack_pays.
 static bool pack_first(int T, int out_dim, int in_dim, int epilogue) {
   const bool pair = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
-  return !(epilogue & FFMI_X_PACKED) && T > 128 && in_dim % 32 == 0 &&
-         (double)T * out_dim * in_dim * (pair ? 2 : 1) >= 2.5e9;
+  if ((epilogue & FFMI_X_PACKED) || T <= 128 || in_dim % 32) return false;
+  return (double)T * out_dim * in_dim * (pair ? 2 : 1) >= 2.5e9 || ffmi::gemm_pack_pays(T, out_dim, in_dim, epilogue);
 }
 // Bytes of the split-K slabs, and of slabs and packed activations behind them.
 // (Planned once a call: about 1 us above 64 rows.  Up to 64 there are no slabs

@@ -35,10 +35,24 @@ hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float
 int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
   const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
   *slices = 1;
-  if (T <= 64 || K % 32 || !use_tiles(T, N, K, paired, false, false)) return -1;
+  const bool xp = (epilogue & FFMI_X_PACKED) != 0;
+  if (T <= 64 || K % 32 || !use_tiles(T, N, K, paired, xp, false, false)) return -1;
   const TilePlan p = tile_plan(T, N, K, paired, false, false);
   *slices = p.S;
   return p.form;
+}
+
+// A k-step of row-major operands takes the tile kernel about 0.12 us longer, all of a
+// slice's one after another: long slices, and unsplit ones on few CUs.  T = 257, M-split
+// kernel (which split them) / tiles / packed and tiles: 2048 x 2048 16.8 / 21.0 / 16.2 us,
+// 4096 x 2048 21.2 / 21.6 / 16.2, 1024 x 1024 10.8 / 12.2 / 10.8, 768 x 768 10.1 / 10.2 / 9.8; but 512 x 4096
+// in 8 slices 14.0 / 12.6 / 15.4 and 4096 x 1376 14.0 / 12.5 / 12.9.
+bool gemm_pack_pays(int T, int N, int K, int epilogue) {
+  const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
+  if (T <= 64 || K % 32 || !use_tiles(T, N, K, paired, false, false, false)) return false;
+  const TilePlan p = tile_plan(T, N, K, paired, false, false);
+  const int steps = (K / 32 + p.S - 1) / p.S;
+  return steps > 48 || (p.S == 1 && steps >= 24 && p.nbm * p.nbn <= 64);
 }
 
 // Packed activation tiles: Xp[mt][kt][lane][8] = X[mt*16 + (lane&15)][kt*32 + 8(lane>>4) + e]

@@ -1282,7 +1282,7 @@ static constexpr TileForm kTileForms[] = {
 static constexpr int kNumTileForms = sizeof(kTileForms) / sizeof(kTileForms[0]);
 struct TilePlan {
   int form, S, nbm, nbn;
-  bool msplit;  // the M-split kernel is the faster one (msplit_ahead)
+  bool msplit[2];  // [packed activations]: the M-split kernel is the faster one (msplit_ahead)
 };
 // Where the M-split kernel stays ahead of the tile forms (us).
 //  * Up to 192 rows, one row block whose non-temporal weight stream is the time (in
@@ -1291,22 +1291,23 @@ struct TilePlan {
 //    T = 82 K 9600 x N 4096 20.0 against 23.7).
 //  * Two blocks of up to 192 rows of a large unpaired weight (12288 x 4096 at T = 384
 //    46.3 against 51.6, 4096 x 11008 44.9 against 47.5; but gate/up 90.6 against 78.8).
-//  * Two such blocks of a small product: narrow waves, all in one round, up to 44
-//    k-steps a slice and no more slices than the tiles take (or few columns, whose
-//    slabs are small).  The tile kernel fills its ring of stages first, which costs it
-//    about 0.5 us and is not won back in so few steps.  At T = 257 and 384: 2304 x 768
-//    7.1 and 7.2 against 7.6, 2048 x 512 5.8 and 6.0 against 6.3 and 6.4, 8192 x 1024 10.8
-//    and 10.3 against 11.2, 512 x 4096 10.2 and 11.3 against 10.8 and 11.8; but 768 x 768, split by
-//    one kernel only, 8.4 and 8.5 against 7.2, and 6144 x 2048, longer slices, 20.1 and 20.1
-//    against 20.0 and 20.2.
-static bool msplit_ahead(int mtiles, int ntiles, int N, int K, bool paired, bool deferred, const TilePlan &t) {
+//  * Two such blocks of a small product of packed activations: narrow waves, all in
+//    one round, up to 44 k-steps a slice and as many slices as the tiles take (so that
+//    row-major and packed activations give the same bits).  The tile kernel fills its
+//    ring of stages first, which costs it about 0.5 us and is not won back in so few
+//    steps.  At T = 257 and 384: 2304 x 768 7.1 and 7.2 against 7.6, 2048 x 512 5.8 and 6.0
+//    against 6.3 and 6.4, 8192 x 1024 10.8 and 10.3 against 11.2, 512 x 4096 10.2 and 11.3 against
+//    10.8 and 11.8; but 768 x 768, split by one kernel only, 8.4 and 8.5 against 7.2, and 6144 x 2048,
+//    longer slices, 20.1 and 20.1 against 20.0 and 20.2.  Row-major operands cost the M-split
+//    kernel more than that (2304 x 768 12.6 against 10.6, 8192 x 1024 16.8 against 13.8).
+static bool msplit_ahead(int mtiles, int ntiles, int N, int K, bool paired, bool xp, bool deferred, const TilePlan &t) {
   if (mtiles <= 12) return true;
   if (mtiles <= 16 || mtiles > 24) return false;
   if ((long)ntiles * 16 * K >= 1L << 25) return !paired && ntiles <= 1024;
+  if (!xp) return false;
   const MidPlan m = mid_plan(mtiles * 16, N, K, paired, deferred && !paired);
   const int steps = (K / 32 + m.S - 1) / m.S;
-  return m.NTW <= 4 && steps <= 44 && (long)m.nblk * m.S * m.mblocks <= 256 &&
-         (m.S <= t.S || (ntiles <= 32 && t.S > 4));
+  return m.NTW <= 4 && steps <= 44 && (long)m.nblk * m.S * m.mblocks <= 256 && m.S == t.S;
 }
 // f32: the output is slabs in any case; deferred: the consumer sums the slabs
 // (else a reduce pass).  Depends on T by its row tiles only, as workspaces are
@@ -1339,11 +1340,11 @@ static TilePlan tile_plan(int T, int N, int K, bool paired, bool f32, bool defer
       if (S > 1) t += 4.0 * S * mb / 4.5;
       for (int d = 0; d < 2; ++d)
         if (t + (S > 1 && !d ? 3.0 : 0.0) < least[d])
-          least[d] = t + (S > 1 && !d ? 3.0 : 0.0), best[d] = TilePlan{f, S, nbm, nbn, false};
+          least[d] = t + (S > 1 && !d ? 3.0 : 0.0), best[d] = TilePlan{f, S, nbm, nbn, {}};
     }
   }
   for (int d = 0; d < 2; ++d)
-    best[d].msplit = msplit_ahead(mtiles, ntiles, N, K, paired, d != 0, best[d]);
+    for (int x = 0; x < 2; ++x) best[d].msplit[x] = msplit_ahead(mtiles, ntiles, N, K, paired, x, d, best[d]);
   at = Found{mtiles, ntiles, KT, flags, {best[0], best[1]}};
   return best[deferred];
 }
@@ -1352,10 +1353,10 @@ static int tile_mode() {
   const char *e = getenv("FFMI_TILE_GEMM");
   return e ? atoi(e) : 1;
 }
-static bool use_tiles(int T, int N, int K, bool paired, bool f32, bool deferred) {
+static bool use_tiles(int T, int N, int K, bool paired, bool xp, bool f32, bool deferred) {
   const int mode = tile_mode();
   if (mode != 1) return mode == 2;
-  return T > 192 && !tile_plan(T, N, K, paired, f32, deferred).msplit;
+  return T > 192 && !tile_plan(T, N, K, paired, f32, deferred).msplit[xp];
 }
 
 // split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;
@@ -1370,7 +1371,8 @@ static inline size_t gemm_slab_bytes(int T, int N, int K, int epilogue, bool f32
   const int ntiles = (N + 15) / 16 * (epilogue ? 2 : 1);
   int S = 1;
   for (int deferred = f32 ? 1 : 0; deferred <= (epilogue ? 0 : 1); ++deferred) {
-    const bool tiles = K % 32 == 0 && use_tiles(T, N, K, epilogue != 0, f32, deferred);
+    // (of row-major ones: where packed ones go elsewhere, it is with as many slices)
+    const bool tiles = K % 32 == 0 && use_tiles(T, N, K, epilogue != 0, false, f32, deferred);
     if (tiles) S = std::max(S, tile_plan(T, N, K, epilogue != 0, f32, deferred).S);
     if (!tiles || !aligned) S = std::max(S, mid_plan(T, N, K, epilogue, deferred).S);
   }
@@ -1534,7 +1536,7 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   // (the tile kernel's copies to LDS are of 16 bytes)
   const bool aligned = (((uintptr_t)X | (uintptr_t)Wp) & 15) == 0;
   if (mtiles > 4 && K % 32 == 0 && aligned && (xp || E < 2) &&
-      use_tiles(T, N, K, paired, epi_f32<E>, defer != nullptr && !paired))
+      use_tiles(T, N, K, paired, xp, epi_f32<E>, defer != nullptr && !paired))
     return run_tiles<E>(X, Wp, Y, ws, ws_bytes, T, N, K, s, xp, yp, defer, nt, wpitch, lim);
   if (mtiles > 4) {
     const MidPlan p = mid_plan(T, N, K, paired, defer != nullptr && !paired);

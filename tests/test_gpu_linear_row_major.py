@@ -60,6 +60,14 @@ def test_row_major(T, N, k, epi):
     H.hipGraphExecDestroy(ex), H.hipGraphDestroy(g)
 
 
+# products that the tile kernel takes row-major and the M-split kernel packed (short
+# slices), and shorter ones that are packed first
+@pytest.mark.parametrize("T,N,k,epi", [(300, 2304, 768, 0), (257, 512, 4096, 0), (384, 2816, 1024, 1), (300, 1000, 256, 0),
+                                       (350, 72, 4096, 0), (257, 2040, 2080, 0), (270, 1000, 1024, 0), (193, 768, 768, 0)])
+def test_row_major_of_few_steps(T, N, k, epi):
+    test_row_major(T, N, k, epi)
+
+
 @pytest.mark.parametrize("T", [1, 3, 8, 9, 15, 16, 17, 24, 33, 64])
 @pytest.mark.parametrize("epi", [0, 1])
 def test_packed_rows_past_the_last(T, epi):

@@ -15,16 +15,35 @@ def tiles(T, N, K, epi=0):
     return (form, s.value) if form >= 0 else None
 
 
-# two blocks of up to 192 rows: short slices in narrow waves stay with the M-split kernel
+# two blocks of up to 192 rows: short slices of packed activations stay with the M-split kernel
 @pytest.mark.parametrize("T", [257, 300, 352, 384])
 @pytest.mark.parametrize("N,K,epi,ours", [
     (2304, 768, 0, True), (2048, 512, 0, True), (8192, 1024, 0, True), (1024, 256, 0, True), (2816, 1024, 1, True),
     (512, 4096, 0, True), (256, 2048, 0, True), (128, 2048, 0, True), (64, 4096, 0, True),
     (768, 768, 0, False), (768, 3072, 0, False), (1024, 1024, 0, False), (32000, 768, 0, False),
-    (2304, 2048, 0, False), (6144, 2048, 0, False), (4096, 2048, 0, False), (128, 512, 0, False),
-    (12288, 4096, 0, True), (11008, 4096, 1, False)])
+    (2304, 2048, 0, False), (6144, 2048, 0, False), (4096, 2048, 0, False), (128, 512, 0, False)])
 def test_two_row_blocks(T, N, K, epi, ours):
-    assert (tiles(T, N, K, epi) is None) == ours
+    assert (tiles(T, N, K, epi | F.X_PACKED) is None) == ours
+    assert tiles(T, N, K, epi) is not None
+
+
+@pytest.mark.parametrize("flags", [0, F.X_PACKED])
+@pytest.mark.parametrize("T,N,K,epi,ours", [(257, 12288, 4096, 0, True), (384, 4096, 11008, 0, True),
+                                            (384, 11008, 4096, 1, False), (385, 12288, 4096, 0, False)])
+def test_large_weights(T, N, K, epi, ours, flags):
+    assert (tiles(T, N, K, epi | flags) is None) == ours
+
+
+# row-major activations are packed first: workspace for more than the slabs
+@pytest.mark.parametrize("T,N,K,epi,packs", [
+    (257, 2048, 2048, 0, True), (300, 4096, 2048, 0, True), (257, 1024, 1024, 0, True), (193, 768, 768, 0, True),
+    (1024, 768, 768, 0, False), (300, 512, 4096, 0, False), (300, 4096, 1376, 0, False), (300, 2304, 768, 0, False),
+    (192, 2048, 2048, 0, False), (168, 12288, 4096, 0, True), (128, 12288, 4096, 0, False)])
+def test_packed_first(T, N, K, epi, packs):
+    L = F.lib()
+    slabs = L.ffmi_linear_workspace_bytes(T, N, K, epi | F.X_PACKED)
+    both = (slabs + 255) // 256 * 256 + L.ffmi_packed_activation_bytes(T, K)
+    assert L.ffmi_linear_workspace_bytes(T, N, K, epi) == (both if packs else slabs)
 
 
 @pytest.mark.parametrize("T", [1, 64, 65, 192, 193, 256, 385, 1024])
@@ -37,7 +56,7 @@ def test_row_tiles_alone_decide(N, K):
     """A thread keeps its plans by row tiles: they must not depend on which T asked first."""
     def asked(first):
         with ThreadPoolExecutor(1) as one:  # (a thread that has kept none)
-            return one.submit(lambda: [tiles(16 * t + first, N, K) for t in range(12, 30)]).result()
+            return one.submit(lambda: [tiles(16 * t + first, N, K, F.X_PACKED) for t in range(12, 30)]).result()
     assert all(asked(r) == asked(16) for r in range(1, 16))
 
 
