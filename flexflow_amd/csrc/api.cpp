@@ -184,11 +184,19 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
     b->max_q = std::max(b->max_q, (int)d->work[wi].q_count);
     b->max_kv = std::max(b->max_kv, (int)d->work[wi].kv_len);
   }
-  // (a request's place in the key split's scratch is for one item)
-  if (b->max_q == 1 && b->max_kv > 256)
-    for (int wi = 1; wi < d->num_work; ++wi)
-      for (int wj = 0; wj < wi; ++wj)
-        if (d->work[wi].req == d->work[wj].req) b->max_kv = 0;
+  // (a request's place in the key split's scratch is for one item; more than 128 items
+  // are never split)
+  if (b->max_q == 1 && b->max_kv > 256 && d->num_work <= 128) {
+    uint64_t seen[16] = {};
+    for (int wi = 0; wi < d->num_work; ++wi) {
+      const unsigned r = (unsigned)d->work[wi].req;
+      if (r >= 1024 || (seen[r >> 6] >> (r & 63) & 1)) {
+        b->max_kv = 0;
+        break;
+      }
+      seen[r >> 6] |= 1ull << (r & 63);
+    }
+  }
   b->commit_overlap = false;
   for (int c = 0; c < d->num_commits && !b->commit_overlap; ++c)
     for (int t = 0; t < d->num_tokens; ++t)

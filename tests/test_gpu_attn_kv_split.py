@@ -98,3 +98,24 @@ def test_two_streams_on_one_handle(heads, lens):
         assert want.any()
         for o in outs[1:]:
             assert np.array_equal(o.get()[:len(g)].view(np.uint16), want)
+
+
+def test_one_request_in_two_items():
+    """A request's keys are split where one item has them: with the request in two items
+    (apart, over keys of earlier steps) each has a workgroup of its own."""
+    d, n, L = 128, 900, K.L
+    c = AttnCase(F.ATTN_INC, heads=2, d=d, max_seq=1024, max_tokens=1024)
+    rng = np.random.default_rng(5)
+    for r in (0, 1):
+        c.run([(3, p, r, p, p + 1, 0, 0, 0) for p in range(n)], rng=rng)
+    qkv, outs = K.Buf(K.f16(rng.standard_normal((3, 3 * c.Hl)))), []
+    for reqs in ((0, 1, 0), (0, 1)):
+        infos = [(7, n - 1, r, -1, n, 0, 0, 0) for r in reqs]  # (nothing is stored)
+        out = K.Buf(np.full((16, c.Hl), np.nan, np.float16))
+        step_on(c, c.b, None, infos, qkv, out)
+        outs.append(out.get()[:len(reqs)].astype(np.float32))
+        assert np.isfinite(outs[-1]).all()
+    # shared and unshared keys: the other order of sums, one rounding to fp16
+    assert (np.abs(outs[0][:2] - outs[1]) <= 2.0 ** -10 * np.abs(outs[1]) + 2e-6).all()
+    # the third row is another query of the first request
+    assert not np.array_equal(outs[0][0], outs[0][2])
