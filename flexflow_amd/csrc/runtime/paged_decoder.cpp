@@ -332,7 +332,8 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
   } else {
     FFMI_TRY(enqueue(sample));
   }
-  if (!sample) FFMI_TRY(logit_rows.begin(logits, false, Vp, nullptr, n, V, stream));
+  // (the step is on the stream: it is waited for and counted whatever becomes of its rows)
+  const ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream);
   FFMI_HIP(hipStreamSynchronize(stream));
   if (recurrent)
     for (int t = 0; t < bc.num_tokens; ++t) {
@@ -341,7 +342,7 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
         states.done(tk.request_index, tk.abs_depth_in_request + 1, tk.token_id);
     }
   if (dbg) dbg_T = step.T, dbg_R = step.R;
-  return FFMI_OK;
+  return rows_st;
 }
 
 // the output rows of a generation step are the requests' last tokens: only
