@@ -162,7 +162,7 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
                            hipStream_t s);
 hipError_t launch_rmsnorm_f32(const float *x1, const float *x2, const float *w, float *res_out,
                               float *out, int T, int H, float eps, hipStream_t s,
-                              const char *gather = nullptr);
+                              const char *gather = nullptr, const int32_t *rows = nullptr);
 hipError_t launch_silu_mul_f32(const float *A, const float *B, float *out, int T, int F,
                                size_t lda, size_t ldb, hipStream_t s);
 hipError_t launch_kv_update_f32(const char *blob, int T, int C, const float *qkv, const float *rope,
@@ -285,7 +285,9 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
                           uint16_t *res_out, uint16_t *out, int T, int H, float eps,
                           hipStream_t s, bool out_packed = false, Partials x2p = {}, const char *gather = nullptr,
                           char *blob_dst = nullptr, size_t blob_bytes = 0,
-                          const int32_t *gather_prev = nullptr);
+                          const int32_t *gather_prev = nullptr,
+                          // out row i (of T) from input row rows[i] of T_in; res_out is not written
+                          const int32_t *rows = nullptr, int T_in = 0);
 // FFMI_FAULT_RESID_ROUND negative control (tests only; process-wide)
 void set_norm_fault(bool on);
 hipError_t launch_embedding(const char *blob, int T, const uint16_t *table,

@@ -298,9 +298,9 @@ __device__ __forceinline__ V block_reduce256(V v, V *sh, Op op) {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void f32_rmsnorm_kernel(
     const float *x1, const float *__restrict__ x2, const float *__restrict__ w, float *res_out,
-    float *__restrict__ out, int H, float eps, const char *__restrict__ gather) {
+    float *__restrict__ out, int H, float eps, const char *__restrict__ gather, const int32_t *__restrict__ rows) {
   __shared__ double sh[4];
-  const int row = blockIdx.x;
+  const int row = rows ? rows[blockIdx.x] : blockIdx.x;  // (rows: the output's row i is of input row rows[i])
   const float *a = gather ? x1 + (size_t)batch_view(gather).tokens[row].token_id * H
                           : x1 + (size_t)row * H;
   const float *b = x2 ? x2 + (size_t)row * H : nullptr;
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256) void f32_rmsnorm_kernel(
   // (res_out may alias x1: read back this thread's own sums, never x1 + x2 again)
   for (int j = threadIdx.x; j < H; j += blockDim.x) {
     const float v = res_out ? res_out[(size_t)row * H + j] : (b ? __fadd_rn(a[j], b[j]) : a[j]);
-    out[(size_t)row * H + j] = __fmul_rn(__fmul_rn(v, rms), w[j]);
+    out[(size_t)blockIdx.x * H + j] = __fmul_rn(__fmul_rn(v, rms), w[j]);
   }
 }
 
@@ -329,9 +329,9 @@ __global__ __launch_bounds__(256) void f32_rmsnorm_kernel(
 template <int NV>
 __global__ __launch_bounds__(256) void f32_rmsnorm_vec_kernel(
     const float *x1, const float *__restrict__ x2, const float *__restrict__ w, float *res_out,
-    float *__restrict__ out, int H, float eps, const char *__restrict__ gather) {
+    float *__restrict__ out, int H, float eps, const char *__restrict__ gather, const int32_t *__restrict__ rows) {
   __shared__ double sh[4];
-  const size_t row = (size_t)blockIdx.x * H;
+  const size_t row = (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * H;
   const float *a = gather ? x1 + (size_t)batch_view(gather).tokens[blockIdx.x].token_id * H : x1 + row;
   f4 v[NV], y[NV], g[NV];
 #pragma unroll
@@ -363,27 +363,28 @@ __global__ __launch_bounds__(256) void f32_rmsnorm_vec_kernel(
     f4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = __fmul_rn(__fmul_rn(v[i][e], rms), g[i][e]);
-    *reinterpret_cast<f4 *>(out + row + j) = o;
+    *reinterpret_cast<f4 *>(out + (size_t)blockIdx.x * H + j) = o;
   }
 }
 
 hipError_t launch_rmsnorm_f32(const float *x1, const float *x2, const float *w, float *res_out,
                               float *out, int T, int H, float eps, hipStream_t s,
-                              const char *gather) {
+                              const char *gather, const int32_t *rows) {
+  if (rows && (gather || res_out)) return hipErrorInvalidValue;
   if (T <= 0) return hipSuccess;
   // rows and buffers of 16-byte pieces, up to 8 per thread (more would spill)
   const bool vec = H > 0 && H % 4 == 0 && H <= 8192 &&
                    (((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)res_out | (uintptr_t)out) & 15) == 0;
   if (!vec)
-    hipLaunchKernelGGL(f32_rmsnorm_kernel, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather);
+    hipLaunchKernelGGL(f32_rmsnorm_kernel, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
   else if (H <= 1024)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<1>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather);
+    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<1>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
   else if (H <= 2048)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<2>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather);
+    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<2>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
   else if (H <= 4096)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<4>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather);
+    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<4>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
   else
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<8>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather);
+    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<8>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
   return hipGetLastError();
 }
 

@@ -88,16 +88,20 @@ __device__ __forceinline__ T block_sum(T v, T *scratch) {
 //   4 / 5: 1 / 2 with the FFMI_FAULT_RESID_ROUND negative control (tests
 //   only): the sum of squares takes the UNROUNDED fp32 residual sum, where
 //   residual_rms_norm_kernels.cu:112-114 squares the half-rounded one
-template <int NT, int MAXC, int MAXS, int SRC>
+// ROWS: the output's row i is of input row rows[i] of the T_in (a prompt step's final
+// norm, of the rows whose logits somebody reads; the residual is not written)
+template <int NT, int MAXC, int MAXS, int SRC, bool ROWS = false>
 __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     const uint16_t *__restrict__ x1, const uint16_t *__restrict__ x2,
     const uint16_t *__restrict__ w, uint16_t *__restrict__ res_out,
     uint16_t *__restrict__ out, int H, float eps, int out_packed,
     const float *__restrict__ x2p, int pS, int pNP, const char *__restrict__ gather,
-    uint4 *__restrict__ blob_dst, int blob_n16, const int32_t *__restrict__ gprev) {
+    uint4 *__restrict__ blob_dst, int blob_n16, const int32_t *__restrict__ gprev,
+    const int32_t *__restrict__ rows, int T_in) {
   __shared__ double scratch[NT / 64];
-  const int row = blockIdx.x;
-  const int T = gridDim.x;
+  static_assert(!ROWS || SRC <= 2, "rows of a plain or residual norm");
+  const int row = ROWS ? rows[blockIdx.x] : blockIdx.x;
+  const int T = ROWS ? T_in : gridDim.x;
   const int nchunk = H >> 3;
   // gather: x1 is the embedding table and row t reads its token's row (the
   // embedding lookup fused into the first layer's norm; res_out gets the copy)
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
 #pragma unroll
         for (int q = 0; q < 4; ++q) r[q] = __hadd2(pa[q], pb[q]);  // correctly rounded
         xa = *reinterpret_cast<uint4 *>(r);
-        *reinterpret_cast<uint4 *>(res_out + (size_t)row * H + ch * 8) = xa;
+        if constexpr (!ROWS) *reinterpret_cast<uint4 *>(res_out + (size_t)row * H + ch * 8) = xa;
       } else if (S == 3) {
         *reinterpret_cast<uint4 *>(res_out + (size_t)row * H + ch * 8) = xa;
       }
@@ -216,7 +220,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
         float y = h2f_(f2h_(__fmul_rn(h2f_(e[q]), rms)));
         o8[q] = f2h_(__fmul_rn(y, h2f_(we[q])));
       }
-      uint16_t *dst = out_packed ? out + act_packed_off(row, ch * 8, H) : out + (size_t)row * H + ch * 8;
+      const int at = ROWS ? blockIdx.x : row;
+      uint16_t *dst = out_packed ? out + act_packed_off(at, ch * 8, H) : out + (size_t)at * H + ch * 8;
       *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<uint4 *>(o8);
     }
   }
@@ -230,7 +235,9 @@ void set_norm_fault(bool on) { g_norm_fault = on; }
 hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t *w,
                           uint16_t *res_out, uint16_t *out, int T, int H, float eps,
                           hipStream_t s, bool out_packed, Partials x2p, const char *gather,
-                          char *blob_dst, size_t blob_bytes, const int32_t *gather_prev) {
+                          char *blob_dst, size_t blob_bytes, const int32_t *gather_prev, const int32_t *rows,
+                          int T_in) {
+  if (rows && (gather || T_in <= 0)) return hipErrorInvalidValue;
   if (gather && (x2 || x2p.S > 0 || !res_out)) return hipErrorInvalidValue;
   if (blob_dst && (!gather || blob_bytes > (size_t)1 << 30 || (uintptr_t)gather % 16 ||
                    (uintptr_t)blob_dst % 16))
@@ -254,10 +261,20 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
   const int src = gather ? 3 : pp ? 2 : x2 ? 1 : 0;
   const int ms = !pp || x2p.S <= 1 ? 1 : x2p.S <= 2 ? 2 : x2p.S <= 4 ? 4 : x2p.S <= 8 ? 8
                : x2p.S <= 12 ? 12 : 16;
-#define FFMI_RMS3(NT, MC, MS, SR)                                                              \
-  hipLaunchKernelGGL((rmsnorm_kernel<NT, MC, MS, SR>), dim3(T), dim3(NT), 0, s, x1, x2, w,    \
+#define FFMI_RMS4(NT, MC, MS, SR, RW)                                                          \
+  hipLaunchKernelGGL((rmsnorm_kernel<NT, MC, MS, SR, RW>), dim3(T), dim3(NT), 0, s, x1, x2, w, \
                      res_out, out, H, eps, op, pp, x2p.S, x2p.NP, gather,               \
-                     reinterpret_cast<uint4 *>(blob_dst), blob_n16, gather_prev)
+                     reinterpret_cast<uint4 *>(blob_dst), blob_n16, gather_prev, rows, T_in)
+#define FFMI_RMS3(NT, MC, MS, SR)                                    \
+  do {                                                               \
+    if constexpr (SR <= 2) {                                         \
+      if (rows) {                                                    \
+        FFMI_RMS4(NT, MC, MS, SR, true);                             \
+        break;                                                       \
+      }                                                              \
+    }                                                                \
+    FFMI_RMS4(NT, MC, MS, SR, false);                                \
+  } while (0)
 #define FFMI_RMS(NT, MC)                                   \
   do {                                                     \
     if (src == 0) FFMI_RMS3(NT, MC, 1, 0);                 \
@@ -274,7 +291,7 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
     else if (src == 1) FFMI_RMS3(NT, MC, 1, 1);            \
     else FFMI_RMS3(NT, MC, 1, 3);                          \
   } while (0)
-  if (g_norm_fault && (src == 1 || src == 2)) {  // negative control (tests only)
+  if (g_norm_fault && !rows && (src == 1 || src == 2)) {  // negative control (tests only)
 #define FFMI_RMSF(NT)                                      \
   do {                                                     \
     if (src == 1) FFMI_RMS3(NT, 1, 1, 4);                  \
@@ -303,6 +320,7 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
 #undef FFMI_RMS_NOSLAB
 #undef FFMI_RMS
 #undef FFMI_RMS3
+#undef FFMI_RMS4
   return hipGetLastError();
 }
 

@@ -49,6 +49,13 @@ struct LlamaF32 : public ffmi_model {
   int32_t *res_d = nullptr;  // [ids (T*k) | probs (T*k)] of a step
   int32_t *res_h = nullptr;  // pinned copy
   LogitRows logit_rows;      // run_inc_logits
+  // rows whose logits the caller reads, where few of a long step (llama_gpu.cpp): the
+  // step's tail takes those, eager.  201 tokens of which 4 rows are read, 32000 x 2048:
+  // lm_head 331 -> 45 us
+  int32_t *rows_h = nullptr;  // [Tm], behind res_h
+  std::vector<int> last_rows;
+  bool few_rows = false;
+  int tail_n = 0;
   ffmi_batch_dev *batch = nullptr;
   PackedStep ps;
   std::vector<void *> allocs;
@@ -201,8 +208,9 @@ struct LlamaF32 : public ffmi_model {
     TRY(alloc(&mlp, (size_t)Tm * Fl));
     TRY(alloc(&logits, (size_t)Tm * V));
     TRY(alloc(&res_d, (size_t)Tm * 4 * 2));
-    FFMI_HIP(hipHostMalloc((void **)&res_h, (size_t)Tm * 4 * 2 * sizeof(int32_t),
-                           hipHostMallocDefault));
+    FFMI_HIP(hipHostMalloc((void **)&res_h, (size_t)Tm * (4 * 2 + 1) * sizeof(int32_t),
+                           hipHostMallocCoherent | hipHostMallocMapped));
+    rows_h = res_h + (size_t)Tm * 4 * 2;
     // weights: full tensors through a staging buffer, this shard's rows /
     // columns copied out
     float *tmp = nullptr;
@@ -318,18 +326,26 @@ struct LlamaF32 : public ffmi_model {
       FFMI_HIP(launch_gemm_f32(mlp, L.wd, proj, T, H, Fl, stream));
       TRY(allreduce(proj, (size_t)T * H));
     }
-    FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, res, h, T, H, eps, stream));
-    FFMI_HIP(launch_gemm_f32(h, lm, logits, T, V, H, stream));
-    float *probs_d = reinterpret_cast<float *>(res_d + (size_t)T * k);
-    FFMI_HIP(launch_softmax_topk_f32(logits, T, V, k, res_d, probs_d, stream));
-    FFMI_HIP(hipMemcpyAsync(res_h, res_d, (size_t)T * k * 8, hipMemcpyDeviceToHost, stream));
+    const int n = tail_n;
+    if (n == 0) return FFMI_OK;
+    FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, few_rows ? nullptr : res, h, n, H, eps, stream, nullptr,
+                                few_rows ? rows_h : nullptr));
+    FFMI_HIP(launch_gemm_f32(h, lm, logits, n, V, H, stream));
+    if (k == 0) return FFMI_OK;  // logits only
+    float *probs_d = reinterpret_cast<float *>(res_d + (size_t)n * k);
+    FFMI_HIP(launch_softmax_topk_f32(logits, n, V, k, res_d, probs_d, stream));
+    FFMI_HIP(hipMemcpyAsync(res_h, res_d, (size_t)n * k * 8, hipMemcpyDeviceToHost, stream));
 #undef TRY
     return FFMI_OK;
   }
 
-  ffmi_status forward(int k) {
+  // n >= 0: rows[0, n) are the only ones that the caller reads; k = 0: logits only
+  ffmi_status forward(int k, const int *rows = nullptr, int n = -1) {
     const int T = (int)ps.tokens.size();
-    FFMI_CHECK(k >= 1 && k <= 4, FFMI_ERR_INVALID);
+    FFMI_CHECK(k >= (n >= 0 ? 0 : 1) && k <= 4, FFMI_ERR_INVALID);
+    few_rows = n >= 0 && T > 64 && 2 * n <= T && P == 1 && !dbg;
+    tail_n = few_rows ? n : T;
+    if (few_rows && n > 0) memcpy(rows_h, rows, n * sizeof(int32_t));
     ffmi_batch_desc desc;
     ps.desc(&desc);
     for (int t = 0; t < T; ++t)
@@ -340,7 +356,7 @@ struct LlamaF32 : public ffmi_model {
     if (T == 0) return FFMI_OK;
     // graphed at TP = 1 (the host-synchronising local group and the
     // transports stay eager here: this path is not the measured one)
-    const bool graph = use_graphs && !dbg && P == 1;
+    const bool graph = use_graphs && !dbg && P == 1 && !few_rows;
     if (graph) {
       const auto key = std::make_tuple(T, batch->num_work, batch->num_commits, k, bytes);
       auto it = graphs.find(key);
@@ -395,9 +411,18 @@ struct LlamaF32 : public ffmi_model {
     if (mode != FFMI_MODEL_INC) return FFMI_ERR_INVALID;
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
-    ffmi_status st = forward(1);
+    last_rows.clear();
+    for (int t = 0; t < bc.num_tokens; ++t)
+      if (t + 1 == bc.num_tokens || bc.tokensInfo[t + 1].request_index != bc.tokensInfo[t].request_index)
+        last_rows.push_back(t);
+    ffmi_status st = forward(1, last_rows.data(), (int)last_rows.size());
     if (st != FFMI_OK) return st;
-    memcpy(ir->token_ids, res_h, bc.num_tokens * sizeof(int32_t));
+    if (few_rows) {
+      std::fill_n(ir->token_ids, bc.num_tokens, -1);
+      for (int i = 0; i < tail_n; ++i) ir->token_ids[rows_h[i]] = res_h[i];
+    } else {
+      memcpy(ir->token_ids, res_h, bc.num_tokens * sizeof(int32_t));
+    }
     return FFMI_OK;
   }
   int vocab_size() const override { return V; }
@@ -406,9 +431,9 @@ struct LlamaF32 : public ffmi_model {
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
     for (int i = 0; i < n; ++i) FFMI_CHECK(rows[i] >= 0 && rows[i] < bc.num_tokens, FFMI_ERR_INVALID);
-    ffmi_status st = forward(1);
+    ffmi_status st = forward(0, rows, n);
     if (st != FFMI_OK || bc.num_tokens == 0) return st;
-    st = logit_rows.begin(logits, false, V, rows, n, V, stream);
+    st = logit_rows.begin(logits, false, V, few_rows ? nullptr : rows, n, V, stream);
     return st == FFMI_OK ? logit_rows.finish(out) : st;
   }
   ffmi_status run_tree(const TreeVerifyBatchConfig &bc, InferenceResult *ir) override {

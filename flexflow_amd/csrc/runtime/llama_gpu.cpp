@@ -132,6 +132,14 @@ struct LlamaGPU : public ffmi_model {
   bool result_copy = getenv("FFMI_RESULT_COPY") && atoi(getenv("FFMI_RESULT_COPY")) != 0;
   float *probs_h = nullptr;
   LogitRows logit_rows;  // run_inc_logits
+  // The rows whose logits a step's caller reads, where they are few of a long step (a
+  // prompt's last token; what a replay asks for): the final norm, lm_head and sampling
+  // run on those only.  1024 tokens of which one row is read, 32000 x 2048: 129 + 58 + 8 us
+  // -> 30 + 9 + 3; x 4096: 224 + 58 -> 45 + 9.  Up to 64 tokens lm_head is bound by its weights
+  // whatever the rows (and the step is one graph), so those take every row.
+  int32_t *rows_h = nullptr;  // [Tm], behind ids_h, read by the norm's launch
+  bool few_rows = false;      // this step's tail takes rows_h[0, few_n)
+  int few_n = 0;
   ffmi_batch_dev *batch = nullptr;
   PackedStep ps;
   std::vector<void *> allocs;
@@ -607,8 +615,9 @@ struct LlamaGPU : public ffmi_model {
     // coherent (uncached) pinned memory: the sampling kernel's stores go
     // straight over PCIe and are visible to the host once the stream has
     // synchronised, whatever HIP_HOST_COHERENT says
-    FFMI_HIP(hipHostMalloc((void **)&ids_h, (size_t)kChain * Tm * 4 * 2 * sizeof(int32_t),
+    FFMI_HIP(hipHostMalloc((void **)&ids_h, ((size_t)kChain * Tm * 4 * 2 + Tm) * sizeof(int32_t),
                            hipHostMallocCoherent | hipHostMallocMapped));
+    rows_h = ids_h + (size_t)kChain * Tm * 4 * 2;
     if (mode == FFMI_MODEL_BEAM) TRY(alloc(&ids_dev, (size_t)kChain * Tm * 4));
     chain_batch[0] = batch;
     // the chained beam steps' staging batches, created here rather than on a
@@ -913,15 +922,19 @@ struct LlamaGPU : public ffmi_model {
   struct StepTime { long n = 0; double launch = 0, gpu = 0, wait = 0, total = 0; };
   std::map<int, StepTime> st_sum;
   int st_T = 0;
-  ffmi_status forward(int k) {
-    ffmi_status st = forward_launch(k);
+  ffmi_status forward(int k, const int *rows = nullptr, int n = -1) {
+    ffmi_status st = forward_launch(k, rows, n);
     if (st != FFMI_OK) return st;
     return forward_finish();
   }
 
-  ffmi_status forward_launch(int k) {
+  // n >= 0: rows[0, n) are the only ones that the caller reads; k = 0: logits only
+  ffmi_status forward_launch(int k, const int *rows = nullptr, int n = -1) {
     inflight = false;
     const int T = (int)ps.tokens.size();
+    few_rows = n >= 0 && T > 64 && 2 * n <= T && o.tp_size == 1 && !dbg;
+    few_n = few_rows ? n : 0;
+    if (few_rows && n > 0) memcpy(rows_h, rows, n * sizeof(int32_t));
     if (step_timing) {
       if (!st_ev[0]) {
         FFMI_HIP(hipEventCreate(&st_ev[0]));
@@ -946,11 +959,11 @@ struct LlamaGPU : public ffmi_model {
     ffmi_status st = ffmi::batch_stage(batch, &desc, &bytes);
     if (st != FFMI_OK) return st;
     if (T == 0) return FFMI_OK;
-    probs_h = reinterpret_cast<float *>(ids_h + cur_slot * slot_ints() + (size_t)T * k);
+    probs_h = reinterpret_cast<float *>(ids_h + cur_slot * slot_ints() + (size_t)(few_rows ? few_n : T) * k);
     // graphed: small steps, and tree-verify steps of one work item per
     // request (a fixed shape while the batch is full: T = 168 for 8 requests
     // of 21 tree tokens); prefill blocks stay eager (one-off shapes)
-    const bool graph = use_graphs && !dbg && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
+    const bool graph = use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
                        (o.tp_size == 1 || peer || rccl || ffmi::comm_size(o.comm) == 1) &&
                        !prof_on(0, T) &&
                        !prof_on(c.num_layers / 2, T);
@@ -1250,6 +1263,8 @@ struct LlamaGPU : public ffmi_model {
       if (dbg && !arn) TRY(dbg_gemm_out(FFMI_DBG_DOWN, l, proj, down_part, T));
     }
     const int XP = (packed ? FFMI_X_PACKED : 0) | wstream;
+    const int tail_n = few_rows ? few_n : T;
+    if (tail_n == 0) return FFMI_OK;
     // (markers also between the tail's kernels: final norm, lm_head, sampling)
     const bool tail_mark = marker_h == c.hidden && (!marker_t || T == marker_t);
     auto mkt = [&]() {
@@ -1260,9 +1275,9 @@ struct LlamaGPU : public ffmi_model {
       if (fuse)  // res already holds the last residual add
         FFMI_HIP(ffmi::launch_rmsnorm(res, nullptr, final_norm, nullptr, h, T, H, eps, stream, packed));
       else
-        FFMI_HIP(ffmi::launch_rmsnorm(res, proj, final_norm, res, h, T, H, eps, stream, packed,
-                                      down_part));
-      prof_end(pr, NORM, (double)T * H * 2 * 4, 0);
+        FFMI_HIP(ffmi::launch_rmsnorm(res, proj, final_norm, res, h, tail_n, H, eps, stream, packed,
+                                      down_part, nullptr, nullptr, 0, nullptr, few_rows ? rows_h : nullptr, T));
+      prof_end(pr, NORM, (double)tail_n * H * 2 * 4, 0);
     }
     mkt();
     if (dbg) {
@@ -1271,12 +1286,14 @@ struct LlamaGPU : public ffmi_model {
       dbg_T = T;
     }
     pr = prof_begin(ptail);
-    TRY(ffmi_linear_ws(h, lm, logits, T, Vl, H, FFMI_EPI_NONE | XP, ws, ws_bytes, s));
-    prof_end(pr, GEMM_LM_HEAD, gemm_bytes(T, Vl, Vl, H), 2.0 * T * Vl * H);
+    TRY(ffmi_linear_ws(h, lm, logits, tail_n, Vl, H, FFMI_EPI_NONE | XP, ws, ws_bytes, s));
+    prof_end(pr, GEMM_LM_HEAD, gemm_bytes(tail_n, Vl, Vl, H), 2.0 * tail_n * Vl * H);
     mkt();
-    pr = prof_begin(ptail);
-    TRY(enqueue_sampling(k, T));
-    prof_end(pr, SAMPLING, (double)T * V * 2, 0);
+    if (k > 0) {  // (0: the caller takes logits)
+      pr = prof_begin(ptail);
+      TRY(enqueue_sampling(k, tail_n));
+      prof_end(pr, SAMPLING, (double)tail_n * V * 2, 0);
+    }
     mkt();
 #undef TRY
     return FFMI_OK;
@@ -1320,11 +1337,22 @@ struct LlamaGPU : public ffmi_model {
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
     cur_slot = 0;
-    ffmi_status st = forward(1);
+    // (a request's next token is its last token's pick: no other is read)
+    last_rows.clear();
+    for (int t = 0; t < bc.num_tokens; ++t)
+      if (t + 1 == bc.num_tokens || bc.tokensInfo[t + 1].request_index != bc.tokensInfo[t].request_index)
+        last_rows.push_back(t);
+    ffmi_status st = forward(1, last_rows.data(), (int)last_rows.size());
     if (st != FFMI_OK) return st;
-    memcpy(ir->token_ids, ids_h, bc.num_tokens * sizeof(int32_t));
+    if (few_rows) {
+      std::fill_n(ir->token_ids, bc.num_tokens, -1);
+      for (int i = 0; i < few_n; ++i) ir->token_ids[rows_h[i]] = ids_h[i];
+    } else {
+      memcpy(ir->token_ids, ids_h, bc.num_tokens * sizeof(int32_t));
+    }
     return FFMI_OK;
   }
+  std::vector<int> last_rows;
   int vocab_size() const override { return c.vocab_size; }
   ffmi_status run_inc_logits(const BatchConfig &bc, const int *rows, int n, float *out) override {
     if (mode != FFMI_MODEL_INC) return FFMI_ERR_INVALID;
@@ -1333,8 +1361,9 @@ struct LlamaGPU : public ffmi_model {
     pack_inc(bc, o.max_requests, slots, &ps);
     for (int i = 0; i < n; ++i) FFMI_CHECK(rows[i] >= 0 && rows[i] < bc.num_tokens, FFMI_ERR_INVALID);
     cur_slot = 0;
-    ffmi_status st = forward_launch(1);
-    if (st == FFMI_OK && bc.num_tokens > 0) st = logit_rows.begin(logits, true, Vl, rows, n, Vl, stream);
+    ffmi_status st = forward_launch(0, rows, n);
+    if (st == FFMI_OK && bc.num_tokens > 0)
+      st = logit_rows.begin(logits, true, Vl, few_rows ? nullptr : rows, n, Vl, stream);
     const ffmi_status fin = forward_finish();
     if (st == FFMI_OK) st = fin;
     return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish(out) : st;
