@@ -339,8 +339,9 @@ struct LlamaF32 : public ffmi_model {
     return FFMI_OK;
   }
 
-  // n >= 0: rows[0, n) are the only ones that the caller reads; k = 0: logits only
-  ffmi_status forward(int k, const int *rows = nullptr, int n = -1) {
+  // n >= 0: rows[0, n) are the only ones that the caller reads; k = 0: their logits,
+  // begun towards out (logit_rows)
+  ffmi_status forward(int k, const int *rows = nullptr, int n = -1, float *out = nullptr) {
     const int T = (int)ps.tokens.size();
     FFMI_CHECK(k >= (n >= 0 ? 0 : 1) && k <= 4, FFMI_ERR_INVALID);
     few_rows = n >= 0 && T > 64 && 2 * n <= T && P == 1 && !dbg;
@@ -385,11 +386,14 @@ struct LlamaF32 : public ffmi_model {
       st = enqueue(k, bytes, true);
       if (st != FFMI_OK) return st;
     }
+    // (the step is on the stream: it is waited for whatever becomes of its rows)
+    const ffmi_status rows_st =
+        k == 0 ? logit_rows.begin(logits, false, V, few_rows ? nullptr : rows, n, V, stream, out) : FFMI_OK;
     FFMI_HIP(hipStreamSynchronize(stream));
     if (P > 1 && ffmi::comm_peer_attached(o.comm) && (st = ffmi::comm_status(o.comm)) != FFMI_OK)
       return st;
     if (dbg) dbg_T = T;
-    return FFMI_OK;
+    return rows_st;
   }
 
   // --inference-debugging: the last eager step's logits (fp32, full vocab)
@@ -431,10 +435,8 @@ struct LlamaF32 : public ffmi_model {
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
     for (int i = 0; i < n; ++i) FFMI_CHECK(rows[i] >= 0 && rows[i] < bc.num_tokens, FFMI_ERR_INVALID);
-    ffmi_status st = forward(0, rows, n);
-    if (st != FFMI_OK || bc.num_tokens == 0) return st;
-    st = logit_rows.begin(logits, false, V, few_rows ? nullptr : rows, n, V, stream);
-    return st == FFMI_OK ? logit_rows.finish(out) : st;
+    const ffmi_status st = forward(0, rows, n, out);
+    return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish() : st;
   }
   ffmi_status run_tree(const TreeVerifyBatchConfig &bc, InferenceResult *ir) override {
     if (mode != FFMI_MODEL_TREE) return FFMI_ERR_INVALID;

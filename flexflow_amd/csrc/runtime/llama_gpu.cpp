@@ -1363,10 +1363,10 @@ struct LlamaGPU : public ffmi_model {
     cur_slot = 0;
     ffmi_status st = forward_launch(0, rows, n);
     if (st == FFMI_OK && bc.num_tokens > 0)
-      st = logit_rows.begin(logits, true, Vl, few_rows ? nullptr : rows, n, Vl, stream);
+      st = logit_rows.begin(logits, true, Vl, few_rows ? nullptr : rows, n, Vl, stream, out);
     const ffmi_status fin = forward_finish();
     if (st == FFMI_OK) st = fin;
-    return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish(out) : st;
+    return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish() : st;
   }
   ffmi_status run_tree(const TreeVerifyBatchConfig &bc, InferenceResult *ir) override {
     if (mode != FFMI_MODEL_TREE) return FFMI_ERR_INVALID;

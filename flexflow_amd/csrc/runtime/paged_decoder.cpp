@@ -278,7 +278,7 @@ ffmi_status PagedDecoder::enqueue(bool sample) {
   return FFMI_OK;
 }
 
-ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n, bool sample) {
+ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n, bool sample, float *out) {
   if (mode != FFMI_MODEL_INC) return FFMI_ERR_INVALID;
   FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
   const int positions = P > 0 ? P : o.max_seq_len;
@@ -333,7 +333,7 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
     FFMI_TRY(enqueue(sample));
   }
   // (the step is on the stream: it is waited for and counted whatever becomes of its rows)
-  const ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream);
+  const ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream, out);
   FFMI_HIP(hipStreamSynchronize(stream));
   if (recurrent)
     for (int t = 0; t < bc.num_tokens; ++t) {
@@ -353,15 +353,15 @@ ffmi_status PagedDecoder::run_inc(const BatchConfig &bc, InferenceResult *ir) {
     if (t + 1 == bc.num_tokens ||
         bc.tokensInfo[t + 1].request_index != bc.tokensInfo[t].request_index)
       rows.push_back(t);
-  FFMI_TRY(forward(bc, rows.data(), (int)rows.size(), true));
+  FFMI_TRY(forward(bc, rows.data(), (int)rows.size(), true, nullptr));
   for (int t = 0; t < bc.num_tokens; ++t) ir->token_ids[t] = -1;
   for (size_t i = 0; i < rows.size(); ++i) ir->token_ids[rows[i]] = res_h[i];
   return FFMI_OK;
 }
 
 ffmi_status PagedDecoder::run_inc_logits(const BatchConfig &bc, const int *rows, int n, float *out) {
-  FFMI_TRY(forward(bc, rows, n, false));
-  return step.T > 0 && n > 0 ? logit_rows.finish(out) : FFMI_OK;
+  FFMI_TRY(forward(bc, rows, n, false, out));
+  return step.T > 0 && n > 0 ? logit_rows.finish() : FFMI_OK;
 }
 
 ffmi_status PagedDecoder::set_debug(int enable) {

@@ -152,7 +152,8 @@ struct PagedDecoder : public ffmi_model {
   ffmi_status capture(int i, const float *rows);
   bool capturing() const { return dbg != 0; }
   ffmi_status enqueue(bool sample);
-  ffmi_status forward(const BatchConfig &bc, const int *rows, int n, bool sample);
+  // sample: picks of the rows; else their logits, begun towards out (logit_rows)
+  ffmi_status forward(const BatchConfig &bc, const int *rows, int n, bool sample, float *out);
   LogitRows logit_rows;  // run_inc_logits
 
   ffmi_status run_inc(const BatchConfig &bc, InferenceResult *ir) override;
