@@ -160,6 +160,13 @@ float weight_amp(int kind);
 // ---- full-precision path (kernels/f32.hip) ----
 hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int N, int K,
                            hipStream_t s);
+// rows [n0, n0 + rows) of W [N][K] (src: the first of them, rows of ld) to blocks of 8 rows
+// x 32 k (f32.hip); dst holds ceil(N / 8) * 8 * K floats
+hipError_t launch_pack_f32_blocks(const float *src, int ld, float *dst, int N, int n0, int rows, int K, hipStream_t s);
+// launch_gemm_f32's sums of a packed W
+hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int T, int N, int K, hipStream_t s);
+hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu, float *out, int T, int F, int K,
+                                     hipStream_t s);
 hipError_t launch_rmsnorm_f32(const float *x1, const float *x2, const float *w, float *res_out,
                               float *out, int T, int H, float eps, hipStream_t s,
                               const char *gather = nullptr, const int32_t *rows = nullptr);

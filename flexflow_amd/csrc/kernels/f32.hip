@@ -28,6 +28,12 @@ namespace ffmi {
 // ---------------------------------------------------------------------------
 // Linear: Y[T][N] = X[T][K] . W[N][K]^T (linear_kernels.cu:450-582, DT_FLOAT)
 // ---------------------------------------------------------------------------
+// (a * sigmoid(a)) * b
+__device__ __forceinline__ float f32_silu_mul(float a, float b) {
+  const float sg = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf(-a)));
+  return __fmul_rn(__fmul_rn(a, sg), b);
+}
+
 // k quarters summed in wave order: 0 + 1 + 2 + 3 (fixed, deterministic), and stored
 template <int MT, int NT>
 __device__ __forceinline__ void f32_gemm_store(f4 (&acc)[MT][NT], f4 (*red)[MT * NT][64],
@@ -74,7 +80,7 @@ __device__ __forceinline__ void f32_gemm_store(f4 (&acc)[MT][NT], f4 (*red)[MT *
 // 16-byte pieces exchanged by the row's number: the operand reads then hit different
 // banks), and reads the next block's operands while it multiplies this one's.
 // Nothing is shared before the sum, so there is no barrier.
-template <int MT, int NT, int PF>
+template <int MT, int NT, int PF, bool PACKED = false>
 __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restrict__ X,
                                                           const float *__restrict__ W,
                                                           float *__restrict__ Y, int T, int N, int K) {
@@ -86,19 +92,21 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
   const int r = lane & 15, g = lane >> 4;
   const int nb = K >> 5;  // k-blocks of 32 (host-checked K % 32 == 0)
   const int kb0 = wave * nb / 4, n = (wave + 1) * nb / 4 - kb0;
+  const int tiles = (N + 7) >> 3;  // PACKED: of 8 columns
   const float *src[PW];
 #pragma unroll
   for (int p = 0; p < PW; ++p) {
     const int f = p >> 1, row = 8 * (p & 1) + (lane >> 3), piece = (lane ^ row) & 7;
-    src[p] = (f < MT ? X + (size_t)min(row0 + f * 16 + row, T - 1) * K
-                     : W + (size_t)min(col0 + (f - MT) * 16 + row, N - 1) * K) +
-             (size_t)kb0 * 32 + piece * 4;
+    if (f < MT) src[p] = X + (size_t)min(row0 + f * 16 + row, T - 1) * K + (size_t)kb0 * 32;
+    else if (!PACKED) src[p] = W + (size_t)min(col0 + (f - MT) * 16 + row, N - 1) * K + (size_t)kb0 * 32;
+    else src[p] = W + ((size_t)kb0 * tiles + min(((col0 >> 3) + 2 * (f - MT) + (p & 1)), tiles - 1)) * 256 + (lane >> 3) * 32;
+    src[p] += piece * 4;
   }
   auto copy = [&](int kb, int slot) {
 #pragma unroll
     for (int p = 0; p < PW; ++p)
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kb * 32),
+          (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kb * (PACKED && p >= 2 * MT ? tiles * 256 : 32)),
           (__attribute__((address_space(3))) void *)&lds[wave][slot][p >> 1][64 * (p & 1)], 16, 0, 0);
   };
   f4 acc[MT][NT];
@@ -153,6 +161,105 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
   auto red = reinterpret_cast<f4(*)[MT * NT][64]>(&lds[0][0][0][0]);
   static_assert(sizeof(lds) >= 3 * MT * NT * 64 * sizeof(f4), "sum buffer");
   f32_gemm_store<MT, NT>(acc, red, Y, T, N, row0, col0, wave, lane);
+}
+
+// Up to 16 rows (decoding) of packed weights (launch_pack_f32_blocks), where their stream
+// is the time: one tile of 16 x 16, of which only what is needed is copied.  What a CU takes in comes back from its L1 in
+// order, so that rows of X, from the L2, wait behind weights from HBM and take the place
+// of weights in flight: XH (up to 8 rows) leaves out the other 8.  COLS = 8: half a tile of
+// columns (the MFMA multiplies the other half for nothing), for widths whose 16-column
+// workgroups leave CUs idle or unevenly loaded.  PAIR: columns 0..7 of the tile are
+// gate's, 8..15 up's (W: F rows of gate, then F of up), and silu(gate) up goes out
+// (f32_silu_mul_kernel's arithmetic).  The sums are the other forms', in their order.
+template <int PF, bool XH, int COLS, bool PAIR>
+__global__ __launch_bounds__(256) void f32_gemm_few_kernel(const float *__restrict__ X, const float *__restrict__ Wp,
+                                                          float *__restrict__ Y, int T, int N, int K) {
+  static_assert(COLS == 16 || COLS == 8, "columns of a workgroup");
+  static_assert(!PAIR || COLS == 8, "a tile of gate and up columns");
+  constexpr int CX = XH ? 1 : 2, CW = COLS == 8 && !PAIR ? 1 : 2, PW = CX + CW;  // copies of 8 rows
+  static_assert(PF * PW <= 63, "vmcnt");
+  __shared__ f4 lds[4][PF][PW][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col0 = blockIdx.x * COLS, r = lane & 15, g = lane >> 4;
+  const int nb = K >> 5;  // k-blocks of 32 (host-checked K % 32 == 0)
+  const int kb0 = wave * nb / 4, n = (wave + 1) * nb / 4 - kb0;
+  const int tiles = ((PAIR ? 2 * N : N) + 7) >> 3;  // of 8 columns: a k-block of W
+  const float *src[PW];
+#pragma unroll
+  for (int p = 0; p < PW; ++p) {
+    const int row = lane >> 3, piece = (lane ^ row) & 7, c = p - CX;
+    if (c < 0) src[p] = X + (size_t)min(8 * p + row, T - 1) * K + (size_t)kb0 * 32;
+    else src[p] = Wp + ((size_t)kb0 * tiles + (PAIR ? c * (N >> 3) + (col0 >> 3) : min((col0 >> 3) + c, tiles - 1))) * 256 + row * 32;
+    src[p] += piece * 4;
+  }
+  auto copy = [&](int kb, int slot) {
+#pragma unroll
+    for (int p = 0; p < PW; ++p)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kb * (p < CX ? 32 : tiles * 256)),
+          (__attribute__((address_space(3))) void *)&lds[wave][slot][p][0], 16, 0, 0);
+  };
+  f4 acc[1][1] = {{f4{0.f, 0.f, 0.f, 0.f}}};
+  f4 cur[2][2], nxt[2][2];  // [X, W][half of the k-block]
+  // (rows that were not copied: the first 8 again, in rows and columns that nobody takes)
+  const int rx = XH ? 0 : r >> 3, rw = CX + (CW == 1 ? 0 : r >> 3);
+  auto read = [&](int slot, f4 (&v)[2][2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = (r & 7) * 8 + ((4 * h + g) ^ (r & 7));
+      v[0][h] = lds[wave][slot][rx][at];
+      v[1][h] = lds[wave][slot][rw][at];
+    }
+  };
+  auto wait = [](auto V) { __builtin_amdgcn_s_waitcnt((V.value & 15) | 0x0f70 | ((V.value >> 4) << 14)); };
+#pragma unroll
+  for (int i = 0; i < PF; ++i)
+    if (i < n) copy(i, i);
+  if (n >= PF) wait(std::integral_constant<int, (PF - 1) * PW>{});
+  else wait(std::integral_constant<int, 0>{});
+  asm volatile("" ::: "memory");
+  if (n > 0) read(0, cur);
+  int slot = 0;
+  for (int kb = 0; kb < n; ++kb) {
+    const int next = slot + 1 == PF ? 0 : slot + 1;
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this block's operands are in registers
+    asm volatile("" ::: "memory");
+    if (kb + PF < n) {
+      copy(kb + PF, slot);
+      wait(std::integral_constant<int, (PF - 1) * PW>{});
+    } else {
+      wait(std::integral_constant<int, 0>{});
+    }
+    asm volatile("" ::: "memory");
+    if (kb + 1 < n) read(next, nxt);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[0][h][j], cur[1][h][j], acc[0][0], 0, 0, 0);
+#pragma unroll
+    for (int f = 0; f < 2; ++f) cur[f][0] = nxt[f][0], cur[f][1] = nxt[f][1];
+    slot = next;
+  }
+  __syncthreads();
+  auto red = reinterpret_cast<f4(*)[1][64]>(&lds[0][0][0][0]);
+  static_assert(sizeof(lds) >= 3 * 64 * sizeof(f4), "sum buffer");
+  if constexpr (COLS == 16) {
+    f32_gemm_store<1, 1>(acc, red, Y, T, N, 0, col0, wave, lane);
+  } else {
+    if (wave > 0) red[wave - 1][0][lane] = acc[0][0];
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) acc[0][0] += red[s][0][lane];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v = acc[0][0][i];
+      if constexpr (PAIR) v = f32_silu_mul(v, __shfl_xor(v, 8));  // (lanes of columns 0..7 hold gate's)
+      const int row = 4 * g + i, col = col0 + r;
+      if (r < 8 && col < N && row < T) Y[(size_t)row * N + col] = v;
+    }
+  }
 }
 
 // The same sums from operands read straight into registers, for rows that are not of
@@ -217,26 +324,17 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float *__restrict__
   f32_gemm_store<MT, NT>(acc, red, Y, T, N, row0, col0, ks, lane);
 }
 
-hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int N, int K,
-                           hipStream_t s) {
-  if (T <= 0 || N <= 0) return hipSuccess;
-  if (K <= 0 || K % 32) return hipErrorInvalidValue;
+// Forms of more than 16 rows: the one with the least work on the busiest CU, workgroups
+// of a CU in rounds of 256 times a workgroup's tiles, times what a tile costs in that
+// form next to a 4 x 4 one (measured at N 2048-32000, K 2048 and 4096, T 24-1024; 2.3 us
+// a tile at K = 2048).  All forms add up an output in the same order.  T = 201, K = 2048:
+// N = 2048 2 x 4 tiles 23.6 us, 4 x 4 39.9 (41.2 from registers); N = 11264 110 and
+// 117 (123); N = 32000 316 and 312 (329).
+template <bool PACKED>
+static void f32_gemm_many(const float *X, const float *W, float *Y, int T, int N, int K, hipStream_t s) {
   const auto tiles = [&](int mt, int nt) {
     return dim3((N + 16 * nt - 1) / (16 * nt), (T + 16 * mt - 1) / (16 * mt));
   };
-  if (((uintptr_t)X | (uintptr_t)W) & 15) {
-    if (T <= 16)
-      hipLaunchKernelGGL((f32_gemm_kernel<1, 1>), tiles(1, 1), dim3(256), 0, s, X, W, Y, T, N, K);
-    else
-      hipLaunchKernelGGL((f32_gemm_kernel<4, 4>), tiles(4, 4), dim3(256), 0, s, X, W, Y, T, N, K);
-    return hipGetLastError();
-  }
-  // The form with the least work on the busiest CU: workgroups of a CU in rounds of
-  // 256 times a workgroup's tiles, times what a tile costs in that form next to a
-  // 4 x 4 one (measured at N 2048-32000, K 2048 and 4096, T 24-1024; 2.3 us a tile
-  // at K = 2048).  All forms add up an output in the same order.  T = 201, K = 2048:
-  // N = 2048 2 x 4 tiles 23.6 us, 4 x 4 39.9 (41.2 from registers); N = 11264 110 and
-  // 117 (123); N = 32000 316 and 312 (329).
   struct Form {
     int mt, nt;
     double cost;
@@ -249,9 +347,28 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
     const double c = (double)(((size_t)g.x * g.y + 255) / 256) * forms[i].mt * forms[i].nt * forms[i].cost;
     if (c < least) least = c, best = i;
   }
-#define FFMI_F32_GEMM(MT, NT, PF)                                                                \
-  hipLaunchKernelGGL((f32_gemm_lds_kernel<MT, NT, PF>), tiles(MT, NT), dim3(256), 0, s, X, W, Y, \
-                     T, N, K)
+#define FFMI_F32_GEMM(MT, NT, PF)                                                                           \
+  hipLaunchKernelGGL((f32_gemm_lds_kernel<MT, NT, PF, PACKED>), tiles(MT, NT), dim3(256), 0, s, X, W, Y, T, \
+                     N, K)
+  if (best == 0) FFMI_F32_GEMM(4, 4, 2);
+  else if (best == 1) FFMI_F32_GEMM(3, 4, 2);
+  else if (best == 2) FFMI_F32_GEMM(2, 4, 2);
+  else if (best == 3) FFMI_F32_GEMM(3, 2, 2);
+  else if (best == 4) FFMI_F32_GEMM(2, 2, 2);
+  else FFMI_F32_GEMM(2, 1, 3);
+#undef FFMI_F32_GEMM
+}
+
+hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int N, int K,
+                           hipStream_t s) {
+  if (T <= 0 || N <= 0) return hipSuccess;
+  if (K <= 0 || K % 32) return hipErrorInvalidValue;
+  const dim3 one((N + 15) / 16, (T + 15) / 16), four((N + 63) / 64, (T + 63) / 64), block(256);
+  if (((uintptr_t)X | (uintptr_t)W) & 15) {
+    if (T <= 16) hipLaunchKernelGGL((f32_gemm_kernel<1, 1>), one, block, 0, s, X, W, Y, T, N, K);
+    else hipLaunchKernelGGL((f32_gemm_kernel<4, 4>), four, block, 0, s, X, W, Y, T, N, K);
+    return hipGetLastError();
+  }
   // Up to 16 rows: a ring of four k-blocks (N = 2048, K = 5632: 13.9 us, 22.7 from registers)
   // takes 64 KiB, two workgroups to a CU, which is too few where each has little to
   // read: of two for short K (N = 32000, T = 8: K = 512 14.3 us, 18.1 with four, 16.0 from
@@ -259,16 +376,80 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
   // of a load, registers for the shortest (N = 32000, K = 256, T = 1: 7.6, ring of two 8.8,
   // of four 11.7; T = 16 10.4, 9.5 and 12.6).
   if (T <= 4 && K <= 256)
-    hipLaunchKernelGGL((f32_gemm_kernel<1, 1>), tiles(1, 1), dim3(256), 0, s, X, W, Y, T, N, K);
-  else if (T <= 16 && (K <= 512 || (K <= 1024 && N >= 4096))) FFMI_F32_GEMM(1, 1, 2);
-  else if (T <= 16) FFMI_F32_GEMM(1, 1, 4);
-  else if (best == 0) FFMI_F32_GEMM(4, 4, 2);
-  else if (best == 1) FFMI_F32_GEMM(3, 4, 2);
-  else if (best == 2) FFMI_F32_GEMM(2, 4, 2);
-  else if (best == 3) FFMI_F32_GEMM(3, 2, 2);
-  else if (best == 4) FFMI_F32_GEMM(2, 2, 2);
-  else FFMI_F32_GEMM(2, 1, 3);
-#undef FFMI_F32_GEMM
+    hipLaunchKernelGGL((f32_gemm_kernel<1, 1>), one, block, 0, s, X, W, Y, T, N, K);
+  else if (T <= 16 && (K <= 512 || (K <= 1024 && N >= 4096)))
+    hipLaunchKernelGGL((f32_gemm_lds_kernel<1, 1, 2>), one, block, 0, s, X, W, Y, T, N, K);
+  else if (T <= 16)
+    hipLaunchKernelGGL((f32_gemm_lds_kernel<1, 1, 4>), one, block, 0, s, X, W, Y, T, N, K);
+  else
+    f32_gemm_many<false>(X, W, Y, T, N, K, s);
+  return hipGetLastError();
+}
+
+// Packed weights (launch_pack_f32_blocks).  Up to 16 rows, T = 4, us, rows as they lie and
+// packed: 12288 x 4096 43.0 -> 35.6, 22016 x 4096 72.3 -> 64.8, K 11008 x N 4096 46.0 -> 31.2,
+// 4096 x 4096 17.6 -> 16.2, 6144 x 2048 12.4 -> 12.2, 11264 x 2048 19.3 -> 17.8, K 5632 x N 2048
+// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0.
+//  * Half tiles of columns where whole ones are at most half as many as CUs (K 5632 x N 2048
+//    14.4 -> 13.8, T = 16 16.3 -> 14.9; 768 x 3072 9.0 -> 8.5); at 256 and above they lose
+//    (6144 x 2048 13.1 -> 13.7, 11264 x 2048 18.3 -> 22.9).
+//  * A ring of two k-blocks, four workgroups to a CU, where there are several rounds of
+//    them and K is short (6144 x 2048 13.1 -> 12.2, 12288 x 4096 37.1 -> 35.6; but 4096 x
+//    4096, one round, 16.5 and 17.2, and K 11008 32.1 and 40.5).
+static bool short_ring(int workgroups, int K) { return workgroups > 256 && K <= 4096; }
+hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int T, int N, int K, hipStream_t s) {
+  if (T <= 0 || N <= 0) return hipSuccess;
+  if (K <= 0 || K % 32 || (((uintptr_t)X | (uintptr_t)Wp) & 15)) return hipErrorInvalidValue;
+  const int wgs = (N + 15) / 16;
+  if (T > 16) f32_gemm_many<true>(X, Wp, Y, T, N, K, s);
+  else if (wgs <= 128 && T <= 8)
+    hipLaunchKernelGGL((f32_gemm_few_kernel<4, true, 8, false>), dim3((N + 7) / 8), dim3(256), 0, s, X, Wp, Y, T, N, K);
+  else if (wgs <= 128)
+    hipLaunchKernelGGL((f32_gemm_few_kernel<4, false, 8, false>), dim3((N + 7) / 8), dim3(256), 0, s, X, Wp, Y, T, N, K);
+  else if (short_ring(wgs, K))
+    hipLaunchKernelGGL((f32_gemm_few_kernel<2, false, 16, false>), dim3(wgs), dim3(256), 0, s, X, Wp, Y, T, N, K);
+  else
+    hipLaunchKernelGGL((f32_gemm_few_kernel<4, false, 16, false>), dim3(wgs), dim3(256), 0, s, X, Wp, Y, T, N, K);
+  return hipGetLastError();
+}
+
+// out [T][F] = silu(X Wg^T) * (X Wu^T), Wp: the F rows of gate, then up's, packed; gu: room
+// for [T][2 F] (more than 16 rows take the product and its unit one after the other).
+hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu, float *out, int T, int F, int K,
+                                     hipStream_t s) {
+  if (T <= 0 || F <= 0) return hipSuccess;
+  if (T > 16 || F % 8) {
+    const hipError_t e = launch_gemm_f32_packed(X, Wp, gu, T, 2 * F, K, s);
+    return e != hipSuccess ? e : launch_silu_mul_f32(gu, gu + F, out, T, F, 2 * (size_t)F, 2 * (size_t)F, s);
+  }
+  if (K <= 0 || K % 32 || (((uintptr_t)X | (uintptr_t)Wp) & 15)) return hipErrorInvalidValue;
+  if (short_ring(F / 8, K))
+    hipLaunchKernelGGL((f32_gemm_few_kernel<2, false, 8, true>), dim3(F / 8), dim3(256), 0, s, X, Wp, out, T, F, K);
+  else
+    hipLaunchKernelGGL((f32_gemm_few_kernel<4, false, 8, true>), dim3(F / 8), dim3(256), 0, s, X, Wp, out, T, F, K);
+  return hipGetLastError();
+}
+
+// Blocks of 8 columns x 32 k (1 KiB, one copy to LDS), k-block after k-block: column n's
+// element k at ((k / 32 * tiles + n / 8) * 8 + n % 8) * 32 + k % 32, tiles = ceil(N / 8).
+// Read k-block by k-block, the chip walks one band of memory instead of 128 bytes of each
+// of thousands of rows.
+__global__ __launch_bounds__(256) void pack_f32_blocks_kernel(const float *__restrict__ src, int ld, float *__restrict__ dst,
+                                                            int tiles, int n0, int rows, int K) {
+  const size_t pieces = (size_t)rows * (K >> 2);
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < pieces; i += (size_t)gridDim.x * 256) {
+    const int row = (int)(i / (K >> 2)), k = (int)(i % (K >> 2)) * 4, n = n0 + row;
+    const f4 v = *reinterpret_cast<const f4 *>(src + (size_t)row * ld + k);
+    *reinterpret_cast<f4 *>(dst + (((size_t)(k >> 5) * tiles + (n >> 3)) * 8 + (n & 7)) * 32 + (k & 31)) = v;
+  }
+}
+
+hipError_t launch_pack_f32_blocks(const float *src, int ld, float *dst, int N, int n0, int rows, int K, hipStream_t s) {
+  if (rows <= 0) return hipSuccess;
+  if (K <= 0 || K % 32 || ld % 4 || n0 < 0 || n0 + rows > N || (((uintptr_t)src | (uintptr_t)dst) & 15))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(pack_f32_blocks_kernel, dim3((unsigned)std::min<size_t>(((size_t)rows * (K / 4) + 255) / 256, 8192)),
+                     dim3(256), 0, s, src, ld, dst, (N + 7) / 8, n0, rows, K);
   return hipGetLastError();
 }
 
@@ -399,8 +580,7 @@ __global__ void f32_silu_mul_kernel(const float *__restrict__ A, const float *__
        i += (size_t)gridDim.x * blockDim.x) {
     const size_t t = i / F, f = i % F;
     const float a = A[t * lda + f], b = B[t * ldb + f];
-    const float sg = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf(-a)));
-    out[i] = __fmul_rn(__fmul_rn(a, sg), b);
+    out[i] = f32_silu_mul(a, b);
   }
 }
 

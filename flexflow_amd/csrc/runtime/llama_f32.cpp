@@ -151,6 +151,7 @@ struct LlamaF32 : public ffmi_model {
       std::vector<float> v;
       ffmi_status st = load_tensor(v, n, name);
       if (st != FFMI_OK) return st;
+      FFMI_HIP(hipStreamSynchronize(stream));  // (tmp is read until then)
       FFMI_HIP(hipMemcpy(tmp, v.data(), n * 4, hipMemcpyHostToDevice));
       return FFMI_OK;
     }
@@ -158,12 +159,13 @@ struct LlamaF32 : public ffmi_model {
                                     perm_cols, pa, 17, scale));
     return FFMI_OK;
   }
-  // rows [r0, r0 + nr) x columns [c0, c0 + nc) of tmp ([.][ld]) -> dst [nr][nc]
-  ffmi_status take(float *dst, const float *tmp, int ld, int r0, int nr, int c0, int nc) {
-    FFMI_HIP(hipMemcpy2DAsync(dst, (size_t)nc * 4, tmp + (size_t)r0 * ld + c0, (size_t)ld * 4,
-                              (size_t)nc * 4, nr, hipMemcpyDeviceToDevice, stream));
+  // rows [r0, r0 + nr) x columns [c0, c0 + nc) of tmp ([.][ld]) -> rows n0 ... of the
+  // packed weight dst [N][nc]
+  ffmi_status take(float *dst, int N, int n0, const float *tmp, int ld, int r0, int nr, int c0, int nc) {
+    FFMI_HIP(launch_pack_f32_blocks(tmp + (size_t)r0 * ld + c0, ld, dst, N, n0, nr, nc, stream));
     return FFMI_OK;
   }
+  ffmi_status alloc_packed(float **p, int N, int K) { return alloc(p, (size_t)((N + 7) / 8 * 8) * K); }
 
   ffmi_status init() {
     H = c.hidden, F = c.intermediate, V = c.vocab_size, P = o.tp_size;
@@ -227,11 +229,12 @@ struct LlamaF32 : public ffmi_model {
     TRY(full_tensor(embed, V, H, "model.embed_tokens.weight", 0, 0, 1, chain ? chain_scale : 1.f));
     TRY(alloc(&final_norm, H));
     TRY(full_tensor(final_norm, 1, H, "model.norm.weight", 1));
-    TRY(alloc(&lm, (size_t)V * H));
+    TRY(alloc_packed(&lm, V, H));
     if (chain)
-      TRY(full_tensor(lm, V, H, "model.embed_tokens.weight", 0, H, 7919));
+      TRY(full_tensor(tmp, V, H, "model.embed_tokens.weight", 0, H, 7919));
     else
-      TRY(full_tensor(lm, V, H, "lm_head.weight", 0));
+      TRY(full_tensor(tmp, V, H, "lm_head.weight", 0));
+    TRY(take(lm, V, 0, tmp, H, 0, V, 0, H));
     const int s = o.tp_rank;
     layers.resize(c.num_layers);
     for (int l = 0; l < c.num_layers; ++l) {
@@ -242,27 +245,27 @@ struct LlamaF32 : public ffmi_model {
       TRY(alloc(&L.post_norm, H));
       TRY(full_tensor(L.post_norm, 1, H, p + "post_attention_layernorm.weight", 1));
       // qkv: rows [Q_s; K_s; V_s] (file_loader.cc:286-303)
-      TRY(alloc(&L.wqkv, (size_t)3 * Hl * H));
+      TRY(alloc_packed(&L.wqkv, 3 * Hl, H));
       const char *names[3] = {"self_attn.q_proj.weight", "self_attn.k_proj.weight",
                               "self_attn.v_proj.weight"};
       for (int q = 0; q < 3; ++q) {
         TRY(full_tensor(tmp, H, H, p + names[q], 0));
-        TRY(take(L.wqkv + (size_t)q * Hl * H, tmp, H, s * Hl, Hl, 0, H));
+        TRY(take(L.wqkv, 3 * Hl, q * Hl, tmp, H, s * Hl, Hl, 0, H));
       }
       // o_proj row-parallel: columns [s*Hl, (s+1)*Hl)
-      TRY(alloc(&L.wo, (size_t)H * Hl));
+      TRY(alloc_packed(&L.wo, H, Hl));
       TRY(full_tensor(tmp, H, H, p + "self_attn.o_proj.weight", kres));
-      TRY(take(L.wo, tmp, H, 0, H, s * Hl, Hl));
+      TRY(take(L.wo, H, 0, tmp, H, 0, H, s * Hl, Hl));
       // gate rows then up rows of this shard: one GEMM, [T][2 Fl]
-      TRY(alloc(&L.wgu, (size_t)2 * Fl * H));
+      TRY(alloc_packed(&L.wgu, 2 * Fl, H));
       TRY(full_tensor(tmp, F, H, p + "mlp.gate_proj.weight", 0));
-      TRY(take(L.wgu, tmp, H, s * Fl, Fl, 0, H));
+      TRY(take(L.wgu, 2 * Fl, 0, tmp, H, s * Fl, Fl, 0, H));
       TRY(full_tensor(tmp, F, H, p + "mlp.up_proj.weight", 0));
-      TRY(take(L.wgu + (size_t)Fl * H, tmp, H, s * Fl, Fl, 0, H));
+      TRY(take(L.wgu, 2 * Fl, Fl, tmp, H, s * Fl, Fl, 0, H));
       // down row-parallel: columns [s*Fl, (s+1)*Fl) of [H][F]
-      TRY(alloc(&L.wd, (size_t)H * Fl));
+      TRY(alloc_packed(&L.wd, H, Fl));
       TRY(full_tensor(tmp, H, F, p + "mlp.down_proj.weight", kres));
-      TRY(take(L.wd, tmp, F, 0, H, s * Fl, Fl));
+      TRY(take(L.wd, H, 0, tmp, F, 0, H, s * Fl, Fl));
       // the layer's DT_FLOAT attention handle (ffmi_attn_cfg.full_precision)
       ffmi_attn_cfg ac{};
       ac.mode = mode == FFMI_MODEL_TREE ? FFMI_ATTN_TREE
@@ -316,21 +319,20 @@ struct LlamaF32 : public ffmi_model {
         FFMI_HIP(launch_rmsnorm_f32(embed, nullptr, L.in_norm, res, h, T, H, eps, stream, blob));
       else
         FFMI_HIP(launch_rmsnorm_f32(res, proj, L.in_norm, res, h, T, H, eps, stream));
-      FFMI_HIP(launch_gemm_f32(h, L.wqkv, qkv, T, 3 * Hl, H, stream));
+      FFMI_HIP(launch_gemm_f32_packed(h, L.wqkv, qkv, T, 3 * Hl, H, stream));
       TRY(attn_forward(L.attn, batch, qkv, Partials(), att, (ffmi_stream)stream));
-      FFMI_HIP(launch_gemm_f32(att, L.wo, proj, T, H, Hl, stream));
+      FFMI_HIP(launch_gemm_f32_packed(att, L.wo, proj, T, H, Hl, stream));
       TRY(allreduce(proj, (size_t)T * H));
       FFMI_HIP(launch_rmsnorm_f32(res, proj, L.post_norm, res, h, T, H, eps, stream));
-      FFMI_HIP(launch_gemm_f32(h, L.wgu, gu, T, 2 * Fl, H, stream));
-      FFMI_HIP(launch_silu_mul_f32(gu, gu + Fl, mlp, T, Fl, 2 * (size_t)Fl, 2 * (size_t)Fl, stream));
-      FFMI_HIP(launch_gemm_f32(mlp, L.wd, proj, T, H, Fl, stream));
+      FFMI_HIP(launch_gate_up_f32_packed(h, L.wgu, gu, mlp, T, Fl, H, stream));
+      FFMI_HIP(launch_gemm_f32_packed(mlp, L.wd, proj, T, H, Fl, stream));
       TRY(allreduce(proj, (size_t)T * H));
     }
     const int n = tail_n;
     if (n == 0) return FFMI_OK;
     FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, few_rows ? nullptr : res, h, n, H, eps, stream, nullptr,
                                 few_rows ? rows_h : nullptr));
-    FFMI_HIP(launch_gemm_f32(h, lm, logits, n, V, H, stream));
+    FFMI_HIP(launch_gemm_f32_packed(h, lm, logits, n, V, H, stream));
     if (k == 0) return FFMI_OK;  // logits only
     float *probs_d = reinterpret_cast<float *>(res_d + (size_t)n * k);
     FFMI_HIP(launch_softmax_topk_f32(logits, n, V, k, res_d, probs_d, stream));

@@ -1,6 +1,8 @@
 """Long steps of the LLaMA models whose callers read few rows: the final norm, lm_head and
 sampling run on those rows only.  Logits against the same step with every row computed
-(debug capture), tokens of prompts of that kind against prompts in short portions."""
+(debug capture), tokens of prompts of that kind against prompts in short portions.  In full
+precision every form of a product adds up in the same order, so there a token's logits do
+not depend on its step at all."""
 import numpy as np
 import pytest
 
@@ -54,3 +56,21 @@ def test_prompts_together_and_in_portions(full):
         prompts = [[(31 * i + 7 * r) % 490 + 5 for i in range(k)] for r, k in enumerate((150, 33, 60))]
         out.append([r.output_tokens for r in fa.generate(rm, m, prompts, max_new_tokens=8)])
     assert out[0] == out[1]
+
+
+# widths that meet half tiles of columns, whole ones, rings of two and four k-blocks, gate and up columns in one
+# tile, widths that are no multiple of 8 (up to 16 tokens), and the forms of more tokens
+@pytest.mark.parametrize("ff,vocab", [(256, 500), (2080, 2101), (4128, 4101)])
+def test_full_precision_does_not_depend_on_the_step(ff, vocab):
+    m = fa.Model(dict(CFG, intermediate=ff, vocab_size=vocab), "inc", max_requests=1, max_tokens=128, max_seq_len=128,
+                 weight_seed=9, full_precision=True)
+    rm = fa.RequestManager(max_requests_per_batch=1, max_tokens_per_batch=128, max_sequence_length=128)
+    toks = [(37 * i + 11) % vocab for i in range(90)]
+    whole = rm.replay_step(m, [(1, toks, range(90))])
+    rm.replay_end(m, 1)
+    got, at = [], 0
+    for k in (1, 2, 8, 9, 16, 17, 7, 1, 29):
+        got.append(rm.replay_step(m, [(1, toks[at:at + k], range(k))]))
+        at += k
+    rm.replay_end(m, 1)
+    assert at == 90 and np.array_equal(np.concatenate(got), whole) and np.isfinite(whole).all() and whole.std() > 0
