@@ -197,6 +197,10 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
       seen[r >> 6] |= 1ull << (r & 63);
     }
   }
+  b->distinct_reqs = d->num_tokens <= 64;
+  for (int t = 1; t < d->num_tokens && b->distinct_reqs; ++t)
+    for (int u = 0; u < t; ++u)
+      if (d->tokens[u].req == d->tokens[t].req) b->distinct_reqs = false;
   b->commit_overlap = false;
   for (int c = 0; c < d->num_commits && !b->commit_overlap; ++c)
     for (int t = 0; t < d->num_tokens; ++t)
@@ -400,15 +404,13 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
   const int heads = h->cfg.num_heads, d = h->cfg.head_dim;
   if (h->cfg.full_precision) {
     // DT_FLOAT: commits (TREE), then RoPE + KV store (+ staging), then the
-    // attention, each its own launch (kernels/f32.hip)
+    // attention (kernels/f32.hip)
     FFMI_CHECK(qkv && qkvp.S == 0 && !(opa && opa->wo), FFMI_ERR_INVALID);
-    FFMI_HIP(ffmi::launch_kv_update_f32(b->dev, b->num_tokens, tree ? b->num_commits : 0,
-                                        (const float *)qkv, h->rope, h->slots, (float *)h->qbuf,
-                                        (float *)h->kc, (float *)h->vc,
-                                        tree ? (float *)h->stage : nullptr, heads, d, h->slots, s));
-    FFMI_HIP(ffmi::launch_attention_f32(b->dev, b->num_tokens, (const float *)h->qbuf,
-                                        (const float *)h->kc, (const float *)h->vc, (float *)out,
-                                        heads, d, h->slots, h->cfg.qk_scale, s));
+    FFMI_HIP(ffmi::launch_update_attention_f32(b->dev, b->num_tokens, tree ? b->num_commits : 0,
+                                               (const float *)qkv, h->rope, h->slots, (float *)h->qbuf,
+                                               (float *)h->kc, (float *)h->vc,
+                                               tree ? (float *)h->stage : nullptr, (float *)out, heads, d,
+                                               h->slots, h->cfg.qk_scale, b->distinct_reqs, s));
     return FFMI_OK;
   }
   uint16_t *stage_wr = nullptr, *stage_rd = nullptr;

@@ -178,6 +178,11 @@ hipError_t launch_kv_update_f32(const char *blob, int T, int C, const float *qkv
 hipError_t launch_attention_f32(const char *blob, int T, const float *qbuf, const float *kc,
                                 const float *vc, float *out, int heads, int d, int slots,
                                 float scale, hipStream_t s);
+// launch_kv_update_f32, then launch_attention_f32; distinct: no two of the step's tokens
+// are of one request (both in one launch then)
+hipError_t launch_update_attention_f32(const char *blob, int T, int C, const float *qkv, const float *rope,
+                                       int max_rope_pos, float *qbuf, float *kc, float *vc, float *stage, float *out,
+                                       int heads, int d, int slots, float scale, bool distinct, hipStream_t s);
 // rows ids.row[0, n) of logits [.][ld] (fp16 or fp32) as fp32 to dst [n][V]
 struct LogitRowIds {
   static constexpr int kMax = 16;
@@ -369,6 +374,7 @@ struct ffmi_batch_dev {
   int num_tokens = 0, num_work = 0, num_commits = 0, num_mask_reqs = 0;
   bool commit_overlap = false;  // a commit depth is also a slot this step stores
   bool one_item_per_req = false;  // every request's tokens form one attention work item
+  bool distinct_reqs = false;     // (of up to 64 tokens) no two tokens of one request
   bool lds_tail = false;  // every item's writes fit the fused kernel's LDS tail and
                           // its commits the work item (else the two-launch path)
   int max_q = 0;                  // largest work item

@@ -601,16 +601,14 @@ hipError_t launch_silu_mul_f32(const float *A, const float *B, float *out, int T
 // next step's commits (tree_inc...cu:335-396 reads them).  Grid (T, heads),
 // d/2 threads.
 // ---------------------------------------------------------------------------
-__global__ void f32_kv_update_kernel(const char *__restrict__ blob, const float *__restrict__ qkv,
-                                     const float *__restrict__ rope, int max_rope_pos,
-                                     float *__restrict__ qbuf, float *__restrict__ kc,
-                                     float *__restrict__ vc, float *__restrict__ stage, int heads,
-                                     int d, int slots) {
-  const int t = blockIdx.x, hd = blockIdx.y, i = threadIdx.x, half = d / 2;
-  if (i >= half) return;
-  const BatchView bv = batch_view(blob);
-  const ffmi_token_info tk = bv.tokens[t];
-  const int Hl = heads * d;
+struct KvUpdateF32 {  // elements i and i + d / 2 of a (token, head)
+  float q0, q1, k0, k1, va, vb;
+};
+__device__ __forceinline__ KvUpdateF32 f32_kv_update(const ffmi_token_info &tk, int t, int hd, int i,
+                                                     const float *__restrict__ qkv, const float *__restrict__ rope,
+                                                     int max_rope_pos, float *__restrict__ kc, float *__restrict__ vc,
+                                                     float *__restrict__ stage, int heads, int d, int slots) {
+  const int half = d / 2, Hl = heads * d;
   const float *row = qkv + (size_t)t * 3 * Hl + hd * d;
   const int p = min(max(tk.pos, 0), max_rope_pos - 1);
   const float c = rope[((size_t)p * half + i) * 2], sn = rope[((size_t)p * half + i) * 2 + 1];
@@ -621,9 +619,6 @@ __global__ void f32_kv_update_kernel(const char *__restrict__ blob, const float 
   const float q1 = __fadd_rn(__fmul_rn(qa, sn), __fmul_rn(qb, c));
   const float k0 = __fsub_rn(__fmul_rn(ka, c), __fmul_rn(kb, sn));
   const float k1 = __fadd_rn(__fmul_rn(ka, sn), __fmul_rn(kb, c));
-  float *qo = qbuf + (size_t)t * Hl + hd * d;
-  qo[i] = q0;
-  qo[i + half] = q1;
   if (tk.store_slot >= 0 && tk.store_slot < slots) {
     const size_t base = (((size_t)tk.req * heads + hd) * slots + tk.store_slot) * d;
     kc[base + i] = k0;
@@ -638,6 +633,20 @@ __global__ void f32_kv_update_kernel(const char *__restrict__ blob, const float 
     st[Hl + i] = va;
     st[Hl + i + half] = vb;
   }
+  return {q0, q1, k0, k1, va, vb};
+}
+__global__ void f32_kv_update_kernel(const char *__restrict__ blob, const float *__restrict__ qkv,
+                                     const float *__restrict__ rope, int max_rope_pos,
+                                     float *__restrict__ qbuf, float *__restrict__ kc,
+                                     float *__restrict__ vc, float *__restrict__ stage, int heads,
+                                     int d, int slots) {
+  const int t = blockIdx.x, hd = blockIdx.y, i = threadIdx.x;
+  if (i >= d / 2) return;
+  const ffmi_token_info tk = batch_view(blob).tokens[t];
+  const KvUpdateF32 u = f32_kv_update(tk, t, hd, i, qkv, rope, max_rope_pos, kc, vc, stage, heads, d, slots);
+  float *qo = qbuf + (size_t)t * heads * d + hd * d;
+  qo[i] = u.q0;
+  qo[i + d / 2] = u.q1;
 }
 
 // commit_tokens_kernel (tree_inc...cu:335-396): accepted tokens of the
@@ -682,11 +691,19 @@ hipError_t launch_kv_update_f32(const char *blob, int T, int C, const float *qkv
 // passes' loads in flight (a thread per key and a thread per output element, one
 // load after another, took 23.9 us for 4 tokens x 16 heads, d = 128, about 160
 // keys, now 6.5); output groups are summed in group order.
+// UPDATE (a step of one token per request: no other workgroup's keys are this step's):
+// the token's KV update first, its own key and value from LDS, the rest as it lies in the
+// cache -- one launch of 7.8 us for two of 4.0 and 7.0 (4 tokens x 16 heads).
 // ---------------------------------------------------------------------------
-template <int D>
+struct KvUpdateArgs {
+  const float *qkv = nullptr, *rope = nullptr;
+  int max_rope_pos = 0;
+  float *kc = nullptr, *vc = nullptr, *stage = nullptr;
+};
+template <int D, bool UPDATE>
 __global__ __launch_bounds__(256) void f32_attention_kernel(
-    const char *__restrict__ blob, const float *__restrict__ qbuf, const float *__restrict__ kc,
-    const float *__restrict__ vc, float *__restrict__ out, int heads, int slots, float scale) {
+    const char *__restrict__ blob, const float *__restrict__ qbuf, const float *kc,
+    const float *vc, float *__restrict__ out, int heads, int slots, float scale, KvUpdateArgs up) {
   constexpr int U = 4;             // passes in flight
   constexpr int KV = D / 32;       // 16-byte pieces of a key per lane
   constexpr int KP = 256 / 8;      // keys of a score pass
@@ -694,10 +711,22 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(
   extern __shared__ __attribute__((aligned(16))) float sc[];  // scores [slots], then partial outputs [G][D]
   __shared__ float shf[4];
   __shared__ double shd[4];
+  __shared__ __attribute__((aligned(16))) float own[UPDATE ? 3 : 1][UPDATE ? D : 1];  // q, k, v of the token
   const int t = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x;
   const BatchView bv = batch_view(blob);
   const ffmi_token_info tk = bv.tokens[t];
   const int Hl = heads * D;
+  const int mine = UPDATE ? tk.store_slot : -1;  // the slot whose key and value are in LDS
+  if constexpr (UPDATE) {
+    if (tid < D / 2) {
+      const KvUpdateF32 u = f32_kv_update(tk, t, hd, tid, up.qkv, up.rope, up.max_rope_pos, up.kc, up.vc, up.stage,
+                                          heads, D, slots);
+      own[0][tid] = u.q0, own[0][tid + D / 2] = u.q1;
+      own[1][tid] = u.k0, own[1][tid + D / 2] = u.k1;
+      own[2][tid] = u.va, own[2][tid + D / 2] = u.vb;
+    }
+    __syncthreads();
+  }
   int kv_end = max(tk.prefix_len, tk.tree_len > 0 ? tk.tree_base + tk.tree_len : 0);
   kv_end = min(kv_end, slots);
   const float *K = kc + ((size_t)tk.req * heads + hd) * slots * D;
@@ -707,7 +736,8 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(
   f4 q[KV];
 #pragma unroll
   for (int i = 0; i < KV; ++i)
-    q[i] = *reinterpret_cast<const f4 *>(qbuf + (size_t)t * Hl + hd * D + (i * 8 + sub) * 4);
+    q[i] = UPDATE ? *reinterpret_cast<const f4 *>(&own[0][(i * 8 + sub) * 4])
+                  : *reinterpret_cast<const f4 *>(qbuf + (size_t)t * Hl + hd * D + (i * 8 + sub) * 4);
   float mx = NEG;
   for (int j0 = 0; j0 < kv_end; j0 += U * KP) {
     f4 k[U][KV];
@@ -721,6 +751,9 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(
     for (int u = 0; u < U; ++u) {
       const int j = j0 + u * KP + (tid >> 3);
       float acc = 0.f;
+      if (UPDATE && j == mine)
+#pragma unroll
+        for (int i = 0; i < KV; ++i) k[u][i] = *reinterpret_cast<const f4 *>(&own[1][(i * 8 + sub) * 4]);
 #pragma unroll
       for (int i = 0; i < KV; ++i)
 #pragma unroll
@@ -755,6 +788,7 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(
     for (int u = 0; u < U; ++u) {
       const int j = min(j0 + u * G, kv_end - 1);
       v[u] = *reinterpret_cast<const f4 *>(V + (size_t)j * D + i * 4);
+      if (UPDATE && j == mine) v[u] = *reinterpret_cast<const f4 *>(&own[2][i * 4]);
       p[u] = j0 + u * G < kv_end ? sc[j] : 0.f;
     }
 #pragma unroll
@@ -774,22 +808,43 @@ __global__ __launch_bounds__(256) void f32_attention_kernel(
   }
 }
 
+template <bool UPDATE>
+static hipError_t run_attention_f32(const char *blob, int T, const float *qbuf, const float *kc, const float *vc,
+                                    float *out, int heads, int d, int slots, float scale, const KvUpdateArgs &up,
+                                    hipStream_t s) {
+  const size_t lds = (size_t)std::max(slots, 1024) * sizeof(float);  // (partial outputs: 1024)
+  if ((size_t)(d + 256 + slots) * sizeof(float) > 64 * 1024) return hipErrorInvalidValue;
+  const dim3 grid(T, heads), block(256);
+#define FFMI_ATTN_F32(DD)                                                                                             \
+  hipLaunchKernelGGL((f32_attention_kernel<DD, UPDATE>), grid, block, lds, s, blob, qbuf, kc, vc, out, heads, slots, \
+                     scale, up)
+  if (d == 128) FFMI_ATTN_F32(128);
+  else if (d == 64) FFMI_ATTN_F32(64);
+  else if (d == 32) FFMI_ATTN_F32(32);
+  else return hipErrorInvalidValue;
+#undef FFMI_ATTN_F32
+  return hipGetLastError();
+}
+
 hipError_t launch_attention_f32(const char *blob, int T, const float *qbuf, const float *kc,
                                 const float *vc, float *out, int heads, int d, int slots,
                                 float scale, hipStream_t s) {
   if (T <= 0) return hipSuccess;
-  const size_t lds = (size_t)std::max(slots, 1024) * sizeof(float);  // (partial outputs: 1024)
-  if ((size_t)(d + 256 + slots) * sizeof(float) > 64 * 1024) return hipErrorInvalidValue;
-  const dim3 grid(T, heads), block(256);
-  if (d == 128)
-    hipLaunchKernelGGL(f32_attention_kernel<128>, grid, block, lds, s, blob, qbuf, kc, vc, out, heads, slots, scale);
-  else if (d == 64)
-    hipLaunchKernelGGL(f32_attention_kernel<64>, grid, block, lds, s, blob, qbuf, kc, vc, out, heads, slots, scale);
-  else if (d == 32)
-    hipLaunchKernelGGL(f32_attention_kernel<32>, grid, block, lds, s, blob, qbuf, kc, vc, out, heads, slots, scale);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  return run_attention_f32<false>(blob, T, qbuf, kc, vc, out, heads, d, slots, scale, KvUpdateArgs(), s);
+}
+
+hipError_t launch_update_attention_f32(const char *blob, int T, int C, const float *qkv, const float *rope,
+                                       int max_rope_pos, float *qbuf, float *kc, float *vc, float *stage, float *out,
+                                       int heads, int d, int slots, float scale, bool distinct, hipStream_t s) {
+  // (beside the scores: the token's rows and the reductions, 2 KiB)
+  const bool one = distinct && (size_t)std::max(slots, 1024) * sizeof(float) + 2048 <= 64 * 1024;
+  const hipError_t e = launch_kv_update_f32(blob, one ? 0 : T, C, qkv, rope, max_rope_pos, qbuf, kc, vc, stage, heads,
+                                            d, slots, s);
+  if (e != hipSuccess || T <= 0) return e;
+  if (!one) return launch_attention_f32(blob, T, qbuf, kc, vc, out, heads, d, slots, scale, s);
+  KvUpdateArgs up;
+  up.qkv = qkv, up.rope = rope, up.max_rope_pos = max_rope_pos, up.kc = kc, up.vc = vc, up.stage = stage;
+  return run_attention_f32<true>(blob, T, qbuf, kc, vc, out, heads, d, slots, scale, up, s);
 }
 
 // ---------------------------------------------------------------------------

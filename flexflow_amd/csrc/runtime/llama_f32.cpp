@@ -59,7 +59,7 @@ struct LlamaF32 : public ffmi_model {
   ffmi_batch_dev *batch = nullptr;
   PackedStep ps;
   std::vector<void *> allocs;
-  std::map<std::tuple<int, int, int, int, size_t>, hipGraphExec_t> graphs;
+  std::map<std::tuple<int, int, int, int, bool, size_t>, hipGraphExec_t> graphs;
   bool use_graphs = getenv("FFMI_NO_GRAPHS") == nullptr;
   int dbg = 0, dbg_T = -1;
 
@@ -361,7 +361,7 @@ struct LlamaF32 : public ffmi_model {
     // transports stay eager here: this path is not the measured one)
     const bool graph = use_graphs && !dbg && P == 1 && !few_rows;
     if (graph) {
-      const auto key = std::make_tuple(T, batch->num_work, batch->num_commits, k, bytes);
+      const auto key = std::make_tuple(T, batch->num_work, batch->num_commits, k, batch->distinct_reqs, bytes);
       auto it = graphs.find(key);
       if (it == graphs.end()) {
         if (graphs.size() >= 256) {
