@@ -79,7 +79,11 @@ __device__ __forceinline__ void f32_gemm_store(f4 (&acc)[MT][NT], f4 (*red)[MT *
 // an LDS ring of its own, PF of them on their way, a row's 128 bytes to 8 lanes (its
 // 16-byte pieces exchanged by the row's number: the operand reads then hit different
 // banks), and reads the next block's operands while it multiplies this one's.
-// Nothing is shared before the sum, so there is no barrier.
+// Nothing is shared before the sum, so there is no barrier.  Blocks in turn use two sets
+// of registers: moving a set (up to 64 registers a block, on the one wave of a SIMD that
+// also issues the MFMAs) took 3-12% of a product (packed, us: T = 201, 2 x 4 tiles, N = 11264
+// 108.6 -> 104.6, K = 5632 x N = 2048 53.9 -> 51.0; T = 75, 2 x 2, K = 5632 32.3 -> 28.9; T = 1000,
+// 4 x 4, N = 11264 419 -> 406; T = 24, N = 32000, the stream of weights, 51.0 and 52.0).
 template <int MT, int NT, int PF, bool PACKED = false>
 __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restrict__ X,
                                                           const float *__restrict__ W,
@@ -114,7 +118,7 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[m][j] = f4{0.f, 0.f, 0.f, 0.f};
-  f4 cur[F][2], nxt[F][2];
+  f4 va[F][2], vb[F][2];
   auto read = [&](int slot, f4 (&v)[F][2]) {
 #pragma unroll
     for (int f = 0; f < F; ++f)
@@ -129,9 +133,9 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
   if (n >= PF) wait(std::integral_constant<int, (PF - 1) * PW>{});
   else wait(std::integral_constant<int, 0>{});
   asm volatile("" ::: "memory");
-  if (n > 0) read(0, cur);
+  if (n > 0) read(0, va);
   int slot = 0;
-  for (int kb = 0; kb < n; ++kb) {
+  auto step = [&](int kb, f4 (&cur)[F][2], f4 (&nxt)[F][2]) {
     const int next = slot + 1 == PF ? 0 : slot + 1;
     // this block's operands are in registers; its slot takes block kb + PF
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
@@ -153,10 +157,14 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
 #pragma unroll
           for (int i = 0; i < NT; ++i)
             acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[m][h][j], cur[MT + i][h][j], acc[m][i], 0, 0, 0);
-#pragma unroll
-    for (int f = 0; f < F; ++f) cur[f][0] = nxt[f][0], cur[f][1] = nxt[f][1];
     slot = next;
+  };
+  int kb = 0;
+  for (; kb + 1 < n; kb += 2) {
+    step(kb, va, vb);
+    step(kb + 1, vb, va);
   }
+  if (kb < n) step(kb, va, vb);
   __syncthreads();
   auto red = reinterpret_cast<f4(*)[MT * NT][64]>(&lds[0][0][0][0]);
   static_assert(sizeof(lds) >= 3 * MT * NT * 64 * sizeof(f4), "sum buffer");
@@ -328,8 +336,9 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float *__restrict__
 // of a CU in rounds of 256 times a workgroup's tiles, times what a tile costs in that
 // form next to a 4 x 4 one (measured at N 2048-32000, K 2048 and 4096, T 24-1024; 2.3 us
 // a tile at K = 2048).  All forms add up an output in the same order.  T = 201, K = 2048:
-// N = 2048 2 x 4 tiles 23.6 us, 4 x 4 39.9 (41.2 from registers); N = 11264 110 and
-// 117 (123); N = 32000 316 and 312 (329).
+// N = 2048 2 x 4 tiles 21.4 us, 4 x 4 37.1 (41.2 from registers); N = 11264 105 and
+// 112 (123); N = 32000 298 and 306 (329).  Two 2 x 2 workgroups share a CU, and the third
+// round of three shares with none: it counts 1.3 (N = 6144, T = 120 43.5 us, 4 x 4 39.7).
 template <bool PACKED>
 static void f32_gemm_many(const float *X, const float *W, float *Y, int T, int N, int K, hipStream_t s) {
   const auto tiles = [&](int mt, int nt) {
@@ -344,7 +353,8 @@ static void f32_gemm_many(const float *X, const float *W, float *Y, int T, int N
   double least = 1e30;
   for (int i = 0; i < 6; ++i) {
     const dim3 g = tiles(forms[i].mt, forms[i].nt);
-    const double c = (double)(((size_t)g.x * g.y + 255) / 256) * forms[i].mt * forms[i].nt * forms[i].cost;
+    const size_t rounds = ((size_t)g.x * g.y + 255) / 256;
+    const double c = (rounds == 3 && forms[i].mt * forms[i].nt == 4 ? 3.3 : (double)rounds) * forms[i].mt * forms[i].nt * forms[i].cost;
     if (c < least) least = c, best = i;
   }
 #define FFMI_F32_GEMM(MT, NT, PF)                                                                           \
