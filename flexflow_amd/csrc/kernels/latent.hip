@@ -1,5 +1,6 @@
 // latent.hip -- latent attention over a paged cache (latent.h).
 #include <algorithm>
+#include <type_traits>
 
 #include "device_util.h"
 #include "latent.h"
@@ -186,8 +187,8 @@ hipError_t launch_head_gemm_f32(const HeadGemm &hg, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // attention over the pages, MFMA form
 // ---------------------------------------------------------------------------
-// One workgroup of eight waves: up to RT * 16 rows against a range of 64-token
-// pages.  Scores S^T = C . Q'^T (lane: 4 keys of one row), outputs O^T = C^T .
+// Up to 32 rows (RT = 1, 2): one workgroup of eight waves, up to RT * 16 rows against a
+// range of 64-token pages.  Scores S^T = C . Q'^T (lane: 4 keys of one row), outputs O^T = C^T .
 // P^T with C^T read from the row-major page in LDS by the transposing LDS load;
 // the k order of the second product is the key order the scores already have
 // in the lanes (16-lane group g: keys 4g..4g+3 and 16+4g..).
@@ -206,7 +207,7 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
     const uint16_t *__restrict__ cache, uint16_t *__restrict__ O, float *__restrict__ slabs,
     float *__restrict__ ml, int heads, float scale_log2) {
   constexpr int R = RC * 64, KS = RC * 2, LDC = R + kRankPad;
-  constexpr int SR = RT == 4 ? 2 : 1;           // row tiles of a wave's scores
+  constexpr int SR = 1;                         // row tiles of a wave's scores
   constexpr int NT = RC * 4, DT = (NT + 7) / 8;  // column tiles: all, of a wave's outputs
   constexpr int LDP = kPageTokens + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sC[2][64 * LDC];
@@ -220,22 +221,9 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
   const bool scoring = RT > 1 || wr == 0;
   const int32_t *table = reinterpret_cast<const int32_t *>(blob) + bk.table;
 
-  // the next page: through registers, RC 16-byte chunks per thread, or (R ==
-  // 512: a row is one 1 KiB wave access) straight into LDS where those
-  // registers would not fit
-  constexpr bool DMA = RC == 8 && RT == 4;
+  // the next page through registers, RC 16-byte chunks per thread
   auto page_at = [&](int i0) {
     return cache + (size_t)(i0 == 0 ? bk.page0 : table[bk.tile0 + i0]) * (64 * R);
-  };
-  auto dma = [&](int i0, int buf) {
-    const uint16_t *page = page_at(i0);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = wave * 8 + i;
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)(page + (size_t)row * R + lane * 8),
-          (__attribute__((address_space(3))) void *)(&sC[buf][row * LDC]), 16, 0, 0);
-    }
   };
   u4 pre[RC];
   auto fetch = [&](int i0) {
@@ -250,8 +238,7 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
       *reinterpret_cast<u4 *>(&sC[buf][(c / (R / 8)) * LDC + (c % (R / 8)) * 8]) = pre[i];
     }
   };
-  if constexpr (DMA) dma(0, 0);
-  else fetch(0);
+  fetch(0);
   // this wave's rows of Q' as B operands (rows past the block re-read its last)
   bf8 q[SR][KS];
   int qpos[SR];
@@ -273,16 +260,10 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
   for (int i = 0; i < RT; ++i) m[i] = -1e30f;
 #pragma unroll
   for (int i = 0; i < SR; ++i) l[i] = 0.f;
-  if constexpr (DMA) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    stage(0);
-    if (bk.ntiles > 1) fetch(1);
-  }
+  stage(0);
+  if (bk.ntiles > 1) fetch(1);
   __syncthreads();
   for (int it = 0; it < bk.ntiles; ++it) {
-    if constexpr (DMA)  // (its buffer was last read before the previous round's last barrier)
-      if (it + 1 < bk.ntiles) dma(it + 1, (it + 1) & 1);
     const uint16_t *C = sC[it & 1];
     f4 s[SR];
     if (scoring) {
@@ -345,7 +326,7 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
         l[i] = l[i] * ai + sum;
       }
     }
-    if (!DMA && it + 1 < bk.ntiles) {
+    if (it + 1 < bk.ntiles) {
       stage((it + 1) & 1);  // (last read by the outputs of tile it - 1)
       if (it + 2 < bk.ntiles) fetch(it + 2);
     }
@@ -380,10 +361,6 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
           acc[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf8, p[i]),
                                                               acc[i][d], 0, 0, 0);
       }
-    }
-    if constexpr (DMA) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
     }
   }
   if (scoring) {
@@ -422,6 +399,279 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
                        f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
       }
     }
+  }
+}
+
+// More than 32 rows (prompts), 64 a block.  Half pages of 32 tokens: waves 0..3 copy half
+// pages to LDS, score 16 rows each against all 32 keys of a half (so that a row's maximum
+// needs no other wave) and leave the weights in LDS; waves 4..7 add a half's outputs up, a
+// quarter of the latent's columns each, one half behind.  A SIMD has a wave of either kind:
+// one's products run beside the other's exponentials and reads.  One barrier a half; two
+// halves are on their way and one in each kind's hands.  A workgroup takes block after
+// block, the next one's rows of Q' and first half copied while this one's last halves are
+// added up, its outputs stored beside the next one's first scores.
+// What bounds it: the LDS (each scoring wave reads the whole half: 128 of 210 KiB a half
+// at rank 512) at 2300 cycles a half, then Q' and O (64 KiB each a block).  Before, all
+// eight waves took turns (scores, barrier, weights, barrier, outputs, barrier a page), Q'
+// was read as it lies (16 rows a load, 256 loads) and the compiler waited for the next page
+// as soon as it was asked for.  32 heads, rank 512, prompt steps of 1024, 1024 and 620
+// tokens: 70 -> 53 us a launch, of which a page of 64 rows takes 2.2.
+// A half's rows lie one after another, the 16-byte pieces of each 256 bytes (of 128 where rows
+// are whole 128s, so that every other row starts at the other half) exchanged by the
+// row's number: a read of scores takes one piece of 16 rows, of outputs two of 8.
+template <int RC>
+constexpr int kLatentPieces = RC % 2 == 0 ? 16 : 8;
+template <int RC>
+__device__ __forceinline__ int latent_turn(int row) {
+  return RC % 2 == 0 ? (row & 7) << 1 | (row >> 3 & 1) : (row >> 1 & 3) << 1 | (row >> 3 & 1);
+}
+template <int RC>
+constexpr int kLatentWide = RC <= 4 ? 2 : 1;  // workgroups of a CU, by their LDS
+template <int RC>
+__global__ __launch_bounds__(512) void latent_attn_wide_kernel(
+    const char *__restrict__ blob, int off_blocks, int num_blocks, const uint16_t *__restrict__ Q,
+    const uint16_t *__restrict__ cache, uint16_t *__restrict__ O, float *__restrict__ slabs,
+    float *__restrict__ ml, int heads, float scale_log2) {
+  constexpr int R = RC * 64, KS = RC * 2, H = 32;  // H: tokens of a half
+  constexpr int PP = kLatentPieces<RC>, KP = PP / 4, CP = PP / 2;  // pieces, k-steps, column tiles of an exchange
+  constexpr int LDP = H + 8;
+  // (one array: of several the compiler knows which one a copy writes, and waits for all
+  // copies under way before it reads that)
+  __shared__ __attribute__((aligned(16))) uint16_t sh[4 * H * R + 2 * 64 * LDP + 2 * (2 * 64 + 2 * 64)];
+  uint16_t *sP = sh + 4 * H * R;                                // [half & 1][64][LDP]
+  float *sA = reinterpret_cast<float *>(sP + 2 * 64 * LDP);     // [half & 1][64]: what the sums so far shrink by
+  float *sM = sA + 2 * 64, *sL = sM + 64;                       // maximum and sum of a row, at a block's end
+  const PagedBlock *blocks = reinterpret_cast<const PagedBlock *>(blob + off_blocks);
+  const int lane = threadIdx.x & 63, g = lane >> 4, l15 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // this workgroup's k-th block (nrows == 0: none): the list, longest first, dealt out back and
+  // forth; padding is at its end
+  auto block_of = [&](int k) {
+    const int i = k * gridDim.x + (k & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x);
+    PagedBlock bk{};
+    if (i < num_blocks) bk = blocks[i];
+    return bk;
+  };
+  // its halves, up to the last position that its last row sees
+  auto halves_of = [&](const PagedBlock &bk) {
+    const int last = bk.pos0 + (bk.row0 + bk.nrows - 1 - bk.seg_row) / heads - bk.tile0 * 64;
+    return min(2 * bk.ntiles, last / H + 1);
+  };
+  // a barrier that leaves copies to LDS and stores under way
+  auto meet = [] {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  PagedBlock bk = block_of(0);
+  if (bk.nrows <= 0) return;
+  if (wave < 4) {
+    const int32_t *words = reinterpret_cast<const int32_t *>(blob);
+    // rows 0 .. 31 (rows past `most`: that one again) to buffer buf & 3, this wave's quarter
+    auto copy = [&](const uint16_t *src, int buf, int most) {
+#pragma unroll
+      for (int i = 0; i < RC; ++i) {
+        const int n = (wave * RC + i) * 64 + lane, row = n / (8 * RC), p = n % (8 * RC);
+        const int piece = (p & -PP) | ((p ^ latent_turn<RC>(row)) & (PP - 1));
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void *)(src + (size_t)min(row, most) * R + piece * 8),
+            (__attribute__((address_space(3))) void *)(sh + (buf & 3) * H * R + (wave * RC + i) * 512), 16, 0, 0);
+      }
+    };
+    auto copy_rows = [&](const PagedBlock &b, int part, int buf) {  // 32 rows of Q'
+      copy(Q + (size_t)(b.row0 + min(part * H, b.nrows - 1)) * R, buf, max(b.nrows - 1 - part * H, 0));
+    };
+    auto copy_half = [&](int h, int page, int buf) { copy(cache + ((size_t)page * 64 + (h & 1) * H) * R, buf, H - 1); };
+    // s_waitcnt vmcnt(RC) (the last stage asked for may still be under way) or vmcnt(0)
+    auto wait = [](bool more) {
+      if (more) __builtin_amdgcn_s_waitcnt((RC & 15) | 0x0f70 | ((RC >> 4) << 14));
+      else __builtin_amdgcn_s_waitcnt(0x0f70);
+      asm volatile("" ::: "memory");
+    };
+    // this lane's piece of a k-step
+    int at[KP];
+#pragma unroll
+    for (int i = 0; i < KP; ++i) at[i] = l15 * R + ((4 * i + g) ^ latent_turn<RC>(l15)) * 8;
+    auto piece = [&](const uint16_t *rows, int ks) {
+      return *reinterpret_cast<const bf8 *>(rows + at[ks % KP] + ks / KP * KP * 32);
+    };
+    int b0 = 0;  // half 0's buffer; the rows of Q' in the two after half 1's
+    copy_rows(bk, 0, 2);
+    copy_rows(bk, 1, 3);
+    copy_half(0, bk.page0, 0);
+    wait(false);
+    meet();
+    for (int k = 0;; ++k) {
+      const PagedBlock nb = block_of(k + 1);
+      const bool next = nb.nrows > 0;
+      const int nh = halves_of(bk);
+      auto page_of = [&](int h) { return h < 2 ? bk.page0 : words[bk.table + bk.tile0 + (min(h, nh - 1) >> 1)]; };
+      // The stages in turn: this block's halves, the next one's rows of Q' and its half 0, each
+      // in the buffer after the last one's.
+      auto stage = [&](int e, int page) {
+        if (e < nh) copy_half(e, page, b0 + e);
+        else if (next && e < nh + 2) copy_rows(nb, e - nh, b0 + e);
+        else if (next && e == nh + 2) copy_half(0, nb.page0, b0 + e);
+      };
+      auto staged = [&](int e) { return e < nh || (next && e <= nh + 2); };
+      stage(1, bk.page0);
+      int page = page_of(2);  // of the next half to be asked for: read a half ahead
+      bf8 q[KS];              // rows 16 wave + l15 as B operands
+      const uint16_t *rows = sh + ((b0 + 2 + (wave >> 1)) & 3) * H * R + (wave & 1) * 16 * R;
+#pragma unroll
+      for (int i = 0; i < KS; ++i) q[i] = piece(rows, i);
+      wait(staged(1));
+      meet();
+      stage(2, page);
+      page = page_of(3);
+      const int row = min(wave * 16 + l15, bk.nrows - 1);
+      const int see = bk.pos0 + (bk.row0 + row - bk.seg_row) / heads - bk.tile0 * 64 - 4 * g;
+      float m = -1e30f, l = 0.f;
+      auto score = [&](int h) {
+        const uint16_t *C = sh + ((b0 + h) & 3) * H * R;
+        // per 16 keys two chains (even / odd k-steps); operands read D steps ahead
+        constexpr int D = KS < 8 ? KS : 8;
+        f4 s[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) s[t][0] = s[t][1] = f4{0.f, 0.f, 0.f, 0.f};
+        bf8 c[D][2];
+        auto read = [&](int ks) {
+          c[ks % D][0] = piece(C, ks);
+          c[ks % D][1] = piece(C + 16 * R, ks);
+        };
+#pragma unroll
+        for (int ks = 0; ks < D; ++ks) read(ks);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            s[t][ks & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c[ks % D][t], q[ks], s[t][ks & 1], 0, 0, 0);
+          if (ks + D < KS) read(ks + D);
+        }
+        float v[2][4], mx = m;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[t][e] = h * H + t * 16 + e <= see ? (s[t][0][e] + s[t][1][e]) * scale_log2 : -INFINITY;
+            mx = fmaxf(mx, v[t][e]);
+          }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float shrink = __builtin_amdgcn_exp2f(m - mx);
+        float sum = 0.f;
+        uint16_t *P = sP + (((h & 1) * 64) + wave * 16 + l15) * LDP + 4 * g;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          s4 w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float x = __builtin_amdgcn_exp2f(v[t][e] - mx);
+            sum += x;
+            w[e] = (short)f2bf(x);
+          }
+          *reinterpret_cast<s4 *>(P + t * 16) = w;
+        }
+        if (g == 0) sA[(h & 1) * 64 + wave * 16 + l15] = shrink;
+        l = l * shrink + sum;
+        m = mx;
+      };
+      score(0);
+      for (int h = 0; h < nh; ++h) {
+        wait(staged(h + 2));  // stage h + 1 has landed
+        meet();
+        // (its buffer was half h - 1's, whose outputs were added up before the barrier, or Q''s)
+        stage(h + 3, page);
+        page = page_of(h + 4);
+        if (h + 1 < nh) score(h + 1);
+      }
+      l += __shfl_xor(l, 16);
+      l += __shfl_xor(l, 32);
+      if (g == 0) sM[wave * 16 + l15] = m, sL[wave * 16 + l15] = l;
+      wait(next);  // the next block's rows of Q' have landed
+      meet();
+      if (!next) return;
+      b0 = (b0 + nh + 2) & 3;
+      bk = nb;
+    }
+  }
+  const int ct0 = (wave - 4) * RC, trow = 4 * g + (l15 >> 2);
+  const int tturn = latent_turn<RC>(trow) ^ ((l15 & 3) >> 1), tbase = trow * R + (l15 & 1) * 4;
+  int b0 = 0;
+  meet();
+  meet();
+  for (int k = 0;; ++k) {
+    const PagedBlock nb = block_of(k + 1);
+    const int nh = halves_of(bk);
+    f4 acc[4][RC];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int d = 0; d < RC; ++d) acc[i][d] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < nh; ++h) {
+      meet();
+      const uint16_t *C = sh + ((b0 + h) & 3) * H * R, *P = sP + (h & 1) * 64 * LDP;
+      // 16 columns of 32 tokens, transposed: k order as the weights'
+      auto columns = [&](int d) {
+        const int ct = ct0 + d;
+        const uint16_t *p = C + tbase + ct / CP * CP * 16 + ((2 * (ct % CP)) ^ tturn) * 8;
+        const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)(p));
+        const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4 *)(p + 16 * R));
+        return __builtin_bit_cast(bf8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      };
+      bf8 p[4], a[RC];
+      float shrink[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) shrink[i] = sA[(h & 1) * 64 + i * 16 + l15];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint16_t *pr = P + (i * 16 + l15) * LDP + 4 * g;
+        const s4 lo = *reinterpret_cast<const s4 *>(pr), hi = *reinterpret_cast<const s4 *>(pr + 16);
+        p[i] = __builtin_bit_cast(bf8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+#pragma unroll
+      for (int d = 0; d < RC; ++d) a[d] = columns(d);
+      __builtin_amdgcn_sched_barrier(0);
+      if (__any(shrink[0] != 1.f || shrink[1] != 1.f || shrink[2] != 1.f || shrink[3] != 1.f))
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int d = 0; d < RC; ++d) acc[i][d] *= shrink[i];
+#pragma unroll
+      for (int d = 0; d < RC; ++d) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          acc[i][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d], p[i], acc[i][d], 0, 0, 0);
+      }
+    }
+    meet();
+    if (nb.nrows > 0) meet();  // (the next block's scores start beside the stores)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = i * 16 + l15;
+      if (r >= bk.nrows) continue;
+      const float sum = sL[r];
+      if (bk.slot >= 0) {
+        const size_t pr = (size_t)bk.slot * 64 + r;
+#pragma unroll
+        for (int d = 0; d < RC; ++d) *reinterpret_cast<f4 *>(slabs + pr * R + (ct0 + d) * 16 + 4 * g) = acc[i][d];
+        if (wave == 4 && g == 0) ml[pr * 2] = sM[r], ml[pr * 2 + 1] = sum;
+      } else {
+        const float inv = __fdiv_rn(1.0f, sum);
+        uint16_t *o = O + (size_t)(bk.row0 + r) * R + ct0 * 16 + 4 * g;
+#pragma unroll
+        for (int d = 0; d < RC; ++d) {
+          const f4 v = acc[i][d] * inv;
+          *reinterpret_cast<uint2 *>(o + d * 16) =
+              make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+        }
+      }
+    }
+    if (nb.nrows <= 0) return;
+    b0 = (b0 + nh + 2) & 3;
+    bk = nb;
   }
 }
 
@@ -495,7 +745,9 @@ hipError_t launch_latent_attention(const char *blob, const PagedLists &pl, const
   case RC:                                                                                      \
     if (pl.row_tiles == 1) FFMI_LA2(RC, 1);                                                     \
     else if (pl.row_tiles == 2) FFMI_LA2(RC, 2);                                                \
-    else if (pl.row_tiles == 4) FFMI_LA2(RC, 4);                                                \
+    else if (pl.row_tiles == 4)                                                                 \
+      hipLaunchKernelGGL((latent_attn_wide_kernel<RC>), dim3(std::min(pl.num_blocks, 256 * kLatentWide<RC>)), dim3(512), 0, s, \
+                         blob, pl.off_blocks, pl.num_blocks, q, cache, o, slabs, ml, pl.heads, sl); \
     else return hipErrorInvalidValue;                                                           \
     if (pl.num_merges > 0)                                                                      \
       hipLaunchKernelGGL((latent_merge_kernel<RC>), dim3(pl.num_merges, pl.row_tiles * 16),     \

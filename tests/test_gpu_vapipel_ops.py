@@ -137,6 +137,24 @@ def test_latent_attention_batches(heads, rank, full):
     assert np.abs(got - ref).max() < tol * np.abs(ref).max()
 
 
+# Prompts of so many rows that a workgroup takes several blocks one after another, the next one's
+# rows and first keys copied while this one ends: blocks of 1, 2, ... half pages of 32 keys, of the
+# last half only, of 64 rows and of fewer, whole and split (partial results of a few long rows).
+@pytest.mark.parametrize("heads,rank,seqs", [
+    (32, 512, [(300, 0), (270, 31), (1, 700)]), (33, 512, [(520, 63)]), (32, 384, [(33, 0)] * 17),
+    (96, 256, [(360, 5)]), (192, 192, [(200, 1000)]), (160, 128, [(430, 32)]), (96, 64, [(370, 64), (3, 8)]),
+    (40, 512, [(2, 1500), (3, 900)])])
+def test_latent_attention_blocks_in_turn(heads, rank, seqs):
+    rng = np.random.default_rng(heads + rank)
+    pages, n = paged(rng, [p0 + t for t, p0 in seqs])
+    cache = bf16(rng.standard_normal((n, 64, rank)))
+    q = bf16(rng.standard_normal((sum(t for t, _ in seqs) * heads, rank)) * 2.0)
+    got, ref = attention(q, cache, heads, rank ** -0.5, [(t, p0, pg) for (t, p0), pg in zip(seqs, pages)], False)
+    # weights and outputs are rounded to bf16, sums are fp32
+    assert np.linalg.norm(got - ref) < 2.0 ** -8 * np.linalg.norm(ref)
+    assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -8 * np.abs(cache).max()).all()
+
+
 @pytest.mark.parametrize("full", [False, True])
 @pytest.mark.parametrize("heads,rank", [(2, 64), (20, 512), (33, 128), (4, 576)])
 def test_latent_attention_finds_each_key(heads, rank, full):
