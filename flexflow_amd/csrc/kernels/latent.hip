@@ -127,6 +127,124 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const PagedToken *__re
                      (uint16_t *)st.cache, st.rank, st.n, st.eps);
 }
 
+// More than 128 rows: a workgroup takes 128 rows and 128 columns of a head, its rows through
+// LDS in chunks of 64 k, two of them and a chunk of weights on their way.  Read as they lie,
+// rows sent the lanes of a load to 16 places, which the L1 serves one after another,
+// and two k-steps of loads were all that was under way.  A row's eight 16-byte pieces lie
+// exchanged by the row's number; row-major outputs go through LDS as well and leave as
+// whole lines.  A head's workgroups share an XCD where heads are a multiple of 8: its
+// weights are read from memory once.  1024 rows, 32 heads: K = 128, N = 512 with the latents'
+// store 25 -> 21 us, K = 512, N = 128 21 -> 14.
+__device__ __forceinline__ int prep_turn(int row) { return (row >> 1 & 3) << 1 | (row >> 3 & 1); }
+template <int KC>
+__device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *sh) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, l15 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = b % a.heads, rest = b / a.heads, nt0 = (rest % a.gx) * 8, m0 = (rest / a.gx) * 128;
+  const int wm = wave >> 1, wn = wave & 1, K = KC * 64;
+  const uint16_t *x = a.X + (size_t)h * K;
+  auto copy = [&](int c) {  // 4 KiB of the chunk's 16 (8 rows a copy)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (wave * 4 + i) * 8 + (lane >> 3), piece = (lane ^ prep_turn(row)) & 7;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void *)(x + (size_t)min(m0 + row, a.T - 1) * a.ldx + c * 64 + piece * 8),
+          (__attribute__((address_space(3))) void *)(sh + c * 8192 + (wave * 4 + i) * 512), 16, 0, 0);
+    }
+  };
+  const uint16_t *w0[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w0[j] = a.W + ((size_t)h * a.NTt + min(nt0 + wn * 4 + j, a.NTt - 1)) * a.KT * 512 + lane * 8;
+  bf8 w[2][2][4];
+  auto weights = [&](int c) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[c & 1][k][j] = *reinterpret_cast<const bf8 *>(w0[j] + (size_t)(2 * c + k) * 512);
+  };
+  f4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+  copy(0);
+  if (KC > 1) copy(1);
+  weights(0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < KC; ++c) {
+    if (c + 2 < KC) copy(c + 2);
+    if (c + 1 < KC) weights(c + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // chunk c has landed, what was just asked for may be under way: s_waitcnt vmcnt
+    if (c + 2 < KC) __builtin_amdgcn_s_waitcnt(0x0f70 | 12);
+    else if (c + 1 < KC) __builtin_amdgcn_s_waitcnt(0x0f70 | 8);
+    else __builtin_amdgcn_s_waitcnt(0x0f70);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint16_t *xr = sh + c * 8192 + (wm * 64 + l15) * 64;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      bf8 xf[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        xf[i] = *reinterpret_cast<const bf8 *>(xr + i * 1024 + ((4 * k + g) ^ prep_turn(l15)) * 8);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c & 1][k][j], xf[i], acc[i][j], 0, 0, 0);
+    }
+  }
+  const int N = a.NTt * 16, Yw = a.heads * N, n0 = nt0 + wn * 4;  // (column tiles)
+  __syncthreads();
+  uint16_t *mine = sh + wave * 4096;  // 64 rows x 64 columns of this wave, pieces exchanged
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = m0 + wm * 64 + i * 16 + l15;
+    float sc = 1.f;
+    if (a.gate) sc = __fdiv_rn(1.0f, 1.0f + expf(-bf2f(a.gate[(size_t)min(m, a.T - 1) * a.ldg + h])));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f4 v = acc[i][j];
+      const uint2 o = make_uint2(f2bf(v[0] * sc) | ((uint32_t)f2bf(v[1] * sc) << 16),
+                                 f2bf(v[2] * sc) | ((uint32_t)f2bf(v[3] * sc) << 16));
+      if (a.packed) {
+        if (m < a.T && n0 + j < a.NTt)
+          *reinterpret_cast<uint2 *>(a.Y + act_packed_off(m, h * N + (n0 + j) * 16 + 4 * g, Yw)) = o;
+      } else {
+        const int piece = (2 * j + (g >> 1)) ^ prep_turn(l15);
+        *reinterpret_cast<uint2 *>(mine + (i * 16 + l15) * 64 + piece * 8 + 4 * (g & 1)) = o;
+      }
+    }
+  }
+  if (a.packed) return;
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's own writes
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = i * 8 + (lane >> 3), m = m0 + wm * 64 + row, p = lane & 7;
+    const uint4 v = *reinterpret_cast<const uint4 *>(mine + row * 64 + ((p ^ prep_turn(row & 15)) * 8));
+    if (m < a.T && n0 + (p >> 1) < a.NTt)
+      *reinterpret_cast<uint4 *>(a.Y + (size_t)m * Yw + h * N + n0 * 16 + p * 8) = v;
+  }
+}
+template <int KC>
+__global__ __launch_bounds__(256) void latent_prep_tile_kernel(const PagedToken *__restrict__ tok, HgDev a,
+                                                               int nprod, LatentStore st) {
+  __shared__ __attribute__((aligned(16))) uint16_t sh[(KC < 2 ? 2 : KC) * 8192];
+  if ((int)blockIdx.x < nprod) {
+    head_gemm_tile<KC>(a, blockIdx.x, sh);
+    return;
+  }
+  const int t = (blockIdx.x - nprod) * 4 + (threadIdx.x >> 6);
+  if (t >= a.T) return;
+  latent_store_token(tok[t], (const uint16_t *)st.d + (size_t)t * st.ldd, st.w,
+                     (uint16_t *)st.cache, st.rank, st.n, st.eps);
+}
+
 static hipError_t run_prep(const PagedToken *tok, const LatentStore &st, const HeadGemm &hg,
                            hipStream_t s) {
   if (hg.T <= 0) return hipSuccess;
@@ -145,10 +263,24 @@ static hipError_t run_prep(const PagedToken *tok, const LatentStore &st, const H
     hipLaunchKernelGGL((latent_prep_kernel<MT, NT, WM>), dim3(np + nst), dim3(256), 0, s, tok, a, \
                        np, st);                                                                 \
   } while (0)
+// (widths that heads and latents have; their rows have to fit the LDS)
+#define FFMI_PREP_TILE(KC)                                                                      \
+  do {                                                                                          \
+    a.gx = (a.NTt + 7) / 8, a.gz = (hg.T + 127) / 128;                                          \
+    const int np = a.gx * a.heads * a.gz;                                                       \
+    hipLaunchKernelGGL((latent_prep_tile_kernel<KC>), dim3(np + nst), dim3(256), 0, s, tok, a, np, st); \
+  } while (0)
   if (hg.T <= 16) FFMI_PREP(1, 1, 1);
   else if (hg.T <= 32) FFMI_PREP(2, 1, 1);
   else if (hg.T <= 128) FFMI_PREP(2, 2, 1);
+  else if (hg.K == 64) FFMI_PREP_TILE(1);
+  else if (hg.K == 128) FFMI_PREP_TILE(2);
+  else if (hg.K == 192) FFMI_PREP_TILE(3);
+  else if (hg.K == 256) FFMI_PREP_TILE(4);
+  else if (hg.K == 384) FFMI_PREP_TILE(6);
+  else if (hg.K == 512) FFMI_PREP_TILE(8);
   else FFMI_PREP(4, 4, 2);
+#undef FFMI_PREP_TILE
 #undef FFMI_PREP
   return hipGetLastError();
 }

@@ -136,6 +136,23 @@ def test_portions(engine, name, full):
         close(run(engine(name, full), toks, cuts), want, full)
 
 
+# the heads' products of more than 128 rows: a tile of 128 rows and one row more, tiles of 128
+# columns and fewer, rows of 64 k and of 4 and 6 times as many
+TILED = VM.model_config(64, 64, 300, [VM.layer(3, 256, 160, 256, 0.06, 32), VM.layer(9, 64, 256, 384, 0.12, None),
+                                      VM.layer(2, 384, 32, 64, 0.05, 32)])
+
+
+@pytest.mark.parametrize("n", [128, 129, 256])
+def test_prompts_of_whole_row_tiles_and_one_more(tmp_path, n):
+    weights = VM.random_weights(TILED, 5)
+    folder = VM.write_checkpoint(tmp_path / "m", TILED, weights)
+    m = fa.Model(fa.load_config(folder), "inc", max_requests=2, max_tokens=256, max_seq_len=300, weights_folder=folder)
+    rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=256, max_spec_tree_token_num=0,
+                           max_sequence_length=300)
+    toks = tokens(TILED, n, n)
+    close(run((rm, m), toks, [n]), R.forward(TILED, weights, toks, []), False)
+
+
 @pytest.mark.parametrize("full", [True, False])
 def test_first_tokens_and_single_token_prompts(engine, full):
     for t in range(5):
