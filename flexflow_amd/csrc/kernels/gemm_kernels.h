@@ -616,16 +616,26 @@ __global__ __launch_bounds__(WPG * 64) void gemm_wave_kernel(const uint16_t *__r
   }
 }
 
-// Split-K factor of the skinny path: only narrow layers (few column groups,
-// e.g. the 68M SSM's o/down with 48 tiles) and only when the consumer takes
-// the partial slabs (no reduce pass); keeps >= 4 k-steps per wave.
+// Split-K factor of the skinny path, only where the consumer takes the partial
+// slabs (no reduce pass).  Narrow layers (few column groups, e.g. the 68M SSM's
+// o/down with 48 tiles) fill the chip by it.  From 128 tiles on: halves, where they even out
+// what the busiest CU reads (a tile a workgroup: 384 tiles are two on half of the
+// CUs, in halves three on each).  T = 8, cold, us: N 6144 x K 4096 11.8 -> 10.5, 10240 x 4096
+// 16.4 -> 15.2, 4608 x 4096 10.5 -> 9.0, 6144 x 2048 7.4 -> 6.3, 2048 x 2048 4.7 -> 4.0, 2048 x 5632
+// 7.5 -> 6.5; T = 38, 2048 x 2048 8.0 -> 6.2; where they don't, 4096 x 4096 8.2 -> 8.8, 4096 x 11008
+// 15.6 -> 16.1.  Four slices gain little more (6144 x 4096 9.9, 6144 x 2048 6.5) and cost a
+// consumer that reads every sum several times (matrix memories) more than that.
+// A wave keeps 4 k-steps or more.
 static int skinny_split(int T, int N, int K, int epi, bool deferrable) {
   // FFMI_SKINNY_SPLIT=0 keeps every skinny launch unsplit (A/B runs)
   static const bool off = getenv("FFMI_SKINNY_SPLIT") && atoi(getenv("FFMI_SKINNY_SPLIT")) == 0;
   if (off || !deferrable || epi || T > 64) return 1;
   const int ntiles = (N + 15) / 16;
-  if (ntiles >= 128) return 1;
   const int KT = K / 32;
+  if (ntiles >= 128) {  // (tiles of the busiest CU)
+    const int whole = (ntiles + 255) / 256, halves = (2 * ntiles + 255) / 256;
+    return KT >= 32 && halves < 2 * whole ? 2 : 1;
+  }
   int S = 256 / ntiles;
   S = std::min(S, std::max(1, KT / 8));  // >= 1 k-step per wave of an 8-wave slice
   return std::max(1, std::min(S, 8));

@@ -153,6 +153,21 @@ def test_prompts_of_whole_row_tiles_and_one_more(tmp_path, n):
     close(run((rm, m), toks, [n]), R.forward(TILED, weights, toks, []), False)
 
 
+# steps of few rows, whose products of 2048 columns are summed in halves of K by the norms that
+# read them: 64 k-steps, 32 (the fewest that are split) and an odd number, rows of one to four tiles
+HALVES = VM.model_config(64, 2048, 120, [VM.layer(16, 128, 128, 64, 0.09, 1024), VM.layer(3, 352, 352, 64, 0.05, 2080)])
+
+
+def test_products_in_halves(tmp_path):
+    weights = VM.random_weights(HALVES, 6)
+    folder = VM.write_checkpoint(tmp_path / "m", HALVES, weights)
+    m = fa.Model(fa.load_config(folder), "inc", max_requests=2, max_tokens=64, max_seq_len=120, weights_folder=folder)
+    rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=64, max_spec_tree_token_num=0,
+                           max_sequence_length=120)
+    toks = tokens(HALVES, 116, 7)
+    close(run((rm, m), toks, [1, 16, 17, 1, 64, 15, 1, 1]), R.forward(HALVES, weights, toks, []), False)
+
+
 @pytest.mark.parametrize("full", [True, False])
 def test_first_tokens_and_single_token_prompts(engine, full):
     for t in range(5):
