@@ -994,7 +994,8 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 //    the barrier (a counted s_waitcnt vmcnt, never 0 in the steady state, and
 //    a raw s_barrier: __syncthreads would drain the DMAs);
 //  * the loop body has no branches (a step without a next one is a separate
-//    instantiation; waves past the last fragment load it again), and
+//    instantiation; waves past the last fragment load it again, or see
+//    kExactCopies), and
 //    sched_barrier pins MFMA group / LDS read / DMA in turn: left alone the
 //    compiler collects the reads behind the MFMAs and waits for them;
 //  * a wave's MFMA groups run at raised priority, so that of the two waves of
@@ -1013,15 +1014,20 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // copies.  T = 216: K 11008 x N 4096 35.4 us either way, 12288 x 4096 39.2 and 39.1; with
 // two row blocks the second one's reads miss (4096 x 4096 21.3 -> 25.3, gate/up 55.3
 // -> 63.6), which therefore go without the hint.
+// A stage whose fragments the waves do not share evenly: the last waves copy one less
+// (two instances of the loop, one per count; each waits for its own copies).  Twelve
+// waves only, of which 6 and 10 would copy for nothing; the forms of eight gain nothing
+// from it (400 products of 200 .. 1024 rows: 0.2% slower to 0.3% faster a form).
+template <int MI, int NJ, int WR, int WC>
+static constexpr bool kExactCopies = WR * WC > 8 && (MI * WR + NJ * WC) % (WR * WC) != 0;
 template <int EPI, int MI, int NJ, int WR, int WC, int NB, bool NTL>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
     const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wp, uint16_t *__restrict__ Y,
     float *__restrict__ Yf, int T, int N, int KT, int NTILES, int nbm, int S, int xp, int yp,
     size_t wts, size_t wks, float lim) {
   constexpr int NW = WR * WC, FX = MI * WR, F = FX + NJ * WC;  // waves; fragments of a stage
-  constexpr int PW = (F + NW - 1) / NW;                        // DMAs per wave and stage
-  static_assert(NB >= 3 && (NB - 1) * PW < 64, "stages in flight");
-  static_assert(!NTL || FX % NW == 0, "a wave's copy is of X or of weights, known to the compiler");
+  constexpr int PMAX = (F + NW - 1) / NW;                      // DMAs per wave and stage
+  static_assert(NB >= 3 && (NB - 1) * PMAX < 64, "stages in flight");
   __shared__ __attribute__((aligned(1024))) h8 lds[NB][F][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1031,101 +1037,110 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
   const int bm = L % nbm, ks = L / nbm % S, bn = L / (nbm * S);
   // this slice's k-steps: [kb, kb + n), n >= 1 (tile_plan)
   const int per = (KT + S - 1) / S, kb = ks * per, n = min(KT, kb + per) - kb;
-  // this wave's fragments f = wave + NW p of a stage: X row tile f (< FX) or
-  // weight tile f - FX (the last rows / tile again past the end)
-  const uint16_t *src[PW];
-  size_t step[PW];
-#pragma unroll
-  for (int p = 0; p < PW; ++p) {
-    const int f = min(wave + NW * p, F - 1);
-    if (f >= FX) {
-      src[p] = Wp + (size_t)min(bn * (F - FX) + f - FX, NTILES - 1) * wts + (size_t)kb * wks + lane * 8;
-      step[p] = wks;
-    } else if (xp) {
-      src[p] = X + ((size_t)min(bm * FX + f, (T - 1) >> 4) * KT + kb) * 512 + lane * 8;
-      step[p] = 512;
-    } else {
-      const int row = min((bm * FX + f) * 16 + (lane & 15), T - 1);
-      src[p] = X + ((size_t)row * KT + kb) * 32 + 8 * (lane >> 4);
-      step[p] = 32;
-    }
-  }
-  auto issue = [&](int kt, int slot, int p) {
-    const auto from = (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kt * step[p]);
-    const auto to = (__attribute__((address_space(3))) void *)(&lds[slot][min(wave + NW * p, F - 1)][0]);
-    // (cache policy 2: non-temporal)
-    if (NTL && wave + NW * p >= FX) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
-    else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
-  };
   const int wm = wave / WC, wn = wave % WC;
   f4 acc[MI][NJ];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  // (fewer steps than stages: the last step again, into slots nobody reads)
+  auto loop = [&](auto PWc) __attribute__((always_inline)) {
+    constexpr int PW = decltype(PWc)::value;
+    // this wave's fragments f = wave + NW p of a stage: X row tile f (< FX) or
+    // weight tile f - FX (the last rows / tile again past the end)
+    const uint16_t *src[PW];
+    size_t step[PW];
 #pragma unroll
-  for (int kt = 0; kt < NB; ++kt) {
+    for (int p = 0; p < PW; ++p) {
+      const int f = min(wave + NW * p, F - 1);
+      if (f >= FX) {
+        src[p] = Wp + (size_t)min(bn * (F - FX) + f - FX, NTILES - 1) * wts + (size_t)kb * wks + lane * 8;
+        step[p] = wks;
+      } else if (xp) {
+        src[p] = X + ((size_t)min(bm * FX + f, (T - 1) >> 4) * KT + kb) * 512 + lane * 8;
+        step[p] = 512;
+      } else {
+        const int row = min((bm * FX + f) * 16 + (lane & 15), T - 1);
+        src[p] = X + ((size_t)row * KT + kb) * 32 + 8 * (lane >> 4);
+        step[p] = 32;
+      }
+    }
+    auto issue = [&](int kt, int slot, int p) {
+      const auto from = (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kt * step[p]);
+      const auto to = (__attribute__((address_space(3))) void *)(&lds[slot][min(wave + NW * p, F - 1)][0]);
+      // (cache policy 2: non-temporal)
+      if (NTL && wave + NW * p >= FX) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
+      else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+    };
+    // (fewer steps than stages: the last step again, into slots nobody reads)
 #pragma unroll
-    for (int p = 0; p < PW; ++p) issue(min(kt, n - 1), kt, p);
-  }
-  h8 xf[MI], wa[NJ], wb[NJ];
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 1) * PW) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+    for (int kt = 0; kt < NB; ++kt) {
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) wa[j] = lds[0][FX + wn * NJ + j][lane];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) xf[i] = lds[0][wm * MI + i][lane];
-  int slot = 0;
-  // Step kt on xf / wc, with step kt + 1's fragments read into xf / wx.  The
-  // wait leaves the NB - 2 stages after kt + 1 in flight and retires this
-  // wave's own reads of stage kt (issued a step ago); behind the barrier stage
-  // kt + 1 is there for every wave and stage kt's slot is free for kt + NB.
-  // MORE: step kt + NB exists.  (The last step reads a stale slot unused.)
-  auto kstep = [&](auto MOREc, h8(&wc)[NJ], h8(&wx)[NJ], int kt) {
-    constexpr bool MORE = decltype(MOREc)::value;
-    constexpr int VM = MORE ? (NB - 2) * PW : 0;
-    const int nslot = slot + 1 == NB ? 0 : slot + 1;
-    // s_waitcnt vmcnt(VM) lgkmcnt(0)
-    __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+      for (int p = 0; p < PW; ++p) issue(min(kt, n - 1), kt, p);
+    }
+    h8 xf[MI], wa[NJ], wb[NJ];
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 1) * PW) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      __builtin_amdgcn_s_setprio(1);
+    for (int j = 0; j < NJ; ++j) wa[j] = lds[0][FX + wn * NJ + j][lane];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j)  // D = W . X^T (see mid_store)
-        acc[i][j] = mma16<EPI>(wc[j], xf[i], acc[i][j]);
-      xf[i] = lds[nslot][wm * MI + i][lane];
+    for (int i = 0; i < MI; ++i) xf[i] = lds[0][wm * MI + i][lane];
+    int slot = 0;
+    // Step kt on xf / wc, with step kt + 1's fragments read into xf / wx.  The
+    // wait leaves the NB - 2 stages after kt + 1 in flight and retires this
+    // wave's own reads of stage kt (issued a step ago); behind the barrier stage
+    // kt + 1 is there for every wave and stage kt's slot is free for kt + NB.
+    // MORE: step kt + NB exists.  (The last step reads a stale slot unused.)
+    auto kstep = [&](auto MOREc, h8(&wc)[NJ], h8(&wx)[NJ], int kt) {
+      constexpr bool MORE = decltype(MOREc)::value;
+      constexpr int VM = MORE ? (NB - 2) * PW : 0;
+      const int nslot = slot + 1 == NB ? 0 : slot + 1;
+      // s_waitcnt vmcnt(VM) lgkmcnt(0)
+      __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
 #pragma unroll
-      for (int j = i * NJ / MI; j < (i + 1) * NJ / MI; ++j) wx[j] = lds[nslot][FX + wn * NJ + j][lane];
-      if constexpr (MORE) {
+      for (int i = 0; i < MI; ++i) {
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int p = i * PW / MI; p < (i + 1) * PW / MI; ++p) issue(kt + NB, slot, p);
+        for (int j = 0; j < NJ; ++j)  // D = W . X^T (see mid_store)
+          acc[i][j] = mma16<EPI>(wc[j], xf[i], acc[i][j]);
+        xf[i] = lds[nslot][wm * MI + i][lane];
+#pragma unroll
+        for (int j = i * NJ / MI; j < (i + 1) * NJ / MI; ++j) wx[j] = lds[nslot][FX + wn * NJ + j][lane];
+        if constexpr (MORE) {
+#pragma unroll
+          for (int p = i * PW / MI; p < (i + 1) * PW / MI; ++p) issue(kt + NB, slot, p);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_sched_barrier(0);
+      slot = nslot;
+    };
+    const auto yes = std::integral_constant<bool, true>{};
+    const auto no = std::integral_constant<bool, false>{};
+    int kt = 0;
+    for (; kt + 2 + NB <= n; kt += 2) {
+      kstep(yes, wa, wb, kt);
+      kstep(yes, wb, wa, kt + 1);
     }
-    slot = nslot;
-  };
-  const auto yes = std::integral_constant<bool, true>{};
-  const auto no = std::integral_constant<bool, false>{};
-  int kt = 0;
-  for (; kt + 2 + NB <= n; kt += 2) {
-    kstep(yes, wa, wb, kt);
-    kstep(yes, wb, wa, kt + 1);
-  }
-  if (kt + 1 + NB <= n) {
-    kstep(yes, wa, wb, kt++);
+    if (kt + 1 + NB <= n) {
+      kstep(yes, wa, wb, kt++);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
-  }
+      for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
+    }
 #pragma unroll 1
-  for (; kt < n; ++kt) {
-    kstep(no, wa, wb, kt);
+    for (; kt < n; ++kt) {
+      kstep(no, wa, wb, kt);
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
+      for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
+    }
+  };
+  if constexpr (kExactCopies<MI, NJ, WR, WC>) {
+    if (wave < F % NW) loop(std::integral_constant<int, PMAX>{});
+    else loop(std::integral_constant<int, PMAX - 1>{});
+  } else {
+    loop(std::integral_constant<int, PMAX>{});
   }
   mid_store<MI, NJ, EPI>(acc, Y, Yf, T, N, NTILES, S, ks, bn * (F - FX) + wn * NJ,
                          (bm * FX + wm * MI) * 16, lane, yp, lim);
@@ -1369,6 +1384,26 @@ static bool use_tiles(int T, int N, int K, bool paired, bool xp, bool f32, bool 
   return T > 192 && !tile_plan(T, N, K, paired, f32, deferred).msplit[xp];
 }
 
+// Products of 65 .. 192 rows of which the M-split plan gives a workgroup six weight tiles
+// (96 columns): its waves then hold 2 or 3 x 6 accumulators and each copies six KiB of
+// weights and its own rows a step, one stage ahead.  Twelve waves, 2 or 3 x 2
+// accumulators each, keep 3 or 4 stages in flight and share every copy.  Cold weights,
+// M-split / this at T = 82, 128, 168, 192 (us): gate/up 2 x 11008 x 4096 43.2 / 37.2,
+// 44.6 / 39.6, 51.6 / 47.5, 53.0 / 47.4; 12288 x 4096 in 2 slices 23.7 / 21.6, 25.7 / 23.7,
+// 29.3 / 27.4, 30.2 / 28.2; 6144 x 4096 in 4 14.9 / 13.2, 16.0 / 15.1, 17.5 / 16.9, 18.7 / 17.8.
+// Where the plan has other widths the M-split kernel stays ahead of every form tried
+// (32000 x 4096 at T = 168, 128 columns, 62.9 against 62.2 .. 91; 4096 x 11008, 64
+// columns in 8 slices, 24.4 against 25.5 .. 34; 4096 x 4096 13.6 against 14.0 .. 17.6).
+// Over 348 such products (K 128 .. 8192, N 2048 .. 24576) this is 1.10 times as fast: 1.03
+// to 1.09 from K = 2048 on, 1.06 to 1.28 below, the slowest 0.96.
+// Packed activations; no slice without k-steps; not where the M-split kernel is to
+// write its timeline (FFMI_GEMM_STAMP).
+static bool takes_six(int T, int K, int NTW, int S, bool packed) {
+  static const bool stamp = getenv("FFMI_GEMM_STAMP") != nullptr;
+  const int KT = K / 32, steps = (KT + S - 1) / S;
+  return packed && !stamp && K % 32 == 0 && T <= 192 && NTW == 6 && (S - 1) * steps < KT;
+}
+
 // split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;
 // aligned: activations on 16-byte boundaries, as a model's own are (those the tile
 // kernel takes it takes always: the M-split plans, a microsecond, are not asked for)
@@ -1503,6 +1538,34 @@ static hipError_t run_tiles(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, 
   return hipGetLastError();
 }
 
+// Up to 192 rows in one block, 96 columns a workgroup: the tile kernel with 12 waves
+// in the M-split kernel's place, at its split of K (the same bits in the same slabs).
+template <int E>
+static hipError_t run_six(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws, int T, int N, int K,
+                          hipStream_t s, int yp, int S, Partials *defer, bool nt, int wpitch, float lim) {
+  constexpr bool paired = epi_paired<E>, f32 = epi_f32<E>;
+  const int KT = K / 32, ntiles = (N + 15) / 16 * (paired ? 2 : 1);
+  const size_t wts = w_tile_stride(KT), wks = w_k_stride(wpitch ? wpitch : ntiles);
+  const dim3 grid((ntiles + 5) / 6 * S), block(768);
+#define FFMI_SIX(MI, NB, NL)                                                                               \
+  hipLaunchKernelGGL((gemm_tile_kernel<E, MI, 2, 4, 3, NB, NL>), grid, block, 0, s, X, Wp, Y, ws, T, N, KT, \
+                     ntiles, 1, S, 1, yp, wts, wks, lim)
+  if (T <= 128) {
+    if (nt) FFMI_SIX(2, 5, true);
+    else FFMI_SIX(2, 5, false);
+  } else {
+    if (nt) FFMI_SIX(3, 4, true);
+    else FFMI_SIX(3, 4, false);
+  }
+#undef FFMI_SIX
+  if (defer && ((S > 1 && !paired) || f32)) {
+    defer->p = ws, defer->S = S, defer->NP = ntiles * 16;
+    return hipGetLastError();
+  }
+  if (S > 1 && !f32) return run_reduce<E>(ws, Y, T, N, ntiles, S, yp, lim, s);
+  return hipGetLastError();
+}
+
 // E: the epilogue kind.  Kind 4 takes its slab buffer in `ws` (at least
 // T * ntiles * 16 floats) and reports it in *defer; without `defer` it runs
 // unsplit, [T][ntiles * 16] in `ws`.
@@ -1552,7 +1615,11 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
     const MidPlan p = mid_plan(T, N, K, paired, defer != nullptr && !paired);
 #define FFMI_RUN(M, NW) \
   return run_mid<E, M, NW, 4>(X, Wp, Y, ws, ws_bytes, T, N, K, s, xp, yp, SM, defer, nt, wpitch, lim)
-    const int SM = epi_f32<E> && !defer ? 1 : p.S;
+    int SM = epi_f32<E> && !defer ? 1 : p.S;
+    if (SM > 1 && (!ws || ws_bytes < (size_t)SM * T * ((N + 15) / 16 * 16 << paired) * sizeof(float)))
+      SM = 1;  // no workspace: un-split (slower)
+    if (takes_six(T, K, p.NTW, SM, xp && aligned))
+      return run_six<E>(X, Wp, Y, ws, T, N, K, s, yp, SM, defer, nt, wpitch, lim);
     if (p.MTW == 3) {
       if (p.NTW == 2) FFMI_RUN(3, 2);
       if (p.NTW == 4) FFMI_RUN(3, 4);

@@ -107,3 +107,31 @@ def test_weight_stream(T, N, K, epi, form):
         got.append(y.get())
         assert np.isfinite(got[-1][:T]).all() and np.isnan(got[-1][T]).all()
     assert np.array_equal(*(g[:T].view(np.uint16) for g in got))
+
+
+# 65 .. 192 rows, 96 columns a workgroup: edges of the row tiles and of the two row counts,
+# columns past the last whole tile of 96, one k-step to more than the ring's stages, in and
+# out of K slices.  Row-major activations of these sizes take the M-split kernel, whose
+# order of sums is the same.
+@pytest.mark.parametrize("stream", [0, F.W_STREAM])
+@pytest.mark.parametrize("T", [65, 81, 128, 129, 176, 192])
+@pytest.mark.parametrize("N,K,epi", [(16392, 32, 0), (20008, 96, 0), (16392, 160, 0), (16400, 512, 0), (8224, 32, 1),
+                                     (11040, 288, 1), (4120, 2560, 0)])
+def test_twelve_waves(T, N, K, epi, stream):
+    L = F.lib()
+    rng = np.random.default_rng(zlib.crc32(f"{T}:{N}:{K}".encode()))
+    x = f16(rng.standard_normal((T, K)))
+    W = [f16(rng.uniform(-0.05, 0.05, (N, K))) for _ in range(1 + epi)]
+    dev = [Buf(w) for w in W]
+    Wp = Buf.empty(((1 + epi) * L.ffmi_linear_packed_bytes(N, K) // 2,), np.uint16)
+    F.check(L.ffmi_linear_pack_gate_up(dev[0].ptr, dev[1].ptr, N, K, Wp.ptr, None) if epi else
+            L.ffmi_linear_pack_weight(dev[0].ptr, N, K, Wp.ptr, None))
+    Xr, Xp = Buf(x), Buf(pack_act_np(x))
+    y, z = (Buf(np.full((T + 1, N), np.nan, np.float16)) for _ in range(2))
+    F.check(L.ffmi_linear(Xp.ptr, Wp.ptr, y.ptr, T, N, K, epi | F.X_PACKED | stream, None))
+    F.check(L.ffmi_linear(Xr.ptr, Wp.ptr, z.ptr, T, N, K, epi | stream, None))
+    y, z = y.get(), z.get()
+    assert np.isnan(y[T]).all() and np.isfinite(y[:T]).all()
+    assert np.array_equal(y[:T].view(np.uint16), z[:T].view(np.uint16))
+    if not epi and T in (65, 192) and K < 512:
+        close16(y[:T], O.linear(x.astype(np.float32), W[0].astype(np.float32), fp16=1))
