@@ -406,11 +406,15 @@ ffmi_status attn_forward(ffmi_attn *h, const ffmi_batch_dev *b, const void *qkv,
     // DT_FLOAT: commits (TREE), then RoPE + KV store (+ staging), then the
     // attention (kernels/f32.hip)
     FFMI_CHECK(qkv && qkvp.S == 0 && !(opa && opa->wo), FFMI_ERR_INVALID);
+    // (in one launch a token's output is written while others' rows of qkv are still read)
+    const char *in = (const char *)qkv, *to = (const char *)out;
+    const size_t row = (size_t)heads * d * sizeof(float);
+    const bool apart = to + b->num_tokens * row <= in || in + b->num_tokens * 3 * row <= to;
     FFMI_HIP(ffmi::launch_update_attention_f32(b->dev, b->num_tokens, tree ? b->num_commits : 0,
                                                (const float *)qkv, h->rope, h->slots, (float *)h->qbuf,
                                                (float *)h->kc, (float *)h->vc,
                                                tree ? (float *)h->stage : nullptr, (float *)out, heads, d,
-                                               h->slots, h->cfg.qk_scale, b->distinct_reqs, s));
+                                               h->slots, h->cfg.qk_scale, b->distinct_reqs && apart, s));
     return FFMI_OK;
   }
   uint16_t *stage_wr = nullptr, *stage_rd = nullptr;

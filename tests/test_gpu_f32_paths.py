@@ -85,3 +85,17 @@ def test_attention_passes(d, lens):
     infos = [(7, n, r, n, n + 1, 0, 0, 0) for r, n in lens.items()]
     out, qs = c.run(infos, rng=rng)
     c.check(out[:len(infos)], np.stack([c.ref_row(qs[t], i[2], range(i[1] + 1)) for t, i in enumerate(infos)]))
+
+
+# outputs in the queries' own buffer, from its start or overlapping its end: as in a buffer of their own
+@pytest.mark.parametrize("at", [0, 1, 2])
+def test_attention_output_in_its_input(at):
+    T, c = 4, AttnCase(F.ATTN_INC, heads=8, d=128, max_seq=256, max_tokens=512, fp32=True)
+    c.run([(3, p, r, p, p + 1, 0, 0, 0) for r in range(T) for p in range(40 + r)], rng=np.random.default_rng(1))
+    want, _ = c.run([(7, 40 + r, r, 40 + r, 41 + r, 0, 0, 0) for r in range(T)], rng=np.random.default_rng(2))
+    qkv = np.random.default_rng(2).standard_normal((T, 3 * c.Hl)).astype(np.float32)
+    off = (0, 5, 3 * T - 1)[at] * c.Hl
+    buf = Buf(np.concatenate([qkv.ravel(), np.zeros(T * c.Hl, np.float32)]))
+    F.check(K.L.ffmi_attn_inc(c.h, c.b, buf.ptr, ctypes.c_void_p(buf.ptr.value + 4 * off), None))
+    got = buf.get()[off:off + T * c.Hl].reshape(T, c.Hl)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
