@@ -77,6 +77,17 @@ extern "C" ffmi_status ffmi_latent_attention(const void *q, const void *cache, i
   st = step.stage(ids.data(), segs, nullptr, 0);
   if (st != FFMI_OK) return st;
   FFMI_HIP(hipMemcpy(step.dev, step.host, step.bytes, hipMemcpyHostToDevice));
+  // (blocks of 64 rows copy rows and keys to LDS 16 bytes at a time)
+  DeviceBuf qa, ca;
+  auto on16 = [&](const void *&p, DeviceBuf &buf, size_t bytes) {
+    if (!mfma || step.lists(heads).row_tiles < 4 || ((uintptr_t)p & 15) == 0) return FFMI_OK;
+    if (!buf.get(bytes)) return FFMI_ERR_OOM;
+    FFMI_HIP(hipMemcpyAsync(buf.p, p, bytes, hipMemcpyDeviceToDevice, nullptr));
+    p = buf.p;
+    return FFMI_OK;
+  };
+  if ((st = on16(q, qa, (size_t)T * heads * rank * 2)) != FFMI_OK) return st;
+  if ((st = on16(cache, ca, (size_t)pages * kPageTokens * rank * 2)) != FFMI_OK) return st;
   DeviceBuf slabs, ml;
   if (!slabs.get(mfma ? (size_t)kSlots * 64 * rank * 4 : 0) || !ml.get((size_t)kSlots * 64 * 8))
     return FFMI_ERR_OOM;

@@ -188,3 +188,23 @@ def test_latent_attention_rejects_bad_tables():
     L = F.lib()
     assert L.ffmi_latent_attention(q.ptr, c.ptr, 2, q.ptr, 2, 64, 1.0, ctypes.byref(s), 1, 0) == 1
     assert L.ffmi_latent_attention(q.ptr, c.ptr, 2, q.ptr, 2, 72, 1.0, ctypes.byref(s), 1, 0) == 5
+
+
+# rows and keys that start 2, 8 or 14 bytes past a 16-byte boundary, in blocks of 64 rows: the same bits
+@pytest.mark.parametrize("rank", [64, 192, 512])
+def test_latent_attention_off_16_bytes(rank):
+    rng, heads, n = np.random.default_rng(rank), 8, 150
+    pages, total = paged(rng, [n])
+    q, cache = (bf16_bits(bf16(rng.standard_normal(k))) for k in ((n * heads, rank), (total, 64, rank)))
+    table = np.ascontiguousarray(pages[0], np.int32)
+    seq = F.PagedSeq(n, 0, table.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)))
+    got = []
+    for skip in ((0, 0), (1, 0), (0, 4), (7, 1)):
+        bq, bc = (Buf(np.concatenate([np.zeros(k, np.uint16), v.ravel()])) for k, v in zip(skip, (q, cache)))
+        bo = Buf.empty(q.shape, np.uint16)
+        F.check(F.lib().ffmi_latent_attention(ctypes.c_void_p(bq.ptr.value + 2 * skip[0]),
+                                              ctypes.c_void_p(bc.ptr.value + 2 * skip[1]), total, bo.ptr, heads, rank,
+                                              rank ** -0.5, ctypes.byref(seq), 1, 0))
+        got.append(bo.get())
+    assert np.isfinite(to_f32(got[0])).all() and got[0].any()
+    assert all(np.array_equal(got[0], g) for g in got[1:])
