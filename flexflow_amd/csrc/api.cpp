@@ -198,9 +198,12 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
     }
   }
   b->distinct_reqs = d->num_tokens <= 64;
-  for (int t = 1; t < d->num_tokens && b->distinct_reqs; ++t)
-    for (int u = 0; u < t; ++u)
-      if (d->tokens[u].req == d->tokens[t].req) b->distinct_reqs = false;
+  uint64_t met[16] = {};
+  for (int t = 0; t < d->num_tokens && b->distinct_reqs; ++t) {
+    const unsigned r = (unsigned)d->tokens[t].req;
+    b->distinct_reqs = r < 1024 && !(met[r >> 6] >> (r & 63) & 1);
+    if (b->distinct_reqs) met[r >> 6] |= 1ull << (r & 63);
+  }
   b->commit_overlap = false;
   for (int c = 0; c < d->num_commits && !b->commit_overlap; ++c)
     for (int t = 0; t < d->num_tokens; ++t)
