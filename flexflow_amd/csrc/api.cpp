@@ -531,7 +531,7 @@ static size_t packed_behind(size_t slab) { return (slab + 255) & ~(size_t)255; }
 
 extern "C" size_t ffmi_linear_workspace_bytes(int T, int out_dim, int in_dim, int epilogue) {
   if (T <= 0 || out_dim <= 0 || in_dim <= 0) return 0;
-  const size_t slab = ffmi::gemm_workspace_bytes(T, out_dim, in_dim, epilogue);
+  const size_t slab = linear_slab_bytes(T, out_dim, in_dim, epilogue);
   return pack_first(T, out_dim, in_dim, epilogue) ? packed_behind(slab) + ffmi::packed_act_bytes(T, in_dim) : slab;
 }
 

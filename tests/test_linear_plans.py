@@ -74,3 +74,10 @@ def test_every_tile_form_is_tested(epi, monkeypatch):
     for T, N, K, e, form, sliced in G.FORMS:
         got = tiles(T, N, K, e)
         assert (got[0], got[1] > 1) == (form, sliced)
+
+
+# up to 64 rows a call of its own never splits K: nothing to keep
+@pytest.mark.parametrize("T", [1, 16, 64])
+@pytest.mark.parametrize("N,K", [(768, 768), (2048, 2048), (6144, 2048), (12320, 4096), (32000, 768)])
+def test_few_rows_need_no_workspace(T, N, K):
+    assert F.lib().ffmi_linear_workspace_bytes(T, N, K, 0) == 0
