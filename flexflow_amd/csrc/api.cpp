@@ -1237,6 +1237,11 @@ extern "C" int ffmi_debug_linear_tiles(int T, int out_dim, int in_dim, int epilo
   return ffmi::gemm_tile_form(T, out_dim, in_dim, epilogue, slices ? slices : &one);
 }
 
+extern "C" int ffmi_debug_few_rows_slices(int T, int out_dim, int in_dim) {
+  if (T <= 0 || T > 64 || out_dim <= 0 || in_dim <= 0) return -1;
+  return ffmi::gemm_few_rows_slices(T, out_dim, in_dim);
+}
+
 extern "C" long ffmi_debug_gemm_stamps(long long *dst, long max_waves) {
   return ffmi::gemm_debug_stamps(dst, max_waves);
 }

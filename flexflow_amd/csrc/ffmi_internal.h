@@ -254,6 +254,8 @@ hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float
 // The form (kTileForms) and K slices in which the tile kernel takes a product of its
 // own (no consumer of slabs), -1 where another kernel takes it
 int gemm_tile_form(int T, int N, int K, int epilogue, int *slices);
+// K slices of a product of up to 64 rows whose consumer sums the slabs
+int gemm_few_rows_slices(int T, int N, int K);
 // row-major activations are better packed first for the tile kernel
 bool gemm_pack_pays(int T, int N, int K, int epilogue);
 // (aligned: X on a 16-byte boundary)

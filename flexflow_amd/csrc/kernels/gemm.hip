@@ -42,6 +42,8 @@ int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
   return p.form;
 }
 
+int gemm_few_rows_slices(int T, int N, int K) { return skinny_split(T, N, K, 0, true); }
+
 // A k-step of row-major operands takes the tile kernel about 0.12 us longer, all of a
 // slice's one after another: long slices, and unsplit ones on few CUs.  T = 257, M-split
 // kernel (which split them) / tiles / packed and tiles: 2048 x 2048 16.8 / 21.0 / 16.2 us,

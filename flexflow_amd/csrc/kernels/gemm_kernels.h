@@ -620,10 +620,21 @@ __global__ __launch_bounds__(WPG * 64) void gemm_wave_kernel(const uint16_t *__r
 // slabs (no reduce pass).  Narrow layers (few column groups, e.g. the 68M SSM's
 // o/down with 48 tiles) fill the chip by it.  From 128 tiles on: halves, where they even out
 // what the busiest CU reads (a tile a workgroup: 384 tiles are two on half of the
-// CUs, in halves three on each).  T = 8, cold, us: N 6144 x K 4096 11.8 -> 10.5, 10240 x 4096
-// 16.4 -> 15.2, 4608 x 4096 10.5 -> 9.0, 6144 x 2048 7.4 -> 6.3, 2048 x 2048 4.7 -> 4.0, 2048 x 5632
-// 7.5 -> 6.5; T = 38, 2048 x 2048 8.0 -> 6.2; where they don't, 4096 x 4096 8.2 -> 8.8, 4096 x 11008
-// 15.6 -> 16.1.  Four slices gain little more (6144 x 4096 9.9, 6144 x 2048 6.5) and cost a
+// CUs, in halves three on each).  Cold, us, T = 4, 24 and 64: N 6144 x K 4096 11.6 -> 10.3, 15.6 -> 13.5,
+// 23.2 -> 19.3; 4608 x 4096 10.6 -> 9.1, 14.5 -> 12.2, 22.7 -> 18.6; 6144 x 2048 7.5 -> 6.8, 9.6 -> 8.5, 14.1 ->
+// 11.9; 2048 x 2048 4.7 -> 4.0, 6.2 -> 4.9, 8.8 -> 6.7; where they don't, at T = 8, 4096 x 4096 8.2 -> 8.8,
+// 4096 x 11008 15.6 -> 16.1.  From 512 tiles on and more than 16 rows a workgroup takes two
+// tiles (dispatch_nt), and the split is the same for all rows (a row's order of sums does not
+// depend on how many there are), so both grids have to gain: 600 tiles, 9600 x 4096, 15.8 ->
+// 14.3, 22.4 -> 19.1, 31.0 -> 25.1; but 786 tiles, 12576 x 4096, 20.1 -> 18.4, then 23.7 -> 24.6 and 31.9 ->
+// 32.3, and 1376, 22016 x 4096, 29.9 -> 28.1, 33.6 -> 34.2, 45.7 -> 47.9 (two rounds and a half of
+// two tiles are as good as three).  Nor what gemm_wave_kernel takes, whole K only: 22016 x 1024
+// 10.4 -> 11.4, 12.2 -> 17.2, 17.4 -> 21.0.
+// A tensor-parallel layer's column chunk is such a product too, its slabs summed by the
+// all-reduce's copy-in (at most 1 MB more to read): 2048 x 1376 4.9 -> 3.7, 5.9 -> 4.5, 7.8 -> 6.0;
+// 2048 x 2752 5.8 -> 5.3, 7.7 -> 6.4, 10.4 -> 8.0; 2048 x 5504 8.1 -> 6.5, 11.3 -> 8.5, 17.3 -> 10.8; 2048 x 1024
+// 3.7 -> 3.6, 4.6 -> 4.3, 6.4 -> 5.2.
+// Four slices gain little more (6144 x 4096 9.9, 6144 x 2048 6.5) and cost a
 // consumer that reads every sum several times (matrix memories) more than that.
 // A wave keeps 4 k-steps or more.
 static int skinny_split(int T, int N, int K, int epi, bool deferrable) {
@@ -632,9 +643,10 @@ static int skinny_split(int T, int N, int K, int epi, bool deferrable) {
   if (off || !deferrable || epi || T > 64) return 1;
   const int ntiles = (N + 15) / 16;
   const int KT = K / 32;
-  if (ntiles >= 128) {  // (tiles of the busiest CU)
-    const int whole = (ntiles + 255) / 256, halves = (2 * ntiles + 255) / 256;
-    return KT >= 32 && halves < 2 * whole ? 2 : 1;
+  if (ntiles >= 128) {
+    const auto evens = [](int wgs) { return (2 * wgs + 255) / 256 < 2 * ((wgs + 255) / 256); };
+    if (KT < 32 || (ntiles >= 1024 && KT <= 32)) return 1;
+    return evens(ntiles) && (ntiles < 512 || evens((ntiles + 1) / 2)) ? 2 : 1;
   }
   int S = 256 / ntiles;
   S = std::min(S, std::max(1, KT / 8));  // >= 1 k-step per wave of an 8-wave slice

@@ -667,6 +667,8 @@ ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const float *ss_i
 /* Test hook: the tile size (0 ..) and K slices in which ffmi_linear's tile kernel
  * takes a product on 16-byte boundaries, -1 where another kernel takes it. */
 int ffmi_debug_linear_tiles(int T, int out_dim, int in_dim, int epilogue, int *slices);
+/* Test hook: the K slices of a model's product of up to 64 rows whose consumer sums them. */
+int ffmi_debug_few_rows_slices(int T, int out_dim, int in_dim);
 
 /* Diagnostics: with FFMI_GEMM_STAMP set in the environment, M-split GEMM
  * launches record per-wave timestamps; copies the last launch's records

@@ -81,3 +81,14 @@ def test_every_tile_form_is_tested(epi, monkeypatch):
 @pytest.mark.parametrize("N,K", [(768, 768), (2048, 2048), (6144, 2048), (12320, 4096), (32000, 768)])
 def test_few_rows_need_no_workspace(T, N, K):
     assert F.lib().ffmi_linear_workspace_bytes(T, N, K, 0) == 0
+
+
+# halves of K only where the grid that runs gains by them: one tile of 16 columns a workgroup, two from 512
+# tiles and 17 rows on; whole K where a wave takes it; the same for every T
+@pytest.mark.parametrize("N,K,slices", [
+    (2048, 2048, 2), (2048, 1376, 2), (6144, 4096, 2), (4608, 4096, 2), (5632, 2048, 2), (9600, 4096, 2),
+    (8224, 2048, 2), (4096, 4096, 1), (4096, 11008, 1), (12288, 4096, 1), (12320, 2048, 1), (12576, 4096, 1),
+    (22016, 4096, 1), (22016, 1024, 1), (16448, 1024, 1), (16448, 1056, 2), (32000, 4096, 1), (2048, 992, 1)])
+def test_halves_of_few_rows(N, K, slices):
+    L = F.lib()
+    assert {L.ffmi_debug_few_rows_slices(T, N, K) for T in (1, 16, 17, 33, 64)} == {slices}
