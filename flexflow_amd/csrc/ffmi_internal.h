@@ -251,8 +251,9 @@ __device__ __forceinline__ float silu_glu(float gate, float up) {
 hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                        size_t ws_bytes, int T, int N, int K, int epilogue, hipStream_t s,
                        Partials *defer = nullptr, int wpitch = 0, const FuseArgs *fuse = nullptr);
-// The form (kTileForms) and K slices in which the tile kernel takes a product of its
-// own (no consumer of slabs), -1 where another kernel takes it
+// The form (kTileForms; kNumTileForms: twelve waves, takes_six) and K slices in which the
+// tile kernel takes a product of its own (no consumer of slabs), -1 where another kernel
+// takes it
 int gemm_tile_form(int T, int N, int K, int epilogue, int *slices);
 // K slices of a product of up to 64 rows whose consumer sums the slabs
 int gemm_few_rows_slices(int T, int N, int K);

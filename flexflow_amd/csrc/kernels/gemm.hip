@@ -36,7 +36,13 @@ int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
   const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
   *slices = 1;
   const bool xp = (epilogue & FFMI_X_PACKED) != 0;
-  if (T <= 64 || K % 32 || !use_tiles(T, N, K, paired, xp, false, false)) return -1;
+  if (T <= 64 || K % 32) return -1;
+  if (!use_tiles(T, N, K, paired, xp, false, false)) {
+    const MidPlan m = mid_plan(T, N, K, paired);
+    if (!takes_six(T, K, m.NTW, m.S, xp)) return -1;
+    *slices = m.S;
+    return kNumTileForms;
+  }
   const TilePlan p = tile_plan(T, N, K, paired, false, false);
   *slices = p.S;
   return p.form;

@@ -1409,11 +1409,11 @@ static bool use_tiles(int T, int N, int K, bool paired, bool xp, bool f32, bool 
 // Over 348 such products (K 128 .. 8192, N 2048 .. 24576) this is 1.10 times as fast: 1.03
 // to 1.09 from K = 2048 on, 1.06 to 1.28 below, the slowest 0.96.
 // Packed activations; no slice without k-steps; not where the M-split kernel is to
-// write its timeline (FFMI_GEMM_STAMP).
+// write its timeline (FFMI_GEMM_STAMP), nor without the tile kernel (FFMI_TILE_GEMM=0).
 static bool takes_six(int T, int K, int NTW, int S, bool packed) {
   static const bool stamp = getenv("FFMI_GEMM_STAMP") != nullptr;
   const int KT = K / 32, steps = (KT + S - 1) / S;
-  return packed && !stamp && K % 32 == 0 && T <= 192 && NTW == 6 && (S - 1) * steps < KT;
+  return packed && !stamp && K % 32 == 0 && T <= 192 && NTW == 6 && (S - 1) * steps < KT && tile_mode() != 0;
 }
 
 // split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;

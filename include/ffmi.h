@@ -664,8 +664,9 @@ ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const float *ss_i
                                          void *Y, int T, int out_dim, int in_dim, int epilogue,
                                          ffmi_stream stream);
 
-/* Test hook: the tile size (0 ..) and K slices in which ffmi_linear's tile kernel
- * takes a product on 16-byte boundaries, -1 where another kernel takes it. */
+/* Test hook: the tile size (0 .. 9; 10: twelve waves, 65 .. 192 rows) and K slices in
+ * which ffmi_linear's tile kernel takes a product on 16-byte boundaries, -1 where
+ * another kernel takes it. */
 int ffmi_debug_linear_tiles(int T, int out_dim, int in_dim, int epilogue, int *slices);
 /* Test hook: the K slices of a model's product of up to 64 rows whose consumer sums them. */
 int ffmi_debug_few_rows_slices(int T, int out_dim, int in_dim);

@@ -92,3 +92,21 @@ def test_few_rows_need_no_workspace(T, N, K):
 def test_halves_of_few_rows(N, K, slices):
     L = F.lib()
     assert {L.ffmi_debug_few_rows_slices(T, N, K) for T in (1, 16, 17, 33, 64)} == {slices}
+
+
+# 65 .. 192 rows of packed activations, 96 columns a workgroup: twelve waves, unless the tile kernel is off
+@pytest.mark.parametrize("T", [65, 128, 129, 192])
+@pytest.mark.parametrize("N,K,epi,slices", [(11008, 4096, 1, 1), (12288, 4096, 0, 2), (6144, 2048, 0, 4),
+                                            (20480, 4096, 0, 1), (32000, 4096, 0, 0), (4096, 4096, 0, 0)])
+def test_twelve_waves(T, N, K, epi, slices, monkeypatch):
+    assert tiles(T, N, K, epi | F.X_PACKED) == ((10, slices) if slices else None)
+    assert tiles(T, N, K, epi) is None
+    monkeypatch.setenv("FFMI_TILE_GEMM", "0")
+    assert tiles(T, N, K, epi | F.X_PACKED) is None
+
+
+def test_twelve_waves_are_tested():
+    """test_gpu_tile_gemm.py's products are of that form, in and out of K slices."""
+    import test_gpu_tile_gemm as G
+    met = [tiles(T, N, K, epi | F.X_PACKED) for T in G.TWELVE_ROWS for N, K, epi in G.TWELVE]
+    assert {m[0] for m in met} == {10} and {m[1] > 1 for m in met} == {False, True}
