@@ -986,7 +986,8 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
   }
 }
 
-// Tile form of T > 192 (tile_plan, msplit_ahead): one workgroup per output tile of
+// Tile form of T > 192 (tile_plan, msplit_ahead), and with twelve waves of 65 .. 192 rows
+// (takes_six): one workgroup per output tile of
 // WR x MI row tiles by WC x NJ weight tiles, its WR x WC waves MI x NJ MFMA
 // accumulators each.  Every operand fragment (16 x 32, 1 KiB) lands in LDS in
 // the MFMA's order with ONE global_load_lds_dwordx4 wave-instruction
@@ -1027,8 +1028,8 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // two row blocks the second one's reads miss (4096 x 4096 21.3 -> 25.3, gate/up 55.3
 // -> 63.6), which therefore go without the hint.
 // A stage whose fragments the waves do not share evenly: the last waves copy one less
-// (two instances of the loop, one per count; each waits for its own copies).  Twelve
-// waves only, of which 6 and 10 would copy for nothing; the forms of eight gain nothing
+// (an instance of the loop per count, and with NTL per kind; each waits for its own
+// copies).  Twelve waves only, of which 6 and 10 would copy for nothing; the forms of eight gain nothing
 // from it (400 products of 200 .. 1024 rows: 0.2% slower to 0.3% faster a form).
 template <int MI, int NJ, int WR, int WC>
 static constexpr bool kExactCopies = WR * WC > 8 && (MI * WR + NJ * WC) % (WR * WC) != 0;
@@ -1040,6 +1041,8 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
   constexpr int NW = WR * WC, FX = MI * WR, F = FX + NJ * WC;  // waves; fragments of a stage
   constexpr int PMAX = (F + NW - 1) / NW;                      // DMAs per wave and stage
   static_assert(NB >= 3 && (NB - 1) * PMAX < 64, "stages in flight");
+  static_assert(!NTL || FX % NW == 0 || (kExactCopies<MI, NJ, WR, WC> && F % NW <= FX % NW),
+                "a wave's copy is of X or of weights, known to the compiler");
   __shared__ __attribute__((aligned(1024))) h8 lds[NB][F][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1055,10 +1058,11 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  auto loop = [&](auto PWc) __attribute__((always_inline)) {
-    constexpr int PW = decltype(PWc)::value;
+  auto loop = [&](auto PWc, auto PXc) __attribute__((always_inline)) {
+    constexpr int PW = decltype(PWc)::value, PX = decltype(PXc)::value;
     // this wave's fragments f = wave + NW p of a stage: X row tile f (< FX) or
-    // weight tile f - FX (the last rows / tile again past the end)
+    // weight tile f - FX (the last rows / tile again past the end); NTL: the first PX
+    // of X, the others of weights
     const uint16_t *src[PW];
     size_t step[PW];
 #pragma unroll
@@ -1080,7 +1084,7 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
       const auto from = (const __attribute__((address_space(1))) void *)(src[p] + (size_t)kt * step[p]);
       const auto to = (__attribute__((address_space(3))) void *)(&lds[slot][min(wave + NW * p, F - 1)][0]);
       // (cache policy 2: non-temporal)
-      if (NTL && wave + NW * p >= FX) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
+      if (NTL && p >= PX) __builtin_amdgcn_global_load_lds(from, to, 16, 0, 2);
       else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
     };
     // (fewer steps than stages: the last step again, into slots nobody reads)
@@ -1148,11 +1152,21 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
       for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
     }
   };
+  constexpr std::integral_constant<int, PMAX> most{};
+  constexpr std::integral_constant<int, FX / NW> xs{};
   if constexpr (kExactCopies<MI, NJ, WR, WC>) {
-    if (wave < F % NW) loop(std::integral_constant<int, PMAX>{});
-    else loop(std::integral_constant<int, PMAX - 1>{});
+    constexpr std::integral_constant<int, PMAX - 1> less{};
+    if constexpr (!NTL || FX % NW == 0) {
+      if (wave < F % NW) loop(most, xs);
+      else loop(less, xs);
+    } else {  // (a third instance: the last waves copy weights only)
+      constexpr std::integral_constant<int, FX / NW + 1> more{};
+      if (wave < F % NW) loop(most, more);
+      else if (wave < FX % NW) loop(less, more);
+      else loop(less, xs);
+    }
   } else {
-    loop(std::integral_constant<int, PMAX>{});
+    loop(most, xs);
   }
   mid_store<MI, NJ, EPI>(acc, Y, Yf, T, N, NTILES, S, ks, bn * (F - FX) + wn * NJ,
                          (bm * FX + wm * MI) * 16, lane, yp, lim);
