@@ -39,9 +39,7 @@ int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
   if (T <= 64 || K % 32) return -1;
   if (!use_tiles(T, N, K, paired, xp, false, false)) {
     const MidPlan m = mid_plan(T, N, K, paired);
-    if (!takes_six(T, K, m.NTW, m.S, xp)) return -1;
-    *slices = m.S;
-    return kNumTileForms;
+    return takes_six(T, K, m.NTW, m.S, xp) ? kNumTileForms : -1;
   }
   const TilePlan p = tile_plan(T, N, K, paired, false, false);
   *slices = p.S;

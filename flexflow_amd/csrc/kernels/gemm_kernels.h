@@ -1410,24 +1410,27 @@ static bool use_tiles(int T, int N, int K, bool paired, bool xp, bool f32, bool 
   return T > 192 && !tile_plan(T, N, K, paired, f32, deferred).msplit[xp];
 }
 
-// Products of 65 .. 192 rows of which the M-split plan gives a workgroup six weight tiles
-// (96 columns): its waves then hold 2 or 3 x 6 accumulators and each copies six KiB of
+// Unsplit products of 65 .. 192 rows of which the M-split plan gives a workgroup six weight
+// tiles (96 columns): its waves then hold 2 or 3 x 6 accumulators and each copies six KiB of
 // weights and its own rows a step, one stage ahead.  Twelve waves, 2 or 3 x 2
-// accumulators each, keep 3 or 4 stages in flight and share every copy.  Cold weights,
-// M-split / this at T = 82, 128, 168, 192 (us): gate/up 2 x 11008 x 4096 43.2 / 37.2,
-// 44.6 / 39.6, 51.6 / 47.5, 53.0 / 47.4; 12288 x 4096 in 2 slices 23.7 / 21.6, 25.7 / 23.7,
-// 29.3 / 27.4, 30.2 / 28.2; 6144 x 4096 in 4 14.9 / 13.2, 16.0 / 15.1, 17.5 / 16.9, 18.7 / 17.8.
+// accumulators each, keep 3 or 4 stages in flight and share every copy.  Cold streamed
+// weights behind a norm, M-split / this at T = 72, 128, 168, 192 (us), on the better and on the
+// worse of two machines: gate/up 2 x 11008 x 4096 40.2 / 39.0, 45.6 / 41.0, 51.3 / 47.5, 52.4 / 47.9
+// and 42.1 / 40.5, 45.9 / 43.8, 52.1 / 50.3, 53.7 / 50.0; 20480 x 4096 40.5 / 35.2, 45.5 / 41.4, 51.0 / 46.2,
+// 52.0 / 47.0 and 41.9 / 36.7, 45.8 / 42.4, 51.4 / 47.7, 52.9 / 48.2; 2 x 9216 x 1024 15.0 / 12.3, 15.1 / 13.4,
+// 17.7 / 15.5, 17.9 / 15.7 and 15.1 / 13.1, 15.2 / 13.9, 18.1 / 16.3, 18.6 / 16.4; 24576 x 8192 at 168 97.5 / 91.3
+// and 99.6 / 96.5.  Without the hint of a stream 0 to 10% less, 0.95 at worst.
+// In K slices it depends on the machine, so those stay with the M-split kernel:
+// 12288 x 4096 in two at T = 168 30.6 / 29.1 on one, 31.1 / 32.9 on the other (in the model 31.5 / 30.0
+// and 32.0 / 33.7; T = 72 23.8 / 22.5 and 24.9 / 28.4), 6144 x 4096 in four 19.6 / 19.8 and 19.6 / 23.3, 2 x 3072 x 4096 in
+// four 18.8 / 19.2 and 19.7 / 22.9.
 // Where the plan has other widths the M-split kernel stays ahead of every form tried
-// (32000 x 4096 at T = 168, 128 columns, 62.9 against 62.2 .. 91; 4096 x 11008, 64
-// columns in 8 slices, 24.4 against 25.5 .. 34; 4096 x 4096 13.6 against 14.0 .. 17.6).
-// Over 348 such products (K 128 .. 8192, N 2048 .. 24576) this is 1.10 times as fast: 1.03
-// to 1.09 from K = 2048 on, 1.06 to 1.28 below, the slowest 0.96.
-// Packed activations; no slice without k-steps; not where the M-split kernel is to
-// write its timeline (FFMI_GEMM_STAMP), nor without the tile kernel (FFMI_TILE_GEMM=0).
+// (32000 x 4096 at T = 168, 128 columns, 62.9 against 62.2 .. 91).
+// Packed activations; not where the M-split kernel is to write its timeline
+// (FFMI_GEMM_STAMP), nor without the tile kernel (FFMI_TILE_GEMM=0).
 static bool takes_six(int T, int K, int NTW, int S, bool packed) {
   static const bool stamp = getenv("FFMI_GEMM_STAMP") != nullptr;
-  const int KT = K / 32, steps = (KT + S - 1) / S;
-  return packed && !stamp && K % 32 == 0 && T <= 192 && NTW == 6 && (S - 1) * steps < KT && tile_mode() != 0;
+  return packed && !stamp && K % 32 == 0 && T <= 192 && NTW == 6 && S == 1 && tile_mode() != 0;
 }
 
 // split-K workspace of the largest plan (0: unsplit); f32: an epilogue of sums;
@@ -1565,17 +1568,16 @@ static hipError_t run_tiles(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, 
 }
 
 // Up to 192 rows in one block, 96 columns a workgroup: the tile kernel with 12 waves
-// in the M-split kernel's place, at its split of K (the same bits in the same slabs).
+// in the M-split kernel's place, unsplit (the same bits).
 template <int E>
 static hipError_t run_six(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws, int T, int N, int K,
-                          hipStream_t s, int yp, int S, Partials *defer, bool nt, int wpitch, float lim) {
-  constexpr bool paired = epi_paired<E>, f32 = epi_f32<E>;
-  const int KT = K / 32, ntiles = (N + 15) / 16 * (paired ? 2 : 1);
+                          hipStream_t s, int yp, Partials *defer, bool nt, int wpitch, float lim) {
+  const int KT = K / 32, ntiles = (N + 15) / 16 * (epi_paired<E> ? 2 : 1);
   const size_t wts = w_tile_stride(KT), wks = w_k_stride(wpitch ? wpitch : ntiles);
-  const dim3 grid((ntiles + 5) / 6 * S), block(768);
+  const dim3 grid((ntiles + 5) / 6), block(768);
 #define FFMI_SIX(MI, NB, NL)                                                                               \
   hipLaunchKernelGGL((gemm_tile_kernel<E, MI, 2, 4, 3, NB, NL>), grid, block, 0, s, X, Wp, Y, ws, T, N, KT, \
-                     ntiles, 1, S, 1, yp, wts, wks, lim)
+                     ntiles, 1, 1, 1, yp, wts, wks, lim)
   if (T <= 128) {
     if (nt) FFMI_SIX(2, 5, true);
     else FFMI_SIX(2, 5, false);
@@ -1584,11 +1586,7 @@ static hipError_t run_six(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, fl
     else FFMI_SIX(3, 4, false);
   }
 #undef FFMI_SIX
-  if (defer && ((S > 1 && !paired) || f32)) {
-    defer->p = ws, defer->S = S, defer->NP = ntiles * 16;
-    return hipGetLastError();
-  }
-  if (S > 1 && !f32) return run_reduce<E>(ws, Y, T, N, ntiles, S, yp, lim, s);
+  if (defer && epi_f32<E>) defer->p = ws, defer->S = 1, defer->NP = ntiles * 16;
   return hipGetLastError();
 }
 
@@ -1645,7 +1643,7 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
     if (SM > 1 && (!ws || ws_bytes < (size_t)SM * T * ((N + 15) / 16 * 16 << paired) * sizeof(float)))
       SM = 1;  // no workspace: un-split (slower)
     if (takes_six(T, K, p.NTW, SM, xp && aligned))
-      return run_six<E>(X, Wp, Y, ws, T, N, K, s, yp, SM, defer, nt, wpitch, lim);
+      return run_six<E>(X, Wp, Y, ws, T, N, K, s, yp, defer, nt, wpitch, lim);
     if (p.MTW == 3) {
       if (p.NTW == 2) FFMI_RUN(3, 2);
       if (p.NTW == 4) FFMI_RUN(3, 4);

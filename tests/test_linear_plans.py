@@ -94,19 +94,14 @@ def test_halves_of_few_rows(N, K, slices):
     assert {L.ffmi_debug_few_rows_slices(T, N, K) for T in (1, 16, 17, 33, 64)} == {slices}
 
 
-# 65 .. 192 rows of packed activations, 96 columns a workgroup: twelve waves, unless the tile kernel is off
+# 65 .. 192 rows of packed activations, 96 columns a workgroup, whole K: twelve waves, unless the tile kernel
+# is off; what is split in K stays with the M-split kernel
 @pytest.mark.parametrize("T", [65, 128, 129, 192])
-@pytest.mark.parametrize("N,K,epi,slices", [(11008, 4096, 1, 1), (12288, 4096, 0, 2), (6144, 2048, 0, 4),
-                                            (20480, 4096, 0, 1), (32000, 4096, 0, 0), (4096, 4096, 0, 0)])
-def test_twelve_waves(T, N, K, epi, slices, monkeypatch):
-    assert tiles(T, N, K, epi | F.X_PACKED) == ((10, slices) if slices else None)
+@pytest.mark.parametrize("N,K,epi,ours", [(11008, 4096, 1, True), (20480, 4096, 0, True), (18432, 512, 0, True),
+                                          (12288, 4096, 0, False), (6144, 2048, 0, False), (6144, 4096, 0, False),
+                                          (5632, 4096, 1, False), (32000, 4096, 0, False), (4096, 4096, 0, False)])
+def test_twelve_waves(T, N, K, epi, ours, monkeypatch):
+    assert tiles(T, N, K, epi | F.X_PACKED) == ((10, 1) if ours else None)
     assert tiles(T, N, K, epi) is None
     monkeypatch.setenv("FFMI_TILE_GEMM", "0")
     assert tiles(T, N, K, epi | F.X_PACKED) is None
-
-
-def test_twelve_waves_are_tested():
-    """test_gpu_tile_gemm.py's products are of that form, in and out of K slices."""
-    import test_gpu_tile_gemm as G
-    met = [tiles(T, N, K, epi | F.X_PACKED) for T in G.TWELVE_ROWS for N, K, epi in G.TWELVE]
-    assert {m[0] for m in met} == {10} and {m[1] > 1 for m in met} == {False, True}
