@@ -163,6 +163,8 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
 // rows [n0, n0 + rows) of W [N][K] (src: the first of them, rows of ld) to blocks of 8 rows
 // x 32 k (f32.hip); dst holds ceil(N / 8) * 8 * K floats
 hipError_t launch_pack_f32_blocks(const float *src, int ld, float *dst, int N, int n0, int rows, int K, hipStream_t s);
+// whether a model's [.][K] weight is kept in blocks (f32.hip)
+bool f32_in_blocks(int K);
 // launch_gemm_f32's sums of a packed W
 hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int T, int N, int K, hipStream_t s);
 hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu, float *out, int T, int F, int K,

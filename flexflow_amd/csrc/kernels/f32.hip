@@ -174,7 +174,10 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
 // Up to 16 rows (decoding) of packed weights (launch_pack_f32_blocks), where their stream
 // is the time: one tile of 16 x 16, of which only what is needed is copied.  What a CU takes in comes back from its L1 in
 // order, so that rows of X, from the L2, wait behind weights from HBM and take the place
-// of weights in flight: XH (up to 8 rows) leaves out the other 8.  COLS = 8: half a tile of
+// of weights in flight: in half tiles of columns, where they are two copies of three, XH
+// (up to 8 rows) leaves out the other 8; whole tiles and pairs take the same time
+// with and without (T = 8: 6144 x 2048 12.6 and 12.5 us, 12288 x 4096 35.0 and 35.1, gate/up 2 x 5632 x
+// 2048 19.0 and 18.5, 2 x 11008 x 4096 64.3 and 65.1).  COLS = 8: half a tile of
 // columns (the MFMA multiplies the other half for nothing), for widths whose 16-column
 // workgroups leave CUs idle or unevenly loaded.  PAIR: columns 0..7 of the tile are
 // gate's, 8..15 up's (W: F rows of gate, then F of up), and silu(gate) up goes out
@@ -338,7 +341,9 @@ __global__ __launch_bounds__(256) void f32_gemm_kernel(const float *__restrict__
 // a tile at K = 2048).  All forms add up an output in the same order.  T = 201, K = 2048:
 // N = 2048 2 x 4 tiles 21.4 us, 4 x 4 37.1 (41.2 from registers); N = 11264 105 and
 // 112 (123); N = 32000 298 and 306 (329).  Two 2 x 2 workgroups share a CU, and the third
-// round of three shares with none: it counts 1.3 (N = 6144, T = 120 43.5 us, 4 x 4 39.7).
+// round of three shares with none: it counts 1.3 (N = 6144, T = 120 43.3 us, 4 x 4 39.7; of 120
+// products 6 change form by it, 5 to a faster one: 0.2% above the fastest form on average,
+// 0.5% without).
 template <bool PACKED>
 static void f32_gemm_many(const float *X, const float *W, float *Y, int T, int N, int K, hipStream_t s) {
   const auto tiles = [&](int mt, int nt) {
@@ -395,6 +400,16 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
     f32_gemm_many<false>(X, W, Y, T, N, K, s);
   return hipGetLastError();
 }
+
+// Short rows stay as they lie: their workgroups read a few KiB each, in one piece, which
+// blocks scatter over as many bands.  T = 1, 4, 8 and 16, us, rows / blocks: N 32000 x K 256 7.4 / 9.7,
+// 8.1 / 10.0, 8.8 / 10.1, 9.1 / 10.5; x 512 13.2 / 15.2, 13.5 / 15.5, 13.8 / 15.7, 14.4 / 16.4; x 768 19.7 / 20.3 .. 21.9 /
+// 22.3; 2304 x 768 3.8 / 4.0 .. 4.1 / 4.3; 4096 x 1024 5.9 / 6.5 .. 6.2 / 6.7; equal above 16 rows.  From
+// 1280 on blocks are 0.8 (4096 x 2048) to 1.4 times as fast (K 11008 x N 4096), 1.0 to 1.2 from 5120
+// columns on; a model's steps of 1, 4 and 12 tokens are 2, 2 and 2% faster with this line at width 256,
+// 2% at 512, 3% at 768, 1% at 1024.  Gate and up are in blocks whatever K is: 1.1 to 1.5 times as fast as
+// rows and a unit of their own.
+bool f32_in_blocks(int K) { return K >= 1280; }
 
 // Packed weights (launch_pack_f32_blocks).  Up to 16 rows, T = 4, us, rows as they lie and
 // packed: 12288 x 4096 43.0 -> 35.6, 22016 x 4096 72.3 -> 64.8, K 11008 x N 4096 46.0 -> 31.2,

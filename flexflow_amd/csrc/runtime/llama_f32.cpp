@@ -30,7 +30,7 @@ namespace {
 
 struct LayerF {
   float *in_norm = nullptr, *post_norm = nullptr;
-  float *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wd = nullptr;  // row-major [N][K]
+  float *wqkv = nullptr, *wo = nullptr, *wgu = nullptr, *wd = nullptr;  // [N][K] (take)
   ffmi_attn *attn = nullptr;  // DT_FLOAT handle: fp32 KV cache, TREE staging, RoPE table
 };
 
@@ -160,10 +160,19 @@ struct LlamaF32 : public ffmi_model {
     return FFMI_OK;
   }
   // rows [r0, r0 + nr) x columns [c0, c0 + nc) of tmp ([.][ld]) -> rows n0 ... of the
-  // packed weight dst [N][nc]
-  ffmi_status take(float *dst, int N, int n0, const float *tmp, int ld, int r0, int nr, int c0, int nc) {
-    FFMI_HIP(launch_pack_f32_blocks(tmp + (size_t)r0 * ld + c0, ld, dst, N, n0, nr, nc, stream));
+  // weight dst [N][nc], in blocks (f32.hip) or row-major
+  ffmi_status take(float *dst, int N, int n0, const float *tmp, int ld, int r0, int nr, int c0, int nc, bool blocks) {
+    const float *src = tmp + (size_t)r0 * ld + c0;
+    if (blocks)
+      FFMI_HIP(launch_pack_f32_blocks(src, ld, dst, N, n0, nr, nc, stream));
+    else
+      FFMI_HIP(hipMemcpy2DAsync(dst + (size_t)n0 * nc, (size_t)nc * 4, src, (size_t)ld * 4, (size_t)nc * 4, nr,
+                                hipMemcpyDeviceToDevice, stream));
     return FFMI_OK;
+  }
+  hipError_t product(const float *X, const float *W, float *Y, int T, int N, int K) {
+    return f32_in_blocks(K) ? launch_gemm_f32_packed(X, W, Y, T, N, K, stream)
+                            : launch_gemm_f32(X, W, Y, T, N, K, stream);
   }
   ffmi_status alloc_packed(float **p, int N, int K) { return alloc(p, (size_t)((N + 7) / 8 * 8) * K); }
 
@@ -234,7 +243,7 @@ struct LlamaF32 : public ffmi_model {
       TRY(full_tensor(tmp, V, H, "model.embed_tokens.weight", 0, H, 7919));
     else
       TRY(full_tensor(tmp, V, H, "lm_head.weight", 0));
-    TRY(take(lm, V, 0, tmp, H, 0, V, 0, H));
+    TRY(take(lm, V, 0, tmp, H, 0, V, 0, H, f32_in_blocks(H)));
     const int s = o.tp_rank;
     layers.resize(c.num_layers);
     for (int l = 0; l < c.num_layers; ++l) {
@@ -250,22 +259,22 @@ struct LlamaF32 : public ffmi_model {
                               "self_attn.v_proj.weight"};
       for (int q = 0; q < 3; ++q) {
         TRY(full_tensor(tmp, H, H, p + names[q], 0));
-        TRY(take(L.wqkv, 3 * Hl, q * Hl, tmp, H, s * Hl, Hl, 0, H));
+        TRY(take(L.wqkv, 3 * Hl, q * Hl, tmp, H, s * Hl, Hl, 0, H, f32_in_blocks(H)));
       }
       // o_proj row-parallel: columns [s*Hl, (s+1)*Hl)
       TRY(alloc_packed(&L.wo, H, Hl));
       TRY(full_tensor(tmp, H, H, p + "self_attn.o_proj.weight", kres));
-      TRY(take(L.wo, H, 0, tmp, H, 0, H, s * Hl, Hl));
+      TRY(take(L.wo, H, 0, tmp, H, 0, H, s * Hl, Hl, f32_in_blocks(Hl)));
       // gate rows then up rows of this shard: one GEMM, [T][2 Fl]
       TRY(alloc_packed(&L.wgu, 2 * Fl, H));
       TRY(full_tensor(tmp, F, H, p + "mlp.gate_proj.weight", 0));
-      TRY(take(L.wgu, 2 * Fl, 0, tmp, H, s * Fl, Fl, 0, H));
+      TRY(take(L.wgu, 2 * Fl, 0, tmp, H, s * Fl, Fl, 0, H, true));
       TRY(full_tensor(tmp, F, H, p + "mlp.up_proj.weight", 0));
-      TRY(take(L.wgu, 2 * Fl, Fl, tmp, H, s * Fl, Fl, 0, H));
+      TRY(take(L.wgu, 2 * Fl, Fl, tmp, H, s * Fl, Fl, 0, H, true));
       // down row-parallel: columns [s*Fl, (s+1)*Fl) of [H][F]
       TRY(alloc_packed(&L.wd, H, Fl));
       TRY(full_tensor(tmp, H, F, p + "mlp.down_proj.weight", kres));
-      TRY(take(L.wd, H, 0, tmp, F, 0, H, s * Fl, Fl));
+      TRY(take(L.wd, H, 0, tmp, F, 0, H, s * Fl, Fl, f32_in_blocks(Fl)));
       // the layer's DT_FLOAT attention handle (ffmi_attn_cfg.full_precision)
       ffmi_attn_cfg ac{};
       ac.mode = mode == FFMI_MODEL_TREE ? FFMI_ATTN_TREE
@@ -319,20 +328,20 @@ struct LlamaF32 : public ffmi_model {
         FFMI_HIP(launch_rmsnorm_f32(embed, nullptr, L.in_norm, res, h, T, H, eps, stream, blob));
       else
         FFMI_HIP(launch_rmsnorm_f32(res, proj, L.in_norm, res, h, T, H, eps, stream));
-      FFMI_HIP(launch_gemm_f32_packed(h, L.wqkv, qkv, T, 3 * Hl, H, stream));
+      FFMI_HIP(product(h, L.wqkv, qkv, T, 3 * Hl, H));
       TRY(attn_forward(L.attn, batch, qkv, Partials(), att, (ffmi_stream)stream));
-      FFMI_HIP(launch_gemm_f32_packed(att, L.wo, proj, T, H, Hl, stream));
+      FFMI_HIP(product(att, L.wo, proj, T, H, Hl));
       TRY(allreduce(proj, (size_t)T * H));
       FFMI_HIP(launch_rmsnorm_f32(res, proj, L.post_norm, res, h, T, H, eps, stream));
       FFMI_HIP(launch_gate_up_f32_packed(h, L.wgu, gu, mlp, T, Fl, H, stream));
-      FFMI_HIP(launch_gemm_f32_packed(mlp, L.wd, proj, T, H, Fl, stream));
+      FFMI_HIP(product(mlp, L.wd, proj, T, H, Fl));
       TRY(allreduce(proj, (size_t)T * H));
     }
     const int n = tail_n;
     if (n == 0) return FFMI_OK;
     FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, few_rows ? nullptr : res, h, n, H, eps, stream, nullptr,
                                 few_rows ? rows_h : nullptr));
-    FFMI_HIP(launch_gemm_f32_packed(h, lm, logits, n, V, H, stream));
+    FFMI_HIP(product(h, lm, logits, n, V, H));
     if (k == 0) return FFMI_OK;  // logits only
     float *probs_d = reinterpret_cast<float *>(res_d + (size_t)n * k);
     FFMI_HIP(launch_softmax_topk_f32(logits, n, V, k, res_d, probs_d, stream));

@@ -74,3 +74,13 @@ def test_full_precision_does_not_depend_on_the_step(ff, vocab):
         at += k
     rm.replay_end(m, 1)
     assert at == 90 and np.array_equal(np.concatenate(got), whole) and np.isfinite(whole).all() and whole.std() > 0
+
+
+# the same at widths of which every weight is kept in blocks: half tiles of columns (heads, ff), whole ones in
+# rings of two and of four k-blocks (qkv and lm_head), pairs, and columns past the last whole tile
+@pytest.mark.parametrize("hidden,ff,vocab", [(1280, 1312, 2101), (1280, 2080, 4101), (1536, 1280, 4097)])
+def test_full_precision_of_wide_rows_does_not_depend_on_the_step(hidden, ff, vocab, monkeypatch):
+    monkeypatch.setitem(CFG, "hidden", hidden)
+    monkeypatch.setitem(CFG, "num_heads", hidden // 128)
+    monkeypatch.setitem(CFG, "num_kv_heads", hidden // 128)
+    test_full_precision_does_not_depend_on_the_step(ff, vocab)
