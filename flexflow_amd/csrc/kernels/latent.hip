@@ -324,7 +324,7 @@ hipError_t launch_head_gemm_f32(const HeadGemm &hg, hipStream_t s) {
 // P^T with C^T read from the row-major page in LDS by the transposing LDS load;
 // the k order of the second product is the key order the scores already have
 // in the lanes (16-lane group g: keys 4g..4g+3 and 16+4g..).
-//   scores:  wave = (16-key tile, half of the rows); RT == 1: four waves only
+//   scores:  wave = (16-key tile, row tile); RT == 1: four waves only
 //   outputs: each wave an eighth of the latent's columns, all rows
 // Softmax state in fp32, base-2 exponents; weights meet the second product in
 // bf16, the sums take them unrounded.
@@ -339,7 +339,6 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
     const uint16_t *__restrict__ cache, uint16_t *__restrict__ O, float *__restrict__ slabs,
     float *__restrict__ ml, int heads, float scale_log2) {
   constexpr int R = RC * 64, KS = RC * 2, LDC = R + kRankPad;
-  constexpr int SR = 1;                         // row tiles of a wave's scores
   constexpr int NT = RC * 4, DT = (NT + 7) / 8;  // column tiles: all, of a wave's outputs
   constexpr int LDP = kPageTokens + 8;
   __shared__ __attribute__((aligned(16))) uint16_t sC[2][64 * LDC];
@@ -372,62 +371,49 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
   };
   fetch(0);
   // this wave's rows of Q' as B operands (rows past the block re-read its last)
-  bf8 q[SR][KS];
-  int qpos[SR];
+  bf8 q[KS];
+  const int qr = min(wr * 16 + l15, bk.nrows - 1);
+  const uint16_t *qp = Q + (size_t)(bk.row0 + qr) * R + 8 * g;
 #pragma unroll
-  for (int i = 0; i < SR; ++i) {
-    const int r = min((wr * SR + i) * 16 + l15, bk.nrows - 1);
-    const uint16_t *qr = Q + (size_t)(bk.row0 + r) * R + 8 * g;
-#pragma unroll
-    for (int k = 0; k < KS; ++k) q[i][k] = *reinterpret_cast<const bf8 *>(qr + k * 32);
-    qpos[i] = bk.pos0 + (bk.row0 + r - bk.seg_row) / heads;
-  }
+  for (int k = 0; k < KS; ++k) q[k] = *reinterpret_cast<const bf8 *>(qp + k * 32);
+  const int qpos = bk.pos0 + (bk.row0 + qr - bk.seg_row) / heads;
   f4 acc[RT][DT];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int d = 0; d < DT; ++d) acc[i][d] = f4{0.f, 0.f, 0.f, 0.f};
-  float m[RT], l[SR];
+  float m[RT], l = 0.f;
 #pragma unroll
   for (int i = 0; i < RT; ++i) m[i] = -1e30f;
-#pragma unroll
-  for (int i = 0; i < SR; ++i) l[i] = 0.f;
   stage(0);
   if (bk.ntiles > 1) fetch(1);
   __syncthreads();
   for (int it = 0; it < bk.ntiles; ++it) {
     const uint16_t *C = sC[it & 1];
-    f4 s[SR];
+    f4 s;
     if (scoring) {
-      // two chains per row tile (even / odd k-steps)
-      f4 s2[SR];
-#pragma unroll
-      for (int i = 0; i < SR; ++i) s[i] = s2[i] = f4{0.f, 0.f, 0.f, 0.f};
+      // two chains (even / odd k-steps)
+      f4 s2 = f4{0.f, 0.f, 0.f, 0.f};
+      s = s2;
 #pragma unroll
       for (int ks = 0; ks < KS; ks += 2) {
         const uint16_t *cr = &C[(wk * 16 + l15) * LDC + ks * 32 + 8 * g];
         const bf8 c0 = *reinterpret_cast<const bf8 *>(cr), c1 = *reinterpret_cast<const bf8 *>(cr + 32);
-#pragma unroll
-        for (int i = 0; i < SR; ++i) {
-          s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c0, q[i][ks], s[i], 0, 0, 0);
-          s2[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1, q[i][ks + 1], s2[i], 0, 0, 0);
-        }
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c0, q[ks], s, 0, 0, 0);
+        s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1, q[ks + 1], s2, 0, 0, 0);
       }
       // scale, mask, this wave's maximum of every row
       const int key0 = (bk.tile0 + it) * 64 + wk * 16 + 4 * g;
+      float mx = -1e30f;
 #pragma unroll
-      for (int i = 0; i < SR; ++i) {
-        float mx = -1e30f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float v = key0 + e <= qpos[i] ? (s[i][e] + s2[i][e]) * scale_log2 : -INFINITY;
-          s[i][e] = v;
-          mx = fmaxf(mx, v);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        if (g == 0) sM[wk][(wr * SR + i) * 16 + l15] = mx;
+      for (int e = 0; e < 4; ++e) {
+        const float v = key0 + e <= qpos ? (s[e] + s2[e]) * scale_log2 : -INFINITY;
+        s[e] = v;
+        mx = fmaxf(mx, v);
       }
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (g == 0) sM[wk][wr * 16 + l15] = mx;
     }
     __syncthreads();
     float alpha[RT];
@@ -442,21 +428,17 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
       m[i] = mn;
     }
     if (scoring) {
+      const float mi = RT > 1 && wr ? m[RT - 1] : m[0];
+      const float ai = RT > 1 && wr ? alpha[RT - 1] : alpha[0];
+      float p[4], sum = 0.f;
 #pragma unroll
-      for (int i = 0; i < SR; ++i) {
-        const float mi = RT > 1 && wr ? m[RT > 1 ? SR + i : i] : m[i];
-        const float ai = RT > 1 && wr ? alpha[RT > 1 ? SR + i : i] : alpha[i];
-        float p[4], sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          p[e] = __builtin_amdgcn_exp2f(s[i][e] - mi);
-          sum += p[e];
-        }
-        *reinterpret_cast<uint2 *>(&sP[((wr * SR + i) * 16 + l15) * LDP + wk * 16 + 4 * g]) =
-            make_uint2(f2bf(p[0]) | ((uint32_t)f2bf(p[1]) << 16),
-                       f2bf(p[2]) | ((uint32_t)f2bf(p[3]) << 16));
-        l[i] = l[i] * ai + sum;
+      for (int e = 0; e < 4; ++e) {
+        p[e] = __builtin_amdgcn_exp2f(s[e] - mi);
+        sum += p[e];
       }
+      *reinterpret_cast<uint2 *>(&sP[(wr * 16 + l15) * LDP + wk * 16 + 4 * g]) =
+          make_uint2(f2bf(p[0]) | ((uint32_t)f2bf(p[1]) << 16), f2bf(p[2]) | ((uint32_t)f2bf(p[3]) << 16));
+      l = l * ai + sum;
     }
     if (it + 1 < bk.ntiles) {
       stage((it + 1) & 1);  // (last read by the outputs of tile it - 1)
@@ -496,13 +478,9 @@ __global__ __launch_bounds__(512) void latent_attn_kernel(
     }
   }
   if (scoring) {
-#pragma unroll
-    for (int i = 0; i < SR; ++i) {
-      float v = l[i];
-      v += __shfl_xor(v, 16);
-      v += __shfl_xor(v, 32);
-      if (g == 0) sL[wk][(wr * SR + i) * 16 + l15] = v;
-    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) sL[wk][wr * 16 + l15] = l;
   }
   __syncthreads();
 #pragma unroll
