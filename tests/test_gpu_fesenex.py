@@ -12,6 +12,7 @@ import pytest
 import fesenex_models as FM
 import fesenex_ref as R
 import flexflow_amd as fa
+import flexflow_amd.ffmi as F
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -385,6 +386,19 @@ def test_many_heads_of_linear_attention(tmp_path, dim, vdim):
     for rid, toks in reqs.items():
         assert at[rid] == len(toks)
         close(np.concatenate(got[rid]), R.forward(model[0], w, toks), False)
+
+
+# prompts of 65 .. 192 tokens whose first product has 96 columns a workgroup (twelve waves) and leaves its sums
+# to the kernel that reads them
+@pytest.mark.parametrize("n", [100, 150])
+def test_wide_products_of_prompts(tmp_path, n):
+    heads = 34
+    assert F.lib().ffmi_debug_linear_tiles(n, 4 * heads * 128, 64, F.X_PACKED, None) == 10
+    model = FM.model_config(64, 64, [FM.lightning(heads, 128, 128, [0.7 + 0.008 * h for h in range(heads)])])
+    weights = FM.random_weights(model, 4)
+    eng = make_engine(FM.write_checkpoint(tmp_path / "m", model[0], weights), False)
+    toks = tokens(model, n + 2, n)
+    close(run(eng, toks, [n, 1, 1]), R.forward(model[0], weights, toks, []), False)
 
 
 @pytest.mark.parametrize("full", [True, False])

@@ -26,3 +26,10 @@ def test_linear_bf16_swiglu(T, N, K):
     # one rounding to bf16, and the sums' own error through the product's slope
     slope = 2e-5 * (1.0 + np.abs(u) + np.abs(g))
     assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + slope).all(), np.abs(got - want).max()
+
+
+# 96 columns a workgroup: twelve waves (both row counts and their edges)
+@pytest.mark.parametrize("T", [65, 128, 129, 192])
+def test_linear_bf16_swiglu_twelve_waves(T):
+    assert F.lib().ffmi_debug_linear_tiles(T, 8480, 160, F.EPI_SILU_MUL | F.X_PACKED, None) == 10
+    test_linear_bf16_swiglu(T, 8480, 160)

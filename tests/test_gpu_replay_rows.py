@@ -29,6 +29,7 @@ def test_rows_of_a_long_step(T, full):
         for r in range(3):
             rm.replay_end(m, r + 1)
         return np.concatenate([got, more])
+    every = step([range(n[0]), range(10), [0]])  # (every row is wanted, so every row is computed)
     for want in ([[n[0] - 1], [9], [0]], [[], [], [0]], [[], [], []], [list(range(0, n[0], 3)), [4, 2], []],
                  [list(range(max(0, T // 2 - 2))), [0], []], [range(n[0]), range(10), [0]]):
         few = step(want)
@@ -41,9 +42,10 @@ def test_rows_of_a_long_step(T, full):
         bound = (2.0 ** -10 * np.abs(whole) + 2.0 ** -14 * np.abs(whole).max()) if not full else 1e-5 * np.abs(whole).max()
         assert (np.abs(few[:-1] - whole[:-1]) <= bound[:-1] if not full else
                 np.abs(few[:-1] - whole[:-1]) <= bound).all()
-        # (a step after it: its keys and values are the long step's own, computed alike)
-        assert np.array_equal(few[-1], whole[-1]) or np.abs(few[-1] - whole[-1]).max() <= \
-            (2e-2 if not full else 1e-5) * np.abs(whole).max()
+        # a step after it: the long step's own keys and values, whatever rows it was asked for, are the same
+        # bits; those of a step under debug capture (other kernels in 16 bits) are as near as 16 bits are
+        assert np.array_equal(few[-1], every[-1])
+        assert np.abs(few[-1] - whole[-1]).max() <= (2e-2 if not full else 1e-5) * np.abs(whole).max()
 
 
 @pytest.mark.parametrize("full", [False, True])

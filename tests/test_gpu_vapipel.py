@@ -168,6 +168,20 @@ def test_products_in_halves(tmp_path):
     close(run((rm, m), toks, [1, 16, 17, 1, 64, 15, 1, 1]), R.forward(HALVES, weights, toks, []), False)
 
 
+# the slabs' room is for as many tokens as a step may have, whole tiles or not
+@pytest.mark.parametrize("capacity", [8, 40])
+def test_halves_do_not_depend_on_the_capacity(tmp_path, capacity):
+    folder = VM.write_checkpoint(tmp_path / "m", HALVES, VM.random_weights(HALVES, 6))
+    toks, got = tokens(HALVES, capacity, 3), []
+    for most in (capacity, 64):
+        m = fa.Model(fa.load_config(folder), "inc", max_requests=2, max_tokens=most, max_seq_len=120,
+                     weights_folder=folder)
+        rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=most, max_spec_tree_token_num=0,
+                               max_sequence_length=120)
+        got.append(run((rm, m), toks, [capacity]))
+    assert np.array_equal(*got)
+
+
 @pytest.mark.parametrize("full", [True, False])
 def test_first_tokens_and_single_token_prompts(engine, full):
     for t in range(5):

@@ -43,6 +43,13 @@ def test_linear_bf16_epilogues(T, N, K):
     assert (np.abs(q - r * r) <= 2.0 ** -8 * r * r + 2 * (r + 3e-6 * mag) * 3e-6 * mag).all()
 
 
+# 96 columns a workgroup: twelve waves (both row counts and their edges)
+@pytest.mark.parametrize("T", [65, 128, 129, 192])
+def test_linear_bf16_twelve_waves(T):
+    assert F.lib().ffmi_debug_linear_tiles(T, 16928, 160, F.X_PACKED, None) == 10
+    test_linear_bf16_epilogues(T, 16928, 160)
+
+
 def test_linear_bf16_rows_do_not_depend_on_the_batch():
     rng = np.random.default_rng(5)
     X, W = bf16(rng.standard_normal((64, 512))), bf16(rng.standard_normal((288, 512)))
