@@ -414,7 +414,7 @@ bool f32_in_blocks(int K) { return K >= 1280; }
 // Packed weights (launch_pack_f32_blocks).  Up to 16 rows, T = 4, us, rows as they lie and
 // packed: 12288 x 4096 43.0 -> 35.6, 22016 x 4096 72.3 -> 64.8, K 11008 x N 4096 46.0 -> 31.2,
 // 4096 x 4096 17.6 -> 16.2, 6144 x 2048 12.4 -> 12.2, 11264 x 2048 19.3 -> 17.8, K 5632 x N 2048
-// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0.
+// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0; but 4096 x 2048 8.2 -> 10.1 (launches back to back).
 //  * Half tiles of columns where whole ones are at most half as many as CUs (K 5632 x N 2048
 //    14.4 -> 13.8, T = 16 16.3 -> 14.9; 768 x 3072 9.0 -> 8.5); at 256 and above they lose
 //    (6144 x 2048 13.1 -> 13.7, 11264 x 2048 18.3 -> 22.9).

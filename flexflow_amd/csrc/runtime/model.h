@@ -52,6 +52,8 @@ void beam_result_layout(const BeamSearchBatchConfig &bc, std::vector<int> *map);
 struct ffmi_model {
   int mode = FFMI_MODEL_INC;
   virtual ~ffmi_model() {}
+  // an INC step: the pick of every request's last token of the batch, which is what the
+  // scheduler reads (the other entries may be -1: long steps sample no other row)
   virtual ffmi_status run_inc(const ffmi::BatchConfig &bc, ffmi::InferenceResult *ir) = 0;
   virtual ffmi_status run_tree(const ffmi::TreeVerifyBatchConfig &bc,
                                ffmi::InferenceResult *ir) = 0;
