@@ -34,6 +34,19 @@ __device__ __forceinline__ float f32_silu_mul(float a, float b) {
   return __fmul_rn(__fmul_rn(a, sg), b);
 }
 
+// The column block that workgroup b of n takes of a packed weight.  Workgroups go round the
+// eight XCDs, so in their own order an XCD reads 2 KiB (8 columns: 1 KiB) of each 16 (8) of
+// a band, always the same ones where the bands are of a round number of them: a part of its
+// L2's channels.  There an XCD takes an eighth of the columns in one piece.  Rows / blocks in their
+// own order / so, us: T = 4, 4096 x 2048 8.3 / 10.1 / 8.5, x 3072 11.3 / 12.9 / 10.7, x 4096 16.1 / 16.8 /
+// 14.2, x 8192 30.3 / 27.8 / 23.1; 6144 x 2048 12.1 / 12.8 / 11.8; 12288 x 2048 18.9 / 19.9 / 18.7; gate/up 2 x
+// 2048 x 4096 9.8 / 8.9 (blocks); T = 24, 4096 x 2048 10.1 / 11.6 / 10.5.  Other numbers of workgroups
+// gain nothing by it or lose (32000 x 2048 46.2 -> 47.9, 11264 x 2048 18.1 -> 18.4; fewer than 256,
+// 1024 x 3072 at T = 16 9.1 -> 9.4).
+__device__ __forceinline__ int f32_column_block(int b, int n) {
+  return n % 128 == 0 && n >= 256 ? (b & 7) * (n >> 3) + (b >> 3) : b;
+}
+
 // k quarters summed in wave order: 0 + 1 + 2 + 3 (fixed, deterministic), and stored
 template <int MT, int NT>
 __device__ __forceinline__ void f32_gemm_store(f4 (&acc)[MT][NT], f4 (*red)[MT * NT][64],
@@ -92,7 +105,7 @@ __global__ __launch_bounds__(256) void f32_gemm_lds_kernel(const float *__restri
   static_assert(PF * PW <= 63, "vmcnt");
   __shared__ f4 lds[4][PF][F][128];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row0 = blockIdx.y * MT * 16, col0 = blockIdx.x * NT * 16;
+  const int row0 = blockIdx.y * MT * 16, col0 = (PACKED ? f32_column_block(blockIdx.x, gridDim.x) : (int)blockIdx.x) * NT * 16;
   const int r = lane & 15, g = lane >> 4;
   const int nb = K >> 5;  // k-blocks of 32 (host-checked K % 32 == 0)
   const int kb0 = wave * nb / 4, n = (wave + 1) * nb / 4 - kb0;
@@ -191,7 +204,7 @@ __global__ __launch_bounds__(256) void f32_gemm_few_kernel(const float *__restri
   static_assert(PF * PW <= 63, "vmcnt");
   __shared__ f4 lds[4][PF][PW][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col0 = blockIdx.x * COLS, r = lane & 15, g = lane >> 4;
+  const int col0 = f32_column_block(blockIdx.x, gridDim.x) * COLS, r = lane & 15, g = lane >> 4;
   const int nb = K >> 5;  // k-blocks of 32 (host-checked K % 32 == 0)
   const int kb0 = wave * nb / 4, n = (wave + 1) * nb / 4 - kb0;
   const int tiles = ((PAIR ? 2 * N : N) + 7) >> 3;  // of 8 columns: a k-block of W
@@ -414,7 +427,7 @@ bool f32_in_blocks(int K) { return K >= 1280; }
 // Packed weights (launch_pack_f32_blocks).  Up to 16 rows, T = 4, us, rows as they lie and
 // packed: 12288 x 4096 43.0 -> 35.6, 22016 x 4096 72.3 -> 64.8, K 11008 x N 4096 46.0 -> 31.2,
 // 4096 x 4096 17.6 -> 16.2, 6144 x 2048 12.4 -> 12.2, 11264 x 2048 19.3 -> 17.8, K 5632 x N 2048
-// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0; but 4096 x 2048 8.2 -> 10.1 (launches back to back).
+// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0.
 //  * Half tiles of columns where whole ones are at most half as many as CUs (K 5632 x N 2048
 //    14.4 -> 13.8, T = 16 16.3 -> 14.9; 768 x 3072 9.0 -> 8.5); at 256 and above they lose
 //    (6144 x 2048 13.1 -> 13.7, 11264 x 2048 18.3 -> 22.9).

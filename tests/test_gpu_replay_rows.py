@@ -79,8 +79,10 @@ def test_full_precision_does_not_depend_on_the_step(ff, vocab):
 
 
 # the same at widths of which every weight is kept in blocks: half tiles of columns (heads, ff), whole ones in
-# rings of two and of four k-blocks (qkv and lm_head), pairs, and columns past the last whole tile
-@pytest.mark.parametrize("hidden,ff,vocab", [(1280, 1312, 2101), (1280, 2080, 4101), (1536, 1280, 4097)])
+# rings of two and of four k-blocks (qkv and lm_head), pairs, columns past the last whole tile, and numbers of
+# columns that the workgroups of an XCD take in one piece
+@pytest.mark.parametrize("hidden,ff,vocab", [(1280, 1312, 2101), (1280, 2080, 4101), (1536, 1280, 4097),
+                                             (1280, 2048, 4096), (2048, 1280, 6144)])
 def test_full_precision_of_wide_rows_does_not_depend_on_the_step(hidden, ff, vocab, monkeypatch):
     monkeypatch.setitem(CFG, "hidden", hidden)
     monkeypatch.setitem(CFG, "num_heads", hidden // 128)
