@@ -981,37 +981,54 @@ hipError_t launch_softmax_topk_f32(const float *logits, int T, int V, int k, int
   return hipGetLastError();
 }
 
-// Rows of logits as fp32, into pinned host memory: bound by PCIe, so all that
-// matters is whole lines in flight (a wave writes 1 KiB at a time).
+// Rows of logits as fp32, into pinned host memory: bound by PCIe, so what matters is
+// whole lines in flight (a wave writes 1 KiB at a time) and that the host does not wait
+// for the last row before it copies the first.  So all workgroups write one row after the
+// other, and one that has written its columns of a row says so in a word of its own,
+// there[row][blockIdx.x] = mark (no counters to clear, no workgroup waits for another).
+// With rows shared out over 2, 4 and 16 groups of workgroups they end later than one after
+// the other: 24 decode steps of 8 rows of 32000, whole steps, 22.15 ms in one group, 22.18 in
+// two, 22.40 and 22.53 in four and 16 (all rows copied after the kernel: 23.0).
 template <class IN>
 __global__ __launch_bounds__(256) void logit_rows_kernel(const IN *__restrict__ logits, size_t ld, LogitRowIds ids,
-                                                         int V, float *__restrict__ dst) {
-  const IN *src = logits + (size_t)ids.row[blockIdx.y] * ld;
-  float *to = dst + (size_t)blockIdx.y * V;
+                                                         int n, int V, float *__restrict__ dst, uint32_t *there,
+                                                         uint32_t mark) {
   const bool wide = V % 4 == 0 && ld % 4 == 0;
-  for (int i = (blockIdx.x * 256 + threadIdx.x) * 4; i < V; i += gridDim.x * 1024) {
-    if (wide) {
-      f4 v;
-      if constexpr (sizeof(IN) == 4) v = *reinterpret_cast<const f4 *>(src + i);
-      else
+  for (int row = 0; row < n; ++row) {
+    const IN *src = logits + (size_t)ids.row[row] * ld;
+    float *to = dst + (size_t)row * V;
+    for (int i = (blockIdx.x * 256 + threadIdx.x) * 4; i < V; i += gridDim.x * 1024) {
+      if (wide) {
+        f4 v;
+        if constexpr (sizeof(IN) == 4) v = *reinterpret_cast<const f4 *>(src + i);
+        else
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (float)src[i + j];
-      *reinterpret_cast<f4 *>(to + i) = v;
-    } else {
-      for (int j = i; j < min(i + 4, V); ++j) to[j] = (float)src[j];
+          for (int j = 0; j < 4; ++j) v[j] = (float)src[i + j];
+        *reinterpret_cast<f4 *>(to + i) = v;
+      } else {
+        for (int j = i; j < min(i + 4, V); ++j) to[j] = (float)src[j];
+      }
     }
+    // every wave's writes are there, then the word (a release for the host)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(there + row * LogitRowIds::kParts + blockIdx.x, mark, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
 hipError_t launch_logit_rows(const void *logits, bool half, size_t ld, const LogitRowIds &ids, int n, int V,
-                             float *dst, hipStream_t s) {
+                             float *dst, uint32_t *there, uint32_t mark, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (n > LogitRowIds::kMax) return hipErrorInvalidValue;
-  const dim3 grid(std::min((V + 1023) / 1024, 32), n);
+  const dim3 grid(LogitRowIds::parts(V));
   if (half)
-    hipLaunchKernelGGL(logit_rows_kernel<_Float16>, grid, dim3(256), 0, s, (const _Float16 *)logits, ld, ids, V, dst);
+    hipLaunchKernelGGL(logit_rows_kernel<_Float16>, grid, dim3(256), 0, s, (const _Float16 *)logits, ld, ids, n, V,
+                       dst, there, mark);
   else
-    hipLaunchKernelGGL(logit_rows_kernel<float>, grid, dim3(256), 0, s, (const float *)logits, ld, ids, V, dst);
+    hipLaunchKernelGGL(logit_rows_kernel<float>, grid, dim3(256), 0, s, (const float *)logits, ld, ids, n, V, dst,
+                       there, mark);
   return hipGetLastError();
 }
 

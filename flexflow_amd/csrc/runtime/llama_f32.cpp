@@ -398,9 +398,10 @@ struct LlamaF32 : public ffmi_model {
       if (st != FFMI_OK) return st;
     }
     // (the step is on the stream: it is waited for whatever becomes of its rows)
-    const ffmi_status rows_st =
+    ffmi_status rows_st =
         k == 0 ? logit_rows.begin(logits, false, V, few_rows ? nullptr : rows, n, V, stream, out) : FFMI_OK;
-    FFMI_HIP(hipStreamSynchronize(stream));
+    if (k == 0 && rows_st == FFMI_OK) rows_st = logit_rows.finish();
+    if (k > 0 || n <= 0 || rows_st != FFMI_OK) FFMI_HIP(hipStreamSynchronize(stream));
     if (P > 1 && ffmi::comm_peer_attached(o.comm) && (st = ffmi::comm_status(o.comm)) != FFMI_OK)
       return st;
     if (dbg) dbg_T = T;
@@ -446,8 +447,7 @@ struct LlamaF32 : public ffmi_model {
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
     for (int i = 0; i < n; ++i) FFMI_CHECK(rows[i] >= 0 && rows[i] < bc.num_tokens, FFMI_ERR_INVALID);
-    const ffmi_status st = forward(0, rows, n, out);
-    return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish() : st;
+    return forward(0, rows, n, out);
   }
   ffmi_status run_tree(const TreeVerifyBatchConfig &bc, InferenceResult *ir) override {
     if (mode != FFMI_MODEL_TREE) return FFMI_ERR_INVALID;

@@ -1064,12 +1064,13 @@ struct LlamaGPU : public ffmi_model {
     return FFMI_OK;
   }
 
-  ffmi_status forward_finish() {
+  // waited: the stream's work of the step is done already
+  ffmi_status forward_finish(bool waited = false) {
     if (!inflight) return FFMI_OK;
     inflight = false;
     ffmi_status st;
     const double tw = step_timing ? now_us() : 0;
-    FFMI_HIP(hipStreamSynchronize(stream));
+    if (!waited) FFMI_HIP(hipStreamSynchronize(stream));
     if (step_timing) {
       const double te = now_us();
       float ms = 0;
@@ -1364,9 +1365,9 @@ struct LlamaGPU : public ffmi_model {
     ffmi_status st = forward_launch(0, rows, n);
     if (st == FFMI_OK && bc.num_tokens > 0)
       st = logit_rows.begin(logits, true, Vl, few_rows ? nullptr : rows, n, Vl, stream, out);
-    const ffmi_status fin = forward_finish();
-    if (st == FFMI_OK) st = fin;
-    return st == FFMI_OK && bc.num_tokens > 0 ? logit_rows.finish() : st;
+    if (st == FFMI_OK && bc.num_tokens > 0) st = logit_rows.finish();
+    const ffmi_status fin = forward_finish(st == FFMI_OK && bc.num_tokens > 0 && n > 0);
+    return st == FFMI_OK ? fin : st;
   }
   ffmi_status run_tree(const TreeVerifyBatchConfig &bc, InferenceResult *ir) override {
     if (mode != FFMI_MODEL_TREE) return FFMI_ERR_INVALID;

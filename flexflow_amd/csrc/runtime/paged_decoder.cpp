@@ -333,8 +333,9 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
     FFMI_TRY(enqueue(sample));
   }
   // (the step is on the stream: it is waited for and counted whatever becomes of its rows)
-  const ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream, out);
-  FFMI_HIP(hipStreamSynchronize(stream));
+  ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream, out);
+  if (!sample && rows_st == FFMI_OK) rows_st = logit_rows.finish();
+  if (sample || n <= 0 || rows_st != FFMI_OK) FFMI_HIP(hipStreamSynchronize(stream));
   if (recurrent)
     for (int t = 0; t < bc.num_tokens; ++t) {
       const auto &tk = bc.tokensInfo[t];
@@ -360,8 +361,7 @@ ffmi_status PagedDecoder::run_inc(const BatchConfig &bc, InferenceResult *ir) {
 }
 
 ffmi_status PagedDecoder::run_inc_logits(const BatchConfig &bc, const int *rows, int n, float *out) {
-  FFMI_TRY(forward(bc, rows, n, false, out));
-  return step.T > 0 && n > 0 ? logit_rows.finish() : FFMI_OK;
+  return forward(bc, rows, n, false, out);
 }
 
 ffmi_status PagedDecoder::set_debug(int enable) {

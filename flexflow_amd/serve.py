@@ -4,6 +4,7 @@ python/flexflow/serve/serve.py LLM/SSM).  All work happens in the C++
 runtime and HIP kernels; this file only marshals arguments.
 """
 import ctypes
+import struct
 import json
 import os
 from dataclasses import dataclass
@@ -360,27 +361,35 @@ class RequestManager:
         returns the wanted logits [rows, vocab] fp32, in the order of the
         entries and of `want` (include/ffmi.h ffmi_rm_replay_step)."""
         import numpy as np
-        arr = (F.ReplayEntry * max(1, len(entries)))()
-        keep, rows, order, ascending = [], 0, [], True
-        for a, (rid, tokens, want) in zip(arr, entries):
+        n = len(entries)
+        # one buffer of every entry's tokens and rows (an address costs more than the
+        # rest), and the records as 8-byte words: id, tokens, num_tokens, want, num_want
+        parts, at, rows, words, first, turned = [], 0, 0, [], [], {}
+        for i, (rid, tokens, want) in enumerate(entries):
             t = np.ascontiguousarray(tokens, np.int32)
             w = np.ascontiguousarray(want, np.int32).reshape(-1)
             if w.size > 1 and not (w[1:] > w[:-1]).all():  # the library takes them ascending
                 w, back = np.unique(w, return_inverse=True)
-                w, ascending = np.ascontiguousarray(w, np.int32), False
-                order.append(rows + back.reshape(-1))
-            else:
-                order.append(np.arange(rows, rows + len(w)))  # (whole numbers, also of no rows)
-            keep += [t, w]
-            a.id, a.num_tokens, a.num_want = rid, len(t), len(w)
-            a.tokens = ctypes.cast(t.ctypes.data, ctypes.POINTER(ctypes.c_int32))
-            a.want = ctypes.cast(w.ctypes.data, ctypes.POINTER(ctypes.c_int32))
-            rows += len(w)
+                w = np.ascontiguousarray(w, np.int32)
+                turned[i] = rows + back.reshape(-1)
+            words += (ctypes.c_int64(rid).value, at, len(t), at + t.size, w.size)
+            parts += (t, w)
+            first.append(rows)
+            at += t.size + w.size
+            rows += w.size
+        data = b"".join(parts)
+        base = ctypes.cast(data, ctypes.c_void_p).value
+        words[1::5] = [base + 4 * p for p in words[1::5]]
+        words[3::5] = [base + 4 * p for p in words[3::5]]
+        arr = (F.ReplayEntry * max(1, n)).from_buffer_copy(struct.pack(f"{5 * max(1, n)}q", *(words or [0] * 5)))
         out = np.empty((rows, llm.vocab_size), np.float32)
-        F.check(F.lib().ffmi_rm_replay_step(self.handle, llm.handle, arr, len(entries),
-                                            out.ctypes.data_as(ctypes.c_void_p), rows),
-                "replay step")
-        return out if ascending else out[np.concatenate(order)]
+        F.check(F.lib().ffmi_rm_replay_step(self.handle, llm.handle, arr, n,
+                                            ctypes.addressof(ctypes.c_char.from_buffer(out)) if out.size else None,
+                                            rows), "replay step")
+        if not turned:
+            return out
+        ends = first[1:] + [rows]
+        return out[np.concatenate([turned.get(i, np.arange(*p)) for i, p in enumerate(zip(first, ends))])]
 
     def replay_end(self, llm: Model, rid: int):
         """The replayed request is finished: its slot and pages are free."""

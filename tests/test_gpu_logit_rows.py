@@ -14,7 +14,7 @@ LLAMA = dict(num_layers=1, num_heads=2, num_kv_heads=2, hidden=128, intermediate
 
 
 @pytest.mark.parametrize("kind", ["fp16", "fp32", "paged"])
-@pytest.mark.parametrize("vocab", [500, 1203])
+@pytest.mark.parametrize("vocab", [500, 1203, 33001])
 def test_many_rows(kind, vocab):
     cfg = model_config(vocab, 96, 128, [layer(3, 24, 16, 40, 0.2, 160)]) if kind == "paged" else \
         dict(LLAMA, vocab_size=vocab)
