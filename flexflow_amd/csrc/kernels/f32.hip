@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void f32_gemm_few_kernel(const float *__restri
           (__attribute__((address_space(3))) void *)&lds[wave][slot][p][0], 16, 0, 0);
   };
   f4 acc[1][1] = {{f4{0.f, 0.f, 0.f, 0.f}}};
-  f4 cur[2][2], nxt[2][2];  // [X, W][half of the k-block]
+  f4 va[2][2], vb[2][2];  // [X, W][half of the k-block], of blocks in turn
   // (rows that were not copied: the first 8 again, in rows and columns that nobody takes)
   const int rx = XH ? 0 : r >> 3, rw = CX + (CW == 1 ? 0 : r >> 3);
   auto read = [&](int slot, f4 (&v)[2][2]) {
@@ -235,36 +235,67 @@ __global__ __launch_bounds__(256) void f32_gemm_few_kernel(const float *__restri
       v[1][h] = lds[wave][slot][rw][at];
     }
   };
-  auto wait = [](auto V) { __builtin_amdgcn_s_waitcnt((V.value & 15) | 0x0f70 | ((V.value >> 4) << 14)); };
+  auto wait = [](auto V) {  // vmcnt(V) alone
+    __builtin_amdgcn_s_waitcnt((V.value & 15) | 0x0f70 | ((V.value >> 4) << 14));
+    asm volatile("" ::: "memory");
+  };
 #pragma unroll
   for (int i = 0; i < PF; ++i)
     if (i < n) copy(i, i);
   if (n >= PF) wait(std::integral_constant<int, (PF - 1) * PW>{});
   else wait(std::integral_constant<int, 0>{});
-  asm volatile("" ::: "memory");
-  if (n > 0) read(0, cur);
+  if (n > 0) read(0, va);
   int slot = 0;
-  for (int kb = 0; kb < n; ++kb) {
+  // Block kb.  Its eight products are one chain (the sums' order), 32 cycles each, which is the
+  // time where few columns leave a wave alone on its SIMD: copies, waits and reads go into the
+  // gaps between them, and blocks in turn use two sets of registers (moved from one set to
+  // the other, and everything before the first product: K 5632 x N 2048 13.3 us at T = 4, so 10.9, 0.12 us
+  // a block of which the chain is all; 2048 x 2048 6.6 and 5.5, 6144 x 2048 11.6 and 10.9).
+  // MORE: block kb + PF exists; V: copies that may be out when block kb + 1 is read.
+  auto step = [&](auto MORE, auto V, int kb, const f4 (&cur)[2][2], f4 (&nxt)[2][2]) {
     const int next = slot + 1 == PF ? 0 : slot + 1;
+    const auto mul = [&](int h, int j) {
+      __builtin_amdgcn_sched_barrier(0);
+      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[0][h][j], cur[1][h][j], acc[0][0], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this block's operands are in registers
     asm volatile("" ::: "memory");
-    if (kb + PF < n) {
-      copy(kb + PF, slot);
-      wait(std::integral_constant<int, (PF - 1) * PW>{});
-    } else {
-      wait(std::integral_constant<int, 0>{});
-    }
-    asm volatile("" ::: "memory");
-    if (kb + 1 < n) read(next, nxt);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[0][h][j], cur[1][h][j], acc[0][0], 0, 0, 0);
-#pragma unroll
-    for (int f = 0; f < 2; ++f) cur[f][0] = nxt[f][0], cur[f][1] = nxt[f][1];
+    mul(0, 0);
+    if constexpr (MORE.value) copy(kb + PF, slot);
+    mul(0, 1);
+    wait(V);
+    read(next, nxt);  // (behind the last block: a slot that nobody needs)
+    mul(0, 2), mul(0, 3);
+    mul(1, 0), mul(1, 1), mul(1, 2), mul(1, 3);
     slot = next;
+  };
+  const std::true_type yes{};
+  const std::integral_constant<int, (PF - 1) * PW> all{};
+  int kb = 0;
+  for (; kb + 1 + PF < n; kb += 2) {
+    step(yes, all, kb, va, vb);
+    step(yes, all, kb + 1, vb, va);
   }
+  const auto turn = [&] {
+#pragma unroll
+    for (int f = 0; f < 2; ++f) va[f][0] = vb[f][0], va[f][1] = vb[f][1];
+  };
+  if (kb + PF < n) {
+    step(yes, all, kb++, va, vb);
+    turn();
+  }
+  // the last PF blocks, without copies
+  const auto drain = [&](auto REM) {
+    if (n - kb != REM.value) return;
+    step(std::false_type{}, std::integral_constant<int, (REM.value > 2 ? REM.value - 2 : 0) * PW>{}, kb++, va, vb);
+    turn();
+  };
+  const auto drains = [&](const auto &self, auto REM) -> void {
+    drain(REM);
+    if constexpr (REM.value > 1) self(self, std::integral_constant<int, REM.value - 1>{});
+  };
+  drains(drains, std::integral_constant<int, PF>{});
   __syncthreads();
   auto red = reinterpret_cast<f4(*)[1][64]>(&lds[0][0][0][0]);
   static_assert(sizeof(lds) >= 3 * 64 * sizeof(f4), "sum buffer");
@@ -425,15 +456,16 @@ hipError_t launch_gemm_f32(const float *X, const float *W, float *Y, int T, int 
 bool f32_in_blocks(int K) { return K >= 1280; }
 
 // Packed weights (launch_pack_f32_blocks).  Up to 16 rows, T = 4, us, rows as they lie and
-// packed: 12288 x 4096 43.0 -> 35.6, 22016 x 4096 72.3 -> 64.8, K 11008 x N 4096 46.0 -> 31.2,
-// 4096 x 4096 17.6 -> 16.2, 6144 x 2048 12.4 -> 12.2, 11264 x 2048 19.3 -> 17.8, K 5632 x N 2048
-// 14.2 -> 13.8, 2048 x 2048 7.0 and 7.0.
-//  * Half tiles of columns where whole ones are at most half as many as CUs (K 5632 x N 2048
-//    14.4 -> 13.8, T = 16 16.3 -> 14.9; 768 x 3072 9.0 -> 8.5); at 256 and above they lose
-//    (6144 x 2048 13.1 -> 13.7, 11264 x 2048 18.3 -> 22.9).
+// packed: 12288 x 4096 43.0 -> 34.4, 22016 x 4096 72.3 -> 62.7, K 11008 x N 4096 46.0 -> 29.3,
+// 4096 x 4096 17.6 -> 13.4, 6144 x 2048 12.4 -> 10.9, 11264 x 2048 19.3 -> 18.1, K 5632 x N 2048
+// 14.2 -> 10.2, 2048 x 2048 7.0 -> 5.5.
+//  * Half tiles of columns where whole ones are at most half as many as CUs; at 256 and above
+//    they lose (4096 x 4096 13.4 -> 14.7, K 11008 x N 4096 29.3 -> 33.1).  A workgroup is then alone
+//    on its CU: a ring of six k-blocks (K 5632 x N 2048 10.9 -> 10.2, 768 x 3072 6.7 -> 6.5; above 8
+//    rows, which copy more of X, of four: 12.6 and 12.7).
 //  * A ring of two k-blocks, four workgroups to a CU, where there are several rounds of
-//    them and K is short (6144 x 2048 13.1 -> 12.2, 12288 x 4096 37.1 -> 35.6; but 4096 x
-//    4096, one round, 16.5 and 17.2, and K 11008 32.1 and 40.5).
+//    them and K is short (6144 x 2048 11.4 -> 10.9, 32000 x 4096 96.1 -> 91.1; but 4096 x
+//    4096, one round, 13.4 and 14.9, and K 11008 29.3 and 34.6).
 static bool short_ring(int workgroups, int K) { return workgroups > 256 && K <= 4096; }
 hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int T, int N, int K, hipStream_t s) {
   if (T <= 0 || N <= 0) return hipSuccess;
@@ -441,7 +473,7 @@ hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int
   const int wgs = (N + 15) / 16;
   if (T > 16) f32_gemm_many<true>(X, Wp, Y, T, N, K, s);
   else if (wgs <= 128 && T <= 8)
-    hipLaunchKernelGGL((f32_gemm_few_kernel<4, true, 8, false>), dim3((N + 7) / 8), dim3(256), 0, s, X, Wp, Y, T, N, K);
+    hipLaunchKernelGGL((f32_gemm_few_kernel<6, true, 8, false>), dim3((N + 7) / 8), dim3(256), 0, s, X, Wp, Y, T, N, K);
   else if (wgs <= 128)
     hipLaunchKernelGGL((f32_gemm_few_kernel<4, false, 8, false>), dim3((N + 7) / 8), dim3(256), 0, s, X, Wp, Y, T, N, K);
   else if (short_ring(wgs, K))
@@ -453,6 +485,8 @@ hipError_t launch_gemm_f32_packed(const float *X, const float *Wp, float *Y, int
 
 // out [T][F] = silu(X Wg^T) * (X Wu^T), Wp: the F rows of gate, then up's, packed; gu: room
 // for [T][2 F] (more than 16 rows take the product and its unit one after the other).
+// Rings of two and of four k-blocks, T = 4: 2 x 3072 x 768 6.1 and 6.3 us, 2 x 5632 x 2048 18.4 and
+// 18.1 (T = 1 18.1 and 17.2), 2 x 11008 x 4096 63.7 and 62.7.
 hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu, float *out, int T, int F, int K,
                                      hipStream_t s) {
   if (T <= 0 || F <= 0) return hipSuccess;
@@ -461,7 +495,7 @@ hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu,
     return e != hipSuccess ? e : launch_silu_mul_f32(gu, gu + F, out, T, F, 2 * (size_t)F, 2 * (size_t)F, s);
   }
   if (K <= 0 || K % 32 || (((uintptr_t)X | (uintptr_t)Wp) & 15)) return hipErrorInvalidValue;
-  if (short_ring(F / 8, K))
+  if (F / 8 > 256 && K < 2048)
     hipLaunchKernelGGL((f32_gemm_few_kernel<2, false, 8, true>), dim3(F / 8), dim3(256), 0, s, X, Wp, out, T, F, K);
   else
     hipLaunchKernelGGL((f32_gemm_few_kernel<4, false, 8, true>), dim3(F / 8), dim3(256), 0, s, X, Wp, out, T, F, K);
