@@ -96,9 +96,11 @@ inline size_t memory_chunks_max(int T, int spans) { return (size_t)T / kMemoryCh
 hipError_t launch_memory_steps(const char *blob, int off_spans, int num_spans, const Memory &a,
                                const MemoryScratch *w, bool f32, int limit, bool *left, hipStream_t s);
 // Chunks (bf16 model): spans of more than `limit` >= kShortSpan tokens; num_chunks: the
-// step's (PagedSpan::chunk0 counts them).  The outputs are left in w.o.
+// step's (PagedSpan::chunk0 counts them).  The outputs are left in w.o.  left: the other spans
+// too, as launch_memory_steps would, in the same launch; where memory_mixes says so.
+bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit);
 hipError_t launch_memory_chunks(const char *blob, int off_spans, int num_spans, int num_chunks, const Memory &a,
-                                const MemoryScratch &w, int limit, hipStream_t s);
+                                const MemoryScratch &w, int limit, bool *left, hipStream_t s);
 // norm and gate of w.o, for the tokens of spans of more than `above` tokens
 hipError_t launch_memory_out(const char *blob, const Memory &a, const MemoryScratch &w, int above, hipStream_t s);
 

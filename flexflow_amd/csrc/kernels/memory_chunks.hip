@@ -18,7 +18,7 @@
 #include <algorithm>
 
 #include "conv_rows.h"
-#include "memory_util.h"
+#include "memory_steps.h"
 
 namespace ffmi {
 
@@ -108,30 +108,40 @@ __global__ __launch_bounds__(256) void memory_gates_kernel(const char *__restric
   }
 }
 
-// A workgroup per (chunk, head); wave b has the chunk's block of 16 tokens b.
+// LDS of a chunk's workgroup, in bytes
 template <MemoryRule RULE, int KS>
-__global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void memory_chunk_kernel(const char *__restrict__ blob, int off_spans,
-                                                                            int num_spans, Memory a, MemoryScratch w,
-                                                                            int limit) {
+struct ChunkLds {
+  static constexpr int DK = KS * 32, LDK = DK + 8, LDG = DK + 4, LDA = C + 4, VW = 64, LDV = VW + 8;
+  static constexpr int GB = C * LDG * 4, AB = C * LDA * 4 + C * LDV * 2;
+  static constexpr int kK = C * LDK * 2, kX = 2 * kK, kTot = kX + (GB > AB ? GB : AB), kBeta = kTot + 4 * DK * 4;
+  static constexpr int kBytes = kBeta + C * 4;
+  static_assert(kX % 16 == 0 && kTot % 16 == 0, "16-byte pieces");
+};
+
+// A workgroup's first four waves per (chunk, head); wave b has the chunk's block of 16 tokens b.
+template <MemoryRule RULE, int KS>
+__device__ __forceinline__ void memory_chunk(const char *__restrict__ blob, int off_spans, int num_spans,
+                                             const Memory &a, const MemoryScratch &w, int limit, int at_chunk, int h,
+                                             char *smem) {
   constexpr bool DELTA = RULE == kMemoryDelta;
-  constexpr int DK = KS * 32, LDK = DK + 8, LDG = DK + 4, LDA = C + 4, VW = 64, LDV = VW + 8;
-  constexpr int GB = C * LDG * 4, AB = C * LDA * 4 + C * LDV * 2;
-  __shared__ __attribute__((aligned(16))) uint16_t sQ[C * LDK], sK[C * LDK];
-  __shared__ __attribute__((aligned(16))) char sX[GB > AB ? GB : AB];
-  __shared__ __attribute__((aligned(16))) float tot[4][DK];
-  __shared__ float sbeta[C];
+  typedef ChunkLds<RULE, KS> L;
+  constexpr int DK = L::DK, LDK = L::LDK, LDG = L::LDG, LDA = L::LDA, VW = L::VW, LDV = L::LDV;
+  uint16_t *sQ = reinterpret_cast<uint16_t *>(smem), *sK = reinterpret_cast<uint16_t *>(smem + L::kK);
+  char *sX = smem + L::kX;
+  auto tot = reinterpret_cast<float(*)[DK]>(smem + L::kTot);
+  float *sbeta = reinterpret_cast<float *>(smem + L::kBeta);
   float *sG = reinterpret_cast<float *>(sX), *sA = sG;                       // (one after the other)
   uint16_t *sV = reinterpret_cast<uint16_t *>(sX + C * LDA * 4);
   const PagedSpan *spans = reinterpret_cast<const PagedSpan *>(blob + off_spans);
-  const int si = span_of_chunk(spans, num_spans, blockIdx.x);
+  const int si = span_of_chunk(spans, num_spans, at_chunk);
   if (si < 0) return;
   const PagedSpan sp = spans[si];
-  const int t0 = (blockIdx.x - sp.chunk0) * C, h = blockIdx.y, n = min(C, sp.n - t0);
+  const int t0 = (at_chunk - sp.chunk0) * C, n = min(C, sp.n - t0);
   if (sp.n <= limit) return;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l15 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hq = h / (a.H / a.G), cols = memory_columns(a);
-  const size_t id = (size_t)blockIdx.x * a.H + h, row0 = sp.t0 + t0;
+  const size_t id = (size_t)at_chunk * a.H + h, row0 = sp.t0 + t0;
   const size_t slab = (size_t)a.T * a.y.NP, zslab = (size_t)a.T * a.z.NP;
 
   // queries, keys, log decays: sixteen lanes a row, a wave's sixteen rows; everything is
@@ -483,6 +493,34 @@ __global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void memory_chunk_kernel(cons
   }
 }
 
+template <MemoryRule RULE, int KS>
+__global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void memory_chunk_kernel(const char *__restrict__ blob, int off_spans,
+                                                                            int num_spans, Memory a, MemoryScratch w,
+                                                                            int limit) {
+  __shared__ __attribute__((aligned(16))) char smem[ChunkLds<RULE, KS>::kBytes];
+  memory_chunk<RULE, KS>(blob, off_spans, num_spans, a, w, limit, blockIdx.x, blockIdx.y, smem);
+}
+// The same, and the short spans' tokens beside the chunks (launch_memory_steps' work): neither
+// fills the chip, each is a chain of 10-20 us, and they share nothing.  A prompt's portion of
+// 33 tokens beside 5 decoding requests, us: delta rule, 16 heads of 128, 16.6 + 21.2 -> 21.9; normed,
+// 4 of 128, 10.5 + 11.6 -> 12.9; gated, 4 of 256, 11.3 + 22.9 -> 26.3 (13 registers in scratch).
+template <MemoryRule RULE, int KS, bool SPLIT>
+__global__ __launch_bounds__(NT, 1) void memory_mixed_kernel(const char *__restrict__ blob, int off_spans, int num_spans,
+                                                             int num_chunks, Memory a, MemoryScratch w, int limit,
+                                                             MemoryStepsPlan plan) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int chunks = num_chunks * a.H, b = blockIdx.x;
+  if (b < chunks) {
+    if (threadIdx.x < 256)
+      memory_chunk<RULE, KS>(blob, off_spans, num_spans, a, w, limit, b % num_chunks, b / num_chunks,
+                             reinterpret_cast<char *>(lds));
+    return;
+  }
+  const int at = (b - chunks) / a.H;
+  memory_steps<RULE, uint16_t, 8, SPLIT>(blob, off_spans, a, w, limit, plan, (b - chunks) % a.H, at % num_spans,
+                                         at / num_spans, lds);
+}
+
 // The pass over the chunks: a workgroup per (head, VS state columns, span); a head's are
 // mostly on one XCD, which then reads the chunk's operands once.  Wave w: rows
 // 16 w .. of u and o, and of the state 16 columns and an even share of the rows, in
@@ -708,7 +746,7 @@ __global__ __launch_bounds__(256) void memory_out_kernel(const char *__restrict_
 
 template <MemoryRule RULE>
 hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_chunks, const Memory &a,
-                      const MemoryScratch &w, int limit, hipStream_t s) {
+                      const MemoryScratch &w, int limit, const MemoryStepsPlan *steps, hipStream_t s) {
   if (RULE == kMemoryNormed)
     hipLaunchKernelGGL(memory_gates_kernel, dim3(a.H, num_spans), dim3(256), 0, s, blob, off_spans, a, w, limit);
   if (RULE == kMemoryDelta) {
@@ -722,10 +760,24 @@ hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_ch
 #define FFMI_MS(KS, VS)                                                                                             \
   hipLaunchKernelGGL((memory_scan_kernel<RULE, KS, VS>), dim3(a.H, (a.vs + VS - 1) / VS, num_spans), dim3(256), 0, s, \
                      blob, off_spans, a, w, limit)
+  // (where memory_mixes says so)
+  const auto mixed = [&](auto KSc, auto SPLITc) {
+    constexpr int KS = decltype(KSc)::value;
+    constexpr bool SPLIT = decltype(SPLITc)::value;
+    if constexpr ((KS <= 4 || RULE == kMemoryGated) && !(SPLIT && RULE == kMemoryDelta))
+      hipLaunchKernelGGL((memory_mixed_kernel<RULE, KS, SPLIT>),
+                         dim3(a.H * (num_chunks + num_spans * steps->parts)), dim3(NT),
+                         std::max<size_t>(steps->bytes, ChunkLds<RULE, KS>::kBytes), s, blob, off_spans, num_spans,
+                         num_chunks, a, w, limit, *steps);
+  };
 #define FFMI_MC(KS)                                                                                              \
   do {                                                                                                           \
-    hipLaunchKernelGGL((memory_chunk_kernel<RULE, KS>), dim3(num_chunks, a.H), dim3(256), 0, s, blob, off_spans, \
-                       num_spans, a, w, limit);                                                                  \
+    constexpr std::integral_constant<int, KS> ks{};                                                              \
+    if (!steps)                                                                                                  \
+      hipLaunchKernelGGL((memory_chunk_kernel<RULE, KS>), dim3(num_chunks, a.H), dim3(256), 0, s, blob, off_spans, \
+                         num_spans, a, w, limit);                                                                \
+    else if (steps->parts > 1) mixed(ks, std::true_type{});                                                      \
+    else mixed(ks, std::false_type{});                                                                           \
     if (wide) FFMI_MS(KS, 32);                                                                                   \
     else FFMI_MS(KS, 16);                                                                                        \
   } while (0)
@@ -742,8 +794,17 @@ hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_ch
 
 }  // namespace
 
+// One workgroup of either kind fits a CU: one round of them, as a second would cost more than the
+// launch saved.  The chunks of 256 state rows need more registers than two waves of a SIMD
+// have: 16 too many with the gated rule, over 100 with the delta rule.
+bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit) {
+  const MemoryStepsPlan p = memory_steps_plan(a, num_spans, limit, true);
+  return a.dg <= (a.rule == kMemoryGated ? 256 : 128) && p.rows <= 8 && p.bytes <= 64 * 1024 && (p.parts == 1 || a.rule != kMemoryDelta) &&
+         (long)a.H * (num_chunks + (long)num_spans * p.parts) <= 256;
+}
+
 hipError_t launch_memory_chunks(const char *blob, int off_spans, int num_spans, int num_chunks, const Memory &a,
-                                const MemoryScratch &w, int limit, hipStream_t s) {
+                                const MemoryScratch &w, int limit, bool *left, hipStream_t s) {
   if (num_spans <= 0 || num_chunks <= 0) return hipSuccess;
   if (a.H < 1 || a.G < 1 || a.H % a.G || a.dg % 32 || a.vg % 32 || a.dg > kMemoryMaxChunkDim || a.dim > a.dg ||
       a.vdim > a.vg || a.vs != memory_state_columns(a.rule, a.vdim) || a.y.S < 1 || a.y.NP % 4 || a.col % 4 ||
@@ -753,9 +814,18 @@ hipError_t launch_memory_chunks(const char *blob, int off_spans, int num_spans, 
       !w.o || (a.rule == kMemoryDelta && (!w.w || !w.u || !w.rows || !a.rate)) ||
       (a.rule == kMemoryNormed && !w.gates) || num_chunks > 65535)
     return hipErrorInvalidValue;
-  if (a.rule == kMemoryGated) return run_chunks<kMemoryGated>(blob, off_spans, num_spans, num_chunks, a, w, limit, s);
-  if (a.rule == kMemoryDelta) return run_chunks<kMemoryDelta>(blob, off_spans, num_spans, num_chunks, a, w, limit, s);
-  return run_chunks<kMemoryNormed>(blob, off_spans, num_spans, num_chunks, a, w, limit, s);
+  MemoryStepsPlan plan;
+  if (left) {
+    if (bad_steps_shape(a) || !memory_mixes(a, num_spans, num_chunks, limit)) return hipErrorInvalidValue;
+    plan = memory_steps_plan(a, num_spans, limit, true);
+    *left = plan.parts > 1;
+  }
+  const MemoryStepsPlan *const steps = left ? &plan : nullptr;
+#define FFMI_MR(RULE) return run_chunks<RULE>(blob, off_spans, num_spans, num_chunks, a, w, limit, steps, s)
+  if (a.rule == kMemoryGated) FFMI_MR(kMemoryGated);
+  if (a.rule == kMemoryDelta) FFMI_MR(kMemoryDelta);
+  FFMI_MR(kMemoryNormed);
+#undef FFMI_MR
 }
 
 hipError_t launch_memory_out(const char *blob, const Memory &a, const MemoryScratch &w, int above, hipStream_t s) {

@@ -479,12 +479,13 @@ struct Pekarax : public PagedDecoder {
       FFMI_TRY(gemm_sum_to(low, L.wlow, L.nz, L.low, &a.z, zs, zs_bytes));
     }
     bool left = false;
-    if (shorts)
+    const bool mixed = shorts && longs && memory_mixes(a, step.num_spans, step.num_chunks, limit);
+    if (shorts && !mixed)
       FFMI_HIP(launch_memory_steps(step.dev, step.off_spans, step.num_spans, a, chunks ? &scratch : nullptr, f32,
                                    limit, &left, stream));
     if (longs)
       FFMI_HIP(launch_memory_chunks(step.dev, step.off_spans, step.num_spans, step.num_chunks, a, scratch, limit,
-                                    stream));
+                                    mixed ? &left : nullptr, stream));
     if (left || longs) FFMI_HIP(launch_memory_out(step.dev, a, scratch, left ? 0 : limit, stream));
     return FFMI_OK;
   }
