@@ -174,6 +174,7 @@ ffmi_status batch_stage(ffmi_batch_dev *b, const ffmi_batch_desc *d, size_t *byt
   memcpy(b->host, &h, sizeof(h));
   FFMI_CHECK(off <= b->cap, FFMI_ERR_INVALID);
   b->num_tokens = d->num_tokens;
+  b->off_tokens = h.off_tokens;
   b->num_work = d->num_work;
   b->num_commits = d->num_commits;
   b->num_mask_reqs = d->num_mask_reqs;

@@ -171,7 +171,17 @@ hipError_t launch_gate_up_f32_packed(const float *X, const float *Wp, float *gu,
                                      hipStream_t s);
 hipError_t launch_rmsnorm_f32(const float *x1, const float *x2, const float *w, float *res_out,
                               float *out, int T, int H, float eps, hipStream_t s,
-                              const char *gather = nullptr, const int32_t *rows = nullptr);
+                              const int32_t *rows = nullptr);
+// The same of the rows of x1 that the step's tokens name: its blob, staged at `host`
+// (mapped), is copied to `dev` for the kernels after this one.
+struct BlobFetch {
+  const char *host;
+  char *dev;
+  size_t bytes;
+  int off_tokens;
+};
+hipError_t launch_embed_rmsnorm_f32(const float *table, const BlobFetch &blob, const float *w, float *res_out,
+                                    float *out, int T, int H, float eps, hipStream_t s);
 hipError_t launch_silu_mul_f32(const float *A, const float *B, float *out, int T, int F,
                                size_t lda, size_t ldb, hipStream_t s);
 hipError_t launch_kv_update_f32(const char *blob, int T, int C, const float *qkv, const float *rope,
@@ -304,7 +314,7 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
                           uint16_t *res_out, uint16_t *out, int T, int H, float eps,
                           hipStream_t s, bool out_packed = false, Partials x2p = {}, const char *gather = nullptr,
                           char *blob_dst = nullptr, size_t blob_bytes = 0,
-                          const int32_t *gather_prev = nullptr,
+                          const int32_t *gather_prev = nullptr, int gather_tokens = 0,
                           // out row i (of T) from input row rows[i] of T_in; res_out is not written
                           const int32_t *rows = nullptr, int T_in = 0);
 // FFMI_FAULT_RESID_ROUND negative control (tests only; process-wide)
@@ -379,6 +389,7 @@ struct ffmi_batch_dev {
   int max_tokens = 0, max_requests = 0;
   // host-visible counts of the last upload (launch geometry)
   int num_tokens = 0, num_work = 0, num_commits = 0, num_mask_reqs = 0;
+  int off_tokens = 0;  // of the tokens in the blob (of num_work alone)
   bool commit_overlap = false;  // a commit depth is also a slot this step stores
   bool one_item_per_req = false;  // every request's tokens form one attention work item
   bool distinct_reqs = false;     // (of up to 64 tokens) no two tokens of one request

@@ -579,13 +579,27 @@ __global__ __launch_bounds__(256) void f32_rmsnorm_kernel(
 // 16 bytes per load and all loads in flight together, and stays in registers.  A row
 // of 2048 (4 tokens, residual): 8.4 us an element at a time, 4.7 this way, which is
 // three round trips to memory and the launch.
-template <int NV>
+// FETCH: the rows that the step's tokens name (BlobFetch).  A token's id is one trip to
+// the host's memory, on which the blob's copy goes along (a copy before, the header's
+// offset and the id from device memory: 2.8 us of their own and two trips more here).
+template <int NV, bool FETCH = false>
 __global__ __launch_bounds__(256) void f32_rmsnorm_vec_kernel(
     const float *x1, const float *__restrict__ x2, const float *__restrict__ w, float *res_out,
-    float *__restrict__ out, int H, float eps, const char *__restrict__ gather, const int32_t *__restrict__ rows) {
+    float *__restrict__ out, int H, float eps, std::conditional_t<FETCH, BlobFetch, const int32_t *> from) {
   __shared__ double sh[4];
-  const size_t row = (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * H;
-  const float *a = gather ? x1 + (size_t)batch_view(gather).tokens[blockIdx.x].token_id * H : x1 + row;
+  size_t row;
+  const float *a;
+  if constexpr (FETCH) {
+    row = (size_t)blockIdx.x * H;
+    a = x1 + (size_t)reinterpret_cast<const ffmi_token_info *>(from.host + from.off_tokens)[blockIdx.x].token_id * H;
+    const uint4 *src = reinterpret_cast<const uint4 *>(from.host);
+    const int n16 = (int)((from.bytes + 15) / 16);
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n16; i += gridDim.x * 256)
+      reinterpret_cast<uint4 *>(from.dev)[i] = src[i];
+  } else {
+    row = (size_t)(from ? from[blockIdx.x] : blockIdx.x) * H;
+    a = x1 + row;
+  }
   f4 v[NV], y[NV], g[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -620,24 +634,45 @@ __global__ __launch_bounds__(256) void f32_rmsnorm_vec_kernel(
   }
 }
 
+// rows and buffers of 16-byte pieces, up to 8 per thread (more would spill)
+static bool f32_rows_in_pieces(const float *x1, const float *x2, const float *w, const float *res_out,
+                               const float *out, int H) {
+  return H > 0 && H % 4 == 0 && H <= 8192 &&
+         (((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)res_out | (uintptr_t)out) & 15) == 0;
+}
 hipError_t launch_rmsnorm_f32(const float *x1, const float *x2, const float *w, float *res_out,
-                              float *out, int T, int H, float eps, hipStream_t s,
-                              const char *gather, const int32_t *rows) {
-  if (rows && (gather || res_out)) return hipErrorInvalidValue;
+                              float *out, int T, int H, float eps, hipStream_t s, const int32_t *rows) {
+  if (rows && res_out) return hipErrorInvalidValue;
   if (T <= 0) return hipSuccess;
-  // rows and buffers of 16-byte pieces, up to 8 per thread (more would spill)
-  const bool vec = H > 0 && H % 4 == 0 && H <= 8192 &&
-                   (((uintptr_t)x1 | (uintptr_t)x2 | (uintptr_t)w | (uintptr_t)res_out | (uintptr_t)out) & 15) == 0;
-  if (!vec)
-    hipLaunchKernelGGL(f32_rmsnorm_kernel, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
-  else if (H <= 1024)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<1>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
-  else if (H <= 2048)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<2>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
-  else if (H <= 4096)
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<4>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
-  else
-    hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<8>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, gather, rows);
+#define FFMI_NORM(NV) \
+  hipLaunchKernelGGL(f32_rmsnorm_vec_kernel<NV>, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, rows)
+  if (!f32_rows_in_pieces(x1, x2, w, res_out, out, H))
+    hipLaunchKernelGGL(f32_rmsnorm_kernel, dim3(T), dim3(256), 0, s, x1, x2, w, res_out, out, H, eps, nullptr, rows);
+  else if (H <= 1024) FFMI_NORM(1);
+  else if (H <= 2048) FFMI_NORM(2);
+  else if (H <= 4096) FFMI_NORM(4);
+  else FFMI_NORM(8);
+#undef FFMI_NORM
+  return hipGetLastError();
+}
+hipError_t launch_embed_rmsnorm_f32(const float *table, const BlobFetch &blob, const float *w, float *res_out,
+                                    float *out, int T, int H, float eps, hipStream_t s) {
+  if (!res_out || blob.off_tokens <= 0 || blob.bytes > (size_t)1 << 30 ||
+      (((uintptr_t)blob.host | (uintptr_t)blob.dev) & 15))
+    return hipErrorInvalidValue;
+  if (T <= 0) return hipSuccess;
+#define FFMI_NORM(NV)                                                                                                 \
+  hipLaunchKernelGGL((f32_rmsnorm_vec_kernel<NV, true>), dim3(T), dim3(256), 0, s, table, nullptr, w, res_out, out, H, \
+                     eps, blob)
+  if (!f32_rows_in_pieces(table, nullptr, w, res_out, out, H)) {
+    if (const hipError_t e = hipMemcpyAsync(blob.dev, blob.host, blob.bytes, hipMemcpyHostToDevice, s)) return e;
+    hipLaunchKernelGGL(f32_rmsnorm_kernel, dim3(T), dim3(256), 0, s, table, nullptr, w, res_out, out, H, eps,
+                       (const char *)blob.dev, nullptr);
+  } else if (H <= 1024) FFMI_NORM(1);
+  else if (H <= 2048) FFMI_NORM(2);
+  else if (H <= 4096) FFMI_NORM(4);
+  else FFMI_NORM(8);
+#undef FFMI_NORM
   return hipGetLastError();
 }
 

@@ -113,8 +113,10 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   // step's top-k ids, gprev, which the host could not know when it staged
   // this step; ffmi_model beam_launch_chained)
   int gid = 0;
+  // (their place in the blob, pNP, is known at launch: read from the blob's header it was one
+  // more trip to the host's memory before the row could be asked for)
   if (S == 3) {
-    gid = batch_view(gather).tokens[row].token_id;
+    gid = reinterpret_cast<const ffmi_token_info *>(gather + pNP)[row].token_id;
     if (gid < 0) gid = gprev[-1 - gid];
   }
   const uint16_t *a = S == 3 ? x1 + (size_t)gid * H : x1 + (size_t)row * H;
@@ -237,10 +239,10 @@ void set_norm_fault(bool on) { g_norm_fault = on; }
 hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t *w,
                           uint16_t *res_out, uint16_t *out, int T, int H, float eps,
                           hipStream_t s, bool out_packed, Partials x2p, const char *gather,
-                          char *blob_dst, size_t blob_bytes, const int32_t *gather_prev, const int32_t *rows,
-                          int T_in) {
+                          char *blob_dst, size_t blob_bytes, const int32_t *gather_prev, int gather_tokens,
+                          const int32_t *rows, int T_in) {
   if (rows && (gather || T_in <= 0)) return hipErrorInvalidValue;
-  if (gather && (x2 || x2p.S > 0 || !res_out)) return hipErrorInvalidValue;
+  if (gather && (x2 || x2p.S > 0 || !res_out || gather_tokens <= 0)) return hipErrorInvalidValue;
   if (blob_dst && (!gather || blob_bytes > (size_t)1 << 30 || (uintptr_t)gather % 16 ||
                    (uintptr_t)blob_dst % 16))
     return hipErrorInvalidValue;
@@ -265,7 +267,7 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
                : x2p.S <= 12 ? 12 : 16;
 #define FFMI_RMS4(NT, MC, MS, SR, RW)                                                          \
   hipLaunchKernelGGL((rmsnorm_kernel<NT, MC, MS, SR, RW>), dim3(T), dim3(NT), 0, s, x1, x2, w, \
-                     res_out, out, H, eps, op, pp, x2p.S, x2p.NP, gather,               \
+                     res_out, out, H, eps, op, pp, x2p.S, gather ? gather_tokens : x2p.NP, gather, \
                      reinterpret_cast<uint4 *>(blob_dst), rows ? T_in : blob_n16, rows ? rows : gather_prev)
 #define FFMI_RMS3(NT, MC, MS, SR)                                    \
   do {                                                               \

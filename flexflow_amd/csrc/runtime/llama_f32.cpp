@@ -318,15 +318,16 @@ struct LlamaF32 : public ffmi_model {
     ffmi_status st;
 #define TRY(x) \
   do { if ((st = (x)) != FFMI_OK) return st; } while (0)
-    TRY(batch_copy(batch, blob_bytes, stream, record_upload));
-    const char *blob = batch->dev;
     for (int l = 0; l < c.num_layers; ++l) {
       LayerF &L = layers[l];
       // layer 0: embedding gather into the first norm; then the residual norm
       // of the previous layer's down projection
-      if (l == 0)
-        FFMI_HIP(launch_rmsnorm_f32(embed, nullptr, L.in_norm, res, h, T, H, eps, stream, blob));
-      else
+      if (l == 0) {
+        // (which brings the step's blob to the device)
+        const BlobFetch blob = {batch->host, batch->dev, blob_bytes, batch->off_tokens};
+        FFMI_HIP(launch_embed_rmsnorm_f32(embed, blob, L.in_norm, res, h, T, H, eps, stream));
+        if (record_upload) FFMI_HIP(hipEventRecord(batch->uploaded, stream));
+      } else
         FFMI_HIP(launch_rmsnorm_f32(res, proj, L.in_norm, res, h, T, H, eps, stream));
       FFMI_HIP(product(h, L.wqkv, qkv, T, 3 * Hl, H));
       TRY(attn_forward(L.attn, batch, qkv, Partials(), att, (ffmi_stream)stream));
@@ -339,7 +340,7 @@ struct LlamaF32 : public ffmi_model {
     }
     const int n = tail_n;
     if (n == 0) return FFMI_OK;
-    FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, few_rows ? nullptr : res, h, n, H, eps, stream, nullptr,
+    FFMI_HIP(launch_rmsnorm_f32(res, proj, final_norm, few_rows ? nullptr : res, h, n, H, eps, stream,
                                 few_rows ? rows_h : nullptr));
     FFMI_HIP(product(h, lm, logits, n, V, H));
     if (k == 0) return FFMI_OK;  // logits only

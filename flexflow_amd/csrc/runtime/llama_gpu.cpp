@@ -1164,7 +1164,8 @@ struct LlamaGPU : public ffmi_model {
                                       l == 0 ? (blob_fetch ? batch->host : batch->dev) : nullptr,
                                       l == 0 && blob_fetch ? batch->dev : nullptr, blob_bytes,
                                       cur_slot > 0 ? ids_dev + (size_t)(cur_slot - 1) * (slot_ints() / 2)
-                                                   : nullptr));
+                                                   : nullptr,
+                                      batch->off_tokens));
         // the staging is free for the next step once the fetch has read it
         if (l == 0 && blob_fetch && record_upload) FFMI_HIP(hipEventRecord(batch->uploaded, stream));
         prof_end(pr, NORM, (double)T * H * 2 * (l == 0 ? 3 : 4), 0);
@@ -1277,7 +1278,7 @@ struct LlamaGPU : public ffmi_model {
         FFMI_HIP(ffmi::launch_rmsnorm(res, nullptr, final_norm, nullptr, h, T, H, eps, stream, packed));
       else
         FFMI_HIP(ffmi::launch_rmsnorm(res, proj, final_norm, res, h, tail_n, H, eps, stream, packed,
-                                      down_part, nullptr, nullptr, 0, nullptr, few_rows ? rows_h : nullptr, T));
+                                      down_part, nullptr, nullptr, 0, nullptr, 0, few_rows ? rows_h : nullptr, T));
       prof_end(pr, NORM, (double)tail_n * H * 2 * 4, 0);
     }
     mkt();
