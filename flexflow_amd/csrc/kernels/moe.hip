@@ -24,8 +24,8 @@ __device__ __forceinline__ float slab_total(const Partials &z, const float *p, s
 extern "C" __device__ float __ockl_wfred_max_f32(float);
 // the wave's largest value, NV a lane (column i * 64 + lane; the lowest among equals).
 // Picks follow one another, so a pick's latency counts: the maximum in the register
-// file and a ballot for its place.  (Six steps of two shuffles through LDS: the lists
-// of 38 tokens, 12 picks each, 17.2 us, now 9.9.)
+// file and a ballot for its place.  (Six steps of two shuffles through LDS: 38 tokens
+// of 12 picks in one workgroup 17.2 us instead of 9.9.)
 template <int NV>
 __device__ __forceinline__ int best_column(const float (&v)[NV], float &best) {
   float m = v[0];
@@ -41,10 +41,10 @@ __device__ __forceinline__ int best_column(const float (&v)[NV], float &best) {
   return at;
 }
 // A wave picks a token's experts: NV logits a lane, the best of the wave `top`
-// times over.
+// times over.  A lane's pick, the lane-th of the token (-1: none).
 template <int NV>
-__device__ __forceinline__ void pick_experts(const Partials &z, const float *__restrict__ bias, const MoeSizes &n,
-                                             int t, const MoeLists &l) {
+__device__ __forceinline__ int pick_experts(const Partials &z, const float *__restrict__ bias, const MoeSizes &n,
+                                            int t, const MoeLists &l) {
   const int lane = threadIdx.x & 63;
   const size_t slab = (size_t)n.T * z.NP;
   const float *row = z.p + (size_t)t * z.NP;
@@ -71,16 +71,14 @@ __device__ __forceinline__ void pick_experts(const Partials &z, const float *__r
     for (int i = 0; i < NV; ++i)
       if (at == i * 64 + lane) v[i] = -INFINITY;
   }
-  if (lane < n.top) {
-    l.picked[(size_t)t * n.top + lane] = min(mine_e, n.experts - 1);
-    l.wt[(size_t)t * n.top + lane] = __fdiv_rn(mine, sum);
-  }
+  if (lane < n.top) l.wt[(size_t)t * n.top + lane] = __fdiv_rn(mine, sum);
   if (n.shared && lane == 0) l.gate[t] = __fdiv_rn(1.0f, 1.0f + expf(-gate));
+  return lane < n.top ? min(mine_e, n.experts - 1) : -1;
 }
 // the same by scores
 template <int NV>
-__device__ __forceinline__ void pick_experts(const Partials &z, const MoeScores &sc, const MoeSizes &n, int t,
-                                             const MoeLists &l) {
+__device__ __forceinline__ int pick_experts(const Partials &z, const MoeScores &sc, const MoeSizes &n, int t,
+                                            const MoeLists &l) {
   const int lane = threadIdx.x & 63, cols = n.experts + n.identity, size = cols / sc.groups;
   const size_t slab = (size_t)n.T * z.NP;
   const float *row = z.p + (size_t)t * z.NP;
@@ -133,65 +131,94 @@ __device__ __forceinline__ void pick_experts(const Partials &z, const MoeScores 
     if (lane == k) mine = w, mine_e = at;
   }
   const float f = __fdiv_rn(sc.scale, total + 1e-20f);
-  if (lane < n.top) {
-    const bool real = mine_e < n.experts;
-    l.picked[(size_t)t * n.top + lane] = real ? mine_e : -1;
-    l.wt[(size_t)t * n.top + lane] = real ? mine * f : 0.f;
-  }
+  const bool real = lane < n.top && mine_e < n.experts;
+  if (lane < n.top) l.wt[(size_t)t * n.top + lane] = real ? mine * f : 0.f;
   if (n.identity && lane == 0) l.own[t] = own * f;
+  return real ? mine_e : -1;
 }
 // How: `const float *` (bias) or MoeScores
 template <int NV, class How>
 __global__ __launch_bounds__(256) void moe_pick_kernel(Partials z, How how, MoeSizes n, MoeLists l) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t < n.T) pick_experts<NV>(z, how, n, t, l);
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= n.T) return;
+  const int e = pick_experts<NV>(z, how, n, t, l);
+  if (lane < n.top) l.picked[(size_t)t * n.top + lane] = e;
 }
 
-// One workgroup: tokens by expert.  PICK: it picks the experts as well (few tokens).
-template <int NV, bool PICK, class How>
+// first slot of every expert, from its count (a scan over the first wave), and the tiles
+__device__ __forceinline__ void list_tiles(const int *count, int *next, const MoeSizes &n, const MoeLists &l,
+                                           int rows) {
+  const int tid = threadIdx.x, st = n.shared_tiles(rows);
+  if (tid >= 64) {
+    for (int i = tid - 64; i < st; i += 960)
+      l.tiles[i] = MoeTile{n.experts, i * rows, min(rows, n.T - i * rows), 0};
+    return;
+  }
+  const int per = (n.experts + 63) / 64, e0 = tid * per, e1 = min(e0 + per, n.experts);
+  int slots = 0, tiles = 0;
+  for (int e = e0; e < e1; ++e) slots += (count[e] + 15) & ~15, tiles += (count[e] + rows - 1) / rows;
+  const int own_s = slots, own_t = tiles;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int a = __shfl_up(slots, o), b = __shfl_up(tiles, o);
+    if (tid >= o) slots += a, tiles += b;
+  }
+  if (tid == 63) *l.num_tiles = st + tiles;
+  slots -= own_s, tiles += st - own_t;
+  for (int e = e0; e < e1; ++e) {
+    next[e] = slots;
+    for (int r = 0; r < count[e]; r += rows)
+      l.tiles[tiles++] = MoeTile{e, slots + r, min(rows, count[e] - r), 0};
+    slots += (count[e] + 15) & ~15;
+  }
+}
+// One workgroup: tokens by expert.  A pick's place among its expert's rows comes with
+// the count.
+//   NV > 0: it picks the experts as well, a token a wave (at most 16)
+//   NV = 0: of picks made before, U a thread;  U = 0: of any number
+template <int NV, int U, class How>
 __global__ __launch_bounds__(1024) void moe_lists_kernel(Partials z, How how, MoeSizes n, MoeLists l,
                                                          int rows) {
-  __shared__ int count[kMoeMaxExperts], next[kMoeMaxExperts], total;
-  const int tid = threadIdx.x, A = n.T * n.top, st = n.shared_tiles(rows);
+  __shared__ int count[kMoeMaxExperts], next[kMoeMaxExperts];
+  const int tid = threadIdx.x, A = n.T * n.top;
   for (int e = tid; e < n.experts; e += 1024) count[e] = 0;
-  if constexpr (PICK)
-    for (int t = tid >> 6; t < n.T; t += 16)
-      pick_experts<NV>(z, how, n, t, l);
-  __syncthreads();
-  for (int a = tid; a < A; a += 1024)
-    if (l.picked[a] >= 0) atomicAdd(&count[l.picked[a]], 1);
-  __syncthreads();
-  if (tid < 64) {  // first slot and first tile of every expert: a scan over the wave
-    const int per = (n.experts + 63) / 64, e0 = tid * per, e1 = min(e0 + per, n.experts);
-    int slots = 0, tiles = 0;
-    for (int e = e0; e < e1; ++e) slots += (count[e] + 15) & ~15, tiles += (count[e] + rows - 1) / rows;
-    const int own_s = slots, own_t = tiles;
+  constexpr int R = U ? U : 1;
+  int e[R], place[R];
+  const int t = tid >> 6;
+  if constexpr (NV) {
+    e[0] = -1;
+    if (t < n.T) e[0] = pick_experts<NV>(z, how, n, t, l);
+  } else if constexpr (U) {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int a = __shfl_up(slots, o), b = __shfl_up(tiles, o);
-      if (tid >= o) slots += a, tiles += b;
-    }
-    if (tid == 63) total = tiles;
-    slots -= own_s, tiles += st - own_t;
-    for (int e = e0; e < e1; ++e) {
-      next[e] = slots;
-      for (int r = 0; r < count[e]; r += rows)
-        l.tiles[tiles++] = MoeTile{e, slots + r, min(rows, count[e] - r), 0};
-      slots += (count[e] + 15) & ~15;
-    }
+    for (int u = 0; u < U; ++u) e[u] = tid + u * 1024 < A ? l.picked[tid + u * 1024] : -1;
   }
   __syncthreads();
-  for (int i = tid; i < st; i += 1024)
-    l.tiles[i] = MoeTile{n.experts, i * rows, min(rows, n.T - i * rows), 0};
-  if (tid == 0) *l.num_tiles = st + total;
-  for (int a = tid; a < A; a += 1024) {
-    if (l.picked[a] < 0) {
-      l.at[a] = -1;
-      continue;
-    }
-    const int slot = atomicAdd(&next[l.picked[a]], 1);
-    l.slot_token[slot] = a / n.top;
+  if constexpr (U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e[u] >= 0) place[u] = atomicAdd(&count[e[u]], 1);
+  } else {
+    for (int a = tid; a < A; a += 1024)
+      if (l.picked[a] >= 0) atomicAdd(&count[l.picked[a]], 1);
+  }
+  __syncthreads();
+  list_tiles(count, next, n, l, rows);
+  __syncthreads();
+  const auto put = [&](int a, int token, int slot) {
+    if (slot >= 0) l.slot_token[slot] = token;
     l.at[a] = slot;
+  };
+  if constexpr (NV) {
+    const int lane = tid & 63;
+    if (t < n.T && lane < n.top) put(t * n.top + lane, t, e[0] >= 0 ? next[e[0]] + place[0] : -1);
+  } else if constexpr (U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int a = tid + u * 1024;
+      if (a < A) put(a, a / n.top, e[u] >= 0 ? next[e[u]] + place[u] : -1);
+    }
+  } else {
+    for (int a = tid; a < A; a += 1024) put(a, a / n.top, l.picked[a] >= 0 ? atomicAdd(&next[l.picked[a]], 1) : -1);
   }
 }
 
@@ -204,13 +231,24 @@ static hipError_t route(const Partials &z, How how, const MoeSizes &n, const Moe
       (n.shared && n.gate_col >= z.NP) || (n.identity && !l.own))
     return hipErrorInvalidValue;
   const int rows = n.tile_rows();
+  // Picks are vector instructions, 50 and more each: a workgroup's four SIMDs take as
+  // long for 38 tokens (7.6 us, 4 of 32 experts; 50 for 64 tokens, 10 of 512) as the
+  // workgroups of a launch before it would for hundreds (5.7; 13.6 both launches).  One
+  // launch is the faster while a wave has one token (4.9 us for 16 tokens, 5.5 in two for
+  // 17), with more than 64 columns or 16 picks up to about half the waves (128 columns, 8
+  // picks: 5.1 for 8 tokens, 6.5 in two; 20 picks 10.6 for 16, 8.5 in two).
+  const bool together = n.T <= (cols <= 64 && n.top <= 16 ? 16 : 8);
+#define FFMI_ML(NV, U) \
+  hipLaunchKernelGGL((moe_lists_kernel<NV, U, How>), dim3(1), dim3(1024), 0, s, z, how, n, l, rows)
 #define FFMI_MR(NV)                                                                                          \
   do {                                                                                                       \
-    if (n.T <= 64) {                                                                                         \
-      hipLaunchKernelGGL((moe_lists_kernel<NV, true, How>), dim3(1), dim3(1024), 0, s, z, how, n, l, rows);  \
+    if (together) {                                                                                          \
+      FFMI_ML(NV, 1);                                                                                        \
     } else {                                                                                                 \
       hipLaunchKernelGGL((moe_pick_kernel<NV, How>), dim3((n.T + 3) / 4), dim3(256), 0, s, z, how, n, l);    \
-      hipLaunchKernelGGL((moe_lists_kernel<1, false, How>), dim3(1), dim3(1024), 0, s, z, how, n, l, rows);  \
+      if (n.T * n.top <= 1024) FFMI_ML(0, 1);                                                                \
+      else if (n.T * n.top <= 4096) FFMI_ML(0, 4);                                                           \
+      else FFMI_ML(0, 0);                                                                                    \
     }                                                                                                        \
   } while (0)
   if (cols <= 64) FFMI_MR(1);
@@ -218,6 +256,7 @@ static hipError_t route(const Partials &z, How how, const MoeSizes &n, const Moe
   else if (cols <= 256) FFMI_MR(4);
   else FFMI_MR(16);
 #undef FFMI_MR
+#undef FFMI_ML
   return hipGetLastError();
 }
 hipError_t launch_moe_route(const Partials &z, const float *bias, const MoeSizes &n, const MoeLists &l,
