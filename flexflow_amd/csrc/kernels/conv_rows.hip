@@ -6,10 +6,12 @@
 namespace ffmi {
 
 // A thread has 8 columns of TB tokens.  PAST: taps - 1, the earlier rows and the weights in
-// registers; or -1: read again.
-template <int PAST, bool F32>
+// registers; or -1: read again.  The tokens come one after another, and one that starts a
+// portion reads its carried rows first: a chain, so that a step of few columns has fewer
+// tokens a thread (launch_conv_rows).
+template <int TB, int PAST, bool F32>
 __global__ __launch_bounds__(256) void conv_rows_kernel(const char *__restrict__ blob, ConvRows a) {
-  constexpr int TB = 8, H = PAST > 0 ? PAST : 1;
+  constexpr int H = PAST > 0 ? PAST : 1;
   const int c = (blockIdx.x * 256 + threadIdx.x) * 8, t0 = blockIdx.y * TB;
   if (c >= a.cols) return;
   const PagedToken *tok = reinterpret_cast<const PagedToken *>(blob + a.off_tokens);
@@ -101,11 +103,23 @@ hipError_t launch_conv_rows(const char *blob, const ConvRows &a, hipStream_t s) 
   if (a.cols <= 0 || a.cols % 8 || a.col % 4 || a.u.NP % 4 || a.u.S < 1 || a.col + a.cols > a.u.NP || a.taps < 1 ||
       !a.conv || (a.taps > 1 && !a.carry) || (a.hb != nullptr) == (a.hf != nullptr))
     return hipErrorInvalidValue;
-  const dim3 grid((a.cols + 2047) / 2048, (a.T + 7) / 8);
-#define FFMI_CR(PAST)                                                                           \
-  do {                                                                                          \
-    if (a.hf) hipLaunchKernelGGL((conv_rows_kernel<PAST, true>), grid, dim3(256), 0, s, blob, a); \
-    else hipLaunchKernelGGL((conv_rows_kernel<PAST, false>), grid, dim3(256), 0, s, blob, a);   \
+  // Four taps, a portion and 7 single tokens, us with 1, 2, 4 and 8 tokens a thread:
+  //   38 x 6144    3.3   4.1   6.5   7.9      200 x 3072   3.9   4.2   6.5   9.3
+  //   400 x 6144   8.4   6.6   8.6  10.5      800 x 6144  14.7  11.5  12.3  14.6
+  //   1600 x 6144 25.5  19.1  18.3  20.5  (a portion alone: 24.8  17.8  15.6  16.6)
+  const long size = (long)a.T * a.cols;
+  const int tb = size <= 640 << 10 ? 1 : size <= 5 << 20 ? 2 : 4;
+  const dim3 grid((a.cols + 2047) / 2048, (a.T + tb - 1) / tb);
+#define FFMI_CT(TB, PAST)                                                                             \
+  do {                                                                                                \
+    if (a.hf) hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, true>), grid, dim3(256), 0, s, blob, a); \
+    else hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, false>), grid, dim3(256), 0, s, blob, a);     \
+  } while (0)
+#define FFMI_CR(PAST)                   \
+  do {                                  \
+    if (tb == 1) FFMI_CT(1, PAST);      \
+    else if (tb == 2) FFMI_CT(2, PAST); \
+    else FFMI_CT(4, PAST);              \
   } while (0)
   if (a.taps == 1) FFMI_CR(0);
   else if (a.taps == 2) FFMI_CR(1);
@@ -113,6 +127,7 @@ hipError_t launch_conv_rows(const char *blob, const ConvRows &a, hipStream_t s) 
   else if (a.taps == 4) FFMI_CR(3);
   else FFMI_CR(-1);
 #undef FFMI_CR
+#undef FFMI_CT
   return hipGetLastError();
 }
 
