@@ -63,6 +63,21 @@ struct MoeScores {
 };
 hipError_t launch_moe_route_scores(const Partials &z, const MoeScores &sc, const MoeSizes &n, const MoeLists &l,
                                    hipStream_t s);
+// The same in the kernel that makes a token's row: the product, the picks, their weights
+// (MoeLists); the lists are then a launch of their own.
+struct RouterWeights {
+  const uint16_t *w = nullptr;  // bf16 packed, `steps` k-steps of 32 columns
+  size_t tile = 0, step = 0;    // elements from tile to tile, k-step to k-step
+  int steps = 0;
+};
+struct RouteScores {
+  RouterWeights w;
+  MoeSizes n;
+  MoeScores scores;
+  MoeLists lists;
+};
+bool route_with_row(const MoeSizes &n, int H);  // (the rule) rows of H columns
+hipError_t launch_moe_lists(const MoeSizes &n, const MoeLists &l, hipStream_t s);
 
 // One product of every slot with its expert's matrix.
 //   first  (gated): Y[slot] = silu(X W_gate) (X W_up), X the token's row (row-major),

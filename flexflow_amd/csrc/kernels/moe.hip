@@ -4,144 +4,36 @@
 #include <algorithm>
 
 #include "device_util.h"
+#include "router.h"
 
 namespace ffmi {
 
 // ---------------------------------------------------------------------------
 // routing
 // ---------------------------------------------------------------------------
-// a column's sum over the slabs, their loads together
-__device__ __forceinline__ float slab_total(const Partials &z, const float *p, size_t slab) {
-  float v[8];
+// a column's sum over the slabs of a token's row, their loads together
+struct SlabTotal {
+  const float *row;
+  size_t slab;
+  int S;
+  __device__ __forceinline__ SlabTotal(const Partials &z, int T, int t)
+      : row(z.p + (size_t)t * z.NP), slab((size_t)T * z.NP), S(z.S) {}
+  __device__ __forceinline__ float operator()(int e) const {
+    float v[8];
 #pragma unroll
-  for (int s = 0; s < 8; ++s) v[s] = p[min(s, z.S - 1) * slab];
+    for (int s = 0; s < 8; ++s) v[s] = row[e + min(s, S - 1) * slab];
 #pragma unroll
-  for (int s = 1; s < 8; ++s)
-    if (s < z.S) v[0] += v[s];
-  return v[0];
-}
-// wave-wide maximum on DPP (device library), the same in every lane
-extern "C" __device__ float __ockl_wfred_max_f32(float);
-// the wave's largest value, NV a lane (column i * 64 + lane; the lowest among equals).
-// Picks follow one another, so a pick's latency counts: the maximum in the register
-// file and a ballot for its place.  (Six steps of two shuffles through LDS: 38 tokens
-// of 12 picks in one workgroup 17.2 us instead of 9.9.)
-template <int NV>
-__device__ __forceinline__ int best_column(const float (&v)[NV], float &best) {
-  float m = v[0];
-#pragma unroll
-  for (int i = 1; i < NV; ++i) m = fmaxf(m, v[i]);
-  best = __ockl_wfred_max_f32(m);
-  int at = 0;
-#pragma unroll
-  for (int i = NV - 1; i >= 0; --i) {
-    const unsigned long long where = __ballot(v[i] == best);
-    if (where) at = i * 64 + __builtin_ctzll(where);
+    for (int s = 1; s < 8; ++s)
+      if (s < S) v[0] += v[s];
+    return v[0];
   }
-  return at;
-}
-// A wave picks a token's experts: NV logits a lane, the best of the wave `top`
-// times over.  A lane's pick, the lane-th of the token (-1: none).
-template <int NV>
-__device__ __forceinline__ int pick_experts(const Partials &z, const float *__restrict__ bias, const MoeSizes &n,
-                                            int t, const MoeLists &l) {
-  const int lane = threadIdx.x & 63;
-  const size_t slab = (size_t)n.T * z.NP;
-  const float *row = z.p + (size_t)t * z.NP;
-  const float gate = n.shared ? slab_total(z, row + n.gate_col, slab) : 0.f;
-  float v[NV];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int e = i * 64 + lane;
-    v[i] = -INFINITY;
-    if (e < n.experts) {
-      v[i] = slab_total(z, row + e, slab) + bias[e];
-    }
-  }
-  float top0 = 0.f, sum = 0.f, mine = 0.f;  // lane k: the k-th pick
-  int mine_e = 0;
-  for (int k = 0; k < n.top; ++k) {
-    float best;
-    const int at = best_column<NV>(v, best);
-    if (k == 0) top0 = best;
-    const float p = expf(best - top0);
-    sum += p;
-    if (lane == k) mine = p, mine_e = at;
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (at == i * 64 + lane) v[i] = -INFINITY;
-  }
-  if (lane < n.top) l.wt[(size_t)t * n.top + lane] = __fdiv_rn(mine, sum);
-  if (n.shared && lane == 0) l.gate[t] = __fdiv_rn(1.0f, 1.0f + expf(-gate));
-  return lane < n.top ? min(mine_e, n.experts - 1) : -1;
-}
-// the same by scores
-template <int NV>
-__device__ __forceinline__ int pick_experts(const Partials &z, const MoeScores &sc, const MoeSizes &n, int t,
-                                            const MoeLists &l) {
-  const int lane = threadIdx.x & 63, cols = n.experts + n.identity, size = cols / sc.groups;
-  const size_t slab = (size_t)n.T * z.NP;
-  const float *row = z.p + (size_t)t * z.NP;
-  float s[NV], v[NV];
-  float mx = -INFINITY, sum = 0.f;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int e = i * 64 + lane;
-    s[i] = e < cols ? slab_total(z, row + e, slab) : -INFINITY;
-    mx = fmaxf(mx, s[i]);
-  }
-  mx = __ockl_wfred_max_f32(mx);
-#pragma unroll
-  for (int i = 0; i < NV; ++i) s[i] = expf(s[i] - mx), sum += s[i];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int e = i * 64 + lane;
-    s[i] = __fdiv_rn(s[i], sum);
-    v[i] = e < cols ? s[i] + sc.correction[e] : -INFINITY;
-  }
-  if (sc.keep < sc.groups) {  // the group of the best column left, `keep` times over
-    float left[NV];
-    bool in[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) left[i] = v[i], in[i] = false;
-    for (int k = 0; k < sc.keep; ++k) {
-      float best;
-      const int g = best_column<NV>(left, best) / size;
-#pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if ((i * 64 + lane) / size == g) in[i] = true, left[i] = -INFINITY;
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (!in[i]) v[i] = -INFINITY;
-  }
-  float mine = 0.f, total = 0.f, own = 0.f;
-  int mine_e = 0;
-  for (int k = 0; k < n.top; ++k) {
-    float best, w = 0.f;
-    const int at = best_column<NV>(v, best);
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (at == i * 64 + lane) v[i] = -INFINITY, w = s[i];
-    w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), at & 63));
-    total += w;
-    if (at >= n.experts) own += w;
-    if (lane == k) mine = w, mine_e = at;
-  }
-  const float f = __fdiv_rn(sc.scale, total + 1e-20f);
-  const bool real = lane < n.top && mine_e < n.experts;
-  if (lane < n.top) l.wt[(size_t)t * n.top + lane] = real ? mine * f : 0.f;
-  if (n.identity && lane == 0) l.own[t] = own * f;
-  return real ? mine_e : -1;
-}
+};
 // How: `const float *` (bias) or MoeScores
 template <int NV, class How>
 __global__ __launch_bounds__(256) void moe_pick_kernel(Partials z, How how, MoeSizes n, MoeLists l) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= n.T) return;
-  const int e = pick_experts<NV>(z, how, n, t, l);
+  const int e = pick_experts<NV>(SlabTotal(z, n.T, t), how, n, t, l);
   if (lane < n.top) l.picked[(size_t)t * n.top + lane] = e;
 }
 
@@ -187,7 +79,7 @@ __global__ __launch_bounds__(1024) void moe_lists_kernel(Partials z, How how, Mo
   const int t = tid >> 6;
   if constexpr (NV) {
     e[0] = -1;
-    if (t < n.T) e[0] = pick_experts<NV>(z, how, n, t, l);
+    if (t < n.T) e[0] = pick_experts<NV>(SlabTotal(z, n.T, t), how, n, t, l);
   } else if constexpr (U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) e[u] = tid + u * 1024 < A ? l.picked[tid + u * 1024] : -1;
@@ -222,6 +114,17 @@ __global__ __launch_bounds__(1024) void moe_lists_kernel(Partials z, How how, Mo
   }
 }
 
+// lists of picks made before
+static void lists_of(const MoeSizes &n, const MoeLists &l, int rows, hipStream_t s) {
+#define FFMI_ML(U)                                                                                              \
+  hipLaunchKernelGGL((moe_lists_kernel<0, U, const float *>), dim3(1), dim3(1024), 0, s, Partials(), nullptr, n, l, \
+                     rows)
+  const long picks = (long)n.T * n.top;
+  if (picks <= 1024) FFMI_ML(1);
+  else if (picks <= 4096) FFMI_ML(4);
+  else FFMI_ML(0);
+#undef FFMI_ML
+}
 template <class How>
 static hipError_t route(const Partials &z, How how, const MoeSizes &n, const MoeLists &l, hipStream_t s) {
   if (n.T <= 0) return hipSuccess;
@@ -246,9 +149,7 @@ static hipError_t route(const Partials &z, How how, const MoeSizes &n, const Moe
       FFMI_ML(NV, 1);                                                                                        \
     } else {                                                                                                 \
       hipLaunchKernelGGL((moe_pick_kernel<NV, How>), dim3((n.T + 3) / 4), dim3(256), 0, s, z, how, n, l);    \
-      if (n.T * n.top <= 1024) FFMI_ML(0, 1);                                                                \
-      else if (n.T * n.top <= 4096) FFMI_ML(0, 4);                                                           \
-      else FFMI_ML(0, 0);                                                                                    \
+      lists_of(n, l, rows, s);                                                                               \
     }                                                                                                        \
   } while (0)
   if (cols <= 64) FFMI_MR(1);
@@ -257,6 +158,14 @@ static hipError_t route(const Partials &z, How how, const MoeSizes &n, const Moe
   else FFMI_MR(16);
 #undef FFMI_MR
 #undef FFMI_ML
+  return hipGetLastError();
+}
+hipError_t launch_moe_lists(const MoeSizes &n, const MoeLists &l, hipStream_t s) {
+  if (n.T <= 0) return hipSuccess;
+  if (n.experts < 1 || n.identity < 0 || n.experts + n.identity > kMoeMaxExperts || n.top < 1 ||
+      n.top > std::min(n.experts + n.identity, kMoeMaxTop))
+    return hipErrorInvalidValue;
+  lists_of(n, l, n.tile_rows(), s);
   return hipGetLastError();
 }
 hipError_t launch_moe_route(const Partials &z, const float *bias, const MoeSizes &n, const MoeLists &l,

@@ -1,5 +1,6 @@
 // residual.h -- the 32-bit residual stream: launchers (residual.hip).
 #pragma once
+#include "moe.h"
 #include "paged.h"
 
 namespace ffmi {
@@ -45,7 +46,8 @@ struct SumNorm {
   uint16_t *hb = nullptr, *hrow = nullptr;
   int T = 0, H = 0, n = 0;  // columns, the first n of them real
 };
-hipError_t launch_sum_norm(const SumNorm &a, hipStream_t s);
+// route (where route_with_row; not with rows): the new rows' experts as well
+hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream_t s);
 // packed bf16 rows of the columns [col, col + n) of deferred sums, n a multiple of 32
 hipError_t launch_pack_sums(const Partials &y, int col, uint16_t *out, int T, int n, hipStream_t s);
 hipError_t launch_relu2_f32(float *u, size_t n, hipStream_t s);

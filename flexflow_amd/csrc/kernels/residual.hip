@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "device_util.h"
+#include "router.h"
 
 namespace ffmi {
 
@@ -217,16 +218,21 @@ hipError_t launch_row_norm(const char *blob, int off_rows, const float *x, const
 }
 
 // One workgroup per row, a thread's chunks of 8 columns; all loads before the
-// reduction, of slabs MAXS at a time.
-template <int NT, int MAXC, int MAXS>
-__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a) {
+// reduction, of slabs MAXS at a time.  RT > 0: the row's experts as well, of a router of
+// up to 16 RT columns.
+template <int NT, int MAXC, int MAXS, int RT = 0>
+__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores route) {
   constexpr int U = 4;  // expert rows in flight
   __shared__ float sh[NT / 64];
+  constexpr int NW = NT / 64, RTS = RT ? RT : 1;
+  __shared__ __attribute__((aligned(16))) uint16_t own_row[RT ? NT * 8 : 8];
+  __shared__ __attribute__((aligned(16))) float sums[NW * 16 * RTS];
+  RouterRow<RTS, NW> router;
   const int row = blockIdx.x, H = a.H, nchunk = H >> 3;
   f4 x[MAXC][2], wv[MAXC][2];
   float ss = 0.f;
   const float alpha = a.own ? a.alpha + a.own[row] : a.alpha;
-  const int32_t *at = a.rows ? a.at + (size_t)row * a.top : nullptr;
+  const int32_t *at = !RT && a.rows ? a.at + (size_t)row * a.top : nullptr;
   const float *wt = a.rows ? a.wt + (size_t)row * a.top : nullptr;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
@@ -245,6 +251,7 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a) {
       x[c][h] = *reinterpret_cast<const f4 *>(a.x + (size_t)row * H + ch * 8 + 4 * h) * alpha;
       wv[c][h] = *reinterpret_cast<const f4 *>(a.w + ch * 8 + 4 * h);
     }
+    if constexpr (RT > 0) router.begin(route.w);
     f4 y[2];
     y[0] = y[1] = f4{0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; at && k0 < a.top; k0 += U) {
@@ -294,15 +301,60 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a) {
     const uint4 b = pack8_bf16(x[c][0], x[c][1]);
     if (a.hb) *reinterpret_cast<uint4 *>(a.hb + act_packed_off(row, ch * 8, H)) = b;
     if (a.hrow) *reinterpret_cast<uint4 *>(a.hrow + (size_t)row * H + ch * 8) = b;
+    if constexpr (RT > 0) *reinterpret_cast<uint4 *>(own_row + ch * 8) = b;
+  }
+  if constexpr (RT > 0) {
+    __syncthreads();
+    router.product(route.w, own_row, sums);
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int e = pick_experts<1>(RouterTotal<RT, NW>{sums}, route.scores, route.n, row, route.lists);
+    if ((int)threadIdx.x < route.n.top) route.lists.picked[(size_t)row * route.n.top + threadIdx.x] = e;
   }
 }
-hipError_t launch_sum_norm(const SumNorm &a, hipStream_t s) {
+// Every row's workgroup reads the whole router (from the L2, 64 bytes a clock), which must
+// cost less than the launches saved: one, and with more than 16 tokens that of the picks.
+// A graph's time of norm, router, picks and lists, us, apart and so:
+//   12 x 2048   1 token 8.9  7.6   16 tokens 10.9  8.2    38 12.0  8.2   160 13.6  9.2
+//   36 x 2048           8.8  8.8             10.8  9.4       11.9  9.4       13.8 10.6
+//   64 x 2048           8.8  9.5             10.8 10.1       11.9 10.2       13.7 11.2
+//   64 x 4096           9.5 11.9             11.8 12.5       13.2 12.9       16.4 14.6
+bool route_with_row(const MoeSizes &n, int H) {
+  const int cols = n.shared ? n.gate_col + 1 : n.experts + n.identity, tiles = (cols + 15) / 16;
+  return n.T <= 256 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144);
+}
+hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;
   if (a.H % 32 || !a.x || !a.w || a.y.S < 0 || a.y.S > 8 || (a.y.S > 0 && (a.y.NP < a.H || a.y.NP % 4)) ||
       (a.rows && (a.top < 1 || !a.at || !a.wt)))
     return hipErrorInvalidValue;
   const int nchunk = a.H / 8;
-#define FFMI_SM(NT, MC, MS) hipLaunchKernelGGL((sum_norm_kernel<NT, MC, MS>), dim3(a.T), dim3(NT), 0, s, a)
+  if (route) {
+    const MoeSizes &n = route->n;
+    const MoeScores &sc = route->scores;
+    const int cols = n.experts + n.identity;
+    if (!route_with_row(n, a.H) || n.T != a.T || n.shared || a.rows || route->w.steps * 32 != a.H || !route->w.w ||
+        n.experts < 1 || n.identity < 0 || n.top < 1 || sc.groups < 1 || cols % sc.groups || sc.keep < 1 ||
+        sc.keep > sc.groups || n.top > cols / sc.groups * sc.keep || !sc.correction ||
+        (n.identity && !route->lists.own))
+      return hipErrorInvalidValue;
+#define FFMI_SR(MS, RT) hipLaunchKernelGGL((sum_norm_kernel<512, 1, MS, RT>), dim3(a.T), dim3(512), 0, s, a, *route)
+#define FFMI_SRS(RT)                 \
+  do {                               \
+    if (a.y.S == 0) FFMI_SR(0, RT);  \
+    else if (a.y.S == 1) FFMI_SR(1, RT); \
+    else FFMI_SR(4, RT);             \
+  } while (0)
+    if (cols <= 16) FFMI_SRS(1);
+    else if (cols <= 32) FFMI_SRS(2);
+    else if (cols <= 48) FFMI_SRS(3);
+    else FFMI_SRS(4);
+#undef FFMI_SRS
+#undef FFMI_SR
+    return hipGetLastError();
+  }
+#define FFMI_SM(NT, MC, MS) \
+  hipLaunchKernelGGL((sum_norm_kernel<NT, MC, MS>), dim3(a.T), dim3(NT), 0, s, a, RouteScores())
 #define FFMI_SMS(NT, MC)                 \
   do {                                   \
     if (a.y.S == 0) FFMI_SM(NT, MC, 0);  \

@@ -489,12 +489,17 @@ struct Pekarax : public PagedDecoder {
     if (left || longs) FFMI_HIP(launch_memory_out(step.dev, a, scratch, left ? 0 : limit, stream));
     return FFMI_OK;
   }
-  ffmi_status experts(const PekaraxLayer &L) {
+  // routed: the picks are made
+  ffmi_status experts(const PekaraxLayer &L, bool routed) {
     const MoeSizes n = sizes(L, step.T);
     const MoeLists &l = moe.lists;
-    Partials z;
-    FFMI_TRY(gemm_sum(rows_in(), L.wrouter, L.nr, Wp, &z));
-    FFMI_HIP(launch_moe_route_scores(z, L.scores, n, l, stream));
+    if (routed) {
+      FFMI_HIP(launch_moe_lists(n, l, stream));
+    } else {
+      Partials z;
+      FFMI_TRY(gemm_sum(rows_in(), L.wrouter, L.nr, Wp, &z));
+      FFMI_HIP(launch_moe_route_scores(z, L.scores, n, l, stream));
+    }
     MoeGemm a;
     a.experts = L.experts, a.slot_token = l.slot_token, a.tiles = l.tiles, a.num_tiles = l.num_tiles;
     a.limit = L.limit;
@@ -523,13 +528,17 @@ struct Pekarax : public PagedDecoder {
       SumNorm n = sum_norm(L.norm1);
       FFMI_TRY(gemm_sum(cat, L.wout, Wp, L.no, &n.y));
       if (L.experts) n.hrow = hrow;
-      FFMI_HIP(launch_sum_norm(n, stream));
+      RouteScores route;
+      route.n = sizes(L, step.T), route.scores = L.scores, route.lists = moe.lists;
+      route.w = {(const uint16_t *)L.wrouter, w_tile_stride(Wp / 32), w_k_stride(L.nr / 16), Wp / 32};
+      const bool routed = L.experts && !f32 && route_with_row(route.n, Wp);
+      FFMI_HIP(launch_sum_norm(n, routed ? &route : nullptr, stream));
       if (L.experts) {
-        FFMI_TRY(experts(L));
+        FFMI_TRY(experts(L, routed));
         n = sum_norm(L.norm2);
         n.rows = moe.rows, n.rows_f32 = f32, n.at = moe.lists.at, n.wt = moe.lists.wt, n.top = L.top;
         if (L.identity) n.own = moe.lists.own;
-        FFMI_HIP(launch_sum_norm(n, stream));
+        FFMI_HIP(launch_sum_norm(n, nullptr, stream));
       }
       FFMI_TRY(capture_layer((int)i));
     }

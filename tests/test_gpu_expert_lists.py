@@ -1,5 +1,6 @@
-"""Experts' lists: picked in their launch or in one before (up to 16 tokens at 64 columns and 16
-picks, up to 8 otherwise), one, four and any number of picks a thread (1024, 4096)."""
+"""Experts: the router beside the norm that makes its rows; the lists, picked in their launch or in
+one before (up to 16 tokens at 64 columns and 16 picks, up to 8 otherwise), of one, four and any
+number of picks a thread (1024, 4096)."""
 import pytest
 
 import nomutar_models as NM
@@ -24,4 +25,17 @@ def test_lists(tmp_path, n, top, T):
     w = PM.random_weights(cfg, 7)
     toks = tokens_p(cfg, T, 5)
     eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=256, positions=256)
+    close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
+
+
+@pytest.mark.parametrize("n,identity,width,T", [
+    (12, 4, 96, 1), (12, 5, 100, 16), (30, 4, 352, 17), (47, 2, 1500, 16), (60, 4, 1536, 16), (60, 4, 1568, 16),
+    (60, 4, 1568, 17), (61, 4, 96, 9), (33, 2, 4096, 256), (33, 2, 4096, 257), (33, 2, 4128, 20)])
+def test_router_beside_the_norm(tmp_path, n, identity, width, T):
+    """Up to 64 columns, 256 tokens and 4096 channels, with up to 16 tokens 6144 channels of 16
+    columns; what lies past each."""
+    cfg = PM.model_config(60, width, [PM.experts(PM.gla(1, 16, 16), n, 3, 32, identity=identity, groups=(1, 1))])
+    w = PM.random_weights(cfg, 9)
+    toks = tokens_p(cfg, T, 6)
+    eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=320, positions=320)
     close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
