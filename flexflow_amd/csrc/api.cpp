@@ -688,7 +688,7 @@ extern "C" ffmi_status ffmi_arg_topk_ws(const void *logits, int T, int V, int k,
 }
 
 // Test hooks of the residual RMSNorm folded into the decode GEMMs (the pair
-// llama_gpu.cpp runs at T <= 32): the producer adds its rounded output to
+// llama_gpu.cpp runs at T <= 16): the producer adds its rounded output to
 // the residual in place and leaves per-(row, 16-column tile) sums of
 // squares; the consumer normalises the residual from those sums in its
 // prologue.  Row-major fp16 throughout.

@@ -237,15 +237,17 @@ hipError_t launch_pack_weight(const uint16_t *src, int ld, int row0, int col0,
 // over the two GEMMs around it:
 //  * producer (o / down projection, EPI 0): Y = half(res_in + half(X.W^T))
 //    (Y may alias res_in) and, per row and 16-column tile, the fp32 sum of
-//    squares of those fp16 values -> ss_out[T][N/16];
-//  * consumer (the next qkv or gate/up): X is that residual, row-major; the
-//    prologue turns the row's ss_in partials into rms = half(1/sqrt(sum/K +
+//    squares of those fp16 values -> ss_out[T][N/16]; a copy in packed tiles
+//    for the consumer -> res_packed (N a multiple of 32);
+//  * consumer (the next qkv or gate/up): X is that residual, row-major or
+//    packed; the prologue turns the row's ss_in partials into rms = half(1/sqrt(sum/K +
 //    eps)) and every X fragment becomes half(half(x * rms) * w[k]) before its
 //    MFMA -- the norm kernel's arithmetic, fp16 multiplies.
 struct FuseArgs {
   int kind = 0;                     // 0 none, 1 producer, 2 consumer
   const uint16_t *res_in = nullptr;  // producer: [T][N] residual
   float *ss_out = nullptr;          // producer: [T][N/16]
+  uint16_t *res_packed = nullptr;   // producer: the new residual in packed tiles (null: not wanted)
   const float *ss_in = nullptr;     // consumer: [T][nss]
   int nss = 0;                      // consumer: partials per row (= K/16)
   const uint16_t *wnorm = nullptr;  // consumer: norm weight [K]

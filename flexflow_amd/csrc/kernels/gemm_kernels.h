@@ -115,7 +115,7 @@ __device__ __forceinline__ float lane_f(float v, int l) {
 }
 
 // FZ (FuseArgs, ffmi_internal.h): 1 = residual-add producer epilogue (EPI 0,
-// unsplit), 2 = RMSNorm consumer prologue on row-major X.  Y is restrict-
+// unsplit), 2 = RMSNorm consumer prologue.  Y is restrict-
 // qualified except in the producer, where it aliases fz.res_in (the residual
 // is updated in place).
 template <int FZ>
@@ -158,8 +158,18 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   constexpr int RPW = (MT * 16 + KW - 1) / KW;
   __shared__ float sRms[FZ == 2 ? MT * 16 : 1];
   float pv[FZ == 2 ? RPW : 1][4];
+  // The norm weight comes once per workgroup and lies in LDS (8 KiB: K <= 4096).  A load of
+  // its fragment per k-step, 64 bytes for 64 lanes, takes the L1 as long as one of X.
+  // 12288 x 4096 and gate / up of 11008 x 4096, 8 rows: so and X in rows 20.6 and 31.3 us;
+  // from LDS 19.0 and 29.9, X packed too 18.0 and 29.6; without a norm 17.1 and 28.9.
+  constexpr int WPT = FZ == 2 ? 4096 / 8 / (KW * 64) : 1;
+  __shared__ h8 sWn[FZ == 2 ? 4096 / 8 : 1];
+  h8 wpre[WPT];
   bool rdone = FZ != 2;
   if constexpr (FZ == 2) {
+#pragma unroll
+    for (int c = 0; c < WPT; ++c)
+      wpre[c] = *reinterpret_cast<const h8 *>(fz.wnorm + (size_t)min((int)threadIdx.x + c * KW * 64, K / 8 - 1) * 8);
 #pragma unroll
     for (int rr = 0; rr < RPW; ++rr) {
       const int m = min(wave + rr * KW, T - 1);
@@ -183,6 +193,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     if constexpr (FZ == 2) {
       if (rdone) return;
       rdone = true;
+#pragma unroll
+      for (int c = 0; c < WPT; ++c) sWn[threadIdx.x + c * KW * 64] = wpre[c];
 #pragma unroll
       for (int rr = 0; rr < RPW; ++rr) {
         const int m = wave + rr * KW;
@@ -210,9 +222,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     }
   };
   // norm weight fragment of k-step k (this lane's 8 columns)
-  auto ldwn = [&](int k) -> h8 {
-    return *reinterpret_cast<const h8 *>(fz.wnorm + (size_t)k * 32 + 8 * (lane >> 4));
-  };
+  auto ldwn = [&](int k) -> h8 { return sWn[k * 4 + (lane >> 4)]; };
   // y = half(half(x * rms) * w): two fp16 multiplies, as the norm kernel
   auto nrm = [&](h8 &a, int i, const h8 &w) {
     if constexpr (FZ == 2) a = (a * rms8[i]) * w;
@@ -261,26 +271,28 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     const int nb = (ke - kt) / UP;
     if (nb > 0) {
       h8 bA[UP][NT], aA[UP][MT], bB[UP][NT], aB[UP][MT];
-      h8 wA[FZ == 2 ? UP : 1], wB[FZ == 2 ? UP : 1];
-      auto ld = [&](h8(&bb)[UP][NT], h8(&aa)[UP][MT], h8(&ww)[FZ == 2 ? UP : 1], int k0) {
+      auto ld = [&](h8(&bb)[UP][NT], h8(&aa)[UP][MT], int k0) {
 #pragma unroll
         for (int u = 0; u < UP; ++u)
 #pragma unroll
           for (int j = 0; j < NT; ++j)
             bb[u][j] = ld_weight<NTL>(wrow[j] + (size_t)(k0 + u) * wks);
 #pragma unroll
-        for (int u = 0; u < UP; ++u) {
+        for (int u = 0; u < UP; ++u)
 #pragma unroll
           for (int i = 0; i < MT; ++i)
             aa[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)(k0 + u) * XS);
-          if constexpr (FZ == 2) ww[u] = ldwn(k0 + u);
-        }
       };
-      auto mm = [&](h8(&bb)[UP][NT], h8(&aa)[UP][MT], h8(&ww)[FZ == 2 ? UP : 1]) {
+      auto mm = [&](h8(&bb)[UP][NT], h8(&aa)[UP][MT], int k0) {
+        if constexpr (FZ == 2) {
+          h8 ww[UP];
 #pragma unroll
-        for (int u = 0; u < UP; ++u)
+          for (int u = 0; u < UP; ++u) ww[u] = ldwn(k0 + u);
 #pragma unroll
-          for (int i = 0; i < MT; ++i) nrm(aa[u][i], i, ww[FZ == 2 ? u : 0]);
+          for (int u = 0; u < UP; ++u)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) nrm(aa[u][i], i, ww[u]);
+        }
 #pragma unroll
         for (int u = 0; u < UP; ++u)
 #pragma unroll
@@ -289,30 +301,30 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
             for (int j = 0; j < NT; ++j)
               acc[i][j] = mma16<EPI>(aa[u][i], bb[u][j], acc[i][j]);
       };
-      ld(bA, aA, wA, kt);
+      ld(bA, aA, kt);
       rms_finish();
       int q = 0;
       for (; q + 2 < nb; q += 2) {
-        ld(bB, aB, wB, kt + UP);
+        ld(bB, aB, kt + UP);
         __builtin_amdgcn_sched_barrier(0);
-        mm(bA, aA, wA);
+        mm(bA, aA, kt);
         __builtin_amdgcn_sched_barrier(0);
-        ld(bA, aA, wA, kt + 2 * UP);
+        ld(bA, aA, kt + 2 * UP);
         __builtin_amdgcn_sched_barrier(0);
-        mm(bB, aB, wB);
+        mm(bB, aB, kt + UP);
         __builtin_amdgcn_sched_barrier(0);
         kt += 2 * UP;
       }
       if (q + 1 < nb) {  // two batches left
-        ld(bB, aB, wB, kt + UP);
+        ld(bB, aB, kt + UP);
         __builtin_amdgcn_sched_barrier(0);
-        mm(bA, aA, wA);
+        mm(bA, aA, kt);
         __builtin_amdgcn_sched_barrier(0);
-        mm(bB, aB, wB);
+        mm(bB, aB, kt + UP);
         kt += 2 * UP;
       } else {  // one batch left
         __builtin_amdgcn_sched_barrier(0);
-        mm(bA, aA, wA);
+        mm(bA, aA, kt);
         kt += UP;
       }
     }
@@ -320,28 +332,28 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   for (; kt + U <= ke; kt += U) {
     h8 b[U][NT];
     h8 a[U][MT];
-    h8 wn[FZ == 2 ? U : 1];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int j = 0; j < NT; ++j)
         b[u][j] = ld_weight<NTL>(wrow[j] + (size_t)(kt + u) * wks);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)(kt + u) * XS);
-      if constexpr (FZ == 2) wn[u] = ldwn(kt + u);
-    }
     rms_finish();
     // keep the whole batch of loads ahead of the MFMAs: left alone the
     // scheduler interleaves them and reuses registers, leaving ~7 loads in
     // flight per wave with a vmcnt wait before almost every MFMA
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FZ == 2)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u) {
+        const h8 wn = ldwn(kt + u);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) nrm(a[u][i], i, wn[FZ == 2 ? u : 0]);
+        for (int i = 0; i < MT; ++i) nrm(a[u][i], i, wn);
+      }
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -358,7 +370,6 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     const int rem = ke - kt;
     h8 b[U - 1][NT];
     h8 a[U - 1][MT];
-    h8 wn[FZ == 2 ? U - 1 : 1];
 #pragma unroll
     for (int u = 0; u < U - 1; ++u) {
       const int kk = min(kt + u, ke - 1);
@@ -368,15 +379,17 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)kk * XS);
-      if constexpr (FZ == 2) wn[u] = ldwn(kk);
     }
     rms_finish();
     __builtin_amdgcn_sched_barrier(0);
     const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    if constexpr (FZ == 2)
 #pragma unroll
-    for (int u = 0; u < U - 1; ++u)
+      for (int u = 0; u < U - 1; ++u) {
+        const h8 wn = ldwn(min(kt + u, ke - 1));
 #pragma unroll
-      for (int i = 0; i < MT; ++i) nrm(a[u][i], i, wn[FZ == 2 ? u : 0]);
+        for (int i = 0; i < MT; ++i) nrm(a[u][i], i, wn);
+      }
 #pragma unroll
     for (int u = 0; u < U - 1; ++u) {
       if (u >= rem)
@@ -450,6 +463,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
           float sq = 0.f;
           if (nok && m < T) {
             reinterpret_cast<_Float16 *>(Y)[(size_t)m * N + n] = rh;
+            if (fz.res_packed) reinterpret_cast<_Float16 *>(fz.res_packed)[act_packed_off(m, n, N)] = rh;
             const float f = (float)rh;
             sq = f * f;
           }
@@ -1612,12 +1626,12 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   if ((xp && K % 32) || (yp && (N % 32 || yp % 32 || yp < N))) return hipErrorInvalidValue;
   if constexpr (E < 2)
   if (fuse && fuse->kind) {
-    // producer: row-major residual out, plain epilogue; consumer: row-major X
-    // (the residual), K = the norm width; both unsplit, T <= 32
+    // producer: row-major residual out, plain epilogue; consumer: X is the
+    // residual, K = the norm width; both unsplit, T <= 32
     if (mtiles > 2 || N % 16 || K % 32) return hipErrorInvalidValue;
-    if (fuse->kind == 1 && (paired || yp || !fuse->res_in || !fuse->ss_out))
+    if (fuse->kind == 1 && (paired || yp || !fuse->res_in || !fuse->ss_out || (fuse->res_packed && N % 32)))
       return hipErrorInvalidValue;
-    if (fuse->kind == 2 && (xp || !fuse->ss_in || !fuse->wnorm || fuse->nss <= 0 || fuse->nss > 256))
+    if (fuse->kind == 2 && (!fuse->ss_in || !fuse->wnorm || fuse->nss <= 0 || fuse->nss > 256 || K > 4096))
       return hipErrorInvalidValue;
     const int wp = wpitch ? wpitch : (paired ? 2 : 1) * ((N + 15) / 16);
 #define FFMI_FZ(MTV, FZV) \

@@ -77,9 +77,12 @@ struct LlamaGPU : public ffmi_model {
   // (its all-reduce synchronises the host) and runs eager and unsplit
   bool rccl = false;
   bool solo = false;  // TP shard over a 1-rank communicator without transport or RCCL
-  // residual norms folded into the skinny GEMMs around them (T <= 32, TP = 1):
+  // residual norms folded into the skinny GEMMs around them (T <= 16, TP = 1):
   // per-tile sums of squares of the residual after o (ss_o) and after down
-  // (ss_d), [32][H/16] each.  Only where o/down run unsplit anyway (H/16 >=
+  // (ss_d), [32][H/16] each.  With more rows a wave norms its operands for two
+  // row tiles, and qkv and gate/up of H = 4096 at 24 and 32 rows take 69.8 and
+  // 74.0 us, as products of normed rows 57.0 and 59.7 (two norm launches: 6-7);
+  // of H = 2048 29.4 and 31.2 against 23.1 and 24.2.  Only where o/down run unsplit anyway (H/16 >=
   // 128 tiles: LLaMA-7B decode, +1.9% incr decoding -- the A/B of record is
   // profiles/r03_fused_norm_ab.log, quoted in DESIGN.md §5); the 68M SSM's
   // o/down split K over workgroups, and unsplitting them to fuse cost more
@@ -871,7 +874,7 @@ struct LlamaGPU : public ffmi_model {
   // the residual norms folded into the GEMMs around them (see fuse_norms)
   bool fused_norms(int T) const {
     const int H = c.hidden;
-    return (fuse_norms == 2 || (fuse_norms == 1 && H >= 2048)) && !dbg && o.tp_size == 1 && T <= 32 &&
+    return (fuse_norms == 2 || (fuse_norms == 1 && H >= 2048)) && !dbg && o.tp_size == 1 && T <= 16 &&
            H % 32 == 0 && Hl % 32 == 0 && H <= 4096;
   }
   ffmi::OprojArgs oproj_args(const Layer &L, int T) const {
@@ -1148,6 +1151,7 @@ struct LlamaGPU : public ffmi_model {
         fz_o.kind = fz_d.kind = 1;
         fz_o.res_in = fz_d.res_in = res;
         fz_o.ss_out = ss_o, fz_d.ss_out = ss_d;
+        if (packed) fz_o.res_packed = fz_d.res_packed = h;
         fz_qkv.kind = fz_gu.kind = 2;
         fz_qkv.ss_in = ss_d, fz_gu.ss_in = ss_o;
         fz_qkv.nss = fz_gu.nss = H / 16;
@@ -1179,8 +1183,8 @@ struct LlamaGPU : public ffmi_model {
       }
       pr = prof_begin(on);
       ffmi::Partials qkv_part;
-      FFMI_HIP(ffmi::launch_gemm(fz_in ? res : h, L.wqkv, qkv, (float *)ws, ws_bytes, T, 3 * Hl, H,
-                                 fz_in ? wstream : XP, stream, &qkv_part, 0,
+      FFMI_HIP(ffmi::launch_gemm(fz_in && !packed ? res : h, L.wqkv, qkv, (float *)ws, ws_bytes, T, 3 * Hl, H,
+                                 XP, stream, &qkv_part, 0,
                                  fz_in ? &fz_qkv : nullptr));
       prof_end(pr, GEMM_QKV, gemm_bytes(T, 3 * Hl, 3 * Hl, H), 2.0 * T * 3 * Hl * H);
       mk();
@@ -1229,8 +1233,8 @@ struct LlamaGPU : public ffmi_model {
       pr = prof_begin(on);
       const int YP = packed ? FFMI_Y_PACKED : 0;
       if (fuse)
-        FFMI_HIP(ffmi::launch_gemm(res, L.wgu, mlp, (float *)ws, ws_bytes, T, Fl, H,
-                                   FFMI_EPI_SILU_MUL | YP | wstream, stream, nullptr, 0, &fz_gu));
+        FFMI_HIP(ffmi::launch_gemm(packed ? h : res, L.wgu, mlp, (float *)ws, ws_bytes, T, Fl, H,
+                                   FFMI_EPI_SILU_MUL | XP | YP, stream, nullptr, 0, &fz_gu));
       else
         TRY(ffmi_linear_ws(h, L.wgu, mlp, T, Fl, H, FFMI_EPI_SILU_MUL | XP | YP, ws, ws_bytes, s));
       prof_end(pr, GEMM_GATE_UP, gemm_bytes(T, 2 * Fl, Fl, H), 2.0 * T * 2 * Fl * H);
