@@ -243,8 +243,18 @@ hipError_t launch_pack_weight(const uint16_t *src, int ld, int row0, int col0,
 //    packed; the prologue turns the row's ss_in partials into rms = half(1/sqrt(sum/K +
 //    eps)) and every X fragment becomes half(half(x * rms) * w[k]) before its
 //    MFMA -- the norm kernel's arithmetic, fp16 multiplies.
+// The same of an fp32 residual and bf16 operands (one row tile, T <= 16, unsplit
+// producer; the norm's arithmetic but for the place of the rms):
+//  * 3, producer (fp32 sums): x += X.W^T, hb = bf16(x * w32) in packed tiles and the
+//    sums of squares of x (w32 null: x alone);
+//  * 4, consumer: X is that hb; the sums are multiplied by the row's
+//    1 / sqrt(sum / width + eps), as a factor of a whole row commutes with the product.
 struct FuseArgs {
-  int kind = 0;                     // 0 none, 1 producer, 2 consumer
+  int kind = 0;                     // 0 none, 1, 3 producer, 2, 4 consumer
+  float *x = nullptr;               // 3: [T][N]
+  const float *w32 = nullptr;       // 3: norm weight [N]
+  uint16_t *hb = nullptr;           // 3
+  int width = 0;                    // 4: real columns of the residual
   const uint16_t *res_in = nullptr;  // producer: [T][N] residual
   float *ss_out = nullptr;          // producer: [T][N/16]
   uint16_t *res_packed = nullptr;   // producer: the new residual in packed tiles (null: not wanted)
@@ -290,12 +300,13 @@ hipError_t launch_gemm_bf16_relu2(const uint16_t *X, const uint16_t *Wp, uint16_
                                   Partials *defer = nullptr);
 hipError_t launch_gemm_bf16_f32(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                                 size_t ws_bytes, int T, int N, int K, int flags, hipStream_t s,
-                                Partials *defer = nullptr);
+                                Partials *defer = nullptr, const FuseArgs *fuse = nullptr);
 // Wp: gate and up tiles interleaved (2 N columns); Y bf16 = clamped_glu
 size_t gemm_bf16_glu_workspace_bytes(int T, int N, int K);
 hipError_t launch_gemm_bf16_glu(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float *ws,
                                 size_t ws_bytes, int T, int N, int K, int flags, float limit,
-                                hipStream_t s);
+                                hipStream_t s,
+                                const FuseArgs *fuse = nullptr);
 // The same with a SiLU gate.  y_width: width of the packed rows that Y is the
 // first N columns of (0: N)
 size_t gemm_bf16_swiglu_workspace_bytes(int T, int N, int K);

@@ -115,7 +115,8 @@ __device__ __forceinline__ float lane_f(float v, int l) {
 }
 
 // FZ (FuseArgs, ffmi_internal.h): 1 = residual-add producer epilogue (EPI 0,
-// unsplit), 2 = RMSNorm consumer prologue.  Y is restrict-
+// unsplit), 2 = RMSNorm consumer prologue, 3 and 4 = the pair of an fp32 residual
+// (EPI 4; EPI 4 and 5).  Y is restrict-
 // qualified except in the producer, where it aliases fz.res_in (the residual
 // is updated in place).
 template <int FZ>
@@ -145,6 +146,22 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
       }
     }
   }
+  // FZ == 3: the residual and the norm weight of wave 0's epilogue
+  float xpre[FZ == 3 ? MT : 1][FZ == 3 ? NT : 1][4], wpre3[FZ == 3 ? NT : 1];
+  if constexpr (FZ == 3) {
+    if (wave == 0) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int n = min((int)(blockIdx.x * NT + j) * 16 + (lane & 15), N - 1);
+        wpre3[j] = fz.w32 ? fz.w32[n] : 0.f;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            xpre[i][j][r] = fz.x[(size_t)min(i * 16 + (lane >> 4) * 4 + r, T - 1) * N + n];
+      }
+    }
+  }
   // FZ == 2: rms of every row (the norm kernel's arithmetic on the
   // producer's per-tile sums of squares, summed in a fixed order), then the
   // rms of this lane's rows as an fp16 multiplier of its X fragments
@@ -156,8 +173,9 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   // so waiting for these does not wait for those): the two round trips
   // overlap instead of adding up.  Every wave calls rms_finish exactly once.
   constexpr int RPW = (MT * 16 + KW - 1) / KW;
-  __shared__ float sRms[FZ == 2 ? MT * 16 : 1];
-  float pv[FZ == 2 ? RPW : 1][4];
+  constexpr bool RMS = FZ == 2 || FZ == 4;
+  __shared__ float sRms[RMS ? MT * 16 : 1];
+  float pv[RMS ? RPW : 1][4];
   // The norm weight comes once per workgroup and lies in LDS (8 KiB: K <= 4096).  A load of
   // its fragment per k-step, 64 bytes for 64 lanes, takes the L1 as long as one of X.
   // 12288 x 4096 and gate / up of 11008 x 4096, 8 rows: so and X in rows 20.6 and 31.3 us;
@@ -170,6 +188,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
 #pragma unroll
     for (int c = 0; c < WPT; ++c)
       wpre[c] = *reinterpret_cast<const h8 *>(fz.wnorm + (size_t)min((int)threadIdx.x + c * KW * 64, K / 8 - 1) * 8);
+  }
+  if constexpr (RMS) {
 #pragma unroll
     for (int rr = 0; rr < RPW; ++rr) {
       const int m = min(wave + rr * KW, T - 1);
@@ -178,6 +198,18 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
         pv[rr][c] = fz.ss_in[(size_t)m * fz.nss + min(lane + 64 * c, fz.nss - 1)];
     }
   }
+  // a row's sum of squares: 16-lane DPP rows, then the four row sums in row order
+  auto square_sum = [&](int rr) {
+    float v = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (lane + 64 * c < fz.nss) v += pv[RMS ? rr : 0][c];
+    v += row_ror_f<1>(v);
+    v += row_ror_f<2>(v);
+    v += row_ror_f<4>(v);
+    v += row_ror_f<8>(v);
+    return ((lane_f(v, 0) + lane_f(v, 16)) + lane_f(v, 32)) + lane_f(v, 48);
+  };
   // rms_finish contains the workgroup's only __syncthreads before the
   // cross-wave reduction.  It is called at several points (after the first
   // batch of loads of the pipelined loop, the batched loop or the tail, and
@@ -198,16 +230,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
 #pragma unroll
       for (int rr = 0; rr < RPW; ++rr) {
         const int m = wave + rr * KW;
-        float v = 0.f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (lane + 64 * c < fz.nss) v += pv[rr][c];
-        // 16-lane DPP rows, then the four row sums in row order
-        v += row_ror_f<1>(v);
-        v += row_ror_f<2>(v);
-        v += row_ror_f<4>(v);
-        v += row_ror_f<8>(v);
-        v = ((lane_f(v, 0) + lane_f(v, 16)) + lane_f(v, 32)) + lane_f(v, 48);
+        const float v = square_sum(rr);
         if (lane == 0 && m < T) {
           const float rf = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(v, (float)K), fz.eps)));
           sRms[m] = __half2float(__float2half_rn(rf));
@@ -404,6 +427,15 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   }
 
   rms_finish();  // (a wave with an empty k-range still meets the barrier)
+  if constexpr (FZ == 4) {  // (read behind the reduction's barrier)
+    static_assert(KW > 1, "");
+#pragma unroll
+    for (int rr = 0; rr < RPW; ++rr) {
+      const int m = wave + rr * KW;
+      const float v = square_sum(rr);
+      if (lane == 0 && m < T) sRms[m] = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(v, (float)fz.width) + fz.eps));
+    }
+  }
   // Cross-wave K reduction in a fixed order (wave 0 + 1 + ... + KW-1).
   if (KW > 1) {
     constexpr int REGS = MT * NT * 4;
@@ -430,6 +462,43 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   }
 
   // Epilogue: C/D layout col = lane&15, row = (lane>>4)*4 + r.
+  if constexpr (FZ == 3) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int n = (tile0 + j) * 16 + (lane & 15);
+      const bool nok = tile0 + j < NTILES && n < N;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + i * 16 + (lane >> 4) * 4 + r;
+          const float x = xpre[i][j][r] + acc[i][j][r];
+          float sq = 0.f;
+          if (nok && m < T) {
+            fz.x[(size_t)m * N + n] = x;
+            if (fz.w32) fz.hb[act_packed_off(m, n, N)] = f2bf(x * wpre3[j]);
+            sq = x * x;
+          }
+          if (!fz.w32) continue;
+          sq += row_ror_f<1>(sq);
+          sq += row_ror_f<2>(sq);
+          sq += row_ror_f<4>(sq);
+          sq += row_ror_f<8>(sq);
+          if ((lane & 15) == 0 && m < T && tile0 + j < NTILES) fz.ss_out[(size_t)m * NTILES + tile0 + j] = sq;
+        }
+    }
+    return;
+  }
+  if constexpr (FZ == 4) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float f = sRms[min(m0 + i * 16 + (lane >> 4) * 4 + r, T - 1)];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j][r] *= f;
+      }
+  }
   if (S > 1 || epi_f32<EPI>) {  // unpaired EPI only (host-checked)
     const int NP = NTILES * 16;
 #pragma unroll
@@ -1643,6 +1712,30 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
     if (fuse->kind == 1) FFMI_FZ(2, 1);
     FFMI_FZ(2, 2);
 #undef FFMI_FZ
+  }
+  if constexpr (E == 4 || E == 5)
+  if (fuse && fuse->kind) {
+    const int ntiles = (N + 15) / 16, wp = wpitch ? wpitch : (paired ? 2 : 1) * ntiles;
+    const bool producer = fuse->kind == 3;
+    if (mtiles > 1 || !xp || (producer ? E != 4 || N % 32 || !fuse->x || (fuse->w32 && (!fuse->hb || !fuse->ss_out))
+                                       : fuse->kind != 4 || !fuse->ss_in || fuse->nss < 1 || fuse->nss > 256 ||
+                                             fuse->width < 1))
+      return hipErrorInvalidValue;
+    if constexpr (E == 5) {
+      return run<1, 2, 4, 8, E, 4>(X, Wp, Y, ws, T, N, K, KT, 2 * ntiles, 1, s, 1, yp, nt, wp, *fuse);
+    } else {
+      // (dispatch_nt's forms)
+      int S = producer ? 1 : skinny_split(T, N, K, paired, defer != nullptr);
+      if (S > 1 && ws_bytes < (size_t)S * T * ntiles * 16 * sizeof(float)) S = 1;
+      const bool eight = ntiles < 512 && (KT + S - 1) / S >= 64 && !nt;
+      hipError_t e;
+      if (producer && eight) e = run<1, 1, 8, 8, E, 3>(X, Wp, Y, ws, T, N, K, KT, ntiles, S, s, 1, 0, nt, wp, *fuse);
+      else if (producer) e = run<1, 1, 4, 8, E, 3>(X, Wp, Y, ws, T, N, K, KT, ntiles, S, s, 1, 0, nt, wp, *fuse);
+      else if (eight) e = run<1, 1, 8, 8, E, 4>(X, Wp, Y, ws, T, N, K, KT, ntiles, S, s, 1, 0, nt, wp, *fuse);
+      else e = run<1, 1, 4, 8, E, 4>(X, Wp, Y, ws, T, N, K, KT, ntiles, S, s, 1, 0, nt, wp, *fuse);
+      if (!producer && defer && e == hipSuccess) defer->p = ws, defer->S = S, defer->NP = ntiles * 16;
+      return e;
+    }
   }
   // (the tile kernel's copies to LDS are of 16 bytes)
   const bool aligned = (((uintptr_t)X | (uintptr_t)Wp) & 15) == 0;
