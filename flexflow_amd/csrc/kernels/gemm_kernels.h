@@ -836,9 +836,13 @@ static hipError_t dispatch_nt(const uint16_t *X, const uint16_t *Wp, uint16_t *Y
     return hipGetLastError();
   }
   // wide layers (lm_head): two tiles per workgroup once there are >= 2 row
-  // tiles (SSM lm_head at T = 24: 16.1 -> 12.3 us warm; at one row tile a
-  // single tile stays faster: LLaMA-7B lm_head T = 8 cold 47.8 vs 55.8 us)
-  if (MT >= 2 && ntiles >= 512)
+  // tiles (SSM lm_head at T = 24: 16.1 -> 12.3 us warm), or more than half of one
+  // and tiles for three rounds of pairs (cold, 9 to 16 rows alike: 32000 x 4096
+  // 48.8 -> 40.8 us, 24576 x 4096 34.3 -> 31.8, 50272 x 4096 71.0 -> 66.2, 128256 x
+  // 4096 179 -> 169; at 16 rows 20480 x 4096 30.6 -> 31.3, 12288 x 4096 19.5 ->
+  // 21.5).  Up to 8 rows a single tile is the faster for most widths (12288 to
+  // 128256 x 4096 lose 4-13 %, 32000 gains 8)
+  if (MT >= 2 ? ntiles >= 512 : T > 8 && ntiles >= 1536)
     return run<MT, 2, 4, U, E>(X, Wp, Y, ws, T, N, K, KT, ntiles, S, s, xp, yp, nt, wpitch);
   // 8-wave groups only where the accumulators fit 2 waves/SIMD (no spills)
   if (ntiles >= 512 || MT >= 8)
