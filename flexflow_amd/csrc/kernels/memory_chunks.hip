@@ -119,7 +119,8 @@ struct ChunkLds {
 };
 
 // A workgroup's first four waves per (chunk, head); wave b has the chunk's block of 16 tokens b.
-template <MemoryRule RULE, int KS>
+// FEW: in half the registers that rows of 256 columns take.
+template <MemoryRule RULE, int KS, bool FEW = false>
 __device__ __forceinline__ void memory_chunk(const char *__restrict__ blob, int off_spans, int num_spans,
                                              const Memory &a, const MemoryScratch &w, int limit, int at_chunk, int h,
                                              char *smem) {
@@ -148,9 +149,8 @@ __device__ __forceinline__ void memory_chunk(const char *__restrict__ blob, int 
   // asked for before anything is used
   constexpr int NI = (DK + 127) / 128;
   const f4 nil = {0.f, 0.f, 0.f, 0.f};
-  f4 lq[4][NI][2], lk[4][NI][2], lg[4][NI][2];
-  uint4 bq[4][NI], bk[4][NI];
-  f4 gn[4];  // normed: gates of a row
+  // a thread's four rows, R at a time, the loads of R together
+  constexpr int R = FEW ? 2 : 4;
   float beta = 0.f;
   constexpr int NV = C * VW / 8 / 256;  // 16-byte pieces of a slice of values per thread
   uint4 lv[NV];
@@ -163,112 +163,120 @@ __device__ __forceinline__ void memory_chunk(const char *__restrict__ blob, int 
         lv[i] = *reinterpret_cast<const uint4 *>(w.rows + (row0 + r) * cols + 2 * a.G * a.dg + h * a.vg + c);
     }
   };
-#pragma unroll
-  for (int i4 = 0; i4 < 4; ++i4) {
-    const int r = wave * 16 + i4 * 4 + g;
-    const size_t t = row0 + min(r, n - 1);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int c = min((l15 + 16 * i) * 8, a.dg - 8);
-      if constexpr (DELTA) {
-        bq[i4][i] = *reinterpret_cast<const uint4 *>(w.rows + t * cols + hq * a.dg + c);
-        bk[i4][i] = *reinterpret_cast<const uint4 *>(w.rows + t * cols + (a.G + hq) * a.dg + c);
-      } else {
-        load8(a.y.p + t * a.y.NP + a.col + hq * a.dg + c, lq[i4][i]);
-        load8(a.y.p + t * a.y.NP + a.col + (a.G + hq) * a.dg + c, lk[i4][i]);
-      }
-      if constexpr (RULE != kMemoryNormed) load8(a.z.p + t * a.z.NP + a.decay.zcol + h * a.dg + c, lg[i4][i]);
-    }
-    if constexpr (RULE == kMemoryNormed) {
-      const float *gt = w.gates + (t * a.H + h) * 3;
-      gn[i4] = f4{gt[0], gt[1], 0.f, 0.f};
-    }
-  }
-  if constexpr (DELTA) {
-    if (tid < n) beta = a.y.p[(row0 + tid) * a.y.NP + a.col_beta + h];
-    fetch_values(0);
-  }
   f4 lb[NI][2];
-  if constexpr (RULE != kMemoryNormed)
-#pragma unroll
-    for (int i = 0; i < NI; ++i) load8(a.dbias + (size_t)h * a.dg + min((l15 + 16 * i) * 8, a.dg - 8), lb[i]);
   const float rate = DELTA ? a.rate[h] : 0.f;
-  // (products split over K: the other slabs)
-  for (int s = 1; s < a.y.S; ++s) {
-    if constexpr (DELTA) {
-      if (tid < n) beta += a.y.p[s * slab + (row0 + tid) * a.y.NP + a.col_beta + h];
-    } else {
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
+  for (int i0 = 0; i0 < 4; i0 += R) {
+    f4 lq[R][NI][2], lk[R][NI][2], lg[R][NI][2];
+    uint4 bq[R][NI], bk[R][NI];
+    f4 gn[R];  // normed: gates of a row
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const size_t t = row0 + min(wave * 16 + i4 * 4 + g, n - 1);
-          const int c = min((l15 + 16 * i) * 8, a.dg - 8);
-          f4 v[2];
-          load8(a.y.p + s * slab + t * a.y.NP + a.col + hq * a.dg + c, v);
-          lq[i4][i][0] += v[0], lq[i4][i][1] += v[1];
-          load8(a.y.p + s * slab + t * a.y.NP + a.col + (a.G + hq) * a.dg + c, v);
-          lk[i4][i][0] += v[0], lk[i4][i][1] += v[1];
+    for (int j4 = 0; j4 < R; ++j4) {
+      const int r = wave * 16 + (i0 + j4) * 4 + g;
+      const size_t t = row0 + min(r, n - 1);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int c = min((l15 + 16 * i) * 8, a.dg - 8);
+        if constexpr (DELTA) {
+          bq[j4][i] = *reinterpret_cast<const uint4 *>(w.rows + t * cols + hq * a.dg + c);
+          bk[j4][i] = *reinterpret_cast<const uint4 *>(w.rows + t * cols + (a.G + hq) * a.dg + c);
+        } else {
+          load8(a.y.p + t * a.y.NP + a.col + hq * a.dg + c, lq[j4][i]);
+          load8(a.y.p + t * a.y.NP + a.col + (a.G + hq) * a.dg + c, lk[j4][i]);
         }
+        if constexpr (RULE != kMemoryNormed) load8(a.z.p + t * a.z.NP + a.decay.zcol + h * a.dg + c, lg[j4][i]);
+      }
+      if constexpr (RULE == kMemoryNormed) {
+        const float *gt = w.gates + (t * a.H + h) * 3;
+        gn[j4] = f4{gt[0], gt[1], 0.f, 0.f};
+      }
     }
-  }
-  if constexpr (RULE != kMemoryNormed)
-    for (int s = 1; s < a.z.S; ++s)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          f4 v[2];
-          load8(a.z.p + s * zslab + (row0 + min(wave * 16 + i4 * 4 + g, n - 1)) * a.z.NP + a.decay.zcol + h * a.dg +
-                    min((l15 + 16 * i) * 8, a.dg - 8), v);
-          lg[i4][i][0] += v[0], lg[i4][i][1] += v[1];
-        }
-  if constexpr (DELTA)
-    if (tid < C) sbeta[tid] = tid < n ? sigmoid_f(beta) : 0.f;
-#pragma unroll
-  for (int i4 = 0; i4 < 4; ++i4) {
-    const int r = wave * 16 + i4 * 4 + g;
-    const bool real = r < n;
-    f4 q[NI][2], k[NI][2];
-    float qq = 0.f, kk = 0.f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
+    if (i0 == 0) {
       if constexpr (DELTA) {
-        unpack8_bf16(bq[i4][i], q[i][0], q[i][1]);
-        unpack8_bf16(bk[i4][i], k[i][0], k[i][1]);
+        if (tid < n) beta = a.y.p[(row0 + tid) * a.y.NP + a.col_beta + h];
+        fetch_values(0);
+      }
+      if constexpr (RULE != kMemoryNormed)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) load8(a.dbias + (size_t)h * a.dg + min((l15 + 16 * i) * 8, a.dg - 8), lb[i]);
+    }
+    // (products split over K: the other slabs)
+    for (int s = 1; s < a.y.S; ++s) {
+      if constexpr (DELTA) {
+        if (i0 == 0 && tid < n) beta += a.y.p[s * slab + (row0 + tid) * a.y.NP + a.col_beta + h];
       } else {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) q[i][j] = lq[i4][i][j], k[i][j] = lk[i4][i][j];
-      }
-      if (!real || (l15 + 16 * i) * 8 >= a.dg) q[i][0] = q[i][1] = k[i][0] = k[i][1] = nil;
+        for (int j4 = 0; j4 < R; ++j4)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        qq = fmaf(q[i][e >> 2][e & 3], q[i][e >> 2][e & 3], qq);
-        kk = fmaf(k[i][e >> 2][e & 3], k[i][e >> 2][e & 3], kk);
+          for (int i = 0; i < NI; ++i) {
+            const size_t t = row0 + min(wave * 16 + (i0 + j4) * 4 + g, n - 1);
+            const int c = min((l15 + 16 * i) * 8, a.dg - 8);
+            f4 v[2];
+            load8(a.y.p + s * slab + t * a.y.NP + a.col + hq * a.dg + c, v);
+            lq[j4][i][0] += v[0], lq[j4][i][1] += v[1];
+            load8(a.y.p + s * slab + t * a.y.NP + a.col + (a.G + hq) * a.dg + c, v);
+            lk[j4][i][0] += v[0], lk[j4][i][1] += v[1];
+          }
       }
     }
-    float fq = a.q_scale, fk = 1.f;
-    if (a.unit) {
+    if constexpr (RULE != kMemoryNormed)
+      for (int s = 1; s < a.z.S; ++s)
 #pragma unroll
-      for (int o = 1; o < 16; o <<= 1) qq += __shfl_xor(qq, o), kk += __shfl_xor(kk, o);
-      fq *= __fdiv_rn(1.0f, sqrtf(qq + 1e-6f)), fk = __fdiv_rn(1.0f, sqrtf(kk + 1e-6f));
-    }
-    if constexpr (RULE == kMemoryNormed) fk = ex2(gn[i4][1]);
+        for (int j4 = 0; j4 < R; ++j4)
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int c = (l15 + 16 * i) * 8;
-      if (c >= DK) continue;
-      *reinterpret_cast<uint4 *>(&sQ[r * LDK + c]) = pack8_bf16(q[i][0] * fq, q[i][1] * fq);
-      *reinterpret_cast<uint4 *>(&sK[r * LDK + c]) = pack8_bf16(k[i][0] * fk, k[i][1] * fk);
-      f4 d[2];
+          for (int i = 0; i < NI; ++i) {
+            f4 v[2];
+            load8(a.z.p + s * zslab + (row0 + min(wave * 16 + (i0 + j4) * 4 + g, n - 1)) * a.z.NP + a.decay.zcol +
+                      h * a.dg + min((l15 + 16 * i) * 8, a.dg - 8), v);
+            lg[j4][i][0] += v[0], lg[j4][i][1] += v[1];
+          }
+    if constexpr (DELTA)
+      if (i0 == 0 && tid < C) sbeta[tid] = tid < n ? sigmoid_f(beta) : 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = 0.f;
-        if constexpr (RULE == kMemoryNormed) v = gn[i4][0];
-        else v = c + e < a.dim ? log2_decay<RULE>(a, rate, lg[i4][i][e >> 2][e & 3] + lb[i][e >> 2][e & 3]) : 0.f;
-        d[e >> 2][e & 3] = real ? v : 0.f;
+    for (int j4 = 0; j4 < R; ++j4) {
+      const int r = wave * 16 + (i0 + j4) * 4 + g;
+      const bool real = r < n;
+      f4 q[NI][2], k[NI][2];
+      float qq = 0.f, kk = 0.f;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if constexpr (DELTA) {
+          unpack8_bf16(bq[j4][i], q[i][0], q[i][1]);
+          unpack8_bf16(bk[j4][i], k[i][0], k[i][1]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) q[i][j] = lq[j4][i][j], k[i][j] = lk[j4][i][j];
+        }
+        if (!real || (l15 + 16 * i) * 8 >= a.dg) q[i][0] = q[i][1] = k[i][0] = k[i][1] = nil;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          qq = fmaf(q[i][e >> 2][e & 3], q[i][e >> 2][e & 3], qq);
+          kk = fmaf(k[i][e >> 2][e & 3], k[i][e >> 2][e & 3], kk);
+        }
       }
-      *reinterpret_cast<f4 *>(&sG[r * LDG + c]) = d[0], *reinterpret_cast<f4 *>(&sG[r * LDG + c + 4]) = d[1];
+      float fq = a.q_scale, fk = 1.f;
+      if (a.unit) {
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) qq += __shfl_xor(qq, o), kk += __shfl_xor(kk, o);
+        fq *= __fdiv_rn(1.0f, sqrtf(qq + 1e-6f)), fk = __fdiv_rn(1.0f, sqrtf(kk + 1e-6f));
+      }
+      if constexpr (RULE == kMemoryNormed) fk = ex2(gn[j4][1]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int c = (l15 + 16 * i) * 8;
+        if (c >= DK) continue;
+        *reinterpret_cast<uint4 *>(&sQ[r * LDK + c]) = pack8_bf16(q[i][0] * fq, q[i][1] * fq);
+        *reinterpret_cast<uint4 *>(&sK[r * LDK + c]) = pack8_bf16(k[i][0] * fk, k[i][1] * fk);
+        f4 d[2];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float v = 0.f;
+          if constexpr (RULE == kMemoryNormed) v = gn[j4][0];
+          else v = c + e < a.dim ? log2_decay<RULE>(a, rate, lg[j4][i][e >> 2][e & 3] + lb[i][e >> 2][e & 3]) : 0.f;
+          d[e >> 2][e & 3] = real ? v : 0.f;
+        }
+        *reinterpret_cast<f4 *>(&sG[r * LDG + c]) = d[0], *reinterpret_cast<f4 *>(&sG[r * LDG + c + 4]) = d[1];
+      }
     }
   }
   __syncthreads();
@@ -503,7 +511,7 @@ __global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void memory_chunk_kernel(cons
 // The same, and the short spans' tokens beside the chunks (launch_memory_steps' work): neither
 // fills the chip, each is a chain of 10-20 us, and they share nothing.  A prompt's portion of
 // 33 tokens beside 5 decoding requests, us: delta rule, 16 heads of 128, 16.6 + 21.2 -> 21.9; normed,
-// 4 of 128, 10.5 + 11.6 -> 12.9; gated, 4 of 256, 11.3 + 22.9 -> 26.3 (13 registers in scratch).
+// 4 of 128, 10.5 + 11.6 -> 12.9; gated, 4 of 256, 11.3 + 22.9 -> 25.3 (all of a thread's rows at once: 13 registers in scratch, 26.3).
 template <MemoryRule RULE, int KS, bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void memory_mixed_kernel(const char *__restrict__ blob, int off_spans, int num_spans,
                                                              int num_chunks, Memory a, MemoryScratch w, int limit,
@@ -512,8 +520,8 @@ __global__ __launch_bounds__(NT, 1) void memory_mixed_kernel(const char *__restr
   const int chunks = num_chunks * a.H, b = blockIdx.x;
   if (b < chunks) {
     if (threadIdx.x < 256)
-      memory_chunk<RULE, KS>(blob, off_spans, num_spans, a, w, limit, b % num_chunks, b / num_chunks,
-                             reinterpret_cast<char *>(lds));
+      memory_chunk<RULE, KS, (KS > 4)>(blob, off_spans, num_spans, a, w, limit, b % num_chunks, b / num_chunks,
+                                       reinterpret_cast<char *>(lds));
     return;
   }
   const int at = (b - chunks) / a.H;
@@ -796,7 +804,8 @@ hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_ch
 
 // One workgroup of either kind fits a CU: one round of them, as a second would cost more than the
 // launch saved.  The chunks of 256 state rows need more registers than two waves of a SIMD
-// have: 16 too many with the gated rule, over 100 with the delta rule.
+// have, with the delta rule over 100 more; the gated rule's ask for half of a thread's rows at a
+// time there.
 bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit) {
   const MemoryStepsPlan p = memory_steps_plan(a, num_spans, limit, true);
   return a.dg <= (a.rule == kMemoryGated ? 256 : 128) && p.rows <= 8 && p.bytes <= 64 * 1024 && (p.parts == 1 || a.rule != kMemoryDelta) &&
