@@ -511,7 +511,8 @@ __global__ __launch_bounds__(256, KS <= 4 ? 2 : 1) void memory_chunk_kernel(cons
 // The same, and the short spans' tokens beside the chunks (launch_memory_steps' work): neither
 // fills the chip, each is a chain of 10-20 us, and they share nothing.  A prompt's portion of
 // 33 tokens beside 5 decoding requests, us: delta rule, 16 heads of 128, 16.6 + 21.2 -> 21.9; normed,
-// 4 of 128, 10.5 + 11.6 -> 12.9; gated, 4 of 256, 11.3 + 22.9 -> 25.3 (all of a thread's rows at once: 13 registers in scratch, 26.3).
+// 4 of 128, 10.5 + 11.6 -> 12.9; gated, 4 of 256, 11.3 + 22.9 -> 25.3 (all of a thread's rows at
+// once: 13 registers in scratch, 26.3).
 template <MemoryRule RULE, int KS, bool SPLIT>
 __global__ __launch_bounds__(NT, 1) void memory_mixed_kernel(const char *__restrict__ blob, int off_spans, int num_spans,
                                                              int num_chunks, Memory a, MemoryScratch w, int limit,
