@@ -1,4 +1,4 @@
-"""Products of few rows and many columns: two column tiles a workgroup from 9 rows and 1536 tiles on.
+"""Products of few rows: two column tiles a workgroup from 9 rows and 1536 tiles on; three row tiles.
 A row's sums are the same bits however many rows there are."""
 import numpy as np
 import pytest
@@ -34,3 +34,21 @@ def test_rows(n, k, hint):
         assert (np.abs(got[t].astype(np.float64) - want[:t]) <= bound[:t]).all(), t
         if t <= 16:
             assert np.array_equal(got[t].view(np.uint16), got[16][:t].view(np.uint16)), t
+
+
+@pytest.mark.parametrize("n,k,epi,hint", [(6432, 2048, 0, F.W_STREAM), (2048, 4096, 0, 0), (2048, 1056, 0, 0),
+                                          (768, 3072, 0, 0), (8200, 1056, 0, 0), (2304, 768, 1, 0), (16400, 992, 0, 0)])
+def test_rows_of_three_tiles(n, k, epi, hint):
+    """33 to 48 rows have a form of their own; a row's sums are those of 64."""
+    L = K.L
+    rng = np.random.default_rng(n + k)
+    x, w = f16(rng.standard_normal((64, k))), [Buf(f16(rng.uniform(-0.05, 0.05, (n, k)))) for _ in range(1 + epi)]
+    xb, wp = Buf(x), Buf.empty(((1 + epi) * L.ffmi_linear_packed_bytes(n, k) // 2,), np.uint16)
+    F.check(L.ffmi_linear_pack_gate_up(w[0].ptr, w[1].ptr, n, k, wp.ptr, None) if epi else
+            L.ffmi_linear_pack_weight(w[0].ptr, n, k, wp.ptr, None))
+    got = {}
+    for t in (64, 32, 33, 40, 47, 48, 49):
+        y = Buf(np.full((t, n), np.nan, np.float16))
+        F.check(L.ffmi_linear(xb.ptr, wp.ptr, y.ptr, t, n, k, epi | hint, None))
+        got[t] = y.get().view(np.uint16)
+        assert np.array_equal(got[t], got[64][:t]), t
