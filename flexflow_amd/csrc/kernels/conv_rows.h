@@ -22,6 +22,11 @@ struct ConvRows {
   float *hf = nullptr;
   int off_tokens = 0;
   int above = 0;  // only tokens of portions of more than so many tokens
+  // besides (null: nothing): columns [pack_col, pack_col + pack_n) of u in packed bf16 rows, as
+  // launch_pack_sums makes them, on workgroups behind the convolution's (at 38 tokens either is
+  // 15 to 120 workgroups; one launch for two takes 3 us less)
+  uint16_t *pack = nullptr;
+  int pack_col = 0, pack_n = 0;
 };
 hipError_t launch_conv_rows(const char *blob, const ConvRows &a, hipStream_t s);
 

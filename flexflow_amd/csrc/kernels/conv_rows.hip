@@ -10,8 +10,13 @@ namespace ffmi {
 // portion reads its carried rows first: a chain, so that a step of few columns has fewer
 // tokens a thread (launch_conv_rows).
 template <int TB, int PAST, bool F32>
-__global__ __launch_bounds__(256) void conv_rows_kernel(const char *__restrict__ blob, ConvRows a) {
+__global__ __launch_bounds__(256) void conv_rows_kernel(const char *__restrict__ blob, ConvRows a, int blocks) {
   constexpr int H = PAST > 0 ? PAST : 1;
+  if ((int)blockIdx.y >= blocks) {  // (packing: workgroups behind the convolution's)
+    pack_sums_piece(a.u, a.pack_col, a.pack, a.T, a.pack_n,
+                    ((blockIdx.y - blocks) * (long)gridDim.x + blockIdx.x) * 256 + threadIdx.x);
+    return;
+  }
   const int c = (blockIdx.x * 256 + threadIdx.x) * 8, t0 = blockIdx.y * TB;
   if (c >= a.cols) return;
   const PagedToken *tok = reinterpret_cast<const PagedToken *>(blob + a.off_tokens);
@@ -101,7 +106,8 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const char *__restrict__
 hipError_t launch_conv_rows(const char *blob, const ConvRows &a, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;
   if (a.cols <= 0 || a.cols % 8 || a.col % 4 || a.u.NP % 4 || a.u.S < 1 || a.col + a.cols > a.u.NP || a.taps < 1 ||
-      !a.conv || (a.taps > 1 && !a.carry) || (a.hb != nullptr) == (a.hf != nullptr))
+      !a.conv || (a.taps > 1 && !a.carry) || (a.hb != nullptr) == (a.hf != nullptr) ||
+      (a.pack && (a.pack_n <= 0 || a.pack_n % 32 || a.pack_col % 4 || a.pack_col + a.pack_n > a.u.NP)))
     return hipErrorInvalidValue;
   // Four taps, a portion and 7 single tokens, us with 1, 2, 4 and 8 tokens a thread:
   //   38 x 6144    3.3   4.1   6.5   7.9      200 x 3072   3.9   4.2   6.5   9.3
@@ -109,11 +115,15 @@ hipError_t launch_conv_rows(const char *blob, const ConvRows &a, hipStream_t s) 
   //   1600 x 6144 25.5  19.1  18.3  20.5  (a portion alone: 24.8  17.8  15.6  16.6)
   const long size = (long)a.T * a.cols;
   const int tb = size <= 640 << 10 ? 1 : size <= 5 << 20 ? 2 : 4;
-  const dim3 grid((a.cols + 2047) / 2048, (a.T + tb - 1) / tb);
+  const int blocks = (a.T + tb - 1) / tb, wide = (a.cols + 2047) / 2048;
+  const long pieces = a.pack ? (long)a.T * (a.pack_n / 8) : 0, row = 256L * wide;
+  const dim3 grid(wide, blocks + (unsigned)((pieces + row - 1) / row));
 #define FFMI_CT(TB, PAST)                                                                             \
   do {                                                                                                \
-    if (a.hf) hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, true>), grid, dim3(256), 0, s, blob, a); \
-    else hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, false>), grid, dim3(256), 0, s, blob, a);     \
+    if (a.hf) hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, true>), grid, dim3(256), 0, s, blob, a, \
+                                 blocks);                                                             \
+    else hipLaunchKernelGGL((conv_rows_kernel<TB, PAST, false>), grid, dim3(256), 0, s, blob, a,    \
+                            blocks);                                                                  \
   } while (0)
 #define FFMI_CR(PAST)                   \
   do {                                  \

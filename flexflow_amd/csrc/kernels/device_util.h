@@ -43,6 +43,21 @@ __device__ __forceinline__ float sum_at(const Partials &y, size_t slab, size_t a
   return v;
 }
 
+// packed bf16 rows of the columns [col, col + n) of deferred sums: the id-th piece of 8
+__device__ __forceinline__ void pack_sums_piece(const Partials &y, int col, uint16_t *__restrict__ out, int T, int n,
+                                                long id) {
+  const int n8 = n >> 3;
+  if (id >= (long)T * n8) return;
+  const int t = (int)(id / n8), c = (int)(id % n8) * 8;
+  const float *p = y.p + (size_t)t * y.NP + col + c;
+  f4 lo = *reinterpret_cast<const f4 *>(p), hi = *reinterpret_cast<const f4 *>(p + 4);
+  for (int s = 1; s < y.S; ++s) {
+    const float *ps = p + (size_t)s * T * y.NP;
+    lo += *reinterpret_cast<const f4 *>(ps), hi += *reinterpret_cast<const f4 *>(ps + 4);
+  }
+  *reinterpret_cast<uint4 *>(out + act_packed_off(t, c, n)) = pack8_bf16(lo, hi);
+}
+
 template <int NT>
 __device__ __forceinline__ float row_sum(float v, float *sh) {
 #pragma unroll

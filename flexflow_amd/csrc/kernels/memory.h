@@ -95,7 +95,12 @@ inline size_t memory_chunks_max(int T, int spans) { return (size_t)T / kMemoryCh
 // left in w.o (*left) and launch_memory_out has to follow.
 hipError_t launch_memory_steps(const char *blob, int off_spans, int num_spans, const Memory &a,
                                const MemoryScratch *w, bool f32, int limit, bool *left, hipStream_t s);
-// Chunks (bf16 model): spans of more than `limit` >= kShortSpan tokens; num_chunks: the
+// Before the chunks: the delta rule's convolved rows (w.rows) of spans of more than `limit`
+// tokens and, any rule, the narrow products' input (low: packed bf16 rows of the n columns
+// from a.decay.col on; n == 0: none), one launch.
+hipError_t launch_memory_rows(const char *blob, const Memory &a, const MemoryScratch &w, int limit, uint16_t *low,
+                              int n, hipStream_t s);
+// Chunks (bf16 model), behind launch_memory_rows: spans of more than `limit` >= kShortSpan tokens; num_chunks: the
 // step's (PagedSpan::chunk0 counts them).  The outputs are left in w.o.  left: the other spans
 // too, as launch_memory_steps would, in the same launch; where memory_mixes says so.
 bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit);

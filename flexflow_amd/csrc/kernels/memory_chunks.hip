@@ -18,6 +18,7 @@
 #include <algorithm>
 
 #include "conv_rows.h"
+#include "residual.h"
 #include "memory_steps.h"
 
 namespace ffmi {
@@ -758,12 +759,6 @@ hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_ch
                       const MemoryScratch &w, int limit, const MemoryStepsPlan *steps, hipStream_t s) {
   if (RULE == kMemoryNormed)
     hipLaunchKernelGGL(memory_gates_kernel, dim3(a.H, num_spans), dim3(256), 0, s, blob, off_spans, a, w, limit);
-  if (RULE == kMemoryDelta) {
-    ConvRows c;
-    c.u = a.y, c.T = a.T, c.col = a.col, c.cols = 2 * a.G * a.dg + a.H * a.vg, c.taps = a.taps, c.conv = a.conv;
-    c.carry = a.carry, c.silu = a.silu, c.hb = w.rows, c.off_tokens = a.off_tokens, c.above = limit;
-    if (const hipError_t e = launch_conv_rows(blob, c, s)) return e;
-  }
   // narrow workgroups where the spans and heads alone do not fill the chip
   const bool wide = (long)a.H * num_spans * (a.vs / 16) > 512;
 #define FFMI_MS(KS, VS)                                                                                             \
@@ -813,6 +808,16 @@ bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit) {
          (long)a.H * (num_chunks + (long)num_spans * p.parts) <= 256;
 }
 
+hipError_t launch_memory_rows(const char *blob, const Memory &a, const MemoryScratch &w, int limit, uint16_t *low,
+                              int n, hipStream_t s) {
+  if (n > 0 && !low) return hipErrorInvalidValue;
+  if (a.rule != kMemoryDelta) return n > 0 ? launch_pack_sums(a.y, a.decay.col, low, a.T, n, s) : hipSuccess;
+  ConvRows c;
+  c.u = a.y, c.T = a.T, c.col = a.col, c.cols = 2 * a.G * a.dg + a.H * a.vg, c.taps = a.taps, c.conv = a.conv;
+  c.carry = a.carry, c.silu = a.silu, c.hb = w.rows, c.off_tokens = a.off_tokens, c.above = limit;
+  if (n > 0) c.pack = low, c.pack_col = a.decay.col, c.pack_n = n;
+  return launch_conv_rows(blob, c, s);
+}
 hipError_t launch_memory_chunks(const char *blob, int off_spans, int num_spans, int num_chunks, const Memory &a,
                                 const MemoryScratch &w, int limit, bool *left, hipStream_t s) {
   if (num_spans <= 0 || num_chunks <= 0) return hipSuccess;

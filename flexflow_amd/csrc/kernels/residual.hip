@@ -374,17 +374,7 @@ hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream
 
 __global__ __launch_bounds__(256) void pack_sums_kernel(Partials y, int col, uint16_t *__restrict__ out, int T,
                                                         int n) {
-  const int n8 = n >> 3;
-  const long id = blockIdx.x * 256L + threadIdx.x;
-  if (id >= (long)T * n8) return;
-  const int t = (int)(id / n8), c = (int)(id % n8) * 8;
-  const float *p = y.p + (size_t)t * y.NP + col + c;
-  f4 lo = *reinterpret_cast<const f4 *>(p), hi = *reinterpret_cast<const f4 *>(p + 4);
-  for (int s = 1; s < y.S; ++s) {
-    const float *ps = p + (size_t)s * T * y.NP;
-    lo += *reinterpret_cast<const f4 *>(ps), hi += *reinterpret_cast<const f4 *>(ps + 4);
-  }
-  *reinterpret_cast<uint4 *>(out + act_packed_off(t, c, n)) = pack8_bf16(lo, hi);
+  pack_sums_piece(y, col, out, T, n, blockIdx.x * 256L + threadIdx.x);
 }
 hipError_t launch_pack_sums(const Partials &y, int col, uint16_t *out, int T, int n, hipStream_t s) {
   if (T <= 0) return hipSuccess;

@@ -474,8 +474,8 @@ struct Pekarax : public PagedDecoder {
     const bool chunks = chunk_form(a);
     const int limit = chunks ? std::max(kShortSpan, a.taps) : BatchConfig::MAX_NUM_TOKENS;
     const bool longs = chunks && step.long_spans, shorts = !chunks || step.short_spans || limit > kShortSpan;
+    if (longs) FFMI_HIP(launch_memory_rows(step.dev, a, scratch, limit, low, L.low, stream));
     if (longs && L.low) {
-      FFMI_HIP(launch_pack_sums(y, a.decay.col, low, step.T, L.low, stream));
       FFMI_TRY(gemm_sum_to(low, L.wlow, L.nz, L.low, &a.z, zs, zs_bytes));
     }
     bool left = false;
