@@ -24,8 +24,17 @@ struct MoeSizes {
   int identity = 0;  // further outputs of the router, after the experts': the row itself
   bool shared = false;
   int gate_col = 0;  // column of the shared expert's gate in the router's product
+  // Few: a workgroup per 16 rows and 32 columns, which reads an expert's weights again for
+  // every 16 rows; many: once, on a grid that must not be small.  Both products, us, rows an
+  // expert 5, 10, 14, 20 on average, many and few:
+  //    32 experts, 4 taken, 1408 x 2048    52.7 49.5   52.8 51.3   53.4 58.4   54.2 86.0
+  //    32, 4, 2752 x 4096                   200  172    202  182    204  207    206  319
+  //    64, 8, 1024 x 2048                  81.1 69.2   81.1 73.5   81.8 84.0   83.4  112
+  //   128, 8, 1024 x 2048                   150  133    152  143    153  168    156  220
+  // A shared expert has every token's row: few read it T / 16 times (replay of 32 experts, 4
+  // taken, and one of half the units, steps of 82 tokens: 18.3 ms, 19.0).
   int tile_rows() const {
-    return T > 32 && (long)T * top >= 4L * experts ? kMoeMany : kMoeFew;
+    return T > 32 && (long)T * top >= (shared ? 4L : 12L) * experts ? kMoeMany : kMoeFew;
   }
   // upper bounds: slots of the experts (whole 16s), tiles
   __host__ __device__ int slots() const {

@@ -39,3 +39,13 @@ def test_router_beside_the_norm(tmp_path, n, identity, width, T):
     toks = tokens_p(cfg, T, 6)
     eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=320, positions=320)
     close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
+
+
+@pytest.mark.parametrize("n,top,T", [(8, 2, 33), (8, 2, 47), (8, 2, 48), (16, 4, 47), (16, 4, 48), (64, 1, 200)])
+def test_few_and_many_rows_an_expert(tmp_path, n, top, T):
+    """Products of 16 rows a workgroup up to 12 rows an expert on average, from there on of 256."""
+    cfg = PM.model_config(90, 96, [PM.experts(PM.gla(1, 16, 16), n, top, 200, identity=0, groups=(1, 1))])
+    w = PM.random_weights(cfg, 11)
+    toks = tokens_p(cfg, T, 8)
+    eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=256, positions=256)
+    close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
