@@ -24,18 +24,21 @@ struct MoeSizes {
   int identity = 0;  // further outputs of the router, after the experts': the row itself
   bool shared = false;
   int gate_col = 0;  // column of the shared expert's gate in the router's product
-  // Few: a workgroup per 16 rows and 32 columns, which reads an expert's weights again for
-  // every 16 rows; many: once, on a grid that must not be small.  Both products, us, rows an
-  // expert 5, 10, 14, 20 on average, many and few:
-  //    32 experts, 4 taken, 1408 x 2048    52.7 49.5   52.8 51.3   53.4 58.4   54.2 86.0
-  //    32, 4, 2752 x 4096                   200  172    202  182    204  207    206  319
-  //    64, 8, 1024 x 2048                  81.1 69.2   81.1 73.5   81.8 84.0   83.4  112
-  //   128, 8, 1024 x 2048                   150  133    152  143    153  168    156  220
+  // Few: 16 rows a tile, for which an expert's weights are read again every 16 rows; many:
+  // once, on a grid that must not be small.  Both products, us, 5 and 10 rows an expert on
+  // average, many and few (whole_k):
+  //    32 experts, 4 taken, 1408 x 2048    52.7 49.7   52.8 51.0
+  //    32, 4, 2752 x 4096                   200  162    202  167
+  //    64, 8, 1024 x 2048                  81.1 69.2   81.1 76.4
+  //   128, 8, 1024 x 2048                   150  131    152  137
+  // and from 14 rows on, where many experts have over 16, few are the slower.
   // A shared expert has every token's row: few read it T / 16 times (replay of 32 experts, 4
   // taken, and one of half the units, steps of 82 tokens: 18.3 ms, 19.0).
   int tile_rows() const {
     return T > 32 && (long)T * top >= (shared ? 4L : 12L) * experts ? kMoeMany : kMoeFew;
   }
+  // few rows' products in the order of the many's sums
+  bool whole_k() const { return T > 32 && (long)T * top >= 4L * experts; }
   // upper bounds: slots of the experts (whole 16s), tiles
   __host__ __device__ int slots() const {
     const int a = T * top, e = a < experts ? a : experts;

@@ -268,6 +268,76 @@ __global__ __launch_bounds__(256) void moe_few_kernel(MoeGemm a, int first, size
   }
 }
 
+// The same of whole K: a wave has two tiles of its own, its sums in the tile kernel's order (a
+// row's bits do not change where this form takes its place).  Two register sets: the next U
+// k-steps are on their way while these are multiplied.
+template <bool GATED, bool NTL>
+__global__ __launch_bounds__(256) void moe_chain_kernel(MoeGemm a, int first, size_t wts) {
+  constexpr int U = 8;
+  if (first + (int)blockIdx.y >= *a.num_tiles) return;
+  const MoeTile tl = a.tiles[first + blockIdx.y];
+  const bool shared = tl.expert >= a.experts;
+  const MoeGroup &g = a.g[shared];
+  const int lane = threadIdx.x & 63, m = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int KT = g.K >> 5, ntiles = (GATED ? 2 : 1) * (g.N >> 4), pair = blockIdx.x * 4 + wave, tile0 = pair * 2;
+  if (tile0 >= ntiles) return;
+  const size_t wks = wts == 512 ? (size_t)ntiles * 512 : 512, ts = wts == 512 ? 512 : (size_t)KT * 512;
+  const uint16_t *W = (const uint16_t *)g.W + (shared ? 0 : tl.expert * g.w_stride) + lane * 8;
+  const uint16_t *w0 = W + tile0 * ts, *w1 = W + min(tile0 + 1, ntiles - 1) * ts;
+  const uint16_t *x;
+  if constexpr (GATED) {
+    const int slot = tl.slot0 + min(m, tl.rows - 1);
+    x = (const uint16_t *)g.X + (size_t)(shared ? slot : a.slot_token[slot]) * g.K + 8 * (lane >> 4);
+  } else {
+    x = (const uint16_t *)g.X + ((size_t)(tl.slot0 >> 4) * KT * 64 + packed_lane(lane, tl.rows)) * 8;
+  }
+  constexpr int XS = GATED ? 32 : 512;
+  f4 acc[2];
+  acc[0] = acc[1] = f4{0.f, 0.f, 0.f, 0.f};
+  h8 wa[U][2], xa[U], wb[U][2], xb[U];
+  auto load = [&](h8(&b)[U][2], h8(&xv)[U], int k) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t kk = min(k + u, KT - 1);
+      b[u][0] = ld_weight<NTL>(w0 + kk * wks), b[u][1] = ld_weight<NTL>(w1 + kk * wks);
+      xv[u] = *reinterpret_cast<const h8 *>(x + kk * XS);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mul = [&](const h8(&b)[U][2], const h8(&xv)[U], int n) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u >= n) break;
+      acc[0] = moe_mma(b[u][0], xv[u], acc[0]);
+      acc[1] = moe_mma(b[u][1], xv[u], acc[1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int k = 0;
+  load(wa, xa, 0);
+  for (; k + 2 * U < KT; k += 2 * U) {
+    load(wb, xb, k + U);
+    mul(wa, xa, U);
+    load(wa, xa, k + 2 * U);
+    mul(wb, xb, U);
+  }
+  if (k + U < KT) {
+    load(wb, xb, k + U);
+    mul(wa, xa, U);
+    mul(wb, xb, KT - k - U);
+  } else {
+    mul(wa, xa, KT - k);
+  }
+  if (m >= tl.rows) return;
+  const int row = tl.slot0 + m, n = (lane >> 4) * 4;
+  if constexpr (GATED) {
+    moe_store<true>(g, row, pair * 16 + n, shared ? a.gate[row] : 1.0f, a.limit, acc[0], acc[1]);
+  } else {
+    moe_store<false>(g, row, tile0 * 16 + n, 1.0f, 0.f, acc[0], acc[0]);
+    if (tile0 + 1 < ntiles) moe_store<false>(g, row, tile0 * 16 + 16 + n, 1.0f, 0.f, acc[1], acc[1]);
+  }
+}
+
 // Up to 256 rows x 16 tiles a workgroup: eight waves as 2 (every other 16 rows) x 4
 // (weight tiles); both operands' fragments go to LDS as they are stored (row-major
 // rows: a lane fetches its own row's 16 bytes), NB - 1 k-steps in flight across raw
@@ -470,8 +540,13 @@ hipError_t launch_moe_gemm(const MoeGemm &a, const MoeSizes &n, bool gated, bool
       hipLaunchKernelGGL(moe_tile_kernel<false>, grid, dim3(512), 0, s, a, first, st, cols_shared, cols, wts);
     return hipGetLastError();
   }
-  const dim3 grid((per * N / 16 + 1) / 2, st + tiles);
-#define FFMI_MF(G, NL) hipLaunchKernelGGL((moe_few_kernel<G, NL>), grid, dim3(256), 0, s, a, first, wts)
+  const int pairs = (per * N / 16 + 1) / 2;
+  const dim3 grid(pairs, st + tiles), quads((pairs + 3) / 4, st + tiles);
+#define FFMI_MF(G, NL)                                                                              \
+  do {                                                                                              \
+    if (n.whole_k()) hipLaunchKernelGGL((moe_chain_kernel<G, NL>), quads, dim3(256), 0, s, a, first, wts); \
+    else hipLaunchKernelGGL((moe_few_kernel<G, NL>), grid, dim3(256), 0, s, a, first, wts);         \
+  } while (0)
   if (gated && stream_weights) FFMI_MF(true, true);
   else if (gated) FFMI_MF(true, false);
   else if (stream_weights) FFMI_MF(false, true);

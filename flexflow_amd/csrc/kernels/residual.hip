@@ -315,13 +315,15 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores rou
 // Every row's workgroup reads the whole router (from the L2, 64 bytes a clock), which must
 // cost less than the launches saved: one, and with more than 16 tokens that of the picks.
 // A graph's time of norm, router, picks and lists, us, apart and so:
-//   12 x 2048   1 token 8.9  7.6   16 tokens 10.9  8.2    38 12.0  8.2   160 13.6  9.2
-//   36 x 2048           8.8  8.8             10.8  9.4       11.9  9.4       13.8 10.6
-//   64 x 2048           8.8  9.5             10.8 10.1       11.9 10.2       13.7 11.2
-//   64 x 4096           9.5 11.9             11.8 12.5       13.2 12.9       16.4 14.6
+//   12 x 2048   1 token 8.9  7.6   16 tokens 10.9  8.2    38 12.0  8.2
+//   36 x 2048           8.8  8.8             10.8  9.4       11.9  9.4
+//   64 x 2048           8.8  9.5             10.8 10.1       11.9 10.2
+//   64 x 4096           9.5 11.9             11.8 12.5       13.2 12.9
+// Above 64 tokens the router's product is another kernel with other sums, which close calls
+// of the experts would show.
 bool route_with_row(const MoeSizes &n, int H) {
   const int cols = n.shared ? n.gate_col + 1 : n.experts + n.identity, tiles = (cols + 15) / 16;
-  return n.T <= 256 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144);
+  return n.T <= 64 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144);
 }
 hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;

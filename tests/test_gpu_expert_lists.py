@@ -30,9 +30,9 @@ def test_lists(tmp_path, n, top, T):
 
 @pytest.mark.parametrize("n,identity,width,T", [
     (12, 4, 96, 1), (12, 5, 100, 16), (30, 4, 352, 17), (47, 2, 1500, 16), (60, 4, 1536, 16), (60, 4, 1568, 16),
-    (60, 4, 1568, 17), (61, 4, 96, 9), (33, 2, 4096, 256), (33, 2, 4096, 257), (33, 2, 4128, 20)])
+    (60, 4, 1568, 17), (61, 4, 96, 9), (33, 2, 4096, 64), (33, 2, 4096, 65), (33, 2, 4128, 20)])
 def test_router_beside_the_norm(tmp_path, n, identity, width, T):
-    """Up to 64 columns, 256 tokens and 4096 channels, with up to 16 tokens 6144 channels of 16
+    """Up to 64 columns, 64 tokens and 4096 channels, with up to 16 tokens 6144 channels of 16
     columns; what lies past each."""
     cfg = PM.model_config(60, width, [PM.experts(PM.gla(1, 16, 16), n, 3, 32, identity=identity, groups=(1, 1))])
     w = PM.random_weights(cfg, 9)
