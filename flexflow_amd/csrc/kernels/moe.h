@@ -81,6 +81,7 @@ struct RouterWeights {
   const uint16_t *w = nullptr;  // bf16 packed, `steps` k-steps of 32 columns
   size_t tile = 0, step = 0;    // elements from tile to tile, k-step to k-step
   int steps = 0;
+  int slices = 1;  // of K in the product of few rows (gemm_few_rows_slices), at most 8
 };
 struct RouteScores {
   RouterWeights w;
@@ -88,7 +89,7 @@ struct RouteScores {
   MoeScores scores;
   MoeLists lists;
 };
-bool route_with_row(const MoeSizes &n, int H);  // (the rule) rows of H columns
+bool route_with_row(const MoeSizes &n, int H, int slices);  // (the rule) rows of H columns
 hipError_t launch_moe_lists(const MoeSizes &n, const MoeLists &l, hipStream_t s);
 
 // One product of every slot with its expert's matrix.

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores rou
   constexpr int NW = NT / 64, RTS = RT ? RT : 1;
   __shared__ __attribute__((aligned(16))) uint16_t own_row[RT ? NT * 8 : 8];
   __shared__ __attribute__((aligned(16))) float sums[NW * 16 * RTS];
-  RouterRow<RTS, NW> router;
+  RouterRow<RTS> router;
   const int row = blockIdx.x, H = a.H, nchunk = H >> 3;
   f4 x[MAXC][2], wv[MAXC][2];
   float ss = 0.f;
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores rou
     router.product(route.w, own_row, sums);
     __syncthreads();
     if (threadIdx.x >= 64) return;
-    const int e = pick_experts<1>(RouterTotal<RT, NW>{sums}, route.scores, route.n, row, route.lists);
+    const int e = pick_experts<1>(RouterTotal<RT>{sums, route.w.slices}, route.scores, route.n, row, route.lists);
     if ((int)threadIdx.x < route.n.top) route.lists.picked[(size_t)row * route.n.top + threadIdx.x] = e;
   }
 }
@@ -320,10 +320,12 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores rou
 //   64 x 2048           8.8  9.5             10.8 10.1       11.9 10.2
 //   64 x 4096           9.5 11.9             11.8 12.5       13.2 12.9
 // Above 64 tokens the router's product is another kernel with other sums, which close calls
-// of the experts would show.
-bool route_with_row(const MoeSizes &n, int H) {
+// of the experts would show.  (A slice of 64 k-steps and more would be cut in 8: only where
+// FFMI_SKINNY_SPLIT=0 leaves K whole.)
+bool route_with_row(const MoeSizes &n, int H, int slices) {
   const int cols = n.shared ? n.gate_col + 1 : n.experts + n.identity, tiles = (cols + 15) / 16;
-  return n.T <= 64 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144);
+  return n.T <= 64 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144) && slices >= 1 && slices <= 8 &&
+         (H / 32 + slices - 1) / slices < 64;
 }
 hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;
@@ -335,7 +337,7 @@ hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream
     const MoeSizes &n = route->n;
     const MoeScores &sc = route->scores;
     const int cols = n.experts + n.identity;
-    if (!route_with_row(n, a.H) || n.T != a.T || n.shared || a.rows || route->w.steps * 32 != a.H || !route->w.w ||
+    if (!route_with_row(n, a.H, route->w.slices) || n.T != a.T || n.shared || a.rows || route->w.steps * 32 != a.H || !route->w.w ||
         n.experts < 1 || n.identity < 0 || n.top < 1 || sc.groups < 1 || cols % sc.groups || sc.keep < 1 ||
         sc.keep > sc.groups || n.top > cols / sc.groups * sc.keep || !sc.correction ||
         (n.identity && !route->lists.own))

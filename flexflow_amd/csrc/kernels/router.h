@@ -119,63 +119,75 @@ __device__ __forceinline__ int pick_experts(const Z &z, const MoeScores &sc, con
 }
 
 // The router's product for one row, in the kernel that makes the row: the row in bf16 in
-// LDS, the weights' 16 RT columns split over NW waves by their k-steps.  A wave's first U
-// k-steps are fetched (begin) while the row is still being summed and normed.
-// Sums: of up to U / 4 k-steps, those of a wave, those of the waves, in order.
-template <int RT, int NW>
+// LDS, the weights' 16 RT columns.  The sums are those of the product of few rows
+// (gemm_skinny_kernel), bit for bit, so that a token's experts do not depend on how many
+// tokens share its step: K in `slices`, each in kParts parts of consecutive k-steps, a part
+// a chain of products; then the parts of a slice, then the slices, in order.  Wave w has
+// slice w.  Its first kAhead k-steps of every part are fetched (begin) while the row is
+// still being summed and normed (more than that: channels that 1024 does not divide).
+template <int RT>
 struct RouterRow {
-  static constexpr int U = 8;
-  h8 w[U][RT];
-  f4 acc[4][RT];
-  int kb, ke;
-  __device__ __forceinline__ void load(const RouterWeights &r, int k) {
+  static constexpr int kParts = 4, kAhead = 2;
+  h8 w[kParts][kAhead][RT];
+  int kb, ke, per;
+  // k-step j of part i, or none
+  __device__ __forceinline__ bool has(int i, int j) const { return j < per && kb + i * per + j < ke; }
+  __device__ __forceinline__ void load(const RouterWeights &r, int j0) {
     const uint16_t *p = r.w + (threadIdx.x & 63) * 8;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (k + u >= ke) break;
+    for (int i = 0; i < kParts; ++i)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) w[u][j] = *reinterpret_cast<const h8 *>(p + j * r.tile + (k + u) * r.step);
-    }
+      for (int j = 0; j < kAhead; ++j) {
+        if (!has(i, j0 + j)) continue;
+#pragma unroll
+        for (int c = 0; c < RT; ++c)
+          w[i][j][c] = *reinterpret_cast<const h8 *>(p + c * r.tile + (kb + i * per + j0 + j) * r.step);
+      }
   }
   __device__ __forceinline__ void begin(const RouterWeights &r) {
-    const int per = (r.steps + NW - 1) / NW;
-    kb = min(r.steps, (int)(threadIdx.x >> 6) * per), ke = min(r.steps, kb + per);
-    load(r, kb);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), mine = (r.steps + r.slices - 1) / r.slices;
+    kb = wave < r.slices ? min(r.steps, wave * mine) : r.steps, ke = min(r.steps, kb + mine);
+    per = (ke - kb + kParts - 1) / kParts;
+    load(r, 0);
   }
-  // row: the K values; sums [NW][16 RT] (barriers before and after are the caller's)
+  // row: the K values; sums [slices][16 RT] (barriers before and after are the caller's)
   __device__ __forceinline__ void product(const RouterWeights &r, const uint16_t *row, float *sums) {
     const int lane = threadIdx.x & 63;
+    f4 acc[kParts][RT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kParts; ++i)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-    for (int k = kb; k < ke; k += U) {
-      if (k > kb) load(r, k);
+      for (int c = 0; c < RT; ++c) acc[i][c] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < per; j0 += kAhead) {
+      if (j0 > 0) load(r, j0);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (k + u >= ke) break;
-        const h8 x = *reinterpret_cast<const h8 *>(row + (k + u) * 32 + 8 * (lane >> 4));  // every column of 16 the same
+      for (int j = 0; j < kAhead; ++j)
 #pragma unroll
-        for (int j = 0; j < RT; ++j)
-          acc[u / (U / 4)][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf8, w[u][j]), __builtin_bit_cast(bf8, x), acc[u / (U / 4)][j], 0, 0, 0);
-      }
+        for (int i = 0; i < kParts; ++i) {
+          if (!has(i, j0 + j)) continue;
+          // (every column of 16 the same)
+          const h8 x = *reinterpret_cast<const h8 *>(row + (kb + i * per + j0 + j) * 32 + 8 * (lane >> 4));
+#pragma unroll
+          for (int c = 0; c < RT; ++c)
+            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf8, w[i][j][c]), __builtin_bit_cast(bf8, x), acc[i][c], 0, 0, 0);
+        }
     }
-    if (lane & 15) return;
+    const int wave = threadIdx.x >> 6;
+    if ((lane & 15) || wave >= r.slices) return;
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const f4 v = ((acc[0][j] + acc[1][j]) + acc[2][j]) + acc[3][j];
-      *reinterpret_cast<f4 *>(sums + (threadIdx.x >> 6) * 16 * RT + j * 16 + (lane >> 4) * 4) = v;
-    }
+    for (int c = 0; c < RT; ++c)
+      *reinterpret_cast<f4 *>(sums + wave * 16 * RT + c * 16 + (lane >> 4) * 4) =
+          ((acc[0][c] + acc[1][c]) + acc[2][c]) + acc[3][c];
   }
 };
-template <int RT, int NW>
+template <int RT>
 struct RouterTotal {
   const float *sums;
+  int slices;
   __device__ __forceinline__ float operator()(int e) const {
     float v = sums[e];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) v += sums[i * 16 * RT + e];
+    for (int i = 1; i < slices; ++i) v += sums[i * 16 * RT + e];
     return v;
   }
 };

@@ -1,7 +1,10 @@
 """Experts: the router beside the norm that makes its rows; the lists, picked in their launch or in
 one before (up to 16 tokens at 64 columns and 16 picks, up to 8 otherwise), of one, four and any
 number of picks a thread (1024, 4096)."""
+import numpy as np
 import pytest
+
+import flexflow_amd as fa
 
 import nomutar_models as NM
 import nomutar_ref as NR
@@ -49,3 +52,28 @@ def test_few_and_many_rows_an_expert(tmp_path, n, top, T):
     toks = tokens_p(cfg, T, 8)
     eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=256, positions=256)
     close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
+
+
+@pytest.mark.parametrize("n,identity,width", [(12, 4, 100), (40, 4, 544), (40, 4, 1024), (40, 4, 2048), (60, 4, 1568),
+                                              (40, 4, 2080), (40, 4, 3104), (40, 4, 4096), (8, 4, 4096)])
+def test_a_row_does_not_know_its_step(tmp_path, n, identity, width):
+    """What a layer leaves of one token is the same bits in steps of 8 to 64 tokens, whose router is a product of
+    its own or a part of the norm's launch: K whole, in slices, of k-steps that they do not divide."""
+    cfg = PM.model_config(60, width, [PM.experts(PM.gla(1, 16, 16), n, 2, 32, identity=identity, groups=(1, 1))])
+    folder = PM.write_checkpoint(tmp_path / "p", cfg, PM.random_weights(cfg, 9))
+    m = fa.Model(fa.load_config(folder), "inc", max_requests=64, max_tokens=64, max_seq_len=64, weights_folder=folder,
+                 kv_pool_tokens=64 * 64)
+    rm = fa.RequestManager(max_requests_per_batch=64, max_tokens_per_batch=64, max_spec_tree_token_num=0,
+                           max_sequence_length=64)
+    m.set_debug(True)
+    got, rid = {}, 0
+    for T in (8, 16, 17, 32, 64) if n >= 40 else (8, 16, 17, 32):  # (the experts' products in one order of sums)
+        step = [(rid + i, [(7 * i + 5) % 60], [0]) for i in range(1, T + 1)]
+        rm.replay_step(m, step)
+        got[T] = m.debug_tensor("hidden", 0)
+        assert got[T].shape[0] == T and got[T].dtype == np.float32
+        for e in step:
+            rm.replay_end(m, e[0])
+        rid += T
+    for T in got:
+        assert np.array_equal(got[T][:16], got[17][:min(T, 16)]), T
