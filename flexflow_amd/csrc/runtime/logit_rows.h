@@ -23,6 +23,7 @@ class LogitRows {
   ~LogitRows() {
     for (auto e : done_)
       if (e) (void)hipEventDestroy(e);
+    if (step_) (void)hipEventDestroy(step_);
     if (staging_) (void)hipHostFree(staging_);
     if (there_) (void)hipHostFree(there_);
   }
@@ -47,6 +48,17 @@ class LogitRows {
     }
     for (auto &e : done_)
       if (!e) FFMI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // Rows are waited for by looking, the step before them as the device's flags say
+    // (FFMI_SYNC): where threads yield or sleep, by an event of its own.  (HIP's default
+    // keeps the core in either wait, and the event takes up to 4 us a step.)
+    unsigned flags = 0;
+    FFMI_HIP(hipGetDeviceFlags(&flags));
+    sleeps_ = (flags & hipDeviceScheduleMask) == hipDeviceScheduleBlockingSync ||
+              (flags & hipDeviceScheduleMask) == hipDeviceScheduleYield;
+    if (sleeps_) {
+      if (!step_) FFMI_HIP(hipEventCreateWithFlags(&step_, hipEventDisableTiming));
+      FFMI_HIP(hipEventRecord(step_, s));
+    }
     out_ = out, n_ = n;
     const ffmi_status st = put(0, n);
     if (st == FFMI_OK) touch(out, (size_t)n * V * sizeof(float));
@@ -59,6 +71,7 @@ class LogitRows {
     const int n = n_;
     n_ = 0;
     if (n <= 0) return FFMI_OK;
+    if (sleeps_) FFMI_HIP(hipEventSynchronize(step_));
     int half = 0;
     for (int at = 0;; at += kRows, half ^= 1) {
       const uint32_t mark = mark_;
@@ -121,7 +134,8 @@ class LogitRows {
   uint32_t *there_ = nullptr;  // [2][kRows][kParts]
   uint32_t mark_ = 0;          // of the latest kernel
   size_t staged_ = 0;  // row width that the staging holds
-  hipEvent_t done_[2] = {nullptr, nullptr};
+  hipEvent_t done_[2] = {nullptr, nullptr}, step_ = nullptr;
+  bool sleeps_ = false;
   const void *src_ = nullptr;
   const int *rows_ = nullptr;
   bool half_ = false;

@@ -1,6 +1,10 @@
 """Logits of a replay step on their way to the host (runtime/logit_rows.h): more rows
 than the staging's halves hold, any order and repeats of `want`, a vocabulary that is
 no multiple of the kernel's vectors, against the same rows one step at a time."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -36,3 +40,40 @@ def test_many_rows(kind, vocab):
     both = rm.replay_step(m, [(3, toks[0][:30], [29, 2]), (4, toks[1][:30], [1, 28])])
     assert both.shape == (4, vocab) and np.isfinite(both).all()
     assert np.abs(both[:2] - whole[[29, 2]]).max() < (1e-4 if kind == "fp32" else 3e-2) * np.abs(whole).max()
+
+
+WAITS = """
+import time
+import numpy as np
+import flexflow_amd as fa
+from vapipel_models import layer, model_config
+fa.set_device(0)  # (applies FFMI_SYNC)
+LLAMA = dict(num_layers=8, num_heads=16, num_kv_heads=16, hidden=2048, intermediate=5632, rms_eps=1e-6,
+             rope_theta=10000.0, vocab_size=2000)
+cfg = model_config(2000, 2048, 1024, [layer(16, 128, 128, 256, 0.1, 5632)] * 8) if KIND == "paged" else LLAMA
+m = fa.Model(cfg, "inc", max_requests=1, max_tokens=1000, max_seq_len=1024, weight_seed=5,
+             full_precision=KIND == "fp32")
+rm = fa.RequestManager(max_requests_per_batch=1, max_tokens_per_batch=1000, max_spec_tree_token_num=0,
+                       max_sequence_length=1024)
+toks = np.arange(1000, dtype=np.int32)
+wall = cpu = 0.0
+for i in range(24):
+    w, c = time.perf_counter(), time.thread_time()
+    rm.replay_step(m, [(i + 1, toks, [999])])
+    if i >= 4:
+        wall, cpu = wall + time.perf_counter() - w, cpu + time.thread_time() - c
+    rm.replay_end(m, i + 1)
+print("share", cpu / wall, wall / 20)
+"""
+
+
+@pytest.mark.parametrize("kind", ["fp16", "fp32", "paged"])
+def test_a_long_step_is_waited_for_as_asked(kind):
+    """FFMI_SYNC=block: the thread sleeps while a step of milliseconds runs (launching it is what is left)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, FFMI_SYNC="block", PYTHONPATH=os.pathsep.join([root, os.path.join(root, "tests")]))
+    r = subprocess.run([sys.executable, "-c", "KIND = %r\n" % kind + WAITS], env=env, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    print(r.stdout)
+    assert "not applied" not in r.stderr and float(r.stdout.split("share")[1].split()[0]) < 0.75, r.stdout
