@@ -529,10 +529,13 @@ struct Pekarax : public PagedDecoder {
       FFMI_TRY(gemm_sum(cat, L.wout, Wp, L.no, &n.y));
       if (L.experts) n.hrow = hrow;
       RouteScores route;
-      route.n = sizes(L, step.T), route.scores = L.scores, route.lists = moe.lists;
-      route.w = {(const uint16_t *)L.wrouter, w_tile_stride(Wp / 32), w_k_stride(L.nr / 16), Wp / 32,
-                 step.T <= 64 ? gemm_few_rows_slices(step.T, L.nr, Wp) : 1};
-      const bool routed = L.experts && !f32 && route_with_row(route.n, Wp, route.w.slices);
+      bool routed = false;
+      if (L.experts && !f32 && step.T <= 64) {
+        route.n = sizes(L, step.T), route.scores = L.scores, route.lists = moe.lists;
+        route.w = {(const uint16_t *)L.wrouter, w_tile_stride(Wp / 32), w_k_stride(L.nr / 16), Wp / 32,
+                   gemm_few_rows_slices(step.T, L.nr, Wp)};
+        routed = route_with_row(route.n, Wp, route.w.slices);
+      }
       FFMI_HIP(launch_sum_norm(n, routed ? &route : nullptr, stream));
       if (L.experts) {
         FFMI_TRY(experts(L, routed));
