@@ -15,30 +15,39 @@ struct MoeTile {
   int32_t expert;  // == number of experts: the shared one
   int32_t slot0, rows, pad;
 };
-constexpr int kMoeFew = 16, kMoeMany = 256;  // rows of a tile in the two forms
+constexpr int kMoeFew = 16, kMoeSome = 64, kMoeMany = 256;  // rows of a tile in the three forms
 constexpr int kMoeMaxExperts = 1024, kMoeMaxTop = 64;
 
 // a step's sizes: T tokens of which each takes `top` of `experts`
 struct MoeSizes {
   int T = 0, experts = 0, top = 0;
   int identity = 0;  // further outputs of the router, after the experts': the row itself
-  bool shared = false;
+  bool shared = false, f32 = false;
   int gate_col = 0;  // column of the shared expert's gate in the router's product
-  // Few: 16 rows a tile, for which an expert's weights are read again every 16 rows; many:
-  // once, on a grid that must not be small.  Both products, us, 5 and 10 rows an expert on
-  // average, many and few (whole_k):
-  //    32 experts, 4 taken, 1408 x 2048    52.7 49.7   52.8 51.0
-  //    32, 4, 2752 x 4096                   200  162    202  167
-  //    64, 8, 1024 x 2048                  81.1 69.2   81.1 76.4
-  //   128, 8, 1024 x 2048                   150  131    152  137
-  // and from 14 rows on, where many experts have over 16, few are the slower.
+  // Few rows a tile: an expert's weights are read again for every 16 rows, on a large grid.
+  // Many: once, on a grid that must not be small.  Some, between them: once for up to 64
+  // rows, from registers.  Four layers' steps, us, of 4, 6, 8 and 11 rows an expert on
+  // average, tokens all different, of 8 kinds and of 3, many and some:
+  //   32 experts, 4 taken, 2752 x 4096  1639 1481  1725 1584  1728 1625  1790 1702
+  //                                     1224 1087  1241 1134  1269 1182  1313 1294
+  //                                      698  715   759  794   891  947   949 1049
+  //   32, 4, 1408 x 2048                 618  545   656  595   691  624   721  664
+  //                                      440  448   491  496   520  518   558  582
+  //                                      406  345   447  389   472  446   507  493
+  //   64, 8, 1024 x 2048                 726  669   772  720   833  786   871  835
+  //                                      590  531   636  563   606  571   635  618
+  //                                      439  438   464  471   504  554   534  590
+  // (some loses where a handful of experts takes every row.  Tiles of 16 rows there instead:
+  // 11 rows, 3 kinds 1408, 590, 641.)  From 14 rows on many is the faster.
   // A shared expert has every token's row: few read it T / 16 times (replay of 32 experts, 4
   // taken, and one of half the units, steps of 82 tokens: 18.3 ms, 19.0).
+  // fp32 (16 rows a workgroup in any form): up to 12 rows an expert tiles of 16 spread them,
+  // 32 experts, 704 x 2048, 48 tokens 4.9 -> 3.4 ms, 64 experts, 512 x 2048 6.2 -> 3.6.
   int tile_rows() const {
-    return T > 32 && (long)T * top >= (shared ? 4L : 12L) * experts ? kMoeMany : kMoeFew;
+    if (T <= 32 || (long)T * top < 4L * experts) return kMoeFew;
+    if (shared || (long)T * top >= 12L * experts) return kMoeMany;
+    return f32 ? kMoeFew : kMoeSome;
   }
-  // few rows' products in the order of the many's sums
-  bool whole_k() const { return T > 32 && (long)T * top >= 4L * experts; }
   // upper bounds: slots of the experts (whole 16s), tiles
   __host__ __device__ int slots() const {
     const int a = T * top, e = a < experts ? a : experts;

@@ -268,48 +268,52 @@ __global__ __launch_bounds__(256) void moe_few_kernel(MoeGemm a, int first, size
   }
 }
 
-// The same of whole K: a wave has two tiles of its own, its sums in the tile kernel's order (a
-// row's bits do not change where this form takes its place).  Two register sets: the next U
-// k-steps are on their way while these are multiplied.
-template <bool GATED, bool NTL>
-__global__ __launch_bounds__(256) void moe_chain_kernel(MoeGemm a, int first, size_t wts) {
-  constexpr int U = 8;
-  if (first + (int)blockIdx.y >= *a.num_tiles) return;
-  const MoeTile tl = a.tiles[first + blockIdx.y];
-  const bool shared = tl.expert >= a.experts;
-  const MoeGroup &g = a.g[shared];
+// The same of whole K and up to 64 rows, MT times 16: a wave has two tiles of its own, its
+// sums in the tile kernel's order (a row's bits do not change where this form takes its
+// place).  Two register sets: the next U k-steps are on their way while these are multiplied
+// (with 64 rows U = 4 does not fit the registers of two waves a SIMD).
+template <bool GATED, bool NTL, int MT, int U>
+__device__ __forceinline__ void moe_chain(const MoeGemm &a, const MoeTile &tl, size_t wts) {
+  const MoeGroup &g = a.g[0];
   const int lane = threadIdx.x & 63, m = lane & 15, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int KT = g.K >> 5, ntiles = (GATED ? 2 : 1) * (g.N >> 4), pair = blockIdx.x * 4 + wave, tile0 = pair * 2;
   if (tile0 >= ntiles) return;
   const size_t wks = wts == 512 ? (size_t)ntiles * 512 : 512, ts = wts == 512 ? 512 : (size_t)KT * 512;
-  const uint16_t *W = (const uint16_t *)g.W + (shared ? 0 : tl.expert * g.w_stride) + lane * 8;
+  const uint16_t *W = (const uint16_t *)g.W + tl.expert * g.w_stride + lane * 8;
   const uint16_t *w0 = W + tile0 * ts, *w1 = W + min(tile0 + 1, ntiles - 1) * ts;
-  const uint16_t *x;
-  if constexpr (GATED) {
-    const int slot = tl.slot0 + min(m, tl.rows - 1);
-    x = (const uint16_t *)g.X + (size_t)(shared ? slot : a.slot_token[slot]) * g.K + 8 * (lane >> 4);
-  } else {
-    x = (const uint16_t *)g.X + ((size_t)(tl.slot0 >> 4) * KT * 64 + packed_lane(lane, tl.rows)) * 8;
+  const uint16_t *x[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int r0 = min(i * 16, (tl.rows - 1) & ~15);  // (fewer rows than MT holds: the last 16 again)
+    if constexpr (GATED)
+      x[i] = (const uint16_t *)g.X + (size_t)a.slot_token[tl.slot0 + min(r0 + m, tl.rows - 1)] * g.K + 8 * (lane >> 4);
+    else
+      x[i] = (const uint16_t *)g.X + ((size_t)((tl.slot0 + r0) >> 4) * KT * 64 + packed_lane(lane, tl.rows - r0)) * 8;
   }
   constexpr int XS = GATED ? 32 : 512;
-  f4 acc[2];
-  acc[0] = acc[1] = f4{0.f, 0.f, 0.f, 0.f};
-  h8 wa[U][2], xa[U], wb[U][2], xb[U];
-  auto load = [&](h8(&b)[U][2], h8(&xv)[U], int k) {
+  f4 acc[MT][2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i][0] = acc[i][1] = f4{0.f, 0.f, 0.f, 0.f};
+  h8 wa[U][2], xa[U][MT], wb[U][2], xb[U][MT];
+  auto load = [&](h8(&b)[U][2], h8(&xv)[U][MT], int k) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const size_t kk = min(k + u, KT - 1);
       b[u][0] = ld_weight<NTL>(w0 + kk * wks), b[u][1] = ld_weight<NTL>(w1 + kk * wks);
-      xv[u] = *reinterpret_cast<const h8 *>(x + kk * XS);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) xv[u][i] = *reinterpret_cast<const h8 *>(x[i] + kk * XS);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto mul = [&](const h8(&b)[U][2], const h8(&xv)[U], int n) {
+  auto mul = [&](const h8(&b)[U][2], const h8(&xv)[U][MT], int n) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (u >= n) break;
-      acc[0] = moe_mma(b[u][0], xv[u], acc[0]);
-      acc[1] = moe_mma(b[u][1], xv[u], acc[1]);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        acc[i][0] = moe_mma(b[u][0], xv[u][i], acc[i][0]);
+        acc[i][1] = moe_mma(b[u][1], xv[u][i], acc[i][1]);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -328,14 +332,25 @@ __global__ __launch_bounds__(256) void moe_chain_kernel(MoeGemm a, int first, si
   } else {
     mul(wa, xa, KT - k);
   }
-  if (m >= tl.rows) return;
-  const int row = tl.slot0 + m, n = (lane >> 4) * 4;
-  if constexpr (GATED) {
-    moe_store<true>(g, row, pair * 16 + n, shared ? a.gate[row] : 1.0f, a.limit, acc[0], acc[1]);
-  } else {
-    moe_store<false>(g, row, tile0 * 16 + n, 1.0f, 0.f, acc[0], acc[0]);
-    if (tile0 + 1 < ntiles) moe_store<false>(g, row, tile0 * 16 + 16 + n, 1.0f, 0.f, acc[1], acc[1]);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    if (i * 16 + m >= tl.rows) return;
+    const int row = tl.slot0 + i * 16 + m, n = (lane >> 4) * 4;
+    if constexpr (GATED) {
+      moe_store<true>(g, row, pair * 16 + n, 1.0f, a.limit, acc[i][0], acc[i][1]);
+    } else {
+      moe_store<false>(g, row, tile0 * 16 + n, 1.0f, 0.f, acc[i][0], acc[i][0]);
+      if (tile0 + 1 < ntiles) moe_store<false>(g, row, tile0 * 16 + 16 + n, 1.0f, 0.f, acc[i][1], acc[i][1]);
+    }
   }
+}
+template <bool GATED, bool NTL>
+__global__ __launch_bounds__(256, 2) void moe_chain_kernel(MoeGemm a, size_t wts) {
+  if ((int)blockIdx.y >= *a.num_tiles) return;
+  const MoeTile tl = a.tiles[blockIdx.y];
+  if (tl.rows <= 16) moe_chain<GATED, NTL, 1, 8>(a, tl, wts);
+  else if (tl.rows <= 32) moe_chain<GATED, NTL, 2, 4>(a, tl, wts);
+  else moe_chain<GATED, NTL, 4, 2>(a, tl, wts);
 }
 
 // Up to 256 rows x 16 tiles a workgroup: eight waves as 2 (every other 16 rows) x 4
@@ -541,11 +556,11 @@ hipError_t launch_moe_gemm(const MoeGemm &a, const MoeSizes &n, bool gated, bool
     return hipGetLastError();
   }
   const int pairs = (per * N / 16 + 1) / 2;
-  const dim3 grid(pairs, st + tiles), quads((pairs + 3) / 4, st + tiles);
-#define FFMI_MF(G, NL)                                                                              \
-  do {                                                                                              \
-    if (n.whole_k()) hipLaunchKernelGGL((moe_chain_kernel<G, NL>), quads, dim3(256), 0, s, a, first, wts); \
-    else hipLaunchKernelGGL((moe_few_kernel<G, NL>), grid, dim3(256), 0, s, a, first, wts);         \
+  const dim3 grid(pairs, st + tiles), quads((pairs + 3) / 4, tiles);
+#define FFMI_MF(G, NL)                                                                            \
+  do {                                                                                            \
+    if (rows == kMoeSome) hipLaunchKernelGGL((moe_chain_kernel<G, NL>), quads, dim3(256), 0, s, a, wts); \
+    else hipLaunchKernelGGL((moe_few_kernel<G, NL>), grid, dim3(256), 0, s, a, first, wts);       \
   } while (0)
   if (gated && stream_weights) FFMI_MF(true, true);
   else if (gated) FFMI_MF(true, false);

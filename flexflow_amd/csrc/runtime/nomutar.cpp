@@ -271,7 +271,7 @@ struct Nomutar : public PagedDecoder {
   }
   MoeSizes sizes(const NomutarLayer &L, int T) const {
     MoeSizes n;
-    n.T = T, n.experts = L.experts, n.top = L.top, n.shared = L.sff > 0, n.gate_col = L.gate_col;
+    n.T = T, n.experts = L.experts, n.top = L.top, n.shared = L.sff > 0, n.gate_col = L.gate_col, n.f32 = f32;
     return n;
   }
   // rows of the first product's weight: `heads` of n rows, padded to np

@@ -157,7 +157,7 @@ struct Pekarax : public PagedDecoder {
   // ---- buffers and weights ----
   MoeSizes sizes(const PekaraxLayer &L, int T) const {
     MoeSizes n;
-    n.T = T, n.experts = L.experts, n.top = L.top, n.identity = L.identity;
+    n.T = T, n.experts = L.experts, n.top = L.top, n.identity = L.identity, n.f32 = f32;
     return n;
   }
   bool mfma_form(const PekaraxAttention &A) const { return !f32 && attn_width(A.dim) && attn_width(A.vdim); }

@@ -44,14 +44,37 @@ def test_router_beside_the_norm(tmp_path, n, identity, width, T):
     close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
 
 
-@pytest.mark.parametrize("n,top,T", [(8, 2, 33), (8, 2, 47), (8, 2, 48), (16, 4, 47), (16, 4, 48), (64, 1, 200)])
-def test_few_and_many_rows_an_expert(tmp_path, n, top, T):
-    """Products of 16 rows a workgroup up to 12 rows an expert on average, from there on of 256."""
+@pytest.mark.parametrize("n,top,T,kinds", [
+    (8, 2, 33, 90), (8, 2, 47, 90), (8, 2, 48, 90), (16, 4, 47, 90), (16, 4, 48, 90), (64, 1, 200, 90),
+    (16, 4, 47, 2), (40, 4, 47, 1), (40, 1, 160, 1), (40, 1, 200, 2), (40, 2, 160, 6)])
+def test_few_and_many_rows_an_expert(tmp_path, n, top, T, kinds):
+    """Products of 16 rows a workgroup up to 4 rows an expert on average, up to 12 of up to 64 rows
+    (tokens of few kinds: 17 to 64 rows of one expert, and more), from there on of 256."""
     cfg = PM.model_config(90, 96, [PM.experts(PM.gla(1, 16, 16), n, top, 200, identity=0, groups=(1, 1))])
     w = PM.random_weights(cfg, 11)
-    toks = tokens_p(cfg, T, 8)
+    toks = [t % kinds for t in tokens_p(cfg, T, 8)]
     eng = engine_p(PM.write_checkpoint(tmp_path / "p", cfg, w), False, pool=16 * 64, batch=256, positions=256)
     close_p(run_p(eng, toks, [T]), PR.forward(cfg, w, toks), False)
+
+
+def many_requests(tmp_path, cfg):
+    folder = PM.write_checkpoint(tmp_path / "p", cfg, PM.random_weights(cfg, 9))
+    m = fa.Model(fa.load_config(folder), "inc", max_requests=64, max_tokens=64, max_seq_len=64, weights_folder=folder,
+                 kv_pool_tokens=64 * 64)
+    m.set_debug(True)
+    return fa.RequestManager(max_requests_per_batch=64, max_tokens_per_batch=64, max_spec_tree_token_num=0,
+                             max_sequence_length=64), m
+
+
+def hidden(rm, m, toks, rid):
+    """a step of requests of one token each: the residual stream after the first layer"""
+    step = [(rid + i, [t], [0]) for i, t in enumerate(toks)]
+    rm.replay_step(m, step)
+    got = m.debug_tensor("hidden", 0)
+    assert got.shape[0] == len(toks) and got.dtype == np.float32
+    for e in step:
+        rm.replay_end(m, e[0])
+    return got
 
 
 @pytest.mark.parametrize("n,identity,width", [(12, 4, 100), (40, 4, 544), (40, 4, 1024), (40, 4, 2048), (60, 4, 1568),
@@ -60,20 +83,19 @@ def test_a_row_does_not_know_its_step(tmp_path, n, identity, width):
     """What a layer leaves of one token is the same bits in steps of 8 to 64 tokens, whose router is a product of
     its own or a part of the norm's launch: K whole, in slices, of k-steps that they do not divide."""
     cfg = PM.model_config(60, width, [PM.experts(PM.gla(1, 16, 16), n, 2, 32, identity=identity, groups=(1, 1))])
-    folder = PM.write_checkpoint(tmp_path / "p", cfg, PM.random_weights(cfg, 9))
-    m = fa.Model(fa.load_config(folder), "inc", max_requests=64, max_tokens=64, max_seq_len=64, weights_folder=folder,
-                 kv_pool_tokens=64 * 64)
-    rm = fa.RequestManager(max_requests_per_batch=64, max_tokens_per_batch=64, max_spec_tree_token_num=0,
-                           max_sequence_length=64)
-    m.set_debug(True)
-    got, rid = {}, 0
-    for T in (8, 16, 17, 32, 64) if n >= 40 else (8, 16, 17, 32):  # (the experts' products in one order of sums)
-        step = [(rid + i, [(7 * i + 5) % 60], [0]) for i in range(1, T + 1)]
-        rm.replay_step(m, step)
-        got[T] = m.debug_tensor("hidden", 0)
-        assert got[T].shape[0] == T and got[T].dtype == np.float32
-        for e in step:
-            rm.replay_end(m, e[0])
-        rid += T
+    rm, m = many_requests(tmp_path, cfg)
+    # (up to 64 where the experts' products keep one order of sums)
+    got = {T: hidden(rm, m, [(7 * i + 5) % 60 for i in range(T)], 100 * T)
+           for T in ((8, 16, 17, 32, 64) if n >= 40 else (8, 16, 17, 32))}
     for T in got:
         assert np.array_equal(got[T][:16], got[17][:min(T, 16)]), T
+
+
+@pytest.mark.parametrize("kinds", [60, 3, 1])
+def test_some_and_many_rows_have_the_same_bits(tmp_path, kinds):
+    """Experts' products of up to 64 rows a tile (33 and 59 tokens, 2 of 10 experts) and of 256 (60)."""
+    cfg = PM.model_config(60, 544, [PM.experts(PM.gla(1, 16, 16), 10, 2, 328, identity=0, groups=(1, 1))])
+    rm, m = many_requests(tmp_path, cfg)
+    got = [hidden(rm, m, [(7 * i + 5) % kinds for i in range(T)], 100 * T) for T in (60, 59, 33)]
+    for g in got:
+        assert np.array_equal(g, got[0][:len(g)])
