@@ -273,8 +273,14 @@ struct Fesenex : public PagedDecoder {
   // leaves h = x w and the sums of squares of x, the product after it scales its sums by
   // the rms (FuseArgs 3 and 4); 4096 channels, 8 tokens: 2.2 us a norm less.  From 2048
   // columns on: narrower layers split K up to 8 ways, and unsplit would lose more than a
-  // launch.  With more rows a norm's launch is a small part of the products.
-  bool folds() const { return !f32 && step.T <= 16 && Wp >= 2048 && Wp <= 4096; }
+  // launch; so does one of 2048 columns in two slices from K = 8192 on (12 layers, K = 8192
+  // and 11008, us: 1 token 535 -> 509, 590 -> 592; 16 tokens 620 -> 618, 689 -> 719; unsplit
+  // ones of 2560 to 4096 columns gain 5-12 % of a step at 1 to 16 tokens, K 1024 to 11008).
+  // With more rows a norm's launch is a small part of the products.
+  bool folds(int K) const {
+    return !f32 && step.T <= 16 && Wp >= 2048 && Wp <= 4096 &&
+           (K <= 8192 || gemm_few_rows_slices(step.T, Wp, K) == 1);
+  }
   FuseArgs rms;         // of h, where it lacks its rms
   bool lacks = false;
   // y = h W, the sublayer's first product
@@ -286,7 +292,7 @@ struct Fesenex : public PagedDecoder {
   }
   // x += in W, then the next sublayer's input (w null: none follows)
   ffmi_status to_x(const void *in, const void *wt, int K, const float *w) {
-    lacks = folds();
+    lacks = folds(K);
     if (!lacks) {
       Partials y;
       FFMI_TRY(gemm_sum(in, wt, Wp, K, &y));
