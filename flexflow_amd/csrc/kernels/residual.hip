@@ -220,8 +220,9 @@ hipError_t launch_row_norm(const char *blob, int off_rows, const float *x, const
 // One workgroup per row, a thread's chunks of 8 columns; all loads before the
 // reduction, of slabs MAXS at a time.  RT > 0: the row's experts as well, of a router of
 // up to 16 RT columns.
+struct NoRoute {};
 template <int NT, int MAXC, int MAXS, int RT = 0>
-__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, RouteScores route) {
+__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, std::conditional_t<(RT > 0), RouteScores, NoRoute> route) {
   constexpr int U = 4;  // expert rows in flight
   __shared__ float sh[NT / 64];
   constexpr int NW = NT / 64, RTS = RT ? RT : 1;
@@ -358,7 +359,7 @@ hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream
     return hipGetLastError();
   }
 #define FFMI_SM(NT, MC, MS) \
-  hipLaunchKernelGGL((sum_norm_kernel<NT, MC, MS>), dim3(a.T), dim3(NT), 0, s, a, RouteScores())
+  hipLaunchKernelGGL((sum_norm_kernel<NT, MC, MS>), dim3(a.T), dim3(NT), 0, s, a, NoRoute())
 #define FFMI_SMS(NT, MC)                 \
   do {                                   \
     if (a.y.S == 0) FFMI_SM(NT, MC, 0);  \

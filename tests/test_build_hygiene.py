@@ -27,8 +27,8 @@ LLVM = "/opt/rocm/llvm/bin"
 LIB = os.path.join(ROOT, "flexflow_amd", "libffmi.so")
 
 
-def _lib_usage(lib):
-    """{kernel: scratch bytes per lane} from the built library's code objects."""
+def _lib_usage(lib, key="private_segment_fixed_size"):
+    """{kernel: scratch bytes per lane, or another figure} from the built library's code objects."""
     out = {}
     with tempfile.TemporaryDirectory() as d:
         fat = os.path.join(d, "fat.bin")
@@ -53,14 +53,17 @@ def _lib_usage(lib):
                     f.write(data[pos + off:pos + off + size])
                 notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", co], check=True,
                                        capture_output=True, text=True).stdout
-                name = None  # metadata keys are sorted: .name precedes .private_segment_*
+                name = args = None  # metadata keys are sorted: .kernarg_* and then .name precede .private_segment_*
                 for line in notes.splitlines():
                     m = re.match(r"\s+\.name:\s+(\S+)", line)
                     if m:
                         name = m.group(1)
+                    m = re.search(r"\.kernarg_segment_size:\s+(\d+)", line)
+                    if m:
+                        args = int(m.group(1))
                     m = re.search(r"\.private_segment_fixed_size:\s+(\d+)", line)
                     if m and name:
-                        out[name] = int(m.group(1))
+                        out[name] = int(m.group(1)) if key == "private_segment_fixed_size" else args
             pos = data.find(magic, pos + 1)
     return out
 
@@ -102,3 +105,14 @@ def test_no_kernel_uses_scratch():
     bad = {k: v for r in results for k, v in r.items() if v}
     assert sum(len(r) for r in results) > 20
     assert not bad, f"kernels with scratch: {bad}"
+
+
+@pytest.mark.skipif(not os.path.exists(LIB) or not os.path.exists(f"{LLVM}/llvm-readelf"), reason="nothing built")
+def test_norms_without_a_router_do_not_carry_its_arguments():
+    """A launch copies its arguments, and short chains of norms notice: what a router beside the norm
+    needs (weights, sizes, scores, lists) is an argument of its own instantiations alone."""
+    size = {k: v for k, v in _lib_usage(LIB, "kernarg_segment_size").items() if "sum_norm_kernel" in k}
+    columns = {k: int(re.search(r"sum_norm_kernelI(?:Li\d+E){3}Li(\d+)E", k).group(1)) for k in size}  # of 16, the router's
+    plain, routed = ([v for k, v in size.items() if (columns[k] > 0) == r] for r in (False, True))
+    assert len(plain) >= 9 and len(routed) == 12, size
+    assert max(plain) <= min(routed) - 120, size
