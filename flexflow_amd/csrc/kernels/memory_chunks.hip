@@ -801,7 +801,10 @@ hipError_t run_chunks(const char *blob, int off_spans, int num_spans, int num_ch
 // One workgroup of either kind fits a CU: one round of them, as a second would cost more than the
 // launch saved.  The chunks of 256 state rows need more registers than two waves of a SIMD
 // have, with the delta rule over 100 more; the gated rule's ask for half of a thread's rows at a
-// time there.
+// time there.  The short spans' threads have room for 8 rows, also where a state gives them 1 to
+// 4: 12 layers, a portion of 33 and 5 single tokens, us, two launches and one: delta rule, 8 heads of
+// 32 x 32 (1 row) 641 518, of 64 x 64 (2) 669 539, 4 of 64 x 128 (4) 701 562; gated 542 453, 527
+// 442, 550 454; a portion of 20 and three of 16, the longest steps: 1394 1375, 1889 1723, 2141 1952.
 bool memory_mixes(const Memory &a, int num_spans, int num_chunks, int limit) {
   const MemoryStepsPlan p = memory_steps_plan(a, num_spans, limit, true);
   return a.dg <= (a.rule == kMemoryGated ? 256 : 128) && p.rows <= 8 && p.bytes <= 64 * 1024 && (p.parts == 1 || a.rule != kMemoryDelta) &&

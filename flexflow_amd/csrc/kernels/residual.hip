@@ -222,7 +222,8 @@ hipError_t launch_row_norm(const char *blob, int off_rows, const float *x, const
 // up to 16 RT columns.
 struct NoRoute {};
 template <int NT, int MAXC, int MAXS, int RT = 0>
-__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, std::conditional_t<(RT > 0), RouteScores, NoRoute> route) {
+__global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a,
+                                                      std::conditional_t<(RT > 0), RouteScores, NoRoute> route) {
   constexpr int U = 4;  // expert rows in flight
   __shared__ float sh[NT / 64];
   constexpr int NW = NT / 64, RTS = RT ? RT : 1;
@@ -324,9 +325,9 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a, std::conditiona
 // of the experts would show.  (A slice of 64 k-steps and more would be cut in 8: only where
 // FFMI_SKINNY_SPLIT=0 leaves K whole.)
 bool route_with_row(const MoeSizes &n, int H, int slices) {
-  const int cols = n.shared ? n.gate_col + 1 : n.experts + n.identity, tiles = (cols + 15) / 16;
-  return n.T <= 64 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144) && slices >= 1 && slices <= 8 &&
-         (H / 32 + slices - 1) / slices < 64;
+  const int cols = n.experts + n.identity, tiles = (cols + 15) / 16;
+  return !n.shared && n.T <= 64 && cols <= 64 && H <= 4096 && (n.T > 16 || tiles * H <= 6144) && slices >= 1 &&
+         slices <= 8 && (H / 32 + slices - 1) / slices < 64;
 }
 hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream_t s) {
   if (a.T <= 0) return hipSuccess;
@@ -338,7 +339,7 @@ hipError_t launch_sum_norm(const SumNorm &a, const RouteScores *route, hipStream
     const MoeSizes &n = route->n;
     const MoeScores &sc = route->scores;
     const int cols = n.experts + n.identity;
-    if (!route_with_row(n, a.H, route->w.slices) || n.T != a.T || n.shared || a.rows || route->w.steps * 32 != a.H || !route->w.w ||
+    if (!route_with_row(n, a.H, route->w.slices) || n.T != a.T || a.rows || route->w.steps * 32 != a.H || !route->w.w ||
         n.experts < 1 || n.identity < 0 || n.top < 1 || sc.groups < 1 || cols % sc.groups || sc.keep < 1 ||
         sc.keep > sc.groups || n.top > cols / sc.groups * sc.keep || !sc.correction ||
         (n.identity && !route->lists.own))
