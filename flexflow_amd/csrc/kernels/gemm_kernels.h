@@ -121,11 +121,17 @@ __device__ __forceinline__ float lane_f(float v, int l) {
 // is updated in place).
 template <int FZ>
 using SkinnyY = std::conditional_t<FZ == 1, uint16_t *, uint16_t *__restrict__>;
+// what a launch without norms carries of FuseArgs
+struct PlainArgs {
+  float limit;
+};
+template <int FZ>
+using SkinnyArgs = std::conditional_t<FZ != 0, FuseArgs, PlainArgs>;
 template <int MT, int NT, int KW, int U, int EPI, bool PIPE = false, bool NTL = false, int FZ = 0>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wp,
     SkinnyY<FZ> Y, float *__restrict__ Ypart, int T, int N, int K, int KT,
-    int NTILES, int xp, int yp, size_t wts, size_t wks, FuseArgs fz) {
+    int NTILES, int xp, int yp, size_t wts, size_t wks, SkinnyArgs<FZ> fz) {
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -201,9 +207,11 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   // a row's sum of squares: 16-lane DPP rows, then the four row sums in row order
   auto square_sum = [&](int rr) {
     float v = 0.f;
+    if constexpr (RMS) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (lane + 64 * c < fz.nss) v += pv[RMS ? rr : 0][c];
+      for (int c = 0; c < 4; ++c)
+        if (lane + 64 * c < fz.nss) v += pv[rr][c];
+    }
     v += row_ror_f<1>(v);
     v += row_ror_f<2>(v);
     v += row_ror_f<4>(v);
@@ -595,9 +603,12 @@ static hipError_t run(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float 
   static const int force = getenv("FFMI_SKINNY_PIPE") ? atoi(getenv("FFMI_SKINNY_PIPE")) : -1;
   const int per_wave = ((KT + S - 1) / S + KW - 1) / KW;
   const bool pipe = force >= 0 ? force != 0 : per_wave >= 2 * U;
+  SkinnyArgs<FZ> args;
+  if constexpr (FZ != 0) args = fz;
+  else args.limit = fz.limit;
 #define FFMI_SKINNY_LAUNCH(PP, NL)                                                             \
   hipLaunchKernelGGL((gemm_skinny_kernel<MT, NT, KW, U, EPI, PP, NL, FZ>), grid, dim3(KW * 64), \
-                     lds, s, X, Wp, Y, ws, T, N, K, KT, NTILES, xp, yp, wts, wks, fz)
+                     lds, s, X, Wp, Y, ws, T, N, K, KT, NTILES, xp, yp, wts, wks, args)
   if (pipe) {
     if (nt) FFMI_SKINNY_LAUNCH(true, true);
     else FFMI_SKINNY_LAUNCH(true, false);

@@ -108,10 +108,17 @@ def test_no_kernel_uses_scratch():
 
 
 @pytest.mark.skipif(not os.path.exists(LIB) or not os.path.exists(f"{LLVM}/llvm-readelf"), reason="nothing built")
-def test_norms_without_a_router_do_not_carry_its_arguments():
-    """A launch copies its arguments, and short chains of norms notice: what a router beside the norm
-    needs (weights, sizes, scores, lists) is an argument of its own instantiations alone."""
-    size = {k: v for k, v in _lib_usage(LIB, "kernarg_segment_size").items() if "sum_norm_kernel" in k}
+def test_launches_carry_only_their_own_arguments():
+    """A launch copies its arguments, and short chains of launches notice: what a router beside the norm
+    needs (weights, sizes, scores, lists) is an argument of its own instantiations alone, and so is
+    what a product of few rows needs for the norms around it."""
+    every = _lib_usage(LIB, "kernarg_segment_size")
+    skinny = {k: v for k, v in every.items() if "gemm_skinny_kernel" in k}
+    folded = {k: int(re.search(r"gemm_skinny_kernelI(?:Li\d+E){5}(?:Lb[01]E){2}Li(\d)E", k).group(1)) > 0 for k in skinny}
+    plain, normed = ([v for k, v in skinny.items() if folded[k] == f] for f in (False, True))
+    assert len(plain) > 40 and len(normed) > 10, skinny
+    assert max(plain) <= min(normed) - 90, skinny
+    size = {k: v for k, v in every.items() if "sum_norm_kernel" in k}
     columns = {k: int(re.search(r"sum_norm_kernelI(?:Li\d+E){3}Li(\d+)E", k).group(1)) for k in size}  # of 16, the router's
     plain, routed = ([v for k, v in size.items() if (columns[k] > 0) == r] for r in (False, True))
     assert len(plain) >= 9 and len(routed) == 12, size
