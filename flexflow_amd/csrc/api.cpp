@@ -692,19 +692,37 @@ extern "C" ffmi_status ffmi_arg_topk_ws(const void *logits, int T, int V, int k,
 // the residual in place and leaves per-(row, 16-column tile) sums of
 // squares; the consumer normalises the residual from those sums in its
 // prologue.  Row-major fp16 throughout.
+// (models fold up to 16 rows: more go in pieces of 16)
+static ffmi_status fused_residual_linear(const void *X, const void *W_packed, void *residual, void *residual_packed,
+                                         float *ss_out, int T, int out_dim, int in_dim, int flags,
+                                         ffmi_stream stream) {
+  ffmi::FuseArgs fz;
+  fz.kind = 1;
+  for (int t = 0; t < T; t += 16) {
+    fz.res_in = (const uint16_t *)residual + (size_t)t * out_dim;
+    fz.ss_out = ss_out + (size_t)t * (out_dim / 16);
+    fz.res_packed = (uint16_t *)residual_packed;
+    FFMI_HIP(ffmi::launch_gemm((const uint16_t *)X + (size_t)t * in_dim, (const uint16_t *)W_packed,
+                               (uint16_t *)residual + (size_t)t * out_dim, nullptr, 0, std::min(16, T - t), out_dim,
+                               in_dim, FFMI_EPI_NONE | flags, (hipStream_t)stream, nullptr, 0, &fz));
+  }
+  return FFMI_OK;
+}
 extern "C" ffmi_status ffmi_debug_fused_residual_linear(const void *X, const void *W_packed,
                                                         void *residual, float *ss_out, int T,
                                                         int out_dim, int in_dim,
                                                         ffmi_stream stream) {
   FFMI_CHECK(X && W_packed && residual && ss_out && T > 0 && T <= 32, FFMI_ERR_INVALID);
-  ffmi::FuseArgs fz;
-  fz.kind = 1;
-  fz.res_in = (const uint16_t *)residual;
-  fz.ss_out = ss_out;
-  FFMI_HIP(ffmi::launch_gemm((const uint16_t *)X, (const uint16_t *)W_packed, (uint16_t *)residual,
-                             nullptr, 0, T, out_dim, in_dim, FFMI_EPI_NONE, (hipStream_t)stream,
-                             nullptr, 0, &fz));
-  return FFMI_OK;
+  return fused_residual_linear(X, W_packed, residual, nullptr, ss_out, T, out_dim, in_dim, 0, stream);
+}
+extern "C" ffmi_status ffmi_debug_fused_residual_linear_packed(const void *X, const void *W_packed, void *residual,
+                                                               void *residual_packed, float *ss_out, int T,
+                                                               int out_dim, int in_dim, int flags,
+                                                               ffmi_stream stream) {
+  FFMI_CHECK(X && W_packed && residual && residual_packed && ss_out && T > 0 && T <= 16 &&
+                 !(flags & ~(FFMI_X_PACKED | FFMI_W_STREAM)),
+             FFMI_ERR_INVALID);
+  return fused_residual_linear(X, W_packed, residual, residual_packed, ss_out, T, out_dim, in_dim, flags, stream);
 }
 
 extern "C" ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const float *ss_in,
@@ -712,18 +730,21 @@ extern "C" ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const 
                                                     const void *W_packed, void *Y, int T,
                                                     int out_dim, int in_dim, int epilogue,
                                                     ffmi_stream stream) {
-  FFMI_CHECK(residual && ss_in && norm_w && W_packed && Y && T > 0 && T <= 32 &&
-                 (epilogue == FFMI_EPI_NONE || epilogue == FFMI_EPI_SILU_MUL),
+  const int kind = epilogue & ~(FFMI_X_PACKED | FFMI_W_STREAM);
+  FFMI_CHECK(residual && ss_in && norm_w && W_packed && Y && T > 0 &&
+                 T <= (epilogue & FFMI_X_PACKED ? 16 : 32) && (kind == FFMI_EPI_NONE || kind == FFMI_EPI_SILU_MUL),
              FFMI_ERR_INVALID);
   ffmi::FuseArgs fz;
   fz.kind = 2;
-  fz.ss_in = ss_in;
   fz.nss = in_dim / 16;
   fz.wnorm = (const uint16_t *)norm_w;
   fz.eps = eps;
-  FFMI_HIP(ffmi::launch_gemm((const uint16_t *)residual, (const uint16_t *)W_packed, (uint16_t *)Y,
-                             nullptr, 0, T, out_dim, in_dim, epilogue, (hipStream_t)stream,
-                             nullptr, 0, &fz));
+  for (int t = 0; t < T; t += 16) {
+    fz.ss_in = ss_in + (size_t)t * fz.nss;
+    FFMI_HIP(ffmi::launch_gemm((const uint16_t *)residual + (size_t)t * in_dim, (const uint16_t *)W_packed,
+                               (uint16_t *)Y + (size_t)t * out_dim, nullptr, 0, std::min(16, T - t), out_dim, in_dim,
+                               epilogue, (hipStream_t)stream, nullptr, 0, &fz));
+  }
   return FFMI_OK;
 }
 

@@ -232,7 +232,7 @@ hipError_t launch_pack_weight(const uint16_t *src, int ld, int row0, int col0,
 // Y is written and defer->S = 0.  Only for FFMI_EPI_NONE.  wpitch: tiles per
 // k-row of Wp's allocation (0 = the GEMM's own tile count; a column chunk of a
 // wider matrix passes the full matrix's).
-// Residual RMSNorm folded into the skinny GEMMs (T <= 32, unsplit), the
+// Residual RMSNorm folded into the skinny GEMMs (T <= 16, unsplit), the
 // reference's ResidualRMSNorm (residual_rms_norm_kernels.cu:98-131) split
 // over the two GEMMs around it:
 //  * producer (o / down projection, EPI 0): Y = half(res_in + half(X.W^T))

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   // not PCs); the builtin is convergent, so the compiler neither duplicates
   // nor moves it across the rdone branch.  Pinned by
   // test_gpu_kernels.py::test_fused_norm_consumer_empty_wave_ranges (KW 4 /
-  // 8 with waves that own no k-step, T 1..32).
+  // 8 with waves that own no k-step).
   auto rms_finish = [&]() {
     if constexpr (FZ == 2) {
       if (rdone) return;
@@ -747,36 +747,37 @@ static int skinny_split(int T, int N, int K, int epi, bool deferrable) {
   return std::max(1, std::min(S, 8));
 }
 
-// The fused residual/norm forms (FuseArgs; S == 1, T <= 32): the unfused
+// The fused residual/norm forms (FuseArgs; S == 1, T <= 16): the unfused
 // path's tile and wave choices, one instantiation set per role.
-template <int MT, int U, int FZ>
+template <int FZ>
 static hipError_t dispatch_fused(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, int T, int N,
                                  int K, int KT, int epi, hipStream_t s, int xp, int yp, bool nt,
                                  int wpitch, const FuseArgs &fz) {
+  constexpr int U = 8;
   const int ntiles = (N + 15) / 16;
-  // FFMI_FZ_KW8 (A/B): 8 K-split waves instead of 4 for the one-row-tile
-  // consumer launches -- 1: qkv, 2: qkv and gate/up
+  // FFMI_FZ_KW8 (A/B): 8 K-split waves instead of 4 for the consumer launches
+  // -- 1: qkv, 2: qkv and gate/up
   static const int kw8 = getenv("FFMI_FZ_KW8") ? atoi(getenv("FFMI_FZ_KW8")) : 0;
   if (epi == FFMI_EPI_SILU_MUL) {
     if constexpr (FZ == 2) {
-      if (kw8 >= 2 && MT == 1)
-        return run<MT, 2, 8, U, 1, 2>(X, Wp, Y, nullptr, T, N, K, KT, 2 * ntiles, 1, s, xp, yp, nt,
-                                      wpitch, fz);
-      return run<MT, 2, 4, U, 1, 2>(X, Wp, Y, nullptr, T, N, K, KT, 2 * ntiles, 1, s, xp, yp, nt,
-                                    wpitch, fz);
+      if (kw8 >= 2)
+        return run<1, 2, 8, U, 1, 2>(X, Wp, Y, nullptr, T, N, K, KT, 2 * ntiles, 1, s, xp, yp, nt,
+                                     wpitch, fz);
+      return run<1, 2, 4, U, 1, 2>(X, Wp, Y, nullptr, T, N, K, KT, 2 * ntiles, 1, s, xp, yp, nt,
+                                   wpitch, fz);
     }
     return hipErrorInvalidValue;
   }
   if constexpr (FZ == 2)
-    if (kw8 >= 1 && MT == 1 && ntiles >= 512)
-      return run<MT, 1, 8, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
-  // FFMI_FZ_NT2=1: two tiles per workgroup at one row tile too (A/B)
+    if (kw8 >= 1 && ntiles >= 512)
+      return run<1, 1, 8, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
+  // FFMI_FZ_NT2=1: two tiles per workgroup (A/B)
   static const bool nt2 = getenv("FFMI_FZ_NT2") && atoi(getenv("FFMI_FZ_NT2")) != 0;
-  if ((MT >= 2 || nt2) && ntiles >= 512)
-    return run<MT, 2, 4, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
+  if (nt2 && ntiles >= 512)
+    return run<1, 2, 4, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
   if (ntiles < 512 && KT >= 64 && !nt)
-    return run<MT, 1, 8, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
-  return run<MT, 1, 4, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
+    return run<1, 1, 8, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
+  return run<1, 1, 4, U, 0, FZ>(X, Wp, Y, nullptr, T, N, K, KT, ntiles, 1, s, xp, yp, nt, wpitch, fz);
 }
 
 // E: the epilogue kind (1: paired tiles)
@@ -1711,22 +1712,15 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   if constexpr (E < 2)
   if (fuse && fuse->kind) {
     // producer: row-major residual out, plain epilogue; consumer: X is the
-    // residual, K = the norm width; both unsplit, T <= 32
-    if (mtiles > 2 || N % 16 || K % 32) return hipErrorInvalidValue;
+    // residual, K = the norm width; both unsplit, T <= 16
+    if (mtiles > 1 || N % 16 || K % 32) return hipErrorInvalidValue;
     if (fuse->kind == 1 && (paired || yp || !fuse->res_in || !fuse->ss_out || (fuse->res_packed && N % 32)))
       return hipErrorInvalidValue;
     if (fuse->kind == 2 && (!fuse->ss_in || !fuse->wnorm || fuse->nss <= 0 || fuse->nss > 256 || K > 4096))
       return hipErrorInvalidValue;
     const int wp = wpitch ? wpitch : (paired ? 2 : 1) * ((N + 15) / 16);
-#define FFMI_FZ(MTV, FZV) \
-  return dispatch_fused<MTV, 8, FZV>(X, Wp, Y, T, N, K, KT, paired, s, xp, yp, nt, wp, *fuse)
-    if (mtiles <= 1) {
-      if (fuse->kind == 1) FFMI_FZ(1, 1);
-      FFMI_FZ(1, 2);
-    }
-    if (fuse->kind == 1) FFMI_FZ(2, 1);
-    FFMI_FZ(2, 2);
-#undef FFMI_FZ
+    if (fuse->kind == 1) return dispatch_fused<1>(X, Wp, Y, T, N, K, KT, paired, s, xp, yp, nt, wp, *fuse);
+    return dispatch_fused<2>(X, Wp, Y, T, N, K, KT, paired, s, xp, yp, nt, wp, *fuse);
   }
   if constexpr (E == 4 || E == 5)
   if (fuse && fuse->kind) {

@@ -79,10 +79,12 @@ struct LlamaGPU : public ffmi_model {
   bool solo = false;  // TP shard over a 1-rank communicator without transport or RCCL
   // residual norms folded into the skinny GEMMs around them (T <= 16, TP = 1):
   // per-tile sums of squares of the residual after o (ss_o) and after down
-  // (ss_d), [32][H/16] each.  With more rows a wave norms its operands for two
-  // row tiles, and qkv and gate/up of H = 4096 at 24 and 32 rows take 69.8 and
-  // 74.0 us, as products of normed rows 57.0 and 59.7 (two norm launches: 6-7);
-  // of H = 2048 29.4 and 31.2 against 23.1 and 24.2.  Only where o/down run unsplit anyway (H/16 >=
+  // (ss_d), [16][H/16] each.  With more rows a wave would norm its operands for
+  // two row tiles: qkv and gate/up of H = 4096 at 24 and 32 rows took 69.8 and
+  // 74.0 us, as products of normed rows 57.0 and 59.7 (two norm launches: 6-7),
+  // of H = 2048 29.4 and 31.2 against 23.1 and 24.2; decode steps of 8 layers,
+  // 17, 24 and 32 requests, H = 4096 1078, 1135 and 1255 us against 1034, 1085
+  // and 1192, H = 2048 550, 583 and 632 against 553, 564 and 604.  Only where o/down run unsplit anyway (H/16 >=
   // 128 tiles: LLaMA-7B decode, +1.9% incr decoding -- the A/B of record is
   // profiles/r03_fused_norm_ab.log, quoted in DESIGN.md §5); the 68M SSM's
   // o/down split K over workgroups, and unsplitting them to fuse cost more
@@ -549,8 +551,8 @@ struct LlamaGPU : public ffmi_model {
     TRY(alloc(&qkv, (size_t)Tm * 3 * Hl));
     TRY(alloc(&att, (size_t)Tm * Hl));
     TRY(alloc(&proj, (size_t)Tm * H));
-    TRY(alloc(&ss_o, (size_t)2 * 32 * (H / 16)));
-    ss_d = ss_o + (size_t)32 * (H / 16);
+    TRY(alloc(&ss_o, (size_t)2 * 16 * (H / 16)));
+    ss_d = ss_o + (size_t)16 * (H / 16);
     TRY(alloc(&mlp, (size_t)Tm * Fl));
     fuse_ao = P == 1 && d == 64 && H <= 1024 && H % 16 == 0 &&
               !(getenv("FFMI_FUSE_AO") && atoi(getenv("FFMI_FUSE_AO")) == 0);

@@ -239,6 +239,8 @@ SIGNATURES = {
     "ffmi_debug_gemm_stamps": (ctypes.c_long, [c_void_p, ctypes.c_long]),
     "ffmi_debug_fused_residual_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                                                  c_int, c_int, c_void_p]),
+    "ffmi_debug_fused_residual_linear_packed": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                        c_int, c_int, c_int, c_int, c_void_p]),
     "ffmi_debug_fused_norm_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_float, c_void_p,
                                              c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "ffmi_debug_attn_stamps": (ctypes.c_long, [c_void_p, ctypes.c_long]),

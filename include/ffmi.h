@@ -649,16 +649,23 @@ ffmi_status ffmi_rm_get_stats(ffmi_rm *rm, ffmi_serve_stats *s);
 
 
 
-/* Test hooks: the residual RMSNorm folded into the decode GEMMs (T <= 32,
- * the path of LLaMA-7B decode steps; residual_rms_norm_kernels.cu:98-131
+/* Test hooks: the residual RMSNorm folded into the decode GEMMs (T <= 32 in
+ * pieces of 16, the path of LLaMA-7B decode steps; residual_rms_norm_kernels.cu:98-131
  * split over the GEMMs around it).  Producer: residual[T][out] += round(X .
  * W^T) in place (fp16 add) and ss_out[T][out/16] = per 16-column tile sums of
  * squares of the new residual.  Consumer: Y = (rmsnorm(residual) from ss_in
  * [T][in/16], weight norm_w, eps) . W^T, with the epilogue (FFMI_EPI_NONE /
- * FFMI_EPI_SILU_MUL, row-major).  Row-major fp16, no split-K. */
+ * FFMI_EPI_SILU_MUL, row-major).  Row-major fp16, no split-K.
+ * The packed form, as models run it (T <= 16): flags FFMI_X_PACKED, FFMI_W_STREAM, the
+ * new residual also in packed tiles (out a multiple of 32); the consumer reads them with
+ * FFMI_X_PACKED in `epilogue` (and FFMI_W_STREAM). */
 ffmi_status ffmi_debug_fused_residual_linear(const void *X, const void *W_packed, void *residual,
                                              float *ss_out, int T, int out_dim, int in_dim,
                                              ffmi_stream stream);
+ffmi_status ffmi_debug_fused_residual_linear_packed(const void *X, const void *W_packed,
+                                                    void *residual, void *residual_packed,
+                                                    float *ss_out, int T, int out_dim, int in_dim,
+                                                    int flags, ffmi_stream stream);
 ffmi_status ffmi_debug_fused_norm_linear(const void *residual, const float *ss_in,
                                          const void *norm_w, float eps, const void *W_packed,
                                          void *Y, int T, int out_dim, int in_dim, int epilogue,
