@@ -7,7 +7,9 @@ import ctypes
 import numpy as np
 import pytest
 
+import flexflow_amd as fa
 import flexflow_amd.ffmi as F
+import oracle_lib as O
 import test_gpu_kernels as K
 from hip_util import Buf
 from test_gpu_kernels import AttnCase
@@ -99,3 +101,28 @@ def test_attention_output_in_its_input(at):
     F.check(K.L.ffmi_attn_inc(c.h, c.b, buf.ptr, ctypes.c_void_p(buf.ptr.value + 4 * off), None))
     got = buf.get()[off:off + T * c.Hl].reshape(T, c.Hl)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("heads", [128, 129])
+def test_first_norm_of_wide_rows(heads):
+    """A step's first norm gathers the tokens' rows and brings the step's blob to the device; rows of
+    more than 8192 columns take a copy and the scalar kernel.  Steps of several requests, whose
+    tokens lie elsewhere in the blob; 2-norm within 8192 terms' roundings of 2^-24."""
+    cfg = dict(num_layers=1, vocab_size=64, num_heads=heads, num_kv_heads=heads, hidden=64 * heads, intermediate=32,
+               rms_eps=1e-6, rope_theta=10000.0)
+    m = fa.Model(cfg, "inc", max_requests=3, max_tokens=64, max_seq_len=64, weight_seed=11, full_precision=True)
+    rm = fa.RequestManager(max_requests_per_batch=3, max_tokens_per_batch=64, max_spec_tree_token_num=0,
+                           max_sequence_length=64)
+    ref = O.Model(cfg, 11, fp16=0, max_requests=3, max_seq=64)
+    rng = np.random.default_rng(heads)
+    toks, at, got = rng.integers(0, 64, (3, 40)), [0, 0, 0], [[], [], []]
+    for step in ((5, 0, 0), (1, 7, 0), (1, 1, 20), (1, 1, 1), (17, 1, 1)):
+        part = [(r + 1, toks[r][at[r]:at[r] + n], range(n)) for r, n in enumerate(step) if n]
+        rows = np.split(rm.replay_step(m, part), np.cumsum([n for n in step if n])[:-1])
+        for r in (r for r in range(3) if step[r]):
+            got[r].append(rows.pop(0))
+            at[r] += step[r]
+    for r in range(3):
+        want = ref.forward(r, toks[r][:at[r]].astype(np.int32), 0)
+        d = np.linalg.norm(np.concatenate(got[r]) - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert (d <= 8192 ** 0.5 * 2.0 ** -24 * 4).all(), d.max()
