@@ -1786,10 +1786,13 @@ static hipError_t launch_gemm_kind(const uint16_t *X, const uint16_t *Wp, uint16
   else if (mtiles <= 2) e = dispatch_nt<E, 2, 8>(X, Wp, Y, ws, T, N, K, KT, S, s, xi, yp, nt, wpitch, fz);
   else if (mtiles <= 3) {
     // 33 to 48 rows, cold, as four row tiles, three in batches of four k-steps and of eight:
-    // 6432 x 2048 11.5 us, 11.3, 10.8; 2048 x 4096 10.7, 10.5, 10.0; 4096 x 11008 25.4,
-    // 24.8, 24.5; 768 x 3072 (fewer than eight k-steps a wave) 6.7, 5.9, 6.8; two tiles a
-    // workgroup: 32000 x 4096 57.3, 53.5, 54.5, gate and up of 11008 x 4096 42.2, 39.1, 40.1
-    const bool eight = !paired && (N + 15) / 16 < 512 && (KT + S - 1) / S >= 32;
+    // 6432 x 2048 11.5 us, 11.3, 10.8; 2048 x 4096 10.7, 10.5, 10.0; 768 x 3072 (fewer than eight k-steps a
+    // wave) 6.7, 5.9, 6.8; two tiles a workgroup: 32000 x 4096 57.3, 53.5, 54.5, gate and up of
+    // 11008 x 4096 42.2, 39.1, 40.1.  A rest of a batch of eight is worth a batch (a wave's k-steps
+    // in brackets): 3072 x 1536 (12) 5.7, 5.4, 6.1; 6144 x 3072 (12) 17.3, 16.0, 17.5; 6144 x 5632
+    // (22) 26.0, 23.9, 27.7.
+    const int waves = (KT + S - 1) / S >= 64 && !nt ? 8 : 4, mine = ((KT + S - 1) / S + waves - 1) / waves;
+    const bool eight = !paired && (N + 15) / 16 < 512 && mine >= 8 && mine % 8 == 0;
     if (eight) e = dispatch_nt<E, 3, 8>(X, Wp, Y, ws, T, N, K, KT, S, s, xi, yp, nt, wpitch, fz);
     else e = dispatch_nt<E, 3, 4>(X, Wp, Y, ws, T, N, K, KT, S, s, xi, yp, nt, wpitch, fz);
   }

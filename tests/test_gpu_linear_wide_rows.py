@@ -37,7 +37,7 @@ def test_rows(n, k, hint):
 
 
 @pytest.mark.parametrize("n,k,epi,hint", [(6432, 2048, 0, F.W_STREAM), (2048, 4096, 0, 0), (2048, 1056, 0, 0),
-                                          (768, 3072, 0, 0), (8200, 1056, 0, 0), (2304, 768, 1, 0), (16400, 992, 0, 0)])
+                                          (768, 3072, 0, 0), (3072, 1536, 0, 0), (520, 2816, 0, 0), (8200, 1056, 0, 0), (2304, 768, 1, 0), (16400, 992, 0, 0)])
 def test_rows_of_three_tiles(n, k, epi, hint):
     """33 to 48 rows have a form of their own; a row's sums are those of 64."""
     L = K.L
