@@ -195,11 +195,12 @@ hipError_t launch_attention_f32(const char *blob, int T, const float *qbuf, cons
 hipError_t launch_update_attention_f32(const char *blob, int T, int C, const float *qkv, const float *rope,
                                        int max_rope_pos, float *qbuf, float *kc, float *vc, float *stage, float *out,
                                        int heads, int d, int slots, float scale, bool distinct, hipStream_t s);
-// rows ids.row[0, n) of logits [.][ld] (fp16 or fp32) as fp32 to dst [n][V]; row i is there
+// rows ids.row[0, n) of logits [.][ld] (fp16 or fp32) as fp32 to dst [n][pitch(V)]; row i is there
 // when there[i * kParts + p] == mark for every p < parts(V).  dst and there: mapped host memory
 struct LogitRowIds {
   static constexpr int kMax = 16, kParts = 32;
   static int parts(int V) { return V > 1024 * kParts ? kParts : (V + 1023) / 1024; }
+  __host__ __device__ static size_t pitch(int V) { return ((size_t)V + 3) & ~(size_t)3; }
   int row[kMax];
 };
 hipError_t launch_logit_rows(const void *logits, bool half, size_t ld, const LogitRowIds &ids, int n, int V,

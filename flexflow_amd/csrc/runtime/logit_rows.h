@@ -39,12 +39,12 @@ class LogitRows {
       FFMI_HIP(hipHostMalloc((void **)&there_, bytes, hipHostMallocCoherent | hipHostMallocMapped));
       memset(there_, 0, bytes);
     }
-    if (staged_ < (size_t)V) {
+    if (staged_ < LogitRowIds::pitch(V)) {
       if (staging_) (void)hipHostFree(staging_);
       staging_ = nullptr, staged_ = 0;
-      FFMI_HIP(hipHostMalloc((void **)&staging_, (size_t)2 * kRows * V * sizeof(float),
+      FFMI_HIP(hipHostMalloc((void **)&staging_, 2 * kRows * LogitRowIds::pitch(V) * sizeof(float),
                              hipHostMallocCoherent | hipHostMallocMapped));
-      staged_ = V;
+      staged_ = LogitRowIds::pitch(V);
     }
     for (auto &e : done_)
       if (!e) FFMI_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -84,8 +84,13 @@ class LogitRows {
         const ffmi_status st = await(half, i, mark);
         if (st != FFMI_OK) return st;
         for (to = i + 1; to < here && there(half, to, mark);) ++to;
-        memcpy(out_ + (size_t)(at + i) * V_, staging_ + ((size_t)half * kRows + i) * V_,
-               (size_t)(to - i) * V_ * sizeof(float));
+        const size_t pitch = LogitRowIds::pitch(V_);
+        const float *from = staging_ + ((size_t)half * kRows + i) * pitch;
+        if (pitch == (size_t)V_) {
+          memcpy(out_ + (size_t)(at + i) * V_, from, (to - i) * pitch * sizeof(float));
+        } else {
+          for (int k = i; k < to; ++k, from += pitch) memcpy(out_ + (size_t)(at + k) * V_, from, V_ * sizeof(float));
+        }
       }
       if (at + kRows >= n) break;
     }
@@ -125,7 +130,8 @@ class LogitRows {
     LogitRowIds ids;
     const int n = std::min(kRows, all - at);
     for (int i = 0; i < n; ++i) ids.row[i] = rows_ ? rows_[at + i] : at + i;
-    FFMI_HIP(launch_logit_rows(src_, half_, ld_, ids, n, V_, staging_ + (size_t)half * kRows * V_,
+    FFMI_HIP(launch_logit_rows(src_, half_, ld_, ids, n, V_,
+                               staging_ + (size_t)half * kRows * LogitRowIds::pitch(V_),
                                there_ + (size_t)half * kRows * LogitRowIds::kParts, ++mark_, stream_));
     FFMI_HIP(hipEventRecord(done_[half], stream_));
     return FFMI_OK;

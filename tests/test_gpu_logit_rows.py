@@ -4,6 +4,7 @@ no multiple of the kernel's vectors, against the same rows one step at a time.""
 import os
 import subprocess
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -77,3 +78,26 @@ def test_a_long_step_is_waited_for_as_asked(kind):
     assert r.returncode == 0, r.stderr[-2000:]
     print(r.stdout)
     assert "not applied" not in r.stderr and float(r.stdout.split("share")[1].split()[0]) < 0.75, r.stdout
+
+
+def fastest(vocab, rows, times=25):
+    m = fa.Model(dict(LLAMA, vocab_size=vocab), "inc", max_requests=1, max_tokens=256, max_seq_len=256, weight_seed=5)
+    rm = fa.RequestManager(max_requests_per_batch=1, max_tokens_per_batch=256, max_spec_tree_token_num=0,
+                           max_sequence_length=256)
+    best, toks = 1e9, np.arange(max(rows, 4), dtype=np.int32)
+    for i in range(times):
+        t = time.perf_counter()
+        rm.replay_step(m, [(i + 1, toks, range(rows))])
+        best = min(best, time.perf_counter() - t)
+        rm.replay_end(m, i + 1)
+    return best
+
+
+def test_odd_and_short_rows_arrive_as_fast():
+    """Rows that are no whole pieces of 16 bytes, and short ones, which lie in one workgroup: 48 rows of
+    33001 take as long as of 33000 (3 times so in single words), 200 of 1000 less than five steps of
+    one row (6.5 one after the other)."""
+    odd, even = fastest(33001, 48), fastest(33000, 48)
+    one, many = fastest(1000, 1), fastest(1000, 200)
+    print("us", *(round(t * 1e6) for t in (odd, even, one, many)))
+    assert odd < 1.6 * even and many < 5 * one
