@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """LLaMA-7B SpecInfer (LLaMA-68M SSM) decoded tokens/s on MI355X.
 
-Workload (BASELINE.json metric / SURVEY.md §8d): 8 requests, prompt = BOS +
+Workload: 8 requests, prompt = BOS +
 127 ids (splitmix64, seed 20250117), 128 decoded tokens each (max_length
 256), max_tokens_per_batch 1024, max_spec_tree_token_num 23, tree widths
 (1,1,3), 8 SSM steps per verify; synthetic seeded weights (no checkpoints

@@ -1056,8 +1056,8 @@ hipError_t launch_softmax_topk_f32(const float *logits, int T, int V, int k, int
 // the other, and one that has written its columns of a row says so in a word of its own,
 // there[row][blockIdx.x] = mark (no counters to clear, no workgroup waits for another).
 // Up to 32 workgroups a row; short rows side by side, 32 workgroups in all (200 rows of 1000
-// one after the other: whole steps 393 us, so 222).  Rows of dst are whole pieces of four,
-// whatever V is (200 rows of 33001 in single words: 3290 us, so 1120).
+// one after the other: whole steps 393 us, so 173).  Rows of dst are whole pieces of four,
+// whatever V is (200 rows of 33001 in single words: 3290 us, so 870).
 // With rows shared out over 2, 4 and 16 groups of workgroups they end later than one after
 // the other: 24 decode steps of 8 rows of 32000, whole steps, 22.15 ms in one group, 22.18 in
 // two, 22.40 and 22.53 in four and 16 (all rows copied after the kernel: 23.0).

@@ -321,6 +321,7 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a,
 //   36 x 2048           8.8  8.8             10.8  9.4       11.9  9.4
 //   64 x 2048           8.8  9.5             10.8 10.1       11.9 10.2
 //   64 x 4096           9.5 11.9             11.8 12.5       13.2 12.9
+// (Narrow rows leave waves without a slice: a layer of 36 x 512 with 38 tokens 44.9 and 41.2.)
 // Above 64 tokens the router's product is another kernel with other sums, which close calls
 // of the experts would show.  (A slice of 64 k-steps and more would be cut in 8: only where
 // FFMI_SKINNY_SPLIT=0 leaves K whole.)

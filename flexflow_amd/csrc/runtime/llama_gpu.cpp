@@ -84,9 +84,9 @@ struct LlamaGPU : public ffmi_model {
   // 74.0 us, as products of normed rows 57.0 and 59.7 (two norm launches: 6-7),
   // of H = 2048 29.4 and 31.2 against 23.1 and 24.2; decode steps of 8 layers,
   // 17, 24 and 32 requests, H = 4096 1078, 1135 and 1255 us against 1034, 1085
-  // and 1192, H = 2048 550, 583 and 632 against 553, 564 and 604.  Only where o/down run unsplit anyway (H/16 >=
-  // 128 tiles: LLaMA-7B decode, +1.9% incr decoding -- the A/B of record is
-  // profiles/r03_fused_norm_ab.log, quoted in DESIGN.md §5); the 68M SSM's
+  // and 1192, H = 2048 550, 583 and 632 against 553, 564 and 604.  Only
+  // where o/down run unsplit anyway (H/16 >= 128 tiles: LLaMA-7B decode,
+  // +1.9% incr decoding); the 68M SSM's
   // o/down split K over workgroups, and unsplitting them to fuse cost more
   // than the norm launches saved (SSM step +4 us).  FFMI_FUSE_NORM: 0 off,
   // 1 auto (default), 2 every width (tests)

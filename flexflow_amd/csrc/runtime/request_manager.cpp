@@ -1,7 +1,7 @@
 // request_manager.cpp -- continuous batching and the SpecInfer token-tree
 // scheduler, restated from src/runtime/request_manager.cc (reference
 // @2025-01-17).  Each function cites the reference lines whose behaviour it
-// reproduces.  Deliberate differences (documented in DESIGN.md):
+// reproduces.  Deliberate differences:
 //  * bit operations on BitMask words are 64-bit (1ull << j); the reference's
 //    `1 << j` on int breaks for trees deeper than 31 tokens (quirk 6);
 //  * no tokenizer: requests carry token ids (the parity unit);
