@@ -266,6 +266,23 @@ struct FuseArgs {
   float limit = 0.f;                // clamped gated unit (bf16 paired tiles)
   int y_width = 0;                  // packed output: width of the rows Y is part of (0: N)
 };
+// A product whose rows are the residual norm of another one's slabs, made in its prologue:
+// r = res_in + half(sum of the S slabs [S][T][NP]) -> res_out (another buffer: every
+// workgroup reads res_in), X = half(half(r * rms) * wnorm).  T <= 2 rows of up to 1024
+// columns, S <= 16.
+struct SumNormArgs {
+  const uint16_t *res_in;  // [T][K]
+  const float *sums;
+  int S, NP;
+  const uint16_t *wnorm;  // [K]
+  uint16_t *res_out;      // [T][K]
+  float eps;
+};
+// whether launch_gemm_sum_norm takes a product (else the norm is a launch of its own)
+bool gemm_sum_norm_fits(int T, int N, int K, int epilogue, const Partials &sums);
+// Y = X.W^T, the bits of launch_rmsnorm and launch_gemm
+hipError_t launch_gemm_sum_norm(const SumNormArgs &a, const uint16_t *Wp, uint16_t *Y, int T, int N, int K,
+                                int epilogue, hipStream_t s);
 // g = min(gate, limit), u = up within +-limit: g sigmoid(1.702 g) (u + 1)
 __device__ __forceinline__ float clamped_glu(float gate, float up, float limit) {
   const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
@@ -333,6 +350,7 @@ hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t
                           const int32_t *rows = nullptr, int T_in = 0);
 // FFMI_FAULT_RESID_ROUND negative control (tests only; process-wide)
 void set_norm_fault(bool on);
+bool norm_fault();
 hipError_t launch_embedding(const char *blob, int T, const uint16_t *table,
                             uint16_t *out, int H, hipStream_t s);
 hipError_t launch_silu_mul(const uint16_t *a, const uint16_t *b, uint16_t *out,

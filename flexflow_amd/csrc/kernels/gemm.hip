@@ -32,6 +32,55 @@ hipError_t launch_gemm(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float
   return launch_gemm_kind<0>(X, Wp, Y, ws, ws_bytes, T, N, K, epilogue, s, defer, wpitch, fuse);
 }
 
+// FFMI_SUM_NORM=0: the norm is a launch of its own (A/B, tests; read per call)
+bool gemm_sum_norm_fits(int T, int N, int K, int epilogue, const Partials &sums) {
+  const char *e = getenv("FFMI_SUM_NORM");
+  const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
+  if (norm_fault() || (e && !atoi(e)) || T < 1 || T > kSumNormRows || N < 1 || K > kSumNormWidth || K % 32) return false;
+  if (sums.S < 1 || sums.S > (paired ? 16 : 8) || sums.NP < K || sums.NP % 4) return false;
+  // (its slabs could lie where it would write its own)
+  return paired || skinny_split(T, N, K, 0, true) == 1;
+}
+
+hipError_t launch_gemm_sum_norm(const SumNormArgs &a, const uint16_t *Wp, uint16_t *Y, int T, int N, int K,
+                                int epilogue, hipStream_t s) {
+  if (!gemm_sum_norm_fits(T, N, K, epilogue, Partials{a.sums, a.S, a.NP}) || a.res_in == a.res_out)
+    return hipErrorInvalidValue;
+  const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
+  const bool nt = (epilogue & FFMI_W_STREAM) != 0;
+  const int KT = K / 32, ntiles = (N + 15) / 16, yp = epilogue & FFMI_Y_PACKED ? N : 0;
+  if (yp && N % 32) return hipErrorInvalidValue;
+  const size_t wts = w_tile_stride(KT), wks = w_k_stride(paired ? 2 * ntiles : ntiles);
+  float *none = nullptr;
+  const uint16_t *x = nullptr;
+#define FFMI_MADE(NT, E, NL, FZ)                                                                                  \
+  hipLaunchKernelGGL((gemm_skinny_kernel<1, NT, 4, 8, E, false, NL, FZ>), dim3(ntiles), dim3(256),                \
+                     3 * NT * 4 * 64 * sizeof(float), s, x, Wp, Y, none, T, N, K, KT, NT * ntiles, 1, yp, wts, wks, a)
+#define FFMI_MADE_NL(NT, E, FZ)          \
+  do {                                   \
+    if (nt) FFMI_MADE(NT, E, true, FZ);  \
+    else FFMI_MADE(NT, E, false, FZ);    \
+  } while (0)
+  if (paired) {
+    if (a.S <= 8) FFMI_MADE_NL(2, 1, 5);
+    else if (a.S <= 12) FFMI_MADE_NL(2, 1, 6);
+    else FFMI_MADE_NL(2, 1, 7);
+  } else if (ntiles >= 1024) {  // (the wave kernel's, as in dispatch_nt)
+    const dim3 grid(((ntiles + 1) / 2 + 3) / 4);
+    if (nt)
+      hipLaunchKernelGGL((gemm_wave_kernel<1, 2, 4, true, 4, 0, true>), grid, dim3(256), 0, s, x, Wp, Y, none, T, N,
+                         KT, ntiles, 1, yp, wts, wks, a);
+    else
+      hipLaunchKernelGGL((gemm_wave_kernel<1, 2, 4, false, 4, 0, true>), grid, dim3(256), 0, s, x, Wp, Y, none, T, N,
+                         KT, ntiles, 1, yp, wts, wks, a);
+  } else {
+    FFMI_MADE_NL(1, 0, 5);
+  }
+#undef FFMI_MADE_NL
+#undef FFMI_MADE
+  return hipGetLastError();
+}
+
 int gemm_tile_form(int T, int N, int K, int epilogue, int *slices) {
   const bool paired = (epilogue & ~(FFMI_X_PACKED | FFMI_Y_PACKED | FFMI_W_STREAM)) == FFMI_EPI_SILU_MUL;
   *slices = 1;

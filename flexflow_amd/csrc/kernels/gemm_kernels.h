@@ -114,9 +114,75 @@ __device__ __forceinline__ float lane_f(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
+// The operand rows of a product behind a residual norm, made by every workgroup for
+// itself (SumNormArgs): r = residual + half(sum of slabs), h = half(half(r * rms) * w),
+// the norm kernel's arithmetic and order of sums (norm.hip: 128 threads a row).  The first
+// workgroup of the grid stores r.  load() only asks for the two rows, so that the caller's
+// weight loads go out behind it and their way hides the sums.
+// Bound by latency: slabs, a barrier for the sum of squares and one for the rows, about
+// 1.3 us more than the product alone, where the norm's launch took 3 and its boundary.  A
+// model of 768 channels and 2 layers, 16 steps of one row 1434 -> 1381 us, of two 1484 ->
+// 1416.  Three and four rows are two rounds of slabs in every workgroup: 1512 -> 1514 and 1517 ->
+// 1526, so those keep their launches.
+constexpr int kSumNormRows = 2;      // rows at most
+constexpr int kSumNormWidth = 1024;  // columns at most
+template <int MAXS>
+struct SumNormRows {
+  f4 lo[MAXS], hi[MAXS];
+  uint4 x, w;
+  __device__ __forceinline__ void load(const SumNormArgs &a, int T, int H) {
+    const int row = min((int)(threadIdx.x >> 7), T - 1), ch = min((int)threadIdx.x & 127, (H >> 3) - 1);
+    const float *q = a.sums + (size_t)row * a.NP + ch * 8;
+#pragma unroll
+    for (int s = 0; s < MAXS; ++s) {
+      const float *qs = q + (size_t)min(s, a.S - 1) * T * a.NP;
+      lo[s] = *reinterpret_cast<const f4 *>(qs);
+      hi[s] = *reinterpret_cast<const f4 *>(qs + 4);
+    }
+    x = *reinterpret_cast<const uint4 *>(a.res_in + (size_t)row * H + ch * 8);
+    w = *reinterpret_cast<const uint4 *>(a.wnorm + ch * 8);
+  }
+  // rows: LDS, complete behind the last barrier in here
+  __device__ __forceinline__ void finish(const SumNormArgs &a, int T, int H,
+                                         uint16_t (*rows)[kSumNormWidth + 8], bool store) {
+    __shared__ double part[4];
+    const int wave = threadIdx.x >> 6, row = threadIdx.x >> 7, ch = threadIdx.x & 127;
+    const bool mine = ch < (H >> 3), real = mine && row < T;
+#pragma unroll
+    for (int s = 1; s < MAXS; ++s)
+      if (s < a.S) lo[0] += lo[s], hi[0] += hi[s];
+    union Row8 {
+      uint4 v;
+      _Float16 e[8];
+    } r, wn, y;
+    r.v = x, wn.v = w;
+    double ss = 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      r.e[q] = r.e[q] + (_Float16)(q < 4 ? lo[0][q] : hi[0][q - 4]);
+      const float f = (float)r.e[q];
+      if (mine) ss += (double)f * (double)f;
+    }
+    if (store && real) *reinterpret_cast<uint4 *>(a.res_out + (size_t)row * H + ch * 8) = r.v;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    if ((threadIdx.x & 63) == 0) part[wave] = ss;
+    __syncthreads();
+    const float sum = (float)(part[wave & ~1] + part[wave | 1]);
+    const float rms =
+        (float)(_Float16)__fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, (float)H), a.eps)));
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      y.e[q] = (_Float16)__fmul_rn((float)(_Float16)__fmul_rn((float)r.e[q], rms), (float)wn.e[q]);
+    if (real) *reinterpret_cast<uint4 *>(&rows[row][ch * 8]) = y.v;
+    __syncthreads();
+  }
+};
+
 // FZ (FuseArgs, ffmi_internal.h): 1 = residual-add producer epilogue (EPI 0,
 // unsplit), 2 = RMSNorm consumer prologue, 3 and 4 = the pair of an fp32 residual
-// (EPI 4; EPI 4 and 5).  Y is restrict-
+// (EPI 4; EPI 4 and 5), 5 to 7 = rows made from slabs and residual in the prologue, of up
+// to 8, 12 and 16 slabs (SumNormArgs; one row tile, KW 4).  Y is restrict-
 // qualified except in the producer, where it aliases fz.res_in (the residual
 // is updated in place).
 template <int FZ>
@@ -126,7 +192,9 @@ struct PlainArgs {
   float limit;
 };
 template <int FZ>
-using SkinnyArgs = std::conditional_t<FZ != 0, FuseArgs, PlainArgs>;
+using SkinnyArgs = std::conditional_t<FZ >= 5, SumNormArgs, std::conditional_t<FZ != 0, FuseArgs, PlainArgs>>;
+template <int FZ>
+constexpr int sum_norm_slabs = FZ == 5 ? 8 : FZ == 6 ? 12 : FZ == 7 ? 16 : 0;
 template <int MT, int NT, int KW, int U, int EPI, bool PIPE = false, bool NTL = false, int FZ = 0>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wp,
@@ -135,6 +203,12 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  // FZ >= 5: the rows' loads go out first, the sums wait for them behind the first weights'
+  constexpr bool MAKE = FZ >= 5;
+  static_assert(!MAKE || (MT == 1 && KW == 4 && !PIPE), "256 threads: two rows; a short K");
+  __shared__ __attribute__((aligned(16))) uint16_t sRows[MAKE ? kSumNormRows : 1][MAKE ? kSumNormWidth + 8 : 8];
+  SumNormRows<MAKE ? sum_norm_slabs<FZ> : 1> made;
+  if constexpr (MAKE) made.load(fz, T, K);
   // FZ == 1: the residual this wave-0 epilogue adds, loaded up front
   _Float16 rpre[FZ == 1 ? MT : 1][FZ == 1 ? NT : 1][4];
   if constexpr (FZ == 1) {
@@ -189,7 +263,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   constexpr int WPT = FZ == 2 ? 4096 / 8 / (KW * 64) : 1;
   __shared__ h8 sWn[FZ == 2 ? 4096 / 8 : 1];
   h8 wpre[WPT];
-  bool rdone = FZ != 2;
+  bool rdone = FZ != 2 && !MAKE;
   if constexpr (FZ == 2) {
 #pragma unroll
     for (int c = 0; c < WPT; ++c)
@@ -230,6 +304,11 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
   // test_gpu_kernels.py::test_fused_norm_consumer_empty_wave_ranges (KW 4 /
   // 8 with waves that own no k-step).
   auto rms_finish = [&]() {
+    if constexpr (MAKE) {
+      if (rdone) return;
+      rdone = true;
+      made.finish(fz, T, K, sRows, blockIdx.x == 0 && blockIdx.y == 0);
+    }
     if constexpr (FZ == 2) {
       if (rdone) return;
       rdone = true;
@@ -286,6 +365,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
       xrow[i] = X + (size_t)r * K + 8 * (lane >> 4);
     }
   }
+  // (FZ >= 5: from LDS, behind rms_finish)
+  const uint16_t *made_row = &sRows[MAKE ? min(lane & 15, T - 1) : 0][MAKE ? 8 * (lane >> 4) : 0];
   const uint16_t *wrow[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
@@ -368,12 +449,16 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
 #pragma unroll
       for (int j = 0; j < NT; ++j)
         b[u][j] = ld_weight<NTL>(wrow[j] + (size_t)(kt + u) * wks);
+    if constexpr (!MAKE)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-        a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)(kt + u) * XS);
+        for (int i = 0; i < MT; ++i)
+          a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)(kt + u) * XS);
     rms_finish();
+    if constexpr (MAKE)
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[u][0] = *reinterpret_cast<const h8 *>(made_row + (kt + u) * 32);
     // keep the whole batch of loads ahead of the MFMAs: left alone the
     // scheduler interleaves them and reuses registers, leaving ~7 loads in
     // flight per wave with a vmcnt wait before almost every MFMA
@@ -407,11 +492,16 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
 #pragma unroll
       for (int j = 0; j < NT; ++j)
         b[u][j] = ld_weight<NTL>(wrow[j] + (size_t)kk * wks);
+      if constexpr (!MAKE)
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-        a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)kk * XS);
+        for (int i = 0; i < MT; ++i)
+          a[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)kk * XS);
     }
     rms_finish();
+    if constexpr (MAKE)
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        a[u][0] = *reinterpret_cast<const h8 *>(made_row + min(kt + u, ke - 1) * 32);
     __builtin_amdgcn_sched_barrier(0);
     const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (FZ == 2)
@@ -572,6 +662,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
     }
   } else {
     // tiles (2p, 2p+1) = (gate, up) of output columns [16p, 16p+16)
+    float lim = 0.f;
+    if constexpr (!MAKE) lim = fz.limit;
     int n = cb * 16 + (lane & 15);
     if (n < N) {
 #pragma unroll
@@ -581,7 +673,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(
           int m = m0 + i * 16 + (lane >> 4) * 4 + r;
           if (m >= T) continue;
           Y[yp ? act_packed_off(m, n, yp) : (size_t)m * N + n] =
-              pair16<EPI>(acc[i][0][r], acc[i][1][r], fz.limit);
+              pair16<EPI>(acc[i][0][r], acc[i][1][r], lim);
         }
     }
   }
@@ -620,22 +712,32 @@ static hipError_t run(const uint16_t *X, const uint16_t *Wp, uint16_t *Y, float 
   return hipGetLastError();
 }
 
+struct NoArgs {};
+template <bool MAKE>
+using WaveArgs = std::conditional_t<MAKE, SumNormArgs, NoArgs>;
 // Wide, short-K layers (the 68M SSM's lm_head: 2000 tiles, K = 768): one
 // WAVE per group of NT tiles over the whole K (a single MFMA chain per tile,
 // no cross-wave reduction, no LDS), four independent waves per workgroup.
 // The K-split form launches 1000 short 4-wave workgroups whose loads never
 // fill the CU (13 us for 49 MB from the Infinity Cache); here each wave keeps
 // two batches of UB k-steps in flight (double-buffered registers).
-template <int MT, int NT, int UB, bool NTL, int WPG = 4, int EPI = 0>
+// MAKE: X's rows are made in the prologue (SumNormRows, up to 8 slabs), the wave's first
+// weights asked for ahead of the sums.
+template <int MT, int NT, int UB, bool NTL, int WPG = 4, int EPI = 0, bool MAKE = false>
 __global__ __launch_bounds__(WPG * 64) void gemm_wave_kernel(const uint16_t *__restrict__ X,
                                                              const uint16_t *__restrict__ Wp,
                                                              uint16_t *__restrict__ Y,
                                                              float *__restrict__ Yf, int T, int N,
                                                              int KT, int NTILES, int xp, int yp,
-                                                             size_t wts, size_t wks) {
+                                                             size_t wts, size_t wks, WaveArgs<MAKE> a) {
+  static_assert(!MAKE || (MT == 1 && WPG == 4), "256 threads: two rows");
   const int lane = threadIdx.x & 63;
   const int g = blockIdx.x * WPG + (threadIdx.x >> 6);
-  if (g * NT >= NTILES) return;
+  __shared__ __attribute__((aligned(16))) uint16_t sRows[MAKE ? kSumNormRows : 1][MAKE ? kSumNormWidth + 8 : 8];
+  SumNormRows<MAKE ? 8 : 1> made;
+  const uint16_t *made_row = &sRows[MAKE ? min(lane & 15, T - 1) : 0][MAKE ? 8 * (lane >> 4) : 0];
+  if constexpr (MAKE) made.load(a, T, KT * 32);
+  else if (g * NT >= NTILES) return;
   const int XS = xp ? 512 : 32;
   const uint16_t *xrow[MT];
 #pragma unroll
@@ -664,13 +766,15 @@ __global__ __launch_bounds__(WPG * 64) void gemm_wave_kernel(const uint16_t *__r
 #pragma unroll
       for (int j = 0; j < NT; ++j) bb[u][j] = ld_weight<NTL>(wrow[j] + (size_t)kk * wks);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) xx[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)kk * XS);
+      for (int i = 0; i < MT; ++i)
+        if constexpr (!MAKE) xx[u][i] = *reinterpret_cast<const h8 *>(xrow[i] + (size_t)kk * XS);
     }
   };
   const h8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   auto mm = [&](h8(&bb)[UB][NT], h8(&xx)[UB][MT], int k0) {
 #pragma unroll
     for (int u = 0; u < UB; ++u) {
+      if constexpr (MAKE) xx[u][0] = *reinterpret_cast<const h8 *>(made_row + min(k0 + u, KT - 1) * 32);
       if (k0 + u >= KT) {  // past K: re-loaded fragments times a zero weight
 #pragma unroll
         for (int j = 0; j < NT; ++j) bb[u][j] = zero;
@@ -683,6 +787,10 @@ __global__ __launch_bounds__(WPG * 64) void gemm_wave_kernel(const uint16_t *__r
     }
   };
   ld(bA, xA, 0);
+  if constexpr (MAKE) {
+    made.finish(a, T, KT * 32, sRows, blockIdx.x == 0);
+    if (g * NT >= NTILES) return;
+  }
   for (int k0 = 0; k0 < KT; k0 += 2 * UB) {
     if (k0 + UB < KT) ld(bB, xB, k0 + UB);
     __builtin_amdgcn_sched_barrier(0);
@@ -824,7 +932,7 @@ static hipError_t dispatch_nt(const uint16_t *X, const uint16_t *Wp, uint16_t *Y
 #define FFMI_WAVE(NTV, WPGV, NL)                                                               \
   hipLaunchKernelGGL((gemm_wave_kernel<MT, NTV, 4, NL, WPGV, E>),                              \
                      dim3(((ntiles + NTV - 1) / NTV + WPGV - 1) / WPGV), dim3(WPGV * 64), 0, s, X, \
-                     Wp, Y, ws, T, N, KT, ntiles, xp, yp, wts, wks)
+                     Wp, Y, ws, T, N, KT, ntiles, xp, yp, wts, wks, NoArgs())
     if constexpr (E >= 2) {
       if (nt) FFMI_WAVE(2, 4, true);
       else FFMI_WAVE(2, 4, false);

@@ -235,6 +235,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
 // faulted variants (SRC 4 / 5)
 static bool g_norm_fault = false;
 void set_norm_fault(bool on) { g_norm_fault = on; }
+bool norm_fault() { return g_norm_fault; }
 
 hipError_t launch_rmsnorm(const uint16_t *x1, const uint16_t *x2, const uint16_t *w,
                           uint16_t *res_out, uint16_t *out, int T, int H, float eps,

@@ -56,7 +56,7 @@ struct LlamaGPU : public ffmi_model {
   std::vector<Layer> layers;
   uint16_t *embed = nullptr, *final_norm = nullptr, *lm = nullptr;
   // activations
-  uint16_t *res = nullptr, *h = nullptr, *qkv = nullptr, *att = nullptr, *proj = nullptr,
+  uint16_t *res = nullptr, *res2 = nullptr, *h = nullptr, *qkv = nullptr, *att = nullptr, *proj = nullptr,
            *mlp = nullptr, *logits = nullptr;
   int32_t *ids_d = nullptr;
   // softmax top-k workspace (the split-row form for small steps; zeroed once)
@@ -547,6 +547,7 @@ struct LlamaGPU : public ffmi_model {
   do { if ((st = (x)) != FFMI_OK) return st; } while (0)
     TRY(ffmi_batch_create(Tm, o.max_requests, &batch));
     TRY(alloc(&res, (size_t)Tm * H));
+    if (H <= 1024) TRY(alloc(&res2, (size_t)2 * H));  // (SumNormArgs)
     TRY(alloc(&h, (size_t)Tm * H));
     TRY(alloc(&qkv, (size_t)Tm * 3 * Hl));
     TRY(alloc(&att, (size_t)Tm * Hl));
@@ -1129,6 +1130,19 @@ struct LlamaGPU : public ffmi_model {
     const bool fuse = fused_norms(T);
     // the residual norms inside the transport's all-reduces (tp_fuse_norm)
     const bool arn = peer && !solo && o.tp_size > 1 && (tp_fuse_norm == 2 || (tp_fuse_norm == 1 && !dbg));
+    // The residual: a norm in a product's prologue leaves the new one in the other buffer.
+    uint16_t *rs = res, *rs_to = res2;
+    // the norm of the slabs `part` rides in the launch of the product behind it
+    auto takes_norm = [&](const ffmi::Partials &part, int N, int epi) {
+      return rs_to && !fuse && !arn && !dbg && o.tp_size == 1 && ffmi::gemm_sum_norm_fits(T, N, H, epi, part);
+    };
+    auto norm_gemm = [&](const ffmi::Partials &part, const uint16_t *wn, const uint16_t *W, uint16_t *Y, int N,
+                         int epi) -> ffmi_status {
+      FFMI_HIP(ffmi::launch_gemm_sum_norm(ffmi::SumNormArgs{rs, part.p, part.S, part.NP, wn, rs_to, eps}, W, Y, T, N,
+                                          H, epi, stream));
+      std::swap(rs, rs_to);
+      return FFMI_OK;
+    };
     for (int l = 0; l < c.num_layers; ++l) {
       Layer &L = layers[l];
       const bool on = prof_on(l, T);
@@ -1160,11 +1174,12 @@ struct LlamaGPU : public ffmi_model {
         fz_qkv.wnorm = L.in_norm, fz_gu.wnorm = L.post_norm;
         fz_qkv.eps = fz_gu.eps = eps;
       }
-      if (!fz_in && !(arn && l > 0)) {  // (arn: the previous down all-reduce normalised)
+      const bool nq = l > 0 && takes_norm(down_part, 3 * Hl, XP);
+      if (!nq && !fz_in && !(arn && l > 0)) {  // (arn: the previous down all-reduce normalised)
         pr = prof_begin(on);
         // layer 0: the embedding lookup gathers straight into the first norm
         // (embedding_kernels.cu:233-244; res = the looked-up rows)
-        FFMI_HIP(ffmi::launch_rmsnorm(l == 0 ? embed : res, l == 0 ? nullptr : proj, L.in_norm, res,
+        FFMI_HIP(ffmi::launch_rmsnorm(l == 0 ? embed : rs, l == 0 ? nullptr : proj, L.in_norm, rs,
                                       h, T, H, eps, stream, packed,
                                       l == 0 ? ffmi::Partials() : down_part,
                                       l == 0 ? (blob_fetch ? batch->host : batch->dev) : nullptr,
@@ -1185,9 +1200,12 @@ struct LlamaGPU : public ffmi_model {
       }
       pr = prof_begin(on);
       ffmi::Partials qkv_part;
-      FFMI_HIP(ffmi::launch_gemm(fz_in && !packed ? res : h, L.wqkv, qkv, (float *)ws, ws_bytes, T, 3 * Hl, H,
-                                 XP, stream, &qkv_part, 0,
-                                 fz_in ? &fz_qkv : nullptr));
+      if (nq)
+        TRY(norm_gemm(down_part, L.in_norm, L.wqkv, qkv, 3 * Hl, XP));
+      else
+        FFMI_HIP(ffmi::launch_gemm(fz_in && !packed ? res : h, L.wqkv, qkv, (float *)ws, ws_bytes, T, 3 * Hl, H,
+                                   XP, stream, &qkv_part, 0,
+                                   fz_in ? &fz_qkv : nullptr));
       prof_end(pr, GEMM_QKV, gemm_bytes(T, 3 * Hl, 3 * Hl, H), 2.0 * T * 3 * Hl * H);
       mk();
       if (dbg) TRY(dbg_gemm_out(FFMI_DBG_QKV, l, qkv, qkv_part, T));
@@ -1224,17 +1242,20 @@ struct LlamaGPU : public ffmi_model {
         mk();
       }
       if (dbg && !arn) TRY(dbg_gemm_out(FFMI_DBG_O_PROJ, l, proj, o_part, T));
-      if (!fuse && !arn) {
+      const int YP = packed ? FFMI_Y_PACKED : 0;
+      const bool ngu = takes_norm(o_part, Fl, FFMI_EPI_SILU_MUL | XP | YP);
+      if (!ngu && !fuse && !arn) {
         pr = prof_begin(on);
-        FFMI_HIP(ffmi::launch_rmsnorm(res, proj, L.post_norm, res, h, T, H, eps, stream, packed,
+        FFMI_HIP(ffmi::launch_rmsnorm(rs, proj, L.post_norm, rs, h, T, H, eps, stream, packed,
                                       o_part));
         prof_end(pr, NORM, (double)T * H * 2 * 4, 0);
         mk();
       }
       if (dbg) TRY(dbg_copy(FFMI_DBG_FFN_NORM, l, h, T));
       pr = prof_begin(on);
-      const int YP = packed ? FFMI_Y_PACKED : 0;
-      if (fuse)
+      if (ngu)
+        TRY(norm_gemm(o_part, L.post_norm, L.wgu, mlp, Fl, FFMI_EPI_SILU_MUL | XP | YP));
+      else if (fuse)
         FFMI_HIP(ffmi::launch_gemm(packed ? h : res, L.wgu, mlp, (float *)ws, ws_bytes, T, Fl, H,
                                    FFMI_EPI_SILU_MUL | XP | YP, stream, nullptr, 0, &fz_gu));
       else
@@ -1278,12 +1299,13 @@ struct LlamaGPU : public ffmi_model {
     auto mkt = [&]() {
       if (tail_mark) (void)ffmi::launch_marker(mark_i++, stream);
     };
-    if (!arn) {  // (arn: the last down all-reduce applied the final norm)
+    const bool nlm = !few_rows && takes_norm(down_part, Vl, XP);
+    if (!arn && !nlm) {  // (arn: the last down all-reduce applied the final norm)
       pr = prof_begin(ptail);
       if (fuse)  // res already holds the last residual add
         FFMI_HIP(ffmi::launch_rmsnorm(res, nullptr, final_norm, nullptr, h, T, H, eps, stream, packed));
       else
-        FFMI_HIP(ffmi::launch_rmsnorm(res, proj, final_norm, res, h, tail_n, H, eps, stream, packed,
+        FFMI_HIP(ffmi::launch_rmsnorm(rs, proj, final_norm, rs, h, tail_n, H, eps, stream, packed,
                                       down_part, nullptr, nullptr, 0, nullptr, 0, few_rows ? rows_h : nullptr, T));
       prof_end(pr, NORM, (double)tail_n * H * 2 * 4, 0);
     }
@@ -1294,7 +1316,8 @@ struct LlamaGPU : public ffmi_model {
       dbg_T = T;
     }
     pr = prof_begin(ptail);
-    TRY(ffmi_linear_ws(h, lm, logits, tail_n, Vl, H, FFMI_EPI_NONE | XP, ws, ws_bytes, s));
+    if (nlm) TRY(norm_gemm(down_part, final_norm, lm, logits, Vl, XP));
+    else TRY(ffmi_linear_ws(h, lm, logits, tail_n, Vl, H, FFMI_EPI_NONE | XP, ws, ws_bytes, s));
     prof_end(pr, GEMM_LM_HEAD, gemm_bytes(tail_n, Vl, Vl, H), 2.0 * tail_n * Vl * H);
     mkt();
     if (k > 0) {  // (0: the caller takes logits)
