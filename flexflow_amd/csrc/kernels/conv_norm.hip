@@ -29,8 +29,7 @@ __global__ __launch_bounds__(NT) void conv_norm_kernel(ConvNormStep st, ConvNorm
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, H = a.H, nchunk = H >> 3, T = st.T;
   const PagedToken *tok = reinterpret_cast<const PagedToken *>(st.blob + st.off_tokens);
-  const int first = st.out_rows ? st.out_rows[blockIdx.x] : (int)blockIdx.x;
-  const int out = blockIdx.x;
+  const int out = packed_row(blockIdx.x, gridDim.x), first = st.out_rows ? st.out_rows[out] : out;
   const PagedToken raw = tok[first];  // (one token for the whole workgroup)
   if (st.blob_dst) {
     const uint4 *src = reinterpret_cast<const uint4 *>(st.blob);

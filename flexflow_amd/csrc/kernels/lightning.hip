@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const float *__restrict
                                                          float *__restrict__ hf, int H, int n,
                                                          float eps) {
   __shared__ float sh[4];
-  const int t = blockIdx.x, T = gridDim.x;
+  const int T = gridDim.x, t = packed_row(blockIdx.x, T);
   const float *row = o + (size_t)t * H;
   float ss = 0.f;
   for (int c = threadIdx.x; c < H / 4; c += 256) {

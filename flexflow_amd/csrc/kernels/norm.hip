@@ -102,7 +102,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     uint4 *__restrict__ blob_dst, int blob_n16, const int32_t *__restrict__ gprev) {
   __shared__ double scratch[NT / 64];
   static_assert(!ROWS || SRC <= 2, "rows of a plain or residual norm");
-  const int row = ROWS ? gprev[blockIdx.x] : blockIdx.x;
+  const int at = packed_row(blockIdx.x, gridDim.x), row = ROWS ? gprev[at] : at;
   const int T = ROWS ? blob_n16 : gridDim.x;
   const int nchunk = H >> 3;
   // gather: x1 is the embedding table and row t reads its token's row (the
@@ -224,7 +224,6 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
         float y = h2f_(f2h_(__fmul_rn(h2f_(e[q]), rms)));
         o8[q] = f2h_(__fmul_rn(y, h2f_(we[q])));
       }
-      const int at = ROWS ? blockIdx.x : row;
       uint16_t *dst = out_packed ? out + act_packed_off(at, ch * 8, H) : out + (size_t)at * H + ch * 8;
       *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<uint4 *>(o8);
     }

@@ -13,7 +13,7 @@ __global__ __launch_bounds__(256) void embed_pos_kernel(
     const char *__restrict__ blob_src, uint4 *__restrict__ blob_dst, int blob_n16,
     const uint16_t *__restrict__ embed, const uint16_t *__restrict__ pos, float *__restrict__ x,
     uint16_t *__restrict__ xb, int H) {
-  const int t = blockIdx.x;
+  const int t = packed_row(blockIdx.x, gridDim.x);
   const PagedToken tk = reinterpret_cast<const PagedToken *>(blob_src)[t];  // tokens come first
   const uint4 *src = reinterpret_cast<const uint4 *>(blob_src);
   for (int i = t * 256 + threadIdx.x; i < blob_n16; i += gridDim.x * 256) blob_dst[i] = src[i];
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const float *__restrict
                                                          float *__restrict__ hf, int H, int n,
                                                          float eps, EmbedRows em) {
   __shared__ float sh[NT / 64];
-  const int row = blockIdx.x, T = gridDim.x, nchunk = H >> 3;
+  const int T = gridDim.x, row = packed_row(blockIdx.x, T), nchunk = H >> 3;
   const uint16_t *er = nullptr;
   if (PRE && MAXS == 0 && em.table) {
     er = em.table + (size_t)reinterpret_cast<const PagedToken *>(em.blob_src)[row].token * H;
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void row_norm_kernel(const int32_t *__restrict
                                                        float *__restrict__ hf, int H, int n,
                                                        float eps) {
   __shared__ float sh[4];
-  const int i = blockIdx.x;
+  const int i = packed_row(blockIdx.x, gridDim.x);
   const float *xr = x + (size_t)rows[i] * H;
   float ss = 0.f;
   for (int c = threadIdx.x; c < H / 4; c += 256) {
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(NT) void sum_norm_kernel(SumNorm a,
   __shared__ __attribute__((aligned(16))) uint16_t own_row[RT ? NT * 8 : 8];
   __shared__ __attribute__((aligned(16))) float sums[NW * 16 * RTS];
   RouterRow<RTS> router;
-  const int row = blockIdx.x, H = a.H, nchunk = H >> 3;
+  const int row = packed_row(blockIdx.x, gridDim.x), H = a.H, nchunk = H >> 3;
   f4 x[MAXC][2], wv[MAXC][2];
   float ss = 0.f;
   const float alpha = a.own ? a.alpha + a.own[row] : a.alpha;
