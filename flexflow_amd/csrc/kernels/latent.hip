@@ -135,6 +135,10 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const PagedToken *__re
 // whole lines.  A head's workgroups share an XCD where heads are a multiple of 8: its
 // weights are read from memory once.  1024 rows, 32 heads: K = 128, N = 512 with the latents'
 // store 25 -> 21 us, K = 512, N = 128 21 -> 14.
+// Up to two chunks of k (KC <= 2) it is a chain of waits, and workgroups side by side are what
+// hides them: one chunk's weights in registers at a time leave room for four on a CU instead of
+// two (126 registers, 176 before; two and a half rounds of the 1280 before), and the latents'
+// workgroups go first instead of behind the last products: 20.3 -> 16.9 us.
 __device__ __forceinline__ int prep_turn(int row) { return (row >> 1 & 3) << 1 | (row >> 3 & 1); }
 template <int KC>
 __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *sh) {
@@ -156,12 +160,13 @@ __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *
 #pragma unroll
   for (int j = 0; j < 4; ++j)
     w0[j] = a.W + ((size_t)h * a.NTt + min(nt0 + wn * 4 + j, a.NTt - 1)) * a.KT * 512 + lane * 8;
-  bf8 w[2][2][4];
+  constexpr int WB = KC <= 2 ? 1 : 2;
+  bf8 w[WB][2][4];
   auto weights = [&](int c) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[c & 1][k][j] = *reinterpret_cast<const bf8 *>(w0[j] + (size_t)(2 * c + k) * 512);
+      for (int j = 0; j < 4; ++j) w[c % WB][k][j] = *reinterpret_cast<const bf8 *>(w0[j] + (size_t)(2 * c + k) * 512);
   };
   f4 acc[4][4];
 #pragma unroll
@@ -169,17 +174,19 @@ __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
   copy(0);
-  if (KC > 1) copy(1);
+  if (KC > 1 && WB > 1) copy(1);
   weights(0);
+  if (KC > 1 && WB == 1) copy(1);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int c = 0; c < KC; ++c) {
     if (c + 2 < KC) copy(c + 2);
-    if (c + 1 < KC) weights(c + 1);
+    if (WB > 1 && c + 1 < KC) weights(c + 1);
+    if (WB == 1 && c > 0) weights(c);
     __builtin_amdgcn_sched_barrier(0);
     // chunk c has landed, what was just asked for may be under way: s_waitcnt vmcnt
     if (c + 2 < KC) __builtin_amdgcn_s_waitcnt(0x0f70 | 12);
-    else if (c + 1 < KC) __builtin_amdgcn_s_waitcnt(0x0f70 | 8);
+    else if (c + 1 < KC) __builtin_amdgcn_s_waitcnt(0x0f70 | (WB > 1 ? 8 : 4));
     else __builtin_amdgcn_s_waitcnt(0x0f70);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -195,7 +202,7 @@ __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c & 1][k][j], xf[i], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c % WB][k][j], xf[i], acc[i][j], 0, 0, 0);
     }
   }
   const int N = a.NTt * 16, Yw = a.heads * N, n0 = nt0 + wn * 4;  // (column tiles)
@@ -232,14 +239,15 @@ __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *
   }
 }
 template <int KC>
-__global__ __launch_bounds__(256) void latent_prep_tile_kernel(const PagedToken *__restrict__ tok, HgDev a,
+__global__ __launch_bounds__(256, KC <= 2 ? 4 : 1) void latent_prep_tile_kernel(const PagedToken *__restrict__ tok, HgDev a,
                                                                int nprod, LatentStore st) {
   __shared__ __attribute__((aligned(16))) uint16_t sh[(KC < 2 ? 2 : KC) * 8192];
-  if ((int)blockIdx.x < nprod) {
-    head_gemm_tile<KC>(a, blockIdx.x, sh);
+  const int nst = (int)gridDim.x - nprod;
+  if ((int)blockIdx.x >= nst) {
+    head_gemm_tile<KC>(a, blockIdx.x - nst, sh);
     return;
   }
-  const int t = (blockIdx.x - nprod) * 4 + (threadIdx.x >> 6);
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= a.T) return;
   latent_store_token(tok[t], (const uint16_t *)st.d + (size_t)t * st.ldd, st.w,
                      (uint16_t *)st.cache, st.rank, st.n, st.eps);
