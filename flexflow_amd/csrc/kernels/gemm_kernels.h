@@ -1209,10 +1209,12 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // them afterwards is (0.77 us per k-step of 256 x 256 against 0.43 of MFMA
 // issue).  So:
 //  * the fragments of step k + 1 are read while step k is multiplied, each
-//    xf[i] into the registers that row i's MFMAs have just used and the weight
+//    row's into the registers that its MFMAs have just used and the weight
 //    fragments into a second set, with NB - 2 later stages in flight across
 //    the barrier (a counted s_waitcnt vmcnt, never 0 in the steady state, and
-//    a raw s_barrier: __syncthreads would drain the DMAs);
+//    a raw s_barrier: __syncthreads would drain the DMAs).  Waves of three rows and four
+//    weight tiles or more (kTwoX) read the rows into a second set too, and all of it
+//    ahead of the last row's MFMAs, so that no read is waited for at the step's end;
 //  * the loop body has no branches (a step without a next one is a separate
 //    instantiation; waves past the last fragment load it again, or see
 //    kExactCopies), and
@@ -1240,6 +1242,13 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // from it (400 products of 200 .. 1024 rows: 0.2% slower to 0.3% faster a form).
 template <int MI, int NJ, int WR, int WC>
 static constexpr bool kExactCopies = WR * WC > 8 && (MI * WR + NJ * WC) % (WR * WC) != 0;
+// Two sets of row fragments.  One set / two, us at T = 1024, cold weights: 22016 x 4096 in 256 x 192
+// 176.8 / 171.7, 4096 x 11008 in two slices of 256 x 128 91.2 / 89.7 and of 128 x 256 95.8 / 90.6, 11264 x
+// 2048 in 256 x 192 51.0 / 49.2, 4096 x 11008 in 192 x 128 116.0 / 106.3; 12288 x 4096 at 280 rows
+// in 192 x 128 52.0 / 48.8.  Two rows a wave gain nothing (4096 x 4096 in 128 x 128 40.3 / 40.9) or
+// lose (6144 x 2048 in 128 x 192 31.9 / 32.6), as twelve waves do (22016 x 4096 at 168 rows 52.5 / 53.6).
+template <int MI, int NJ, int WR, int WC>
+static constexpr bool kTwoX = MI >= 3 && NJ >= 4 && WR * WC <= 8;
 template <int EPI, int MI, int NJ, int WR, int WC, int NB, bool NTL>
 __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
     const uint16_t *__restrict__ X, const uint16_t *__restrict__ Wp, uint16_t *__restrict__ Y,
@@ -1300,23 +1309,29 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
 #pragma unroll
       for (int p = 0; p < PW; ++p) issue(min(kt, n - 1), kt, p);
     }
-    h8 xf[MI], wa[NJ], wb[NJ];
+    constexpr bool TWO = kTwoX<MI, NJ, WR, WC>;
+    h8 xa[MI], x2[TWO ? MI : 1], wa[NJ], wb[NJ];
+    auto &xb = [&]() -> h8(&)[MI] {
+      if constexpr (TWO) return x2;
+      else return xa;
+    }();
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 1) * PW) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int j = 0; j < NJ; ++j) wa[j] = lds[0][FX + wn * NJ + j][lane];
 #pragma unroll
-    for (int i = 0; i < MI; ++i) xf[i] = lds[0][wm * MI + i][lane];
+    for (int i = 0; i < MI; ++i) xa[i] = lds[0][wm * MI + i][lane];
     int slot = 0;
-    // Step kt on xf / wc, with step kt + 1's fragments read into xf / wx.  The
+    // Step kt on xc / wc, with step kt + 1's fragments read into xx / wx.  The
     // wait leaves the NB - 2 stages after kt + 1 in flight and retires this
     // wave's own reads of stage kt (issued a step ago); behind the barrier stage
     // kt + 1 is there for every wave and stage kt's slot is free for kt + NB.
     // MORE: step kt + NB exists.  (The last step reads a stale slot unused.)
-    auto kstep = [&](auto MOREc, h8(&wc)[NJ], h8(&wx)[NJ], int kt) {
+    auto kstep = [&](auto MOREc, h8(&xc)[MI], h8(&wc)[NJ], h8(&xx)[MI], h8(&wx)[NJ], int kt) {
       constexpr bool MORE = decltype(MOREc)::value;
       constexpr int VM = MORE ? (NB - 2) * PW : 0;
+      constexpr int R = MI + NJ, G = MI > 1 ? MI - 1 : 1;  // reads; the rows they go with (TWO)
       const int nslot = slot + 1 == NB ? 0 : slot + 1;
       // s_waitcnt vmcnt(VM) lgkmcnt(0)
       __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
@@ -1324,13 +1339,21 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
+        if constexpr (TWO) {
+#pragma unroll
+          for (int f = min(i, G) * R / G; f < min(i + 1, G) * R / G; ++f)
+            if (f < NJ) wx[f] = lds[nslot][FX + wn * NJ + f][lane];
+            else xx[f - NJ] = lds[nslot][wm * MI + f - NJ][lane];
+        }
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int j = 0; j < NJ; ++j)  // D = W . X^T (see mid_store)
-          acc[i][j] = mma16<EPI>(wc[j], xf[i], acc[i][j]);
-        xf[i] = lds[nslot][wm * MI + i][lane];
+          acc[i][j] = mma16<EPI>(wc[j], xc[i], acc[i][j]);
+        if constexpr (!TWO) {
+          xx[i] = lds[nslot][wm * MI + i][lane];
 #pragma unroll
-        for (int j = i * NJ / MI; j < (i + 1) * NJ / MI; ++j) wx[j] = lds[nslot][FX + wn * NJ + j][lane];
+          for (int j = i * NJ / MI; j < (i + 1) * NJ / MI; ++j) wx[j] = lds[nslot][FX + wn * NJ + j][lane];
+        }
         if constexpr (MORE) {
 #pragma unroll
           for (int p = i * PW / MI; p < (i + 1) * PW / MI; ++p) issue(kt + NB, slot, p);
@@ -1344,19 +1367,23 @@ __global__ __launch_bounds__(WR * WC * 64, 1) void gemm_tile_kernel(
     const auto no = std::integral_constant<bool, false>{};
     int kt = 0;
     for (; kt + 2 + NB <= n; kt += 2) {
-      kstep(yes, wa, wb, kt);
-      kstep(yes, wb, wa, kt + 1);
+      kstep(yes, xa, wa, xb, wb, kt);
+      kstep(yes, xb, wb, xa, wa, kt + 1);
     }
     if (kt + 1 + NB <= n) {
-      kstep(yes, wa, wb, kt++);
+      kstep(yes, xa, wa, xb, wb, kt++);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) xa[i] = xb[i];
     }
 #pragma unroll 1
     for (; kt < n; ++kt) {
-      kstep(no, wa, wb, kt);
+      kstep(no, xa, wa, xb, wb, kt);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) wa[j] = wb[j];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) xa[i] = xb[i];
     }
   };
   constexpr std::integral_constant<int, PMAX> most{};
