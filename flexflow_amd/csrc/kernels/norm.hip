@@ -117,7 +117,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   // more trip to the host's memory before the row could be asked for)
   if (S == 3) {
     gid = reinterpret_cast<const ffmi_token_info *>(gather + pNP)[row].token_id;
-    if (gid < 0) gid = gprev[-1 - gid];
+    if (gid < 0) gid = max(gprev[-1 - gid], 0);  // (a row of NaN has no pick, -1)
   }
   const uint16_t *a = S == 3 ? x1 + (size_t)gid * H : x1 + (size_t)row * H;
   // blob fetch: gather is the step's staging blob in mapped host memory; the
@@ -407,6 +407,11 @@ extern "C" __device__ unsigned long long __ockl_wfred_max_u64(unsigned long long
 //    the oracle's serial loop): S = float(double sum) in any order, as above.
 //    `part` = [T][G] doubles, `cnt` = [T] counters, zero before the first
 //    launch and left zero.
+//  * A pick is stored at system scope: the host may look for it in pinned memory while
+//    the stream works on.
+__device__ __forceinline__ void store_pick(int32_t *at, int id) {
+  __hip_atomic_store(at, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <int TPB, int NV, int G>
 __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
     const uint16_t *__restrict__ logits, int V, int k, int32_t *__restrict__ ids,
@@ -563,7 +568,7 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
     return ((unsigned long long)(p + 1u) << 32) | (unsigned long long)(0xffffffffu - i);
   };
   auto emit = [&](int rd, unsigned long long b) {
-    ids[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
+    store_pick(ids + (size_t)row * k + rd, (int)(0xffffffffu - (unsigned)(b & 0xffffffffu)));
     if (ids2) ids2[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
     if (probs) probs[(size_t)row * k + rd] = h2f_((uint16_t)((b >> 32) - 1u));
   };
@@ -708,7 +713,7 @@ __global__ __launch_bounds__(TPB) void softmax_topk_kernel(
     return ((unsigned long long)(p + 1u) << 32) | (unsigned long long)(0xffffffffu - i);
   };
   auto emit = [&](int rd, unsigned long long b) {
-    ids[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
+    store_pick(ids + (size_t)row * k + rd, (int)(0xffffffffu - (unsigned)(b & 0xffffffffu)));
     if (ids2) ids2[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
     if (probs) probs[(size_t)row * k + rd] = h2f_((uint16_t)((b >> 32) - 1u));
   };

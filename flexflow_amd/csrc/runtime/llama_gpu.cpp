@@ -133,6 +133,17 @@ struct LlamaGPU : public ffmi_model {
   bool slot_ev_live[kChain] = {};      // slot_ev recorded for the chain in flight
   int last_slot = -1;                  // highest slot launched since the last wait
   bool chain_ok = !getenv("FFMI_SSM_CHAIN") || atoi(getenv("FFMI_SSM_CHAIN")) != 0;
+  // FFMI_INC_AHEAD=0: decoding steps one by one (A/B, tests)
+  bool ahead_ok = !getenv("FFMI_INC_AHEAD") || atoi(getenv("FFMI_INC_AHEAD")) != 0;
+  bool ahead_step = false;  // (the step being launched is one)
+  // the slot whose picks a step's negative token ids name (-1: none)
+  int slot_before(int slot) const {
+    return mode == FFMI_MODEL_INC ? (ids_dev ? 1 - slot : -1) : slot - 1;
+  }
+  const int32_t *ids_before(int slot) const {
+    const int b = slot_before(slot);
+    return b < 0 ? nullptr : ids_dev + (size_t)b * (slot_ints() / 2);
+  }
   size_t slot_ints() const { return (size_t)((o.max_tokens + 15) & ~15) * 4 * 2; }
   bool result_copy = getenv("FFMI_RESULT_COPY") && atoi(getenv("FFMI_RESULT_COPY")) != 0;
   float *probs_h = nullptr;
@@ -625,14 +636,16 @@ struct LlamaGPU : public ffmi_model {
                            hipHostMallocCoherent | hipHostMallocMapped));
     rows_h = ids_h + (size_t)kChain * Tm * 4 * 2;
     if (mode == FFMI_MODEL_BEAM) TRY(alloc(&ids_dev, (size_t)kChain * Tm * 4));
+    if (ahead_ok && mode == FFMI_MODEL_INC && o.tp_size == 1) TRY(alloc(&ids_dev, (size_t)2 * Tm * 4));
     chain_batch[0] = batch;
     // the chained beam steps' staging batches, created here rather than on a
     // chain's first use: creating one clears its device blob on the legacy
     // stream, which fails -- and invalidates the capture -- while another
     // thread's model is capturing a graph (the TP shard threads of one
     // process, ffmi_comm_create_local, beside their SSMs)
-    if (mode == FFMI_MODEL_BEAM && o.tp_size == 1)
-      for (int i = 1; i < kChain; ++i)
+    // (and the second one of decoding steps launched ahead)
+    if (mode == FFMI_MODEL_BEAM ? o.tp_size == 1 : ids_dev != nullptr)
+      for (int i = 1; i < (mode == FFMI_MODEL_BEAM ? kChain : 2); ++i)
         TRY(ffmi_batch_create((o.max_tokens + 15) & ~15, o.max_requests, &chain_batch[i]));
     // weights (seeded synthetic, orc_gen_weight spec), packed for MFMA
     uint16_t *tmp = nullptr;
@@ -956,7 +969,8 @@ struct LlamaGPU : public ffmi_model {
     // the host instead of reading out of bounds on the device
     // (a chained beam step's -1 - i: entry i of the previous slot's ids,
     // themselves top-k picks in range)
-    const long prev_n = cur_slot > 0 ? (long)slot_results[cur_slot - 1] : 0;
+    const int before = mode != FFMI_MODEL_INC || ahead_step ? slot_before(cur_slot) : -1;
+    const long prev_n = before >= 0 ? (long)slot_results[before] : 0;
     for (int t = 0; t < T; ++t)
       FFMI_CHECK((desc.tokens[t].token_id >= 0 && desc.tokens[t].token_id < c.vocab_size) ||
                      (desc.tokens[t].token_id < 0 && -1L - desc.tokens[t].token_id < prev_n),
@@ -969,7 +983,11 @@ struct LlamaGPU : public ffmi_model {
     // graphed: small steps, and tree-verify steps of one work item per
     // request (a fixed shape while the batch is full: T = 168 for 8 requests
     // of 21 tree tokens); prefill blocks stay eager (one-off shapes)
-    const bool graph = use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
+    // (every other decoding step launched ahead goes without one: the host has a step's time
+    // to enqueue it in, and a shape needs no second graph for the other slot's addresses.  16
+    // decoding steps of a 768-channel model 1120 us so, 1155 with a graph for each slot)
+    const bool second = mode == FFMI_MODEL_INC && cur_slot == 1;
+    const bool graph = !second && use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
                        (o.tp_size == 1 || peer || rccl || ffmi::comm_size(o.comm) == 1) &&
                        !prof_on(0, T) &&
                        !prof_on(c.num_layers / 2, T);
@@ -1000,7 +1018,7 @@ struct LlamaGPU : public ffmi_model {
       FFMI_HIP(hipGraphLaunch(it->second, stream));
     } else {
       if (step_timing) FFMI_HIP(hipEventRecord(st_ev[0], stream));
-      st = enqueue(k, bytes, true, T);
+      st = enqueue(k, bytes, !second, T);
       if (st != FFMI_OK) return st;
     }
     if (step_timing) {
@@ -1184,8 +1202,7 @@ struct LlamaGPU : public ffmi_model {
                                       l == 0 ? ffmi::Partials() : down_part,
                                       l == 0 ? (blob_fetch ? batch->host : batch->dev) : nullptr,
                                       l == 0 && blob_fetch ? batch->dev : nullptr, blob_bytes,
-                                      cur_slot > 0 ? ids_dev + (size_t)(cur_slot - 1) * (slot_ints() / 2)
-                                                   : nullptr,
+                                      ids_before(cur_slot),
                                       batch->off_tokens));
         // the staging is free for the next step once the fetch has read it
         if (l == 0 && blob_fetch && record_upload) FFMI_HIP(hipEventRecord(batch->uploaded, stream));
@@ -1348,13 +1365,11 @@ struct LlamaGPU : public ffmi_model {
       // sharded softmax / top-k: three record exchanges, then the merge
       TRY(ffmi_vocab_shard_topk(o.comm, logits, T, Vl, k, ids_o, probs_o, xch, s));
     } else {
-      // the ids also to device memory: the next chained beam step's
-      // embedding gather reads them there
+      // the ids also to device memory: the embedding gather of the next chained
+      // beam step, or decoding step launched ahead, reads them there
       FFMI_CHECK(k >= 1 && k <= 4 && k <= V, FFMI_ERR_INVALID);
       FFMI_HIP(ffmi::launch_argmax(logits, T, V, k, ids_o, probs_o, stream, topk_ws, topk_ws_bytes,
-                                   mode == FFMI_MODEL_BEAM
-                                       ? ids_dev + (size_t)cur_slot * (slot_ints() / 2)
-                                       : nullptr));
+                                   ids_dev ? ids_dev + (size_t)cur_slot * (slot_ints() / 2) : nullptr));
     }
     if (result_copy)
       FFMI_HIP(hipMemcpyAsync(ids_h + cur_slot * slot_ints(), ids_d, (size_t)T * k * 8,
@@ -1380,6 +1395,57 @@ struct LlamaGPU : public ffmi_model {
       for (int i = 0; i < few_n; ++i) ir->token_ids[rows_h[i]] = ids_h[i];
     } else {
       memcpy(ir->token_ids, ids_h, bc.num_tokens * sizeof(int32_t));
+    }
+    return FFMI_OK;
+  }
+  // Steps one by one / ahead (us): 768 channels, 1 request, 16 steps 1357 / 1120, 8 requests, 40 steps
+  // 3990 / 3300; 2048, 1 request, 40 steps 14840 / 14400, 6 requests, 30 steps 12870 / 12390; 4096
+  // (8 layers), 3 requests, 30 steps 22590 / 22130; 4096 (32 layers), 8 requests, 32 steps 103750 / 103140.
+  // Up to 64 tokens, unsharded, unprofiled; not where the device's flags have
+  // threads yield or sleep: picks are waited for by looking.
+  bool can_launch_ahead(int num_tokens) const override {
+    if (!ids_dev || mode != FFMI_MODEL_INC || num_tokens < 1 || num_tokens > std::min(64, (int)o.max_tokens) || dbg ||
+        result_copy || !use_graphs || step_timing || prof_level != 0 || prof_on(0, num_tokens))
+      return false;
+    unsigned flags = 0;
+    if (hipGetDeviceFlags(&flags) != hipSuccess) return false;
+    flags &= hipDeviceScheduleMask;
+    return flags != hipDeviceScheduleYield && flags != hipDeviceScheduleBlockingSync;
+  }
+  ffmi_status inc_launch(const BatchConfig &bc, int slot, bool ahead) override {
+    FFMI_CHECK((slot == 0 || slot == 1) && can_launch_ahead(bc.num_tokens), FFMI_ERR_INVALID);
+    pack_inc(bc, o.max_requests, slots, &ps);
+    int32_t *ids = ids_h + slot * slot_ints();
+    std::fill_n(ids, bc.num_tokens, -1);
+    cur_slot = slot;
+    batch = chain_batch[slot];
+    ahead_step = ahead;
+    const ffmi_status st = forward_launch(1);
+    ahead_step = false;
+    batch = chain_batch[0];
+    cur_slot = 0;
+    slot_results[slot] = st == FFMI_OK ? bc.num_tokens : 0;
+    return st;
+  }
+  // A row's pick is there when it is no longer -1 (the sampling kernel stores it at system
+  // scope).  An event behind every step would be waited for by the GPU, too.  (The stream
+  // is asked now and then, so that one in error ends the wait.)
+  ffmi_status inc_collect(int slot, int32_t *out) override {
+    if (!out) return forward_finish();
+    const int32_t *ids = ids_h + slot * slot_ints();
+    for (size_t i = 0; i < slot_results[slot]; ++i) {
+      for (int spins = 1; (out[i] = __atomic_load_n(ids + i, __ATOMIC_ACQUIRE)) < 0; ++spins) {
+        if (spins % 8192 == 0) {
+          const hipError_t e = hipStreamQuery(stream);
+          if (e == hipSuccess) {  // (a row of NaN has no pick: -1)
+            out[i] = __atomic_load_n(ids + i, __ATOMIC_ACQUIRE);
+            break;
+          }
+          if (e != hipErrorNotReady) FFMI_HIP(e);
+          (void)hipGetLastError();  // (not an error that a later launch should find)
+        }
+        __builtin_ia32_pause();
+      }
     }
     return FFMI_OK;
   }

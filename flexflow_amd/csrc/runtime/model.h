@@ -93,6 +93,23 @@ struct ffmi_model {
     (void)ir;
     return FFMI_ERR_UNSUPPORTED;
   }
+  // Decoding steps launched ahead (serve_incr_decoding): a step of one token a request
+  // goes on the stream before the step ahead of it has been waited for, with token id
+  // -1 - i where its token is row i's pick of that step (the device fills it in).  Two
+  // slots, used in turn; inc_collect waits for a slot's step and gives its rows' picks
+  // (ids: null: everything launched is waited for, nothing is read).
+  virtual bool can_launch_ahead(int num_tokens) const {
+    (void)num_tokens;
+    return false;
+  }
+  virtual ffmi_status inc_launch(const ffmi::BatchConfig &bc, int slot, bool ahead) {
+    (void)bc, (void)slot, (void)ahead;
+    return FFMI_ERR_UNSUPPORTED;
+  }
+  virtual ffmi_status inc_collect(int slot, int32_t *ids) {
+    (void)slot, (void)ids;
+    return FFMI_ERR_UNSUPPORTED;
+  }
   // an INC step whose caller wants the logits of batch tokens rows[0, n):
   // fp32 [n][vocab] to `out` (host)
   virtual ffmi_status run_inc_logits(const ffmi::BatchConfig &bc, const int *rows, int n,

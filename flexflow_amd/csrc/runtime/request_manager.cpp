@@ -25,6 +25,7 @@
 #include <chrono>
 #include <map>
 #include <memory>
+#include <numeric>
 
 void ffmi_set_last_error(const char *msg, const char *file, int line);  // api.cpp
 
@@ -1048,7 +1049,48 @@ const RequestManager::ProfileInfo *RequestManager::get_profile(RequestGuid guid)
   return it == profiling_requests.end() ? nullptr : &it->second;
 }
 
-// request_manager.cc:3012-3080 (synchronous: one batch in flight)
+// The decoding step after `bc` (one token a request, each the pick of row rows[j] of the
+// step in flight: token id -1 - rows[j]) without the requests that their length ends; false
+// where it is not known before the picks are, or the model does not take it.
+bool RequestManager::next_decode_batch(ffmi_model *llm, const BatchConfig &bc, const std::vector<int> &rows,
+                                       BatchConfig *next) {
+  if (!pending_infr_request_queue.empty() || bc.num_tokens != bc.num_generation_tokens) return false;
+  next->num_tokens = 0;
+  for (int j = 0; j < bc.num_tokens; ++j) {
+    const int r = bc.tokensInfo[j].request_index, depth = bc.tokensInfo[j].abs_depth_in_request + 1;
+    if (depth + 1 >= bc.requestsInfo[r].max_length) continue;
+    next->requestsInfo[r].request_guid = bc.requestsInfo[r].request_guid;
+    auto &tk = next->tokensInfo[next->num_tokens++];
+    tk.request_index = r, tk.abs_depth_in_request = depth, tk.token_id = -1 - rows[j];
+  }
+  return next->num_tokens > 0 && llm->can_launch_ahead(next->num_tokens);
+}
+
+// Are all of bc's tokens in the step launched ahead (`ahead`, after one whose picks are
+// `ids`)?  rows: which rows they are.  (It may hold requests more, ended since.)
+static bool find_rows(const BatchConfig &ahead, const std::vector<int32_t> &ids, const BatchConfig &bc,
+                      std::vector<int> *rows) {
+  rows->clear();
+  int q = 0;
+  for (int j = 0; j < bc.num_tokens; ++j, ++q) {
+    const auto &tk = bc.tokensInfo[j];
+    while (q < ahead.num_tokens && ahead.tokensInfo[q].request_index != tk.request_index) ++q;
+    if (q == ahead.num_tokens) return false;
+    const auto &at = ahead.tokensInfo[q];
+    // (a row of NaN has no pick, -1: such a token is refused when it is launched)
+    if (tk.token_id < 0 || ids[-1 - at.token_id] != tk.token_id ||
+        at.abs_depth_in_request != tk.abs_depth_in_request ||
+        ahead.requestsInfo[at.request_index].request_guid != bc.requestsInfo[tk.request_index].request_guid)
+      return false;
+    rows->push_back(q);
+  }
+  return true;
+}
+
+// request_manager.cc:3012-3080.  Where the model takes it (can_launch_ahead), a decoding
+// step is on the stream before the one ahead of it has been waited for, so that the
+// scheduler's work and the launch pass beside the GPU's.  It is used for the requests
+// that go on; one that ended by its token had a row for nothing.
 ffmi_status RequestManager::serve_incr_decoding(ffmi_model *llm) {
   if (!llm) return FFMI_ERR_INVALID;
   apply_limits();
@@ -1063,6 +1105,12 @@ ffmi_status RequestManager::serve_incr_decoding(ffmi_model *llm) {
   BatchConfig *bc = new BatchConfig();
   InferenceResult *ir = new InferenceResult();
   ffmi_status st = FFMI_OK;
+  // the step launched ahead and the one to be, the latest picks, the batch's rows of its step
+  std::unique_ptr<BatchConfig> ahead(new BatchConfig()), then(new BatchConfig());
+  std::vector<int32_t> ids(BatchConfig::MAX_NUM_TOKENS);
+  std::vector<int> rows;
+  bool flying = false;
+  int slot = 0;
   while (!all_done()) {
     BatchConfig *next = new BatchConfig(prepare_next_batch(*bc, *ir));
     delete bc;
@@ -1073,11 +1121,39 @@ ffmi_status RequestManager::serve_incr_decoding(ffmi_model *llm) {
       break;
     }
     const double tl = now_us();
-    st = llm->run_inc(*bc, ir);
+    if (flying && !find_rows(*ahead, ids, *bc, &rows)) {
+      flying = false;
+      if ((st = llm->inc_collect(slot, nullptr)) != FFMI_OK) break;
+    }
+    bool on_stream = flying;
+    if (!on_stream) {
+      rows.resize(bc->num_tokens);
+      std::iota(rows.begin(), rows.end(), 0);
+      if (llm->can_launch_ahead(bc->num_tokens) && next_decode_batch(llm, *bc, rows, then.get())) {
+        if ((st = llm->inc_launch(*bc, slot, false)) != FFMI_OK) break;
+        on_stream = true;
+      }
+    }
+    if (on_stream) {
+      const int here = slot;
+      flying = next_decode_batch(llm, *bc, rows, then.get());
+      if (flying) {
+        slot = 1 - slot;
+        if ((st = llm->inc_launch(*then, slot, true)) != FFMI_OK) break;
+        std::swap(ahead, then);
+      }
+      if ((st = llm->inc_collect(here, ids.data())) != FFMI_OK) break;
+      for (int j = 0; j < bc->num_tokens; ++j) ir->token_ids[j] = ids[rows[j]];
+    } else {
+      st = llm->run_inc(*bc, ir);
+    }
     stats.llm_us += now_us() - tl;
     if (st != FFMI_OK) break;
     stats.llm_steps++;
   }
+  // (a step that is still on the stream, of requests that ended or after an error)
+  const ffmi_status rest = llm->inc_collect(slot, nullptr);
+  if (st == FFMI_OK && rest != FFMI_ERR_UNSUPPORTED) st = rest;
   delete bc;
   delete ir;
   stats.wall_us = now_us() - t0;

@@ -1,0 +1,49 @@
+"""Decoding steps launched ahead of the picks they continue give the tokens of steps run one by
+one: requests that end by length and by token while others go on, more of them than slots."""
+import pytest
+
+import flexflow_amd as fa
+from flexflow_amd import ffmi as F
+
+pytestmark = pytest.mark.gpu
+
+CFG = dict(num_layers=2, vocab_size=500, num_heads=2, num_kv_heads=2, hidden=128, intermediate=256,
+           rms_eps=1e-6, rope_theta=10000.0)
+
+
+def tokens(slots, prompts, lengths, eos):
+    m = fa.Model(CFG, "inc", max_requests=slots, max_tokens=64, max_seq_len=96, weight_seed=9)
+    out = []
+    for _ in range(2):  # (on what the first pass left behind, too)
+        rm = fa.RequestManager(max_requests_per_batch=slots, max_tokens_per_batch=64, max_sequence_length=96,
+                               eos_token_ids=eos)
+        guids = [rm.register_new_request(p, max_length=n) for p, n in zip(prompts, lengths)]
+        rm.serve_incr_decoding(m)
+        out.append([rm.get_generation_result(g).output_tokens for g in guids])
+    return out
+
+
+@pytest.mark.parametrize("slots,requests", [(1, 1), (1, 3), (4, 3), (4, 4), (4, 7), (20, 20)])
+def test_same_tokens_as_one_by_one(slots, requests, monkeypatch):
+    prompts = [[(37 * i + 11 * r) % 480 + 5 for i in range(3 + r % 5)] for r in range(requests)]
+    lengths = [min(96, len(p) + (3, 40, 2, 17, 60)[r % 5]) for r, p in enumerate(prompts)]
+    lengths[0] = 50
+    monkeypatch.setenv("FFMI_INC_AHEAD", "0")
+    plain = tokens(slots, prompts, lengths, [])[0]
+    assert [len(t) for t in plain] == lengths
+    # tokens that end some requests early, at different steps
+    eos = sorted({t[len(t) - len(t) // 3] for t in plain[::2]})
+    short = tokens(slots, prompts, lengths, eos)
+    assert short[0] == short[1] and any(len(a) < len(b) for a, b in zip(short[0], plain))
+    monkeypatch.delenv("FFMI_INC_AHEAD")
+    assert tokens(slots, prompts, lengths, []) == [plain, plain]
+    assert tokens(slots, prompts, lengths, eos) == short
+
+
+def test_refuses_tokens_out_of_range_behind_steps_launched_ahead():
+    m = fa.Model(CFG, "inc", max_requests=2, max_tokens=64, max_seq_len=96, weight_seed=9)
+    for bad in (-1, 500):
+        rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=64, max_sequence_length=96)
+        assert len(fa.generate(rm, m, [[5, 6, 7]], max_length=30)[0].output_tokens) == 30
+        with pytest.raises(F.FFMIError):
+            rm.replay_step(m, [(1, [9, bad], [1])])
