@@ -1368,7 +1368,9 @@ struct LlamaGPU : public ffmi_model {
       // the ids also to device memory: the embedding gather of the next chained
       // beam step, or decoding step launched ahead, reads them there
       FFMI_CHECK(k >= 1 && k <= 4 && k <= V, FFMI_ERR_INVALID);
-      FFMI_HIP(ffmi::launch_argmax(logits, T, V, k, ids_o, probs_o, stream, topk_ws, topk_ws_bytes,
+      // (probabilities: beam steps alone read them)
+      FFMI_HIP(ffmi::launch_argmax(logits, T, V, k, ids_o, mode == FFMI_MODEL_BEAM ? probs_o : nullptr, stream,
+                                   topk_ws, topk_ws_bytes,
                                    ids_dev ? ids_dev + (size_t)cur_slot * (slot_ints() / 2) : nullptr));
     }
     if (result_copy)
