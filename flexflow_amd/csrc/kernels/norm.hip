@@ -415,8 +415,8 @@ extern "C" __device__ unsigned long long __ockl_wfred_max_u64(unsigned long long
 //    workgroups.  One workgroup a row, V = 32000: 1 row 7.8 -> 3.8 us, 8 rows 8.2 -> 4.2,
 //    168 rows 12.2 -> 4.6.  Other rows, and rows with a NaN or without a finite M, take
 //    the whole path.
-//  * A pick is stored at system scope: the host may look for it in pinned memory while
-//    the stream works on.
+//  * PICK stores at system scope: the host may look for a decoding step's picks in pinned
+//    memory while the stream works on.
 __device__ __forceinline__ void store_pick(int32_t *at, int id) {
   __hip_atomic_store(at, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -605,7 +605,9 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
     return ((unsigned long long)(p + 1u) << 32) | (unsigned long long)(0xffffffffu - i);
   };
   auto emit = [&](int rd, unsigned long long b) {
-    store_pick(ids + (size_t)row * k + rd, (int)(0xffffffffu - (unsigned)(b & 0xffffffffu)));
+    const int id = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
+    if (PICK) store_pick(ids + (size_t)row * k + rd, id);
+    else ids[(size_t)row * k + rd] = id;
     if (ids2) ids2[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
     if (probs) probs[(size_t)row * k + rd] = h2f_((uint16_t)((b >> 32) - 1u));
   };
