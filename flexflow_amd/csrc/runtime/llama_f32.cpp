@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "logit_rows.h"
+#include "step_launch.h"
 #include "model.h"
 
 namespace ffmi {
@@ -369,7 +370,11 @@ struct LlamaF32 : public ffmi_model {
     if (T == 0) return FFMI_OK;
     // graphed at TP = 1 (the host-synchronising local group and the
     // transports stay eager here: this path is not the measured one)
-    const bool graph = use_graphs && !dbg && P == 1 && !few_rows;
+    double keys = 0;
+    for (const auto &w : ps.work) keys += w.kv_len;
+    // (7 launches a layer, and 3)
+    const double read = 4.0 * (c.num_layers * (4.0 * Hl * H + 3.0 * Fl * H + 2.0 * keys * Hl) + (double)V * H);
+    const bool graph = use_graphs && !dbg && P == 1 && !few_rows && !launch_one_by_one(read, 7 * c.num_layers + 3);
     if (graph) {
       const auto key = std::make_tuple(T, batch->num_work, batch->num_commits, k, batch->distinct_reqs, bytes);
       auto it = graphs.find(key);

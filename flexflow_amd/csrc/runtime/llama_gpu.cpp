@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "logit_rows.h"
+#include "step_launch.h"
 #include "model.h"
 #include "request_manager.h"  // (now_us)
 
@@ -52,6 +53,7 @@ struct LlamaGPU : public ffmi_model {
   // Infinity Cache (LLaMA-7B: 13.5 GB streamed once per step; the 68M SSM's
   // 87 MB stay cached from step to step and keep the default policy)
   int wstream = 0;
+  double weight_bytes = 0;
   hipStream_t stream = nullptr;
   std::vector<Layer> layers;
   uint16_t *embed = nullptr, *final_norm = nullptr, *lm = nullptr;
@@ -135,7 +137,7 @@ struct LlamaGPU : public ffmi_model {
   bool chain_ok = !getenv("FFMI_SSM_CHAIN") || atoi(getenv("FFMI_SSM_CHAIN")) != 0;
   // FFMI_INC_AHEAD=0: decoding steps one by one (A/B, tests)
   bool ahead_ok = !getenv("FFMI_INC_AHEAD") || atoi(getenv("FFMI_INC_AHEAD")) != 0;
-  bool ahead_step = false;  // (the step being launched is one)
+  bool slotted = false, ahead_step = false;  // (the step being launched has a slot of the two; is ahead)
   // the slot whose picks a step's negative token ids name (-1: none)
   int slot_before(int slot) const {
     return mode == FFMI_MODEL_INC ? (ids_dev ? 1 - slot : -1) : slot - 1;
@@ -549,6 +551,7 @@ struct LlamaGPU : public ffmi_model {
     {
       const double wbytes = 2.0 * c.num_layers * ((double)4 * Hl * H + 3.0 * Fl * H) +
                             2.0 * V * H;
+      weight_bytes = wbytes;
       wstream = wbytes > 192.0 * (1 << 20) ? FFMI_W_STREAM : 0;
       if (const char *e = getenv("FFMI_W_STREAM"))  // A/B override: 0 / 1
         wstream = atoi(e) ? FFMI_W_STREAM : 0;
@@ -987,7 +990,12 @@ struct LlamaGPU : public ffmi_model {
     // to enqueue it in, and a shape needs no second graph for the other slot's addresses.  16
     // decoding steps of a 768-channel model 1120 us so, 1155 with a graph for each slot)
     const bool second = mode == FFMI_MODEL_INC && cur_slot == 1;
-    const bool graph = !second && use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
+    // (5 launches a layer, and 3)
+    double keys = 0;
+    for (const auto &w : ps.work) keys += w.kv_len;
+    const bool eager = second || (mode != FFMI_MODEL_BEAM && o.tp_size == 1 &&
+                                  launch_one_by_one(weight_bytes + 4.0 * keys * Hl * c.num_layers, 5 * c.num_layers + 3));
+    const bool graph = !eager && use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
                        (o.tp_size == 1 || peer || rccl || ffmi::comm_size(o.comm) == 1) &&
                        !prof_on(0, T) &&
                        !prof_on(c.num_layers / 2, T);
@@ -1018,7 +1026,7 @@ struct LlamaGPU : public ffmi_model {
       FFMI_HIP(hipGraphLaunch(it->second, stream));
     } else {
       if (step_timing) FFMI_HIP(hipEventRecord(st_ev[0], stream));
-      st = enqueue(k, bytes, !second, T);
+      st = enqueue(k, bytes, !slotted, T);  // (a slot's step is waited for before the slot is staged again)
       if (st != FFMI_OK) return st;
     }
     if (step_timing) {
@@ -1421,9 +1429,9 @@ struct LlamaGPU : public ffmi_model {
     std::fill_n(ids, bc.num_tokens, -1);
     cur_slot = slot;
     batch = chain_batch[slot];
-    ahead_step = ahead;
+    slotted = true, ahead_step = ahead;
     const ffmi_status st = forward_launch(1);
-    ahead_step = false;
+    slotted = ahead_step = false;
     batch = chain_batch[0];
     cur_slot = 0;
     slot_results[slot] = st == FFMI_OK ? bc.num_tokens : 0;

@@ -1,6 +1,8 @@
 // paged_decoder.cpp -- see paged_decoder.h.
 #include "paged_decoder.h"
+#include "step_launch.h"
 
+#include <math.h>
 #include <algorithm>
 #include <memory>
 #include <set>
@@ -143,7 +145,13 @@ ffmi_status PagedDecoder::expert_matrices(const std::string &p, int experts, int
   return FFMI_OK;
 }
 
+double PagedDecoder::step_bytes(int T) const {
+  return (dense_bytes + expert_bytes * (1 - pow(1 - expert_share, T))) * (f32 ? 2 : 1);
+}
+
 void PagedDecoder::need_experts(MoeSizes n, int fp) {
+  expert_bytes += 6.0 * Wp * n.experts * fp;
+  expert_share = std::min(expert_share, (double)n.top / std::max(1, n.experts));
   for (n.T = 1; n.T <= Tm; ++n.T) {
     moe.num_units = std::max(moe.num_units, (size_t)n.slots() * fp);
     moe.num_slots = std::max(moe.num_slots, (size_t)n.slots());
@@ -210,6 +218,7 @@ ffmi_status PagedDecoder::init_step(const std::vector<RowShape> &shapes, int max
                                     const std::vector<std::pair<int, int>> &gemms,
                                     double weight_bytes) {
   // weights beyond the Infinity Cache: non-temporal loads, as the LLaMA model
+  dense_bytes = weight_bytes + 2.0 * Vp * Wp - expert_bytes;
   wstream = weight_bytes + 2.0 * Vp * Wp > 192.0 * (1 << 20) ? FFMI_W_STREAM : 0;
   const int positions = P > 0 ? std::min(P, o.max_seq_len) : o.max_seq_len;
   FFMI_TRY(step.init(Tm, o.max_requests, positions, shapes, max_slots));
@@ -304,7 +313,7 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
       const int s = bc.tokensInfo[t].request_index;
       states.begin(s, bc.requestsInfo[s].request_guid);
     }
-  if (use_graphs && !dbg && step.T <= 64) {
+  if (use_graphs && !dbg && step.T <= 64 && !launch_one_by_one(step_bytes(step.T), layer_launches * num_layers + 3)) {
     std::vector<int> key = step.shape;
     key.push_back(sample);
     auto it = graphs.find(key);

@@ -90,6 +90,11 @@ struct PagedDecoder : public ffmi_model {
     return FFMI_OK;
   }
   size_t es() const { return f32 ? 4 : 2; }
+  // what a step reads of its weights, for how it is launched (step_launch.h): all of them
+  // but the experts', of which its tokens touch a part
+  int layer_launches = 8;  // kernels of a layer's decoding step
+  double dense_bytes = 0, expert_bytes = 0, expert_share = 1;  // (share: of the experts that a token takes)
+  double step_bytes(int T) const;
   // the page pool, the step's metadata and the buffers above; gemms: the
   // products (N, K) whose fp32 sums pass through ws (ws_bytes: its least size)
   ffmi_status init_step(const std::vector<RowShape> &shapes, int max_slots,
