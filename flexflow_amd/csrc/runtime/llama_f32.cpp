@@ -368,7 +368,7 @@ struct LlamaF32 : public ffmi_model {
     ffmi_status st = batch_stage(batch, &desc, &bytes);
     if (st != FFMI_OK) return st;
     if (T == 0) return FFMI_OK;
-    // graphed at TP = 1 (the host-synchronising local group and the
+    // graphed at TP = 1, unless the launches are long (step_launch.h) (the host-synchronising local group and the
     // transports stay eager here: this path is not the measured one)
     double keys = 0;
     for (const auto &w : ps.work) keys += w.kv_len;

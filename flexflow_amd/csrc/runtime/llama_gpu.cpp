@@ -985,7 +985,8 @@ struct LlamaGPU : public ffmi_model {
     probs_h = reinterpret_cast<float *>(ids_h + cur_slot * slot_ints() + (size_t)(few_rows ? few_n : T) * k);
     // graphed: small steps, and tree-verify steps of one work item per
     // request (a fixed shape while the batch is full: T = 168 for 8 requests
-    // of 21 tree tokens); prefill blocks stay eager (one-off shapes)
+    // of 21 tree tokens), unless their launches are long (step_launch.h); prefill blocks
+    // stay eager (one-off shapes)
     // (every other decoding step launched ahead goes without one: the host has a step's time
     // to enqueue it in, and a shape needs no second graph for the other slot's addresses.  16
     // decoding steps of a 768-channel model 1120 us so, 1155 with a graph for each slot)
@@ -1441,7 +1442,10 @@ struct LlamaGPU : public ffmi_model {
   // scope).  An event behind every step would be waited for by the GPU, too.  (The stream
   // is asked now and then, so that one in error ends the wait.)
   ffmi_status inc_collect(int slot, int32_t *out) override {
-    if (!out) return forward_finish();
+    if (!out) {  // (a launch that failed has left nothing to finish, but a step ahead of it may run)
+      if (ids_dev) FFMI_HIP(hipStreamSynchronize(stream));
+      return forward_finish(ids_dev != nullptr);
+    }
     const int32_t *ids = ids_h + slot * slot_ints();
     for (size_t i = 0; i < slot_results[slot]; ++i) {
       for (int spins = 1; (out[i] = __atomic_load_n(ids + i, __ATOMIC_ACQUIRE)) < 0; ++spins) {

@@ -184,7 +184,8 @@ struct PagedDecoder : public ffmi_model {
   SafeTensors file;
   uint16_t *tmp = nullptr;  // one raw tensor while loading
   size_t tmp_elems = 0;
-  // decode steps replay a captured graph per launch shape
+  // decode steps replay a captured graph per launch shape, unless their launches are long
+  // (step_launch.h)
   std::map<std::vector<int>, hipGraphExec_t> graphs;
   bool use_graphs = getenv("FFMI_NO_GRAPHS") == nullptr;
   // tensor capture (set_debug): the residual stream after every layer

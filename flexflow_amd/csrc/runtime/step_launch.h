@@ -13,7 +13,8 @@ namespace ffmi {
 // 11760 / 11690, 1 request 12250 / 12150.  2048: LLaMA, 4 requests of 1500 tokens (30) 11970 / 11850, in full
 // precision (29) 5920 / 5880, Pekarax, 38 tokens a step (24) 7190 / 7000; but LLaMA, 1 request (21) 6600 / 6650
 // and 6610 / 6560 on another machine, Fesenex, 1 request (17) 5950 / 6050, Vapipel (7) 6260 / 6860, and of 1024
-// channels (2 - 4) 4370 / 5210 and 4440 / 5580.  Not where threads are to yield or sleep (FFMI_SYNC): a graph
+// channels (2 - 4) 4370 / 5210 and 4440 / 5580.  (On a third machine Fesenex's and Pekarax's were the same
+// either way.)  Not where threads are to yield or sleep (FFMI_SYNC): a graph
 // costs the host less.
 // FFMI_STEP_GRAPHS: 1 always graphs, 0 never (A/B, tests; read per call)
 inline bool launch_one_by_one(double bytes, int launches) {
