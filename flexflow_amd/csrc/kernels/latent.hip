@@ -156,17 +156,17 @@ __device__ __forceinline__ void head_gemm_tile(const HgDev &a, int b, uint16_t *
           (__attribute__((address_space(3))) void *)(sh + c * 8192 + (wave * 4 + i) * 512), 16, 0, 0);
     }
   };
-  const uint16_t *w0[4];
+  const uint16_t *w0[4];  // (the wave's; a lane's 16 bytes are lane * 8 on)
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    w0[j] = a.W + ((size_t)h * a.NTt + min(nt0 + wn * 4 + j, a.NTt - 1)) * a.KT * 512 + lane * 8;
+    w0[j] = a.W + ((size_t)h * a.NTt + min(nt0 + wn * 4 + j, a.NTt - 1)) * a.KT * 512;
   constexpr int WB = KC <= 2 ? 1 : 2;
   bf8 w[WB][2][4];
   auto weights = [&](int c) {
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[c % WB][k][j] = *reinterpret_cast<const bf8 *>(w0[j] + (size_t)(2 * c + k) * 512);
+      for (int j = 0; j < 4; ++j) w[c % WB][k][j] = *reinterpret_cast<const bf8 *>(w0[j] + (2 * c + k) * 512 + lane * 8);
   };
   f4 acc[4][4];
 #pragma unroll
