@@ -280,13 +280,11 @@ struct FuseArgs {
 // r = res_in + half(sum of the S slabs [S][T][NP]) -> res_out (another buffer: every
 // workgroup reads res_in), X = half(half(r * rms) * wnorm).  T <= 2 rows of up to 1024
 // columns, S <= 16.
-struct SumNormArgs {
-  const uint16_t *res_in;  // [T][K]
-  const float *sums;
-  int S, NP;
-  const uint16_t *wnorm;  // [K]
-  uint16_t *res_out;      // [T][K]
-  float eps;
+// (res_in, wnorm and eps are FuseArgs')
+struct SumNormArgs : FuseArgs {
+  const float *sums = nullptr;
+  int S = 0, NP = 0;
+  uint16_t *res_out = nullptr;  // [T][K]
 };
 // whether launch_gemm_sum_norm takes a product (else the norm is a launch of its own)
 bool gemm_sum_norm_fits(int T, int N, int K, int epilogue, const Partials &sums);

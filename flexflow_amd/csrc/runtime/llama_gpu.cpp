@@ -1165,8 +1165,10 @@ struct LlamaGPU : public ffmi_model {
     };
     auto norm_gemm = [&](const ffmi::Partials &part, const uint16_t *wn, const uint16_t *W, uint16_t *Y, int N,
                          int epi) -> ffmi_status {
-      FFMI_HIP(ffmi::launch_gemm_sum_norm(ffmi::SumNormArgs{rs, part.p, part.S, part.NP, wn, rs_to, eps}, W, Y, T, N,
-                                          H, epi, stream));
+      ffmi::SumNormArgs a;
+      a.res_in = rs, a.wnorm = wn, a.eps = eps;
+      a.sums = part.p, a.S = part.S, a.NP = part.NP, a.res_out = rs_to;
+      FFMI_HIP(ffmi::launch_gemm_sum_norm(a, W, Y, T, N, H, epi, stream));
       std::swap(rs, rs_to);
       return FFMI_OK;
     };
