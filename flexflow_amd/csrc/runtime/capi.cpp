@@ -39,6 +39,7 @@ extern "C" long ffmi_model_debug_tensor(ffmi_model *m, int which, int layer, flo
 }
 
 extern "C" long ffmi_model_debug_graphs(ffmi_model *m) { return m ? m->debug_graphs() : -1; }
+extern "C" long ffmi_model_debug_count(ffmi_model *m, int what) { return m ? m->debug_count(what) : -1; }
 
 extern "C" long ffmi_model_debug_width(ffmi_model *m, int which) {
   if (!m) return -1;

@@ -138,6 +138,17 @@ struct LlamaGPU : public ffmi_model {
   // FFMI_INC_AHEAD=0: decoding steps one by one (A/B, tests)
   bool ahead_ok = !getenv("FFMI_INC_AHEAD") || atoi(getenv("FFMI_INC_AHEAD")) != 0;
   bool slotted = false, ahead_step = false;  // (the step being launched has a slot of the two; is ahead)
+  // A step whose requests may all end by the picks ahead of it goes on the stream in two
+  // parts (inc_launch, inc_continue): up to a layer's qkv product, and the rest.
+  enum Part { kWhole, kFirst, kRest };
+  Part step_part = kWhole;
+  struct Begun {  // what the rest takes from the first part
+    int layer = 0;
+    size_t bytes = 0;
+    uint16_t *rs = nullptr, *rs_to = nullptr;
+    ffmi::Partials qkv;
+  } begun;
+  long counts[3] = {0, 0, 0};  // FFMI_COUNT_*
   // the slot whose picks a step's negative token ids name (-1: none)
   int slot_before(int slot) const {
     return mode == FFMI_MODEL_INC ? (ids_dev ? 1 - slot : -1) : slot - 1;
@@ -990,7 +1001,12 @@ struct LlamaGPU : public ffmi_model {
     // (every other decoding step launched ahead goes without one: the host has a step's time
     // to enqueue it in, and a shape needs no second graph for the other slot's addresses.  16
     // decoding steps of a 768-channel model 1120 us so, 1155 with a graph for each slot)
-    const bool second = mode == FFMI_MODEL_INC && cur_slot == 1;
+    const bool second = (mode == FFMI_MODEL_INC && cur_slot == 1) || step_part != kWhole;
+    if (step_part == kFirst) {
+      const int launches = 5 * c.num_layers + 3;
+      begun.layer = launches > 16 && weight_bytes < 8e6 * launches ? 2 : 0;
+      begun.bytes = bytes;
+    }
     // (5 launches a layer, and 3)
     double keys = 0;
     for (const auto &w : ps.work) keys += w.kv_len;
@@ -1001,30 +1017,10 @@ struct LlamaGPU : public ffmi_model {
                        !prof_on(0, T) &&
                        !prof_on(c.num_layers / 2, T);
     if (graph) {
-      const GraphKey key{T, batch->num_work, batch->num_commits, k, tree_parity,
-                         batch->commit_overlap ? 1 : 0,
-                         attn_form(T),
-                         batch->max_q, cur_slot, bytes};
-      auto it = graphs.find(key);
-      if (it == graphs.end()) {
-        if (graphs.size() >= 512) clear_graphs();
-        hipGraph_t g = nullptr;
-        FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        st = enqueue(k, bytes, false, T);
-        const hipError_t ce = hipStreamEndCapture(stream, &g);
-        if (st != FFMI_OK || ce != hipSuccess) {
-          if (g) (void)hipGraphDestroy(g);
-          if (st != FFMI_OK) return st;
-          FFMI_HIP(ce);
-        }
-        hipGraphExec_t ex = nullptr;
-        const hipError_t ie = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        FFMI_HIP(ie);
-        it = graphs.emplace(key, ex).first;
-      }
+      hipGraphExec_t ex = nullptr;
+      if ((st = step_graph(k, bytes, T, &ex)) != FFMI_OK) return st;
       if (step_timing) FFMI_HIP(hipEventRecord(st_ev[0], stream));
-      FFMI_HIP(hipGraphLaunch(it->second, stream));
+      FFMI_HIP(hipGraphLaunch(ex, stream));
     } else {
       if (step_timing) FFMI_HIP(hipEventRecord(st_ev[0], stream));
       st = enqueue(k, bytes, !slotted, T);  // (a slot's step is waited for before the slot is staged again)
@@ -1035,6 +1031,34 @@ struct LlamaGPU : public ffmi_model {
       st_t1 = now_us();
     }
     inflight = true;
+    counts[FFMI_COUNT_STEPS] += step_part == kWhole;
+    return FFMI_OK;
+  }
+
+  // the graph of a step, or of its last part (captured when there is none)
+  ffmi_status step_graph(int k, size_t bytes, int T, hipGraphExec_t *ex) {
+    const GraphKey key{T, batch->num_work, batch->num_commits, k, tree_parity,
+                       batch->commit_overlap ? 1 : 0,
+                       attn_form(T),
+                       batch->max_q, step_part == kRest ? 2 + cur_slot : cur_slot, bytes};
+    auto it = graphs.find(key);
+    if (it == graphs.end()) {
+      if (graphs.size() >= 512) clear_graphs();
+      hipGraph_t g = nullptr;
+      FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+      const ffmi_status st = enqueue(k, bytes, false, T);
+      const hipError_t ce = hipStreamEndCapture(stream, &g);
+      if (st != FFMI_OK || ce != hipSuccess) {
+        if (g) (void)hipGraphDestroy(g);
+        if (st != FFMI_OK) return st;
+        FFMI_HIP(ce);
+      }
+      const hipError_t ie = hipGraphInstantiate(ex, g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      FFMI_HIP(ie);
+      it = graphs.emplace(key, *ex).first;
+    }
+    *ex = it->second;
     return FFMI_OK;
   }
 
@@ -1126,6 +1150,7 @@ struct LlamaGPU : public ffmi_model {
   }
 
   long debug_graphs() const override { return (long)(graphs.size() + group_graphs.size()); }
+  long debug_count(int what) const override { return what >= 0 && what < 3 ? counts[what] : -1; }
   void clear_graphs() {
     for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
     graphs.clear();
@@ -1143,7 +1168,7 @@ struct LlamaGPU : public ffmi_model {
   do { if ((st = (x)) != FFMI_OK) return st; } while (0)
     // the step's blob: fetched by the first kernel from the mapped staging
     // (default), or a separate H2D copy (FFMI_BLOB_FETCH=0: A/B)
-    if (!blob_fetch) TRY(ffmi::batch_copy(batch, blob_bytes, stream, record_upload));
+    if (!blob_fetch && step_part != kRest) TRY(ffmi::batch_copy(batch, blob_bytes, stream, record_upload));
     const bool ptail = prof_on(0, T);
     int pr = 0;
     ffmi::Partials down_part;
@@ -1158,7 +1183,7 @@ struct LlamaGPU : public ffmi_model {
     // the residual norms inside the transport's all-reduces (tp_fuse_norm)
     const bool arn = peer && !solo && o.tp_size > 1 && (tp_fuse_norm == 2 || (tp_fuse_norm == 1 && !dbg));
     // The residual: a norm in a product's prologue leaves the new one in the other buffer.
-    uint16_t *rs = res, *rs_to = res2;
+    uint16_t *rs = step_part == kRest ? begun.rs : res, *rs_to = step_part == kRest ? begun.rs_to : res2;
     // the norm of the slabs `part` rides in the launch of the product behind it
     auto takes_norm = [&](const ffmi::Partials &part, int N, int epi) {
       return rs_to && !fuse && !arn && !dbg && o.tp_size == 1 && ffmi::gemm_sum_norm_fits(T, N, H, epi, part);
@@ -1170,9 +1195,10 @@ struct LlamaGPU : public ffmi_model {
       a.sums = part.p, a.S = part.S, a.NP = part.NP, a.res_out = rs_to;
       FFMI_HIP(ffmi::launch_gemm_sum_norm(a, W, Y, T, N, H, epi, stream));
       std::swap(rs, rs_to);
+      ++counts[FFMI_COUNT_MADE_NORMS];
       return FFMI_OK;
     };
-    for (int l = 0; l < c.num_layers; ++l) {
+    for (int l = step_part == kRest ? begun.layer : 0; l < c.num_layers; ++l) {
       Layer &L = layers[l];
       const bool on = prof_on(l, T);
       const bool mark_on = marker_h == c.hidden && l == c.num_layers - 1 && (!marker_t || T == marker_t);
@@ -1203,8 +1229,8 @@ struct LlamaGPU : public ffmi_model {
         fz_qkv.wnorm = L.in_norm, fz_gu.wnorm = L.post_norm;
         fz_qkv.eps = fz_gu.eps = eps;
       }
-      const bool nq = l > 0 && takes_norm(down_part, 3 * Hl, XP);
-      if (!nq && !fz_in && !(arn && l > 0)) {  // (arn: the previous down all-reduce normalised)
+      const bool nq = l > 0 && takes_norm(down_part, 3 * Hl, XP), rest = step_part == kRest && l == begun.layer;
+      if (!rest && !nq && !fz_in && !(arn && l > 0)) {  // (arn: the previous down all-reduce normalised)
         pr = prof_begin(on);
         // layer 0: the embedding lookup gathers straight into the first norm
         // (embedding_kernels.cu:233-244; res = the looked-up rows)
@@ -1228,7 +1254,9 @@ struct LlamaGPU : public ffmi_model {
       }
       pr = prof_begin(on);
       ffmi::Partials qkv_part;
-      if (nq)
+      if (rest)
+        qkv_part = begun.qkv;
+      else if (nq)
         TRY(norm_gemm(down_part, L.in_norm, L.wqkv, qkv, 3 * Hl, XP));
       else
         FFMI_HIP(ffmi::launch_gemm(fz_in && !packed ? res : h, L.wqkv, qkv, (float *)ws, ws_bytes, T, 3 * Hl, H,
@@ -1236,6 +1264,10 @@ struct LlamaGPU : public ffmi_model {
                                    fz_in ? &fz_qkv : nullptr));
       prof_end(pr, GEMM_QKV, gemm_bytes(T, 3 * Hl, 3 * Hl, H), 2.0 * T * 3 * Hl * H);
       mk();
+      if (step_part == kFirst && l == begun.layer) {
+        begun.rs = rs, begun.rs_to = rs_to, begun.qkv = qkv_part;
+        return FFMI_OK;
+      }
       if (dbg) TRY(dbg_gemm_out(FFMI_DBG_QKV, l, qkv, qkv_part, T));
       pr = prof_begin(on);
       ffmi::OprojArgs oa = oproj_args(L, T);
@@ -1425,20 +1457,49 @@ struct LlamaGPU : public ffmi_model {
     flags &= hipDeviceScheduleMask;
     return flags != hipDeviceScheduleYield && flags != hipDeviceScheduleBlockingSync;
   }
-  ffmi_status inc_launch(const BatchConfig &bc, int slot, bool ahead) override {
+  ffmi_status inc_launch(const BatchConfig &bc, int slot, bool ahead, bool whole) override {
     FFMI_CHECK((slot == 0 || slot == 1) && can_launch_ahead(bc.num_tokens), FFMI_ERR_INVALID);
     pack_inc(bc, o.max_requests, slots, &ps);
     int32_t *ids = ids_h + slot * slot_ints();
     std::fill_n(ids, bc.num_tokens, -1);
     cur_slot = slot;
     batch = chain_batch[slot];
-    slotted = true, ahead_step = ahead;
+    slotted = true, ahead_step = ahead, step_part = whole ? kWhole : kFirst;
     const ffmi_status st = forward_launch(1);
-    slotted = ahead_step = false;
+    slotted = ahead_step = false, step_part = kWhole;
     batch = chain_batch[0];
     cur_slot = 0;
     slot_results[slot] = st == FFMI_OK ? bc.num_tokens : 0;
+    counts[FFMI_COUNT_AHEAD] += ahead && st == FFMI_OK;
     return st;
+  }
+  // The first part runs while the host looks at the picks and launches the rest: kernel by
+  // kernel behind the first layer's qkv product (9 us of 768 channels, 24 of 4096), or, where
+  // there are many launches under 8 MB each (the host would not keep ahead of them), as a
+  // graph behind the third's.  Calls that a token ends, steps one by one / whole steps ahead / in
+  // parts (us): 4096 channels, 32 layers, 3 tokens 8632 / 11243 / 8635, 16 tokens 42790 / 45260 /
+  // 42540; 2048, 8 layers, 3 tokens 1212 / 1541 / 1206, 16 tokens 6015 / 6103 / 5778; 768, 2 layers, 16
+  // tokens 1265 / 1074 / 1022 (as a graph 1106).  57 tokens whose ends are not met, 256 channels, 24
+  // layers 24650 / 23820 / 23920 (kernel by kernel 27100), 1024 channels 29800 / 28820 / 28800 (30500).
+  ffmi_status inc_continue(int slot) override {
+    FFMI_CHECK(slot == 0 || slot == 1, FFMI_ERR_INVALID);
+    cur_slot = slot;
+    batch = chain_batch[slot];
+    step_part = kRest;
+    const ffmi_status st = launch_rest((int)slot_results[slot]);
+    step_part = kWhole;
+    batch = chain_batch[0];
+    cur_slot = 0;
+    counts[FFMI_COUNT_STEPS] += st == FFMI_OK;
+    return st;
+  }
+  ffmi_status launch_rest(int T) {
+    if (begun.layer == 0) return enqueue(1, begun.bytes, false, T);
+    hipGraphExec_t ex = nullptr;
+    const ffmi_status st = step_graph(1, begun.bytes, T, &ex);
+    if (st != FFMI_OK) return st;
+    FFMI_HIP(hipGraphLaunch(ex, stream));
+    return FFMI_OK;
   }
   // A row's pick is there when it is no longer -1 (the sampling kernel stores it at system
   // scope).  An event behind every step would be waited for by the GPU, too.  (The stream

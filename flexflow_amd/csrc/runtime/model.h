@@ -97,13 +97,19 @@ struct ffmi_model {
   // goes on the stream before the step ahead of it has been waited for, with token id
   // -1 - i where its token is row i's pick of that step (the device fills it in).  Two
   // slots, used in turn; inc_collect waits for a slot's step and gives its rows' picks
-  // (ids: null: everything launched is waited for, nothing is read).
+  // (ids: null: everything launched is waited for, nothing is read).  Where the picks may
+  // end every request of it, the step is launched in part (whole = false), so far that the
+  // GPU has work while the host looks; inc_continue launches the rest, or nothing does.
   virtual bool can_launch_ahead(int num_tokens) const {
     (void)num_tokens;
     return false;
   }
-  virtual ffmi_status inc_launch(const ffmi::BatchConfig &bc, int slot, bool ahead) {
-    (void)bc, (void)slot, (void)ahead;
+  virtual ffmi_status inc_launch(const ffmi::BatchConfig &bc, int slot, bool ahead, bool whole) {
+    (void)bc, (void)slot, (void)ahead, (void)whole;
+    return FFMI_ERR_UNSUPPORTED;
+  }
+  virtual ffmi_status inc_continue(int slot) {
+    (void)slot;
     return FFMI_ERR_UNSUPPORTED;
   }
   virtual ffmi_status inc_collect(int slot, int32_t *ids) {
@@ -159,6 +165,10 @@ struct ffmi_model {
     return -1;
   }
   virtual long debug_graphs() const { return -1; }
+  virtual long debug_count(int what) const {
+    (void)what;
+    return -1;
+  }
 };
 
 namespace ffmi {

@@ -153,6 +153,7 @@ class RequestManager {
 
   ffmi_status serve_incr_decoding(ffmi_model *llm);
   bool next_decode_batch(ffmi_model *llm, const BatchConfig &bc, const std::vector<int> &rows, BatchConfig *next);
+  bool goes_on(const BatchConfig &ahead, const std::vector<int32_t> &ids) const;
   ffmi_status serve_spec_infer(ffmi_model *llm);
   // replay of given tokens (include/ffmi.h ffmi_rm_replay_step)
   ffmi_status replay_step(ffmi_model *llm, const ffmi_replay_entry *entries, int n, float *logits,

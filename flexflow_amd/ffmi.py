@@ -35,6 +35,7 @@ F16, F32, I32 = 0, 1, 2
 # synthetic weight inits (ffmi_model_opts.weight_init) and fault kinds
 WEIGHT_INITS = {"uniform": 0, "depth_scaled": 1, "token_chain": 2}
 FAULT_NONE, FAULT_ROPE_POS, FAULT_RESID_ROUND, FAULT_TP_HEAD_SWAP, FAULT_TP_AR_DROP = 0, 1, 2, 3, 4
+COUNT_STEPS, COUNT_AHEAD, COUNT_MADE_NORMS = 0, 1, 2  # ffmi_model_debug_count
 # flagged SpecInfer extensions (include/ffmi.h FFMI_SPEC_EXT_*)
 SPEC_EXT_WIDTH4, SPEC_EXT_MULTI_SSM = 1, 2
 ATTN_QTILE = 32
@@ -208,6 +209,7 @@ SIGNATURES = {
     "ffmi_model_debug_tensor": (ctypes.c_long, [c_void_p, c_int, c_int, c_void_p, ctypes.c_long]),
     "ffmi_model_debug_width": (ctypes.c_long, [c_void_p, c_int]),
     "ffmi_model_debug_graphs": (ctypes.c_long, [c_void_p]),
+    "ffmi_model_debug_count": (ctypes.c_long, [c_void_p, c_int]),
     "ffmi_model_debug_fault": (c_int, [c_void_p, c_int, c_int, c_int]),
     "ffmi_set_device": (c_int, [c_int]),
     "ffmi_rm_create": (c_int, [ctypes.POINTER(RMConfig), ctypes.POINTER(c_void_p)]),

@@ -509,6 +509,14 @@ long ffmi_model_debug_tensor(ffmi_model *m, int which, int layer, float *out, lo
 long ffmi_model_debug_width(ffmi_model *m, int which);
 /* Test hook: step graphs that the model holds (-1: this kind of model does not say). */
 long ffmi_model_debug_graphs(ffmi_model *m);
+/* Test hook: how often the model has taken a path (-1: this kind of model does not say).
+ *   FFMI_COUNT_STEPS: steps put on the stream to their end;
+ *   FFMI_COUNT_AHEAD: decoding steps begun ahead of the picks they continue;
+ *   FFMI_COUNT_MADE_NORMS: norms launched, or captured, as part of a product. */
+#define FFMI_COUNT_STEPS 0
+#define FFMI_COUNT_AHEAD 1
+#define FFMI_COUNT_MADE_NORMS 2
+long ffmi_model_debug_count(ffmi_model *m, int what);
 /* Negative-control fault injection (tests only; never set in serving): the
  * parity tests must FAIL on a model with a deliberate bug.
  *   FFMI_FAULT_ROPE_POS, layer, arg: that layer's RoPE rotates tokens at

@@ -47,3 +47,35 @@ def test_refuses_tokens_out_of_range_behind_steps_launched_ahead():
         assert len(fa.generate(rm, m, [[5, 6, 7]], max_length=30)[0].output_tokens) == 30
         with pytest.raises(F.FFMIError):
             rm.replay_step(m, [(1, [9, bad], [1])])
+
+
+# (5 layers: many short launches, whose last part is a graph)
+@pytest.mark.parametrize("requests,layers", [(1, 2), (4, 2), (1, 5), (4, 5)])
+def test_no_step_for_nobody(requests, layers, monkeypatch):
+    """A call that tokens end runs as many steps to their end as one by one: none for nobody."""
+    prompts = [[(37 * i + 11 * r) % 480 + 5 for i in range(3 + r % 5)] for r in range(requests)]
+    runs = []
+    for ahead in ("0", "1"):
+        monkeypatch.setenv("FFMI_INC_AHEAD", ahead)
+        m = fa.Model(dict(CFG, num_layers=layers), "inc", max_requests=requests, max_tokens=64, max_seq_len=96,
+                     weight_seed=9)
+
+        def count(what):
+            return F.lib().ffmi_model_debug_count(m.handle, what)
+
+        def call(eos):
+            rm = fa.RequestManager(max_requests_per_batch=requests, max_tokens_per_batch=64, max_sequence_length=96,
+                                   eos_token_ids=eos)
+            before = [count(F.COUNT_STEPS), count(F.COUNT_AHEAD)]
+            guids = [rm.register_new_request(p, max_length=60) for p in prompts]
+            rm.serve_incr_decoding(m)
+            return ([rm.get_generation_result(g).output_tokens for g in guids], count(F.COUNT_STEPS) - before[0],
+                    count(F.COUNT_AHEAD) - before[1])
+        plain = call([])
+        gen = [t[-(60 - len(p) - 1):] for t, p in zip(plain[0], prompts)]
+        eos = sorted({max(set(g), key=g.index) for g in gen})  # (the latest to come first)
+        runs.append([plain, call(eos), call([499]), call(eos)])
+        assert all(len(t) < 60 for t in runs[-1][1][0])
+        assert (plain[2] > 0) == (runs[-1][1][2] > 0) == (ahead == "1")
+    for one, two in zip(*runs):
+        assert one[0] == two[0] and one[1] == two[1]
