@@ -1043,7 +1043,10 @@ struct LlamaGPU : public ffmi_model {
                        batch->max_q, step_part == kRest ? 2 + cur_slot : cur_slot, bytes};
     auto it = graphs.find(key);
     if (it == graphs.end()) {
-      if (graphs.size() >= 512) clear_graphs();
+      if (graphs.size() >= 512) {
+        FFMI_HIP(hipStreamSynchronize(stream));  // (a step ahead of this one may run from one)
+        clear_graphs();
+      }
       hipGraph_t g = nullptr;
       FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
       const ffmi_status st = enqueue(k, bytes, false, T);
