@@ -167,7 +167,6 @@ struct Fesenex : public PagedDecoder {
     }
     // 16-row slots for the splits of a step whose blocks do not fill the chip
     max_slots = rows_form || shapes.empty() ? 0 : 512 * kAttnTiles / min_groups;
-    layer_launches = 6;
     FFMI_TRY(init_step(shapes, max_slots, gemms, wbytes));
     FFMI_TRY(alloc_zero(&q, (size_t)Tm * qw * es()));
     FFMI_TRY(alloc_zero(&att, (size_t)Tm * ow * es()));

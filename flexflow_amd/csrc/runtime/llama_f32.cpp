@@ -60,13 +60,13 @@ struct LlamaF32 : public ffmi_model {
   ffmi_batch_dev *batch = nullptr;
   PackedStep ps;
   std::vector<void *> allocs;
-  std::map<std::tuple<int, int, int, int, bool, size_t>, hipGraphExec_t> graphs;
+  std::map<std::tuple<int, int, int, int, bool, size_t>, StepGraph> graphs;
   bool use_graphs = getenv("FFMI_NO_GRAPHS") == nullptr;
   int dbg = 0, dbg_T = -1;
 
   ~LlamaF32() override {
     if (stream) (void)hipStreamSynchronize(stream);
-    for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
+    clear_step_graphs(&graphs);
     for (auto &L : layers) ffmi_attn_destroy(L.attn);
     for (void *p : allocs) (void)hipFree(p);
     if (res_h) (void)hipHostFree(res_h);
@@ -368,37 +368,20 @@ struct LlamaF32 : public ffmi_model {
     ffmi_status st = batch_stage(batch, &desc, &bytes);
     if (st != FFMI_OK) return st;
     if (T == 0) return FFMI_OK;
-    // graphed at TP = 1, unless the launches are long (step_launch.h) (the host-synchronising local group and the
-    // transports stay eager here: this path is not the measured one)
+    // graphed at TP = 1, unless its launches are long (step_launch.h); the host-synchronising
+    // local group and the transports stay eager here: this path is not the measured one
     double keys = 0;
     for (const auto &w : ps.work) keys += w.kv_len;
-    // (7 launches a layer, and 3)
     const double read = 4.0 * (c.num_layers * (4.0 * Hl * H + 3.0 * Fl * H + 2.0 * keys * Hl) + (double)V * H);
-    const bool graph = use_graphs && !dbg && P == 1 && !few_rows && !launch_one_by_one(read, 7 * c.num_layers + 3);
-    if (graph) {
+    hipGraphExec_t graph = nullptr;
+    if (use_graphs && !dbg && P == 1 && !few_rows) {
       const auto key = std::make_tuple(T, batch->num_work, batch->num_commits, k, batch->distinct_reqs, bytes);
-      auto it = graphs.find(key);
-      if (it == graphs.end()) {
-        if (graphs.size() >= 256) {
-          for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
-          graphs.clear();
-        }
-        hipGraph_t g = nullptr;
-        FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-        st = enqueue(k, bytes, false);
-        const hipError_t ce = hipStreamEndCapture(stream, &g);
-        if (st != FFMI_OK || ce != hipSuccess) {
-          if (g) (void)hipGraphDestroy(g);
-          if (st != FFMI_OK) return st;
-          FFMI_HIP(ce);
-        }
-        hipGraphExec_t ex = nullptr;
-        const hipError_t ie = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        FFMI_HIP(ie);
-        it = graphs.emplace(key, ex).first;
-      }
-      FFMI_HIP(hipGraphLaunch(it->second, stream));
+      st = step_graph(&graphs, 256, key, read, 10 * c.num_layers + 5, stream,
+                      [&] { return enqueue(k, bytes, false); }, &graph);
+      if (st != FFMI_OK) return st;
+    }
+    if (graph) {
+      FFMI_HIP(hipGraphLaunch(graph, stream));
     } else {
       st = enqueue(k, bytes, true);
       if (st != FFMI_OK) return st;
@@ -448,6 +431,7 @@ struct LlamaF32 : public ffmi_model {
     return FFMI_OK;
   }
   int vocab_size() const override { return V; }
+  long debug_graphs() const override { return count_step_graphs(graphs); }
   ffmi_status run_inc_logits(const BatchConfig &bc, const int *rows, int n, float *out) override {
     if (mode != FFMI_MODEL_INC) return FFMI_ERR_INVALID;
     FFMI_CHECK(bc.num_tokens <= o.max_tokens, FFMI_ERR_INVALID);

@@ -919,7 +919,7 @@ struct LlamaGPU : public ffmi_model {
   // the next step read the half this one wrote); kept here so graph replays
   // and eager steps agree
   int tree_parity = 0;
-  std::map<GraphKey, hipGraphExec_t> graphs;
+  std::map<GraphKey, ffmi::StepGraph> graphs;
   // FFMI_CHAIN_GROUP=g (>= 2): chained beam slots 1 .. kChain-2 are staged and
   // go out g per graph launch (slot kChain-1 alone, behind the collect event):
   // the boundary between two graph launches (4.9 us from one step's last
@@ -1007,18 +1007,13 @@ struct LlamaGPU : public ffmi_model {
       begun.layer = launches > 16 && weight_bytes < 8e6 * launches ? 2 : 0;
       begun.bytes = bytes;
     }
-    // (5 launches a layer, and 3)
-    double keys = 0;
-    for (const auto &w : ps.work) keys += w.kv_len;
-    const bool eager = second || (mode != FFMI_MODEL_BEAM && o.tp_size == 1 &&
-                                  launch_one_by_one(weight_bytes + 4.0 * keys * Hl * c.num_layers, 5 * c.num_layers + 3));
-    const bool graph = !eager && use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
+    const bool graph = !second && use_graphs && !dbg && !few_rows && (T <= 64 || (batch->one_item_per_req && T <= graph_max_t)) &&
                        (o.tp_size == 1 || peer || rccl || ffmi::comm_size(o.comm) == 1) &&
                        !prof_on(0, T) &&
                        !prof_on(c.num_layers / 2, T);
-    if (graph) {
-      hipGraphExec_t ex = nullptr;
-      if ((st = step_graph(k, bytes, T, &ex)) != FFMI_OK) return st;
+    hipGraphExec_t ex = nullptr;
+    if (graph && (st = graph_of(k, bytes, T, &ex)) != FFMI_OK) return st;
+    if (ex) {
       if (step_timing) FFMI_HIP(hipEventRecord(st_ev[0], stream));
       FFMI_HIP(hipGraphLaunch(ex, stream));
     } else {
@@ -1035,34 +1030,19 @@ struct LlamaGPU : public ffmi_model {
     return FFMI_OK;
   }
 
-  // the graph of a step, or of its last part (captured when there is none)
-  ffmi_status step_graph(int k, size_t bytes, int T, hipGraphExec_t *ex) {
+  // the graph of a step, or of its last part; null: it goes kernel by kernel (step_launch.h)
+  ffmi_status graph_of(int k, size_t bytes, int T, hipGraphExec_t *ex) {
     const GraphKey key{T, batch->num_work, batch->num_commits, k, tree_parity,
                        batch->commit_overlap ? 1 : 0,
                        attn_form(T),
                        batch->max_q, step_part == kRest ? 2 + cur_slot : cur_slot, bytes};
-    auto it = graphs.find(key);
-    if (it == graphs.end()) {
-      if (graphs.size() >= 512) {
-        FFMI_HIP(hipStreamSynchronize(stream));  // (a step ahead of this one may run from one)
-        clear_graphs();
-      }
-      hipGraph_t g = nullptr;
-      FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      const ffmi_status st = enqueue(k, bytes, false, T);
-      const hipError_t ce = hipStreamEndCapture(stream, &g);
-      if (st != FFMI_OK || ce != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        if (st != FFMI_OK) return st;
-        FFMI_HIP(ce);
-      }
-      const hipError_t ie = hipGraphInstantiate(ex, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      FFMI_HIP(ie);
-      it = graphs.emplace(key, *ex).first;
-    }
-    *ex = it->second;
-    return FFMI_OK;
+    double keys = 0;
+    for (const auto &w : ps.work) keys += w.kv_len;
+    const bool may = mode != FFMI_MODEL_BEAM && o.tp_size == 1 && step_part == kWhole;
+    const double read = may ? weight_bytes + 4.0 * keys * Hl * c.num_layers : 0;
+    const int bound = fused_norms(T) ? 5 * c.num_layers + 4
+                                     : (7 + !batch->one_item_per_req + batch->commit_overlap) * c.num_layers + 3;
+    return ffmi::step_graph(&graphs, 512, key, read, bound, stream, [&] { return enqueue(k, bytes, false, T); }, ex);
   }
 
   // A chained slot staged for a grouped launch (chain_group): the staging
@@ -1152,11 +1132,10 @@ struct LlamaGPU : public ffmi_model {
     return FFMI_OK;
   }
 
-  long debug_graphs() const override { return (long)(graphs.size() + group_graphs.size()); }
+  long debug_graphs() const override { return ffmi::count_step_graphs(graphs) + (long)group_graphs.size(); }
   long debug_count(int what) const override { return what >= 0 && what < 3 ? counts[what] : -1; }
   void clear_graphs() {
-    for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
-    graphs.clear();
+    ffmi::clear_step_graphs(&graphs);
     for (auto &kv : group_graphs) (void)hipGraphExecDestroy(kv.second);
     group_graphs.clear();
   }
@@ -1499,8 +1478,8 @@ struct LlamaGPU : public ffmi_model {
   ffmi_status launch_rest(int T) {
     if (begun.layer == 0) return enqueue(1, begun.bytes, false, T);
     hipGraphExec_t ex = nullptr;
-    const ffmi_status st = step_graph(1, begun.bytes, T, &ex);
-    if (st != FFMI_OK) return st;
+    const ffmi_status st = graph_of(1, begun.bytes, T, &ex);
+    if (st != FFMI_OK || !ex) return st != FFMI_OK ? st : enqueue(1, begun.bytes, false, T);
     FFMI_HIP(hipGraphLaunch(ex, stream));
     return FFMI_OK;
   }

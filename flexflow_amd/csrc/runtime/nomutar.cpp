@@ -238,7 +238,6 @@ struct Nomutar : public PagedDecoder {
     }
     // 16-row slots for the splits of a step whose blocks do not fill the chip
     max_slots = rows_form ? 0 : 512 * kAttnTiles / min_groups;
-    layer_launches = 10;
     FFMI_TRY(init_step(shapes, max_slots, gemms, wbytes));
     FFMI_TRY(alloc_zero(&x2, (size_t)Tm * Wp * 4));
     xs[0] = x, xs[1] = x2;

@@ -1,6 +1,5 @@
 // paged_decoder.cpp -- see paged_decoder.h.
 #include "paged_decoder.h"
-#include "step_launch.h"
 
 #include <math.h>
 #include <algorithm>
@@ -11,7 +10,7 @@ namespace ffmi {
 
 PagedDecoder::~PagedDecoder() {
   if (stream) (void)hipStreamSynchronize(stream);
-  for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
+  clear_step_graphs(&graphs);
   for (void *p : allocs) (void)hipFree(p);
   if (tmp) (void)hipFree(tmp);
   if (res_h) (void)hipHostFree(res_h);
@@ -313,34 +312,15 @@ ffmi_status PagedDecoder::forward(const BatchConfig &bc, const int *rows, int n,
       const int s = bc.tokensInfo[t].request_index;
       states.begin(s, bc.requestsInfo[s].request_guid);
     }
-  if (use_graphs && !dbg && step.T <= 64 && !launch_one_by_one(step_bytes(step.T), layer_launches * num_layers + 3)) {
+  hipGraphExec_t graph = nullptr;
+  if (use_graphs && !dbg && step.T <= 64) {
     std::vector<int> key = step.shape;
     key.push_back(sample);
-    auto it = graphs.find(key);
-    if (it == graphs.end()) {
-      if (graphs.size() >= 256) {
-        for (auto &kv : graphs) (void)hipGraphExecDestroy(kv.second);
-        graphs.clear();
-      }
-      hipGraph_t g = nullptr;
-      FFMI_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      const ffmi_status st = enqueue(sample);
-      const hipError_t ce = hipStreamEndCapture(stream, &g);
-      if (st != FFMI_OK || ce != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        if (st != FFMI_OK) return st;
-        FFMI_HIP(ce);
-      }
-      hipGraphExec_t ex = nullptr;
-      const hipError_t ie = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      FFMI_HIP(ie);
-      it = graphs.emplace(key, ex).first;
-    }
-    FFMI_HIP(hipGraphLaunch(it->second, stream));
-  } else {
-    FFMI_TRY(enqueue(sample));
+    FFMI_TRY(step_graph(&graphs, 256, key, step_bytes(step.T), 20 * num_layers + 5, stream,
+                        [&] { return enqueue(sample); }, &graph));
   }
+  if (graph) FFMI_HIP(hipGraphLaunch(graph, stream));
+  else FFMI_TRY(enqueue(sample));
   // (the step is on the stream: it is waited for and counted whatever becomes of its rows)
   ffmi_status rows_st = sample ? FFMI_OK : logit_rows.begin(logits, false, Vp, nullptr, n, V, stream, out);
   if (!sample && rows_st == FFMI_OK) rows_st = logit_rows.finish();

@@ -19,6 +19,7 @@
 #include "paged_step.h"
 #include "safetensors.h"
 #include "state_slots.h"
+#include "step_launch.h"
 
 namespace ffmi {
 
@@ -92,7 +93,6 @@ struct PagedDecoder : public ffmi_model {
   size_t es() const { return f32 ? 4 : 2; }
   // what a step reads of its weights, for how it is launched (step_launch.h): all of them
   // but the experts', of which its tokens touch a part
-  int layer_launches = 8;  // kernels of a layer's decoding step
   double dense_bytes = 0, expert_bytes = 0, expert_share = 1;  // (share: of the experts that a token takes)
   double step_bytes(int T) const;
   // the page pool, the step's metadata and the buffers above; gemms: the
@@ -173,6 +173,7 @@ struct PagedDecoder : public ffmi_model {
     return which == FFMI_DBG_LOGITS ? V : which == FFMI_DBG_HIDDEN ? W : -1;
   }
   ffmi_status set_debug(int enable) override;
+  long debug_graphs() const override { return count_step_graphs(graphs); }
   long debug_tensor(int which, int layer, float *out, long cap) override;
 
   // a factory's body: options checked, `m` configured and initialised
@@ -186,7 +187,7 @@ struct PagedDecoder : public ffmi_model {
   size_t tmp_elems = 0;
   // decode steps replay a captured graph per launch shape, unless their launches are long
   // (step_launch.h)
-  std::map<std::vector<int>, hipGraphExec_t> graphs;
+  std::map<std::vector<int>, StepGraph> graphs;
   bool use_graphs = getenv("FFMI_NO_GRAPHS") == nullptr;
   // tensor capture (set_debug): the residual stream after every layer
   int dbg = 0, dbg_T = -1, dbg_R = 0;

@@ -235,7 +235,6 @@ struct Pekarax : public PagedDecoder {
     }
     // 16-row slots for the splits of a step whose blocks do not fill the chip
     max_slots = rows_form || shapes.empty() ? 0 : 512 * kAttnTiles / min_groups;
-    layer_launches = 13;
     FFMI_TRY(init_step(shapes, max_slots, gemms, wbytes));
     FFMI_TRY(alloc_zero(&q, (size_t)Tm * qw * es()));
     FFMI_TRY(alloc_zero(&cat, (size_t)Tm * cw * es()));

@@ -111,7 +111,6 @@ struct Vapipel : public PagedDecoder {
     bool rows_form = f32;  // some layer's attention takes unsplit blocks only
     for (const VapipelLayer &L : layers) rows_form |= !latent_rank_supported(L.rp);
     const int max_slots = rows_form ? 0 : kMaxSlots;
-    layer_launches = 9;
     FFMI_TRY(init_step(shapes, max_slots, gemms, wbytes));
     if (!f32) FFMI_TRY(alloc_zero(&xb, (size_t)Tm * Wp * 2));
     FFMI_TRY(alloc_zero(&qg, (size_t)Tm * nq * es()));
