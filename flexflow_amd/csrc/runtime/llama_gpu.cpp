@@ -1038,7 +1038,7 @@ struct LlamaGPU : public ffmi_model {
                        batch->max_q, step_part == kRest ? 2 + cur_slot : cur_slot, bytes};
     double keys = 0;
     for (const auto &w : ps.work) keys += w.kv_len;
-    const bool may = mode != FFMI_MODEL_BEAM && o.tp_size == 1 && step_part == kWhole;
+    const bool may = mode != FFMI_MODEL_BEAM && o.tp_size == 1;
     const double read = may ? weight_bytes + 4.0 * keys * Hl * c.num_layers : 0;
     const int bound = fused_norms(T) ? 5 * c.num_layers + 4
                                      : (7 + !batch->one_item_per_req + batch->commit_overlap) * c.num_layers + 3;

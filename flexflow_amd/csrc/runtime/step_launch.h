@@ -24,8 +24,9 @@ namespace ffmi {
 // the caller's fresh pages for their logits cost more beside a graph: with kept ones 6650 / 6510 and 11510 / 11320.)
 // Not where threads are to yield or sleep (FFMI_SYNC): a graph costs the host less.
 // FFMI_STEP_GRAPHS: 1 always graphs, 0 never (A/B, tests; read per call)
-// (bytes: what the step reads; launches: its kernels)
+// (bytes: what the step reads, 0: a graph whatever it is; launches: its kernels)
 inline bool launch_one_by_one(double bytes, int launches) {
+  if (bytes <= 0) return false;
   if (const char *e = getenv("FFMI_STEP_GRAPHS")) return !atoi(e);
   if (bytes < 16e6 * launches) return false;
   unsigned flags = 0;
