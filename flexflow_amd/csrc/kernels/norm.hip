@@ -374,6 +374,7 @@ hipError_t launch_silu_mul(const uint16_t *a, const uint16_t *b, uint16_t *out, 
 extern "C" __device__ float __ockl_wfred_max_f32(float);
 extern "C" __device__ double __ockl_wfred_add_f64(double);
 extern "C" __device__ unsigned long long __ockl_wfred_max_u64(unsigned long long);
+extern "C" __device__ unsigned __ockl_wfred_min_u32(unsigned);
 
 // softmax (fp16 output, softmax.cu:262-288) + ArgMax (argmax.cu:62-100) /
 // ArgTopK (arg_topk.cu:339-448), register-resident: one TPB-thread workgroup
@@ -407,14 +408,17 @@ extern "C" __device__ unsigned long long __ockl_wfred_max_u64(unsigned long long
 //    the oracle's serial loop): S = float(double sum) in any order, as above.
 //    `part` = [T][G] doubles, `cnt` = [T] counters, zero before the first
 //    launch and left zero.
-//  * PICK (k = 1, no probabilities wanted, G = 1): x < M has M's fp16 p only if
+//  * PICK (k = 1, no probabilities wanted): x < M has M's fp16 p only if
 //    p(M) - p(x) = (1 - exp(x - M)) / S is not above fp16's spacing at 1 / S, which is
 //    2^-10 / S at most, or 2^-24 where 1 / S is subnormal (S <= V <= 32768 here).  So a row whose logits
 //    other than M all lie further below it (1.1 times that: the float error of exp and the
 //    division is under 2^-20) is picked without S: no exp terms, no hand-off between
-//    workgroups.  One workgroup a row, V = 32000: 1 row 7.8 -> 3.8 us, 8 rows 8.2 -> 4.2,
-//    168 rows 12.2 -> 4.6.  Other rows, and rows with a NaN or without a finite M, take
-//    the whole path.
+//    workgroups (G > 1: each sees the same row, the first stores).  V = 32000: 1 row
+//    7.7 -> 4.0 us, 8 rows 8.1 -> 4.1, 168 rows 12.0 -> 4.6.  Other rows, and rows with a NaN
+//    or without a finite M, take the whole path in as many workgroups as without PICK, but for
+//    a thread's eight registers (V <= 8192), where the hand-off does not pay: logits of 1e-3, 1 row
+//    of 32000 7.7 -> 9.2 us (in one workgroup 12.6), of 2048 5.4 -> 5.0 (in four 6.0); a third
+//    of 32000 logits equal, others near them 21.3 -> 23.0.
 //  * PICK stores at system scope: the host may look for a decoding step's picks in pinned
 //    memory while the stream works on.
 __device__ __forceinline__ void store_pick(int32_t *at, int id) {
@@ -427,7 +431,6 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
     int32_t *__restrict__ ids2) {
   constexpr int NW = TPB / 64;
   constexpr int kCand = 128;
-  static_assert(!PICK || G == 1, "one workgroup a row");
   static_assert(G == 1 || ((NV * 8) % G == 0 && NV * 8 / G >= 2),
                 "split: whole dwords of a thread's elements per workgroup");
   constexpr int E = NV * 8 / G;  // elements of each thread's row part this workgroup sums
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
     const float tie = 1.1f * fmaxf(0x1p-10f, (float)V * 0x1p-24f);
     unsigned at = 0xffffffffu;
 #pragma unroll
-    for (int v = NV - 1; v >= 0; --v)  // (a thread's lowest index last)
+    for (int v = NV - 1; v >= 0; --v)  // (the first workgroup's threads: their lowest index last)
 #pragma unroll
       for (int e = 7; e >= 0; --e) {
         const float d = M - elem(v, e);
@@ -493,11 +496,14 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
         else odd |= d <= tie;
       }
     odd |= !(fabsf(M) < INFINITY);
-    if (at != 0xffffffffu) atomicMin(&first_max, at);
+    if (__any(at != 0xffffffffu)) {  // (one a wave: in a row of equal logits every lane has one)
+      at = __ockl_wfred_min_u32(at);
+      if (lane == 0) atomicMin(&first_max, at);
+    }
     if (__any(odd) && lane == 0) unclear = 1;
     __syncthreads();
     if (!unclear) {
-      if (tid == 0) {
+      if (tid == 0 && chunk == 0) {
         store_pick(ids + row, (int)first_max);
         if (ids2) ids2[row] = (int)first_max;
       }
@@ -838,17 +844,21 @@ hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *i
     return v == 256 || v == 512 ? v : 1024;
   }();
   const int nv = (V / 8 + tpb - 1) / tpb;
-  // (ids alone, one a row: no probabilities, no split)
-  const bool pick = k == 1 && !probs && tpb == 1024 && split_env < 0;
-  if (pick) G = 1;
+  const bool pick = k == 1 && !probs && tpb == 1024;  // (ids alone, one a row)
+  if (pick && nv <= 1) G = 1;  // (see the kernel)
   // (NV = 8 at 1024 threads would spill: larger vocabularies take the loop kernel)
   if (V % 8 == 0 && ((uintptr_t)logits & 15) == 0 && nv * tpb <= 4096) {
 #define FFMI_SMR(TPB, NV)                                                                  \
   hipLaunchKernelGGL((softmax_topk_reg_kernel<TPB, NV, 1>), dim3(T), dim3(TPB), 0, s, logits, V, \
                      k, ids, probs, nullptr, nullptr, ids2)
-#define FFMI_SMG(NV, GG)                                                                     \
-  hipLaunchKernelGGL((softmax_topk_reg_kernel<1024, NV, GG>), dim3(GG, T), dim3(1024), 0, s, \
+#define FFMI_SMG_AS(NV, GG, P)                                                                  \
+  hipLaunchKernelGGL((softmax_topk_reg_kernel<1024, NV, GG, P>), dim3(GG, T), dim3(1024), 0, s, \
                      logits, V, k, ids, probs, part, cnt, ids2)
+#define FFMI_SMG(NV, GG)                  \
+  do {                                    \
+    if (pick) FFMI_SMG_AS(NV, GG, true);  \
+    else FFMI_SMG_AS(NV, GG, false);      \
+  } while (0)
     const int gmax = 4 * std::max(1, nv);  // >= 2 of a thread's 8 NV elements per workgroup
     while (G > 1 && (G > gmax || (G & (G - 1)))) G >>= 1;
     if (tpb == 1024 && G > 1) {
@@ -888,6 +898,7 @@ hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *i
     }
 #undef FFMI_SMR
 #undef FFMI_SMG
+#undef FFMI_SMG_AS
   } else {
     hipLaunchKernelGGL(softmax_topk_kernel<1024>, dim3(T), dim3(1024), 0, s, logits, V, k, ids, probs,
                        ids2);

@@ -47,3 +47,25 @@ def test_rows_without_a_finite_maximum():
     F.check(F.lib().ffmi_argmax(lb.ptr, 5, 1000, ids.ptr, None, None))
     F.check(F.lib().ffmi_argmax(lb.ptr, 5, 1000, both.ptr, pr.ptr, None))
     assert ids.get().tolist() == both.get().tolist()
+
+
+# the forms of one to eight workgroups a row
+@pytest.mark.parametrize("V", [1000, 8200, 32000])
+@pytest.mark.parametrize("T", [1, 8, 33, 64, 65, 128, 129])
+def test_rows_that_may_tie_share_their_sums(T, V):
+    """Rows that need their sum of exponentials spread it over workgroups, as with probabilities (partial sums
+    in the workspace, behind 1 KB of counters that are left zero); the others need none."""
+    x, L = rows(V, np.random.default_rng(T)), F.lib()
+    close, equal, clear = x[8], x[6], x[5]
+    assert 0 < close.max() - np.unique(close)[-2] < 1e-3 and clear.max() - np.unique(clear)[-2] > 0.1
+    n = int(L.ffmi_arg_topk_workspace_bytes(T))
+    for row, sums in ((clear, False), (equal, False), (close, T <= 128 and V > 8192)):
+        lb, ids, both = Buf(np.tile(row, (T, 1))), Buf.empty((T,), np.int32), Buf.empty((T,), np.int32)
+        pr, ws, ws2 = Buf.empty((T,), np.float32), Buf(np.zeros(n, np.uint8)), Buf(np.zeros(n, np.uint8))
+        F.check(L.ffmi_arg_topk_ws(lb.ptr, T, V, 1, ids.ptr, None, ws.ptr, n, None))
+        F.check(L.ffmi_arg_topk_ws(lb.ptr, T, V, 1, both.ptr, pr.ptr, ws2.ptr, n, None))
+        assert ids.get().tolist() == both.get().tolist()
+        got, whole = ws.get(), ws2.get()
+        assert not got[:1024].any() and not whole[:1024].any()
+        assert got[1024:].any() == sums
+        assert not sums or np.array_equal(got, whole)
