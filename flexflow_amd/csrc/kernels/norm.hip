@@ -419,8 +419,8 @@ extern "C" __device__ unsigned __ockl_wfred_min_u32(unsigned);
 //    a thread's eight registers (V <= 8192), where the hand-off does not pay: logits of 1e-3, 1 row
 //    of 32000 7.7 -> 9.2 us (in one workgroup 12.6), of 2048 5.4 -> 5.0 (in four 6.0); a third
 //    of 32000 logits equal, others near them 21.3 -> 23.0.
-//  * PICK stores at system scope: the host may look for a decoding step's picks in pinned
-//    memory while the stream works on.
+//  * Picks without probabilities are stored at system scope, whatever the form: the host may
+//    look for a decoding step's in pinned memory while the stream works on (launch_argmax).
 __device__ __forceinline__ void store_pick(int32_t *at, int id) {
   __hip_atomic_store(at, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -612,8 +612,8 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
   };
   auto emit = [&](int rd, unsigned long long b) {
     const int id = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
-    if (PICK) store_pick(ids + (size_t)row * k + rd, id);
-    else ids[(size_t)row * k + rd] = id;
+    if (probs) ids[(size_t)row * k + rd] = id;
+    else store_pick(ids + (size_t)row * k + rd, id);
     if (ids2) ids2[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
     if (probs) probs[(size_t)row * k + rd] = h2f_((uint16_t)((b >> 32) - 1u));
   };
