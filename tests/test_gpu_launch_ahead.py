@@ -1,5 +1,6 @@
 """Decoding steps launched ahead of the picks they continue give the tokens of steps run one by
 one: requests that end by length and by token while others go on, more of them than slots."""
+import numpy as np
 import pytest
 
 import flexflow_amd as fa
@@ -11,7 +12,12 @@ CFG = dict(num_layers=2, vocab_size=500, num_heads=2, num_kv_heads=2, hidden=128
            rms_eps=1e-6, rope_theta=10000.0)
 
 
+def ahead(m):
+    return F.lib().ffmi_model_debug_count(m.handle, F.COUNT_AHEAD)
+
+
 def tokens(slots, prompts, lengths, eos):
+    """The tokens of two passes, and whether steps were launched ahead."""
     m = fa.Model(CFG, "inc", max_requests=slots, max_tokens=64, max_seq_len=96, weight_seed=9)
     out = []
     for _ in range(2):  # (on what the first pass left behind, too)
@@ -20,7 +26,7 @@ def tokens(slots, prompts, lengths, eos):
         guids = [rm.register_new_request(p, max_length=n) for p, n in zip(prompts, lengths)]
         rm.serve_incr_decoding(m)
         out.append([rm.get_generation_result(g).output_tokens for g in guids])
-    return out
+    return out, ahead(m) > 0
 
 
 @pytest.mark.parametrize("slots,requests", [(1, 1), (1, 3), (4, 3), (4, 4), (4, 7), (20, 20)])
@@ -29,15 +35,17 @@ def test_same_tokens_as_one_by_one(slots, requests, monkeypatch):
     lengths = [min(96, len(p) + (3, 40, 2, 17, 60)[r % 5]) for r, p in enumerate(prompts)]
     lengths[0] = 50
     monkeypatch.setenv("FFMI_INC_AHEAD", "0")
-    plain = tokens(slots, prompts, lengths, [])[0]
+    (plain, _), taken = tokens(slots, prompts, lengths, [])
+    assert not taken
     assert [len(t) for t in plain] == lengths
     # tokens that end some requests early, at different steps
     eos = sorted({t[len(t) - len(t) // 3] for t in plain[::2]})
-    short = tokens(slots, prompts, lengths, eos)
+    short, _ = tokens(slots, prompts, lengths, eos)
     assert short[0] == short[1] and any(len(a) < len(b) for a, b in zip(short[0], plain))
     monkeypatch.delenv("FFMI_INC_AHEAD")
-    assert tokens(slots, prompts, lengths, []) == [plain, plain]
-    assert tokens(slots, prompts, lengths, eos) == short
+    # (three requests by one slot: none while others wait, and the last has two tokens to come)
+    assert tokens(slots, prompts, lengths, []) == ([plain, plain], (slots, requests) != (1, 3))
+    assert tokens(slots, prompts, lengths, eos)[0] == short
 
 
 def test_refuses_tokens_out_of_range_behind_steps_launched_ahead():
@@ -55,8 +63,8 @@ def test_no_step_for_nobody(requests, layers, monkeypatch):
     """A call that tokens end runs as many steps to their end as one by one: none for nobody."""
     prompts = [[(37 * i + 11 * r) % 480 + 5 for i in range(3 + r % 5)] for r in range(requests)]
     runs = []
-    for ahead in ("0", "1"):
-        monkeypatch.setenv("FFMI_INC_AHEAD", ahead)
+    for mode in ("0", "1"):
+        monkeypatch.setenv("FFMI_INC_AHEAD", mode)
         m = fa.Model(dict(CFG, num_layers=layers), "inc", max_requests=requests, max_tokens=64, max_seq_len=96,
                      weight_seed=9)
 
@@ -66,16 +74,53 @@ def test_no_step_for_nobody(requests, layers, monkeypatch):
         def call(eos):
             rm = fa.RequestManager(max_requests_per_batch=requests, max_tokens_per_batch=64, max_sequence_length=96,
                                    eos_token_ids=eos)
-            before = [count(F.COUNT_STEPS), count(F.COUNT_AHEAD)]
+            before = [count(F.COUNT_STEPS), ahead(m)]
             guids = [rm.register_new_request(p, max_length=60) for p in prompts]
             rm.serve_incr_decoding(m)
             return ([rm.get_generation_result(g).output_tokens for g in guids], count(F.COUNT_STEPS) - before[0],
-                    count(F.COUNT_AHEAD) - before[1])
+                    ahead(m) - before[1])
         plain = call([])
         gen = [t[-(60 - len(p) - 1):] for t, p in zip(plain[0], prompts)]
         eos = sorted({max(set(g), key=g.index) for g in gen})  # (the latest to come first)
         runs.append([plain, call(eos), call([499]), call(eos)])
         assert all(len(t) < 60 for t in runs[-1][1][0])
-        assert (plain[2] > 0) == (runs[-1][1][2] > 0) == (ahead == "1")
+        assert (plain[2] > 0) == (runs[-1][1][2] > 0) == (mode == "1")
     for one, two in zip(*runs):
         assert one[0] == two[0] and one[1] == two[1]
+
+
+def test_row_without_a_pick(tmp_path, monkeypatch):
+    """A row of NaN has no pick: the step after it is refused, launched ahead or not."""
+    rng, H = np.random.default_rng(3), CFG["hidden"]
+    st = {}
+    for n, rows, cols in (("model.embed_tokens", 500, H), ("lm_head", 500, H)):
+        st[n + ".weight"] = rng.uniform(-0.5, 0.5, (rows, cols)).astype(np.float32)
+    for l in range(CFG["num_layers"]):
+        p = f"model.layers.{l}."
+        for n in ("input_layernorm", "post_attention_layernorm"):
+            st[p + n + ".weight"] = np.ones(H, np.float32)
+        for n, rows, cols in [("self_attn.%s_proj" % x, H, H) for x in "qkvo"] + \
+                [("mlp.gate_proj", 256, H), ("mlp.up_proj", 256, H), ("mlp.down_proj", H, 256)]:
+            st[p + n + ".weight"] = rng.uniform(-0.1, 0.1, (rows, cols)).astype(np.float32)
+    st["model.norm.weight"] = np.ones(H, np.float32)
+
+    def run(folder, eos):
+        m = fa.Model(CFG, "inc", max_requests=2, max_tokens=64, max_seq_len=96, weights_folder=str(folder))
+        rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=64, max_sequence_length=96,
+                               eos_token_ids=eos)
+        try:
+            return [r.output_tokens for r in fa.generate(rm, m, [[5, 6, 7], [300, 9]], max_length=40)], ahead(m)
+        except F.FFMIError:
+            return None, ahead(m)
+    fa.convert_hf_model(st, str(tmp_path / "a"))
+    plain, _ = run(tmp_path / "a", [])
+    gen = plain[0][-36:-8]  # (the latest to come first, with steps behind it)
+    late = max(set(gen) - set(plain[1]) - {5, 6, 7}, key=gen.index)
+    assert gen.index(late) > 3
+    st["model.embed_tokens.weight"][late] = np.nan
+    fa.convert_hf_model(st, str(tmp_path / "b"))
+    for eos in ([], [499]):
+        for mode in ("0", "1"):
+            monkeypatch.setenv("FFMI_INC_AHEAD", mode)
+            out, taken = run(tmp_path / "b", eos)
+            assert out is None and (taken > 0) == (mode == "1")

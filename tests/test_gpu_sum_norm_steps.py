@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import flexflow_amd as fa
+import flexflow_amd.ffmi as F
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +37,7 @@ def test_same_bits(monkeypatch, hidden, heads, ff, vocab):
             feed((0, 1), (1, 1))
             feed((0, 2), (1, 1))  # three rows: norm launches, whichever buffer the residual was in
         out.append(np.concatenate(parts))
+        assert (F.lib().ffmi_model_debug_count(m.handle, F.COUNT_MADE_NORMS) > 0) == (mode == "1")
         m.close()
     assert np.isfinite(out[0]).all() and np.ptp(out[0]) > 0
     assert np.array_equal(out[0], out[1])
