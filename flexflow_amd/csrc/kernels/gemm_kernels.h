@@ -1242,10 +1242,13 @@ __global__ __launch_bounds__(256, NTW <= 8 && MTW * NTW <= 24 ? 2 : 1) void gemm
 // from it (400 products of 200 .. 1024 rows: 0.2% slower to 0.3% faster a form).
 template <int MI, int NJ, int WR, int WC>
 static constexpr bool kExactCopies = WR * WC > 8 && (MI * WR + NJ * WC) % (WR * WC) != 0;
-// Two sets of row fragments.  One set / two, us at T = 1024, cold weights: 22016 x 4096 in 256 x 192
-// 176.8 / 171.7, 4096 x 11008 in two slices of 256 x 128 91.2 / 89.7 and of 128 x 256 95.8 / 90.6, 11264 x
-// 2048 in 256 x 192 51.0 / 49.2, 4096 x 11008 in 192 x 128 116.0 / 106.3; 12288 x 4096 at 280 rows
-// in 192 x 128 52.0 / 48.8.  Two rows a wave gain nothing (4096 x 4096 in 128 x 128 40.3 / 40.9) or
+// Two sets of row fragments.  One set / two, us, cold weights, both in turn three times.  192 x 128: 11264 x
+// 2048 gate and up at 280 rows 31.9 / 30.6, 6144 x 2048 at 700 34.6 / 33.0.  256 x 128: 4096 x 11008 at 1024
+// 110.5 / 109.3 (two slices), at 400 59.5 / 58.4 (four), 8192 x 2048 at 1024 44.3 / 43.2.  256 x 192: 22016 x 4096 at
+// 1024 183 / 180, at 512 93.2 / 92.2, 11264 x 2048 at 1024 57.1 / 55.5, 12288 x 4096 at 700 86.9 / 85.4.  192 x 256:
+// 22016 x 4096 at 280 81.7 / 81.0, 4096 x 11008 at 700 85 / 85.  256 x 256: 27648 x 5120 at 1024 264 / 263,
+// 5120 x 13824 at 1024 160 / 155 (three slices).  One block of rows: 32000 x 4096 at 256 rows 77 - 80 / 79 - 81, weights
+// streamed 82 - 91 / 72 - 76.  Two rows a wave gain nothing (4096 x 4096 in 128 x 128 40.3 / 40.9) or
 // lose (6144 x 2048 in 128 x 192 31.9 / 32.6), as twelve waves do (22016 x 4096 at 168 rows 52.5 / 53.6).
 template <int MI, int NJ, int WR, int WC>
 static constexpr bool kTwoX = MI >= 3 && NJ >= 4 && WR * WC <= 8;
