@@ -414,11 +414,12 @@ extern "C" __device__ unsigned __ockl_wfred_min_u32(unsigned);
 //    other than M all lie further below it (1.1 times that: the float error of exp and the
 //    division is under 2^-20) is picked without S: no exp terms, no hand-off between
 //    workgroups (G > 1: each sees the same row, the first stores).  V = 32000: 1 row
-//    7.7 -> 4.0 us, 8 rows 8.1 -> 4.1, 168 rows 12.0 -> 4.6.  Other rows, and rows with a NaN
-//    or without a finite M, take the whole path in as many workgroups as without PICK, but for
-//    a thread's eight registers (V <= 8192), where the hand-off does not pay: logits of 1e-3, 1 row
-//    of 32000 7.7 -> 9.2 us (in one workgroup 12.6), of 2048 5.4 -> 5.0 (in four 6.0); a third
-//    of 32000 logits equal, others near them 21.3 -> 23.0.
+//    7.7 -> 3.9 us, 8 rows 8.1 -> 4.1, 168 rows 12.0 -> 4.6.  Other rows, and rows with a NaN
+//    or without a finite M, take the whole path in as many workgroups as without PICK: logits
+//    of 1e-3, 8 rows 9.2 -> 10.7 us (one workgroup a row 13.9); a third of the logits equal,
+//    others near them 22.0 -> 23.6 (29.6).  But one row takes two at most (four and eight cost a
+//    decoding step of 768 channels 0.5 us where there is no tie; 7.7 -> 11.4 us where there may be), and
+//    a thread's eight registers (V <= 8192) one, as the hand-off does not pay (2048 logits 5.4 -> 5.0, in four 6.0).
 //  * Picks without probabilities are stored at system scope, whatever the form: the host may
 //    look for a decoding step's in pinned memory while the stream works on (launch_argmax).
 __device__ __forceinline__ void store_pick(int32_t *at, int id) {
@@ -845,7 +846,7 @@ hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *i
   }();
   const int nv = (V / 8 + tpb - 1) / tpb;
   const bool pick = k == 1 && !probs && tpb == 1024;  // (ids alone, one a row)
-  if (pick && nv <= 1) G = 1;  // (see the kernel)
+  if (pick) G = nv <= 1 ? 1 : T == 1 ? std::min(G, 2) : G;  // (see the kernel)
   // (NV = 8 at 1024 threads would spill: larger vocabularies take the loop kernel)
   if (V % 8 == 0 && ((uintptr_t)logits & 15) == 0 && nv * tpb <= 4096) {
 #define FFMI_SMR(TPB, NV)                                                                  \
