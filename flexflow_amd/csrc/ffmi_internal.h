@@ -365,7 +365,8 @@ hipError_t launch_silu_mul(const uint16_t *a, const uint16_t *b, uint16_t *out,
                            size_t n, hipStream_t s);
 // softmax + argmax / top-k; with a zeroed workspace of argmax_workspace_bytes(T)
 // (left zeroed) rows of a small T are split over several workgroups
-// (probs null: the ids are stored at system scope)
+// (argmax_picks_seen: with k = 1 and no probs the ids are stored at system scope)
+bool argmax_picks_seen(int V);
 hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *ids,
                          float *probs, hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0,
                          int32_t *ids2 = nullptr);  // (ids2: a second copy of the ids)

@@ -420,8 +420,8 @@ extern "C" __device__ unsigned __ockl_wfred_min_u32(unsigned);
 //    others near them 22.0 -> 23.6 (29.6).  But one row takes two at most (four and eight cost a
 //    decoding step of 768 channels 0.5 us where there is no tie; 7.7 -> 11.4 us where there may be), and
 //    a thread's eight registers (V <= 8192) one, as the hand-off does not pay (2048 logits 5.4 -> 5.0, in four 6.0).
-//  * Picks without probabilities are stored at system scope, whatever the form: the host may
-//    look for a decoding step's in pinned memory while the stream works on (launch_argmax).
+//  * PICK stores at system scope: the host may look for a decoding step's picks in pinned
+//    memory while the stream works on (argmax_picks_seen).
 __device__ __forceinline__ void store_pick(int32_t *at, int id) {
   __hip_atomic_store(at, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -613,8 +613,8 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
   };
   auto emit = [&](int rd, unsigned long long b) {
     const int id = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
-    if (probs) ids[(size_t)row * k + rd] = id;
-    else store_pick(ids + (size_t)row * k + rd, id);
+    if (PICK) store_pick(ids + (size_t)row * k + rd, id);
+    else ids[(size_t)row * k + rd] = id;
     if (ids2) ids2[(size_t)row * k + rd] = (int)(0xffffffffu - (unsigned)(b & 0xffffffffu));
     if (probs) probs[(size_t)row * k + rd] = h2f_((uint16_t)((b >> 32) - 1u));
   };
@@ -819,6 +819,18 @@ size_t argmax_workspace_bytes(int T) {
   return T <= 0 ? 0 : kSplitPartOff + (size_t)std::min(T, kSplitRows) * 16 * 8;
 }
 
+// workgroup width (A/B: FFMI_TOPK_TPB = 256 / 512 / 1024)
+static int topk_tpb() {
+  static const int tpb = [] {
+    const char *e = getenv("FFMI_TOPK_TPB");
+    const int v = e ? atoi(e) : 1024;
+    return v == 256 || v == 512 ? v : 1024;
+  }();
+  return tpb;
+}
+// (PICK and the loop kernel)
+bool argmax_picks_seen(int V) { return topk_tpb() == 1024 || V % 8 || V > 32768; }
+
 hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *ids,
                          float *probs, hipStream_t s, void *ws, size_t ws_bytes, int32_t *ids2) {
   if (T <= 0) return hipSuccess;
@@ -838,12 +850,7 @@ hipError_t launch_argmax(const uint16_t *logits, int T, int V, int k, int32_t *i
   if (!ws || ws_bytes < argmax_workspace_bytes(T) || T > kSplitRows) G = 1;
   unsigned *cnt = reinterpret_cast<unsigned *>(ws);
   double *part = ws ? reinterpret_cast<double *>(static_cast<char *>(ws) + kSplitPartOff) : nullptr;
-  // workgroup width (A/B: FFMI_TOPK_TPB = 256 / 512 / 1024)
-  static const int tpb = [] {
-    const char *e = getenv("FFMI_TOPK_TPB");
-    const int v = e ? atoi(e) : 1024;
-    return v == 256 || v == 512 ? v : 1024;
-  }();
+  const int tpb = topk_tpb();
   const int nv = (V / 8 + tpb - 1) / tpb;
   const bool pick = k == 1 && !probs && tpb == 1024;  // (ids alone, one a row)
   if (pick) G = nv <= 1 ? 1 : T == 1 ? std::min(G, 2) : G;  // (see the kernel)

@@ -1432,7 +1432,8 @@ struct LlamaGPU : public ffmi_model {
   // threads yield or sleep: picks are waited for by looking.
   bool can_launch_ahead(int num_tokens) const override {
     if (!ids_dev || mode != FFMI_MODEL_INC || num_tokens < 1 || num_tokens > std::min(64, (int)o.max_tokens) || dbg ||
-        result_copy || !use_graphs || step_timing || prof_level != 0 || prof_on(0, num_tokens))
+        result_copy || !use_graphs || step_timing || prof_level != 0 || prof_on(0, num_tokens) ||
+        !ffmi::argmax_picks_seen(c.vocab_size))
       return false;
     unsigned flags = 0;
     if (hipGetDeviceFlags(&flags) != hipSuccess) return false;

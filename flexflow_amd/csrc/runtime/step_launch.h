@@ -19,16 +19,18 @@ namespace ffmi {
 // Pekarax, 3 (17) 6120 / 5950, LLaMA, 43 tokens a step (16) 13380 / 11780, SpecInfer (16) 5830 / 5860; Fesenex, 47
 // tokens (13) 8810 / 8630, Pekarax, 1 request (11) 4860 / 4930, Vapipel, 2 (9) 6720 / 7180; of 1024
 // channels (2 - 4) 4370 / 5210 and 4440 / 5580.  On other machines single requests of 20 - 22 MB were 1.7 % slower to 0.8 %
-// faster one by one.  So from 16 MB on, where one by one is within 1 % of a graph or faster, and
-// nearly twice what the clear losses read.  (Most of what LLaMA's 12 and 14 requests gain is that
-// the caller's fresh pages for their logits cost more beside a graph: with kept ones 6650 / 6510 and 11510 / 11320.)
+// faster one by one.  So from 14 MB on, half as much again as the clear losses read: there
+// one by one is within 1 % of a graph or faster, and a new shape's first step needs no graph made
+// (SpecInfer of 2048 channels, 3 tokens 3080 / 2750).  (Most of what LLaMA's 12 and 14 requests gain is
+// that the caller's fresh pages for their logits cost more beside a graph: with kept ones 6650 / 6510 and
+// 11510 / 11320.)
 // Not where threads are to yield or sleep (FFMI_SYNC): a graph costs the host less.
 // FFMI_STEP_GRAPHS: 1 always graphs, 0 never (A/B, tests; read per call)
 // (bytes: what the step reads, 0: a graph whatever it is; launches: its kernels)
 inline bool launch_one_by_one(double bytes, int launches) {
   if (bytes <= 0) return false;
   if (const char *e = getenv("FFMI_STEP_GRAPHS")) return !atoi(e);
-  if (bytes < 16e6 * launches) return false;
+  if (bytes < 14e6 * launches) return false;
   unsigned flags = 0;
   if (hipGetDeviceFlags(&flags) != hipSuccess) return false;
   flags &= hipDeviceScheduleMask;

@@ -54,7 +54,7 @@ def test_same_tokens(monkeypatch):
 
 
 def test_form_by_counted_launches():
-    """16 MB a launch, of as many launches as the step has: 24 with one token (norms in the products around
+    """14 MB a launch, of as many launches as the step has: 24 with one token (norms in the products around
     them: 16.4 MB), 31 with 20 (12.7)."""
     cfg = dict(num_layers=4, vocab_size=8000, num_heads=16, num_kv_heads=16, hidden=2048, intermediate=4608,
                rms_eps=1e-6, rope_theta=10000.0)
