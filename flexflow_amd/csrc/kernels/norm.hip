@@ -497,10 +497,12 @@ __global__ __launch_bounds__(TPB) void softmax_topk_reg_kernel(
         else odd |= d <= tie;
       }
     odd |= !(fabsf(M) < INFINITY);
-    if (__any(at != 0xffffffffu)) {  // (one a wave: in a row of equal logits every lane has one)
+    const unsigned long long has = __ballot(at != 0xffffffffu);
+    if (has & (has - 1)) {  // (one a wave: in a row of equal logits every lane has one)
       at = __ockl_wfred_min_u32(at);
-      if (lane == 0) atomicMin(&first_max, at);
+      if (lane != 0) at = 0xffffffffu;
     }
+    if (at != 0xffffffffu) atomicMin(&first_max, at);
     if (__any(odd) && lane == 0) unclear = 1;
     __syncthreads();
     if (!unclear) {
