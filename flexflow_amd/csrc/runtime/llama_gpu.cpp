@@ -1135,6 +1135,7 @@ struct LlamaGPU : public ffmi_model {
   long debug_graphs() const override { return ffmi::count_step_graphs(graphs) + (long)group_graphs.size(); }
   long debug_count(int what) const override { return what >= 0 && what < 3 ? counts[what] : -1; }
   void clear_graphs() {
+    if (stream) (void)hipStreamSynchronize(stream);  // (chained steps ahead may run from some)
     ffmi::clear_step_graphs(&graphs);
     for (auto &kv : group_graphs) (void)hipGraphExecDestroy(kv.second);
     group_graphs.clear();
