@@ -57,8 +57,8 @@ def test_refuses_tokens_out_of_range_behind_steps_launched_ahead():
             rm.replay_step(m, [(1, [9, bad], [1])])
 
 
-# (5 layers: many short launches, whose last part is a graph)
-@pytest.mark.parametrize("requests,layers", [(1, 2), (4, 2), (1, 5), (4, 5)])
+# (5 layers: many short launches, whose last part is a graph; 20 requests: norms of their own)
+@pytest.mark.parametrize("requests,layers", [(1, 2), (4, 2), (1, 5), (4, 5), (20, 5), (20, 3)])
 def test_no_step_for_nobody(requests, layers, monkeypatch):
     """A call that tokens end runs as many steps to their end as one by one: none for nobody."""
     prompts = [[(37 * i + 11 * r) % 480 + 5 for i in range(3 + r % 5)] for r in range(requests)]
