@@ -24,6 +24,9 @@ namespace ffmi {
 // (SpecInfer of 2048 channels, 3 tokens 3080 / 2750).  (Most of what LLaMA's 12 and 14 requests gain is
 // that the caller's fresh pages for their logits cost more beside a graph: with kept ones 6650 / 6510 and
 // 11510 / 11320.)
+// A busy host pays for it only where it has no core left: LLaMA of 2048 channels, 1 request (22) 6421 / 6407,
+// beside 8 busy threads of 16 cores 6446 / 6406, beside 15 6433 / 6546; Pekarax, 3 requests 4705 / 4584, 4759 / 4617 and
+// 4946 / 4873.
 // Not where threads are to yield or sleep (FFMI_SYNC): a graph costs the host less.
 // FFMI_STEP_GRAPHS: 1 always graphs, 0 never (A/B, tests; read per call)
 // (bytes: what the step reads, 0: a graph whatever it is; launches: its kernels)
