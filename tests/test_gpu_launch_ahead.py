@@ -124,3 +124,32 @@ def test_row_without_a_pick(tmp_path, monkeypatch):
             monkeypatch.setenv("FFMI_INC_AHEAD", mode)
             out, taken = run(tmp_path / "b", eos)
             assert out is None and (taken > 0) == (mode == "1")
+
+
+def test_graphs_given_back_between_steps_launched_ahead():
+    """A model keeps 512 step graphs; the shape after those gives them back while steps are on the stream."""
+    prompts = [[5, 6, 7], [300, 9]]
+
+    def graphs(m):
+        return F.lib().ffmi_model_debug_graphs(m.handle)
+
+    def generate(m):
+        rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=64, max_sequence_length=96)
+        before = ahead(m)
+        out = [r.output_tokens for r in fa.generate(rm, m, prompts, max_length=80)]
+        assert ahead(m) > before
+        return out
+    m = fa.Model(CFG, "inc", max_requests=2, max_tokens=64, max_seq_len=96, weight_seed=9)
+    plain = generate(m)
+    m.close()
+    m = fa.Model(CFG, "inc", max_requests=2, max_tokens=64, max_seq_len=96, weight_seed=9)
+    rm = fa.RequestManager(max_requests_per_batch=2, max_tokens_per_batch=64, max_sequence_length=96)
+    for a in range(1, 64):
+        for b in range(1, min(a, 64 - a) + 1):
+            if graphs(m) < 511:  # (the prompts' step is the last before they are given back)
+                rm.replay_step(m, [(1, range(a), range(a)), (2, range(b), range(b))])
+                rm.replay_end(m, 1), rm.replay_end(m, 2)
+    assert graphs(m) == 511
+    assert generate(m) == plain
+    assert 0 < graphs(m) < 20
+    assert generate(m) == plain
